@@ -262,12 +262,12 @@ int qca_qr_site(int side, const void* A, int chil, int chir, int target, void* A
 int qca_exact_apply_h(int precision, const void* psi, void* out, int ncells, int distance, int lo,
                       int hi, void* stream);
 
-/* psi <- exp(-i (pi/2) dt H) psi on the 2^N basis (complex128, device) by
- * Krylov with the closed-form H.  Replaces reference exact.py:15-28.  The
- * step is split into 2^l equal substeps when the Krylov basis (at most 64
- * vectors, at least 24, within 16 GiB) cannot hold the whole step: a substep
- * that reaches the basis limit is discarded and retried at half the length.
- * *iters receives the matvec count summed over the substeps. */
+/* psi <- exp(-i (pi/2) dt H) psi on the 2^N basis (complex128, device) by a
+ * Chebyshev series with the closed-form H (|H| <= ncells), cut where its tail
+ * falls below tol * |psi|.  Replaces reference exact.py:15-28.  A step with
+ * (pi/2) |dt| ncells > 512 is cut into equal substeps.  Uses three vectors of
+ * workspace.  *iters receives the number of H applications.  Amplitudes that
+ * are not finite are an error (-4), and psi is left as it was. */
 int qca_exact_expm(void* psi, int ncells, int distance, int lo, int hi, double dt, double tol,
                    int* iters, void* stream);
 

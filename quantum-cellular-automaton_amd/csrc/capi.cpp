@@ -111,13 +111,13 @@ qca::ContractWs<T> contract_ws(long tsize, long outsize) {
 
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
-qca::LanczosWork lanczos_ws(long n, qca::LanczosCtrl** ctrl_host, int max_m = qca::LZ_MAXK) {
+qca::LanczosWork lanczos_ws(long n, qca::LanczosCtrl** ctrl_host) {
   qca::LanczosWork lw;
   lw.max_n = n;
-  lw.max_m = max_m;
+  lw.max_m = qca::LZ_MAXK;
   lw.max_blocks = qca::lanczos_nblk(n);
   lw.ctrl = sbuf<qca::LanczosCtrl>("lz_ctrl", 1);
-  lw.V = sbuf<qca::c128>("lz_V", (long)max_m * n);
+  lw.V = sbuf<qca::c128>("lz_V", (long)lw.max_m * n);
   lw.w64 = sbuf<qca::c128>("lz_w", n);
   lw.part = sbuf<qca::c128>("lz_part", (long)lw.max_blocks * qca::LZ_MAXK);
   lw.part2 = sbuf<qca::c128>("lz_part2", (long)lw.max_blocks * qca::LZ_MAXK);
@@ -131,19 +131,12 @@ qca::LanczosWork lanczos_ws(long n, qca::LanczosCtrl** ctrl_host, int max_m = qc
   return lw;
 }
 
-struct KrylovOutcome {
-  int m = 0;           // Krylov dimension used
-  bool hit_limit = false;
-};
-
 // Runs the Krylov loop: mv(j, V_j) must enqueue w = H V_j and the iteration
 // tail.  Iterations j = 0 .. max_m-2 may run; the device closes the
-// exponential at the latest at dimension max_m-1 and then flags a limit hit
-// when its error estimate is still above the tolerance.  x is overwritten with
-// the result unless the limit was hit and keep_on_limit is false.
+// exponential at the latest at dimension max_m-1.  x is overwritten with the
+// result.  Returns the Krylov dimension used.
 template <typename MV>
-KrylovOutcome krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::LanczosCtrl* host,
-                          MV&& mv, hipStream_t s, bool keep_on_limit = true) {
+int krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::LanczosCtrl* host, MV&& mv, hipStream_t s) {
   qca::lanczos_begin(x, n, lw, s);
   int j = 0, chunk = 8;
   while (true) {
@@ -156,13 +149,9 @@ KrylovOutcome krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::Lancz
                        "Krylov exponential did not converge (non-finite input?)");
     chunk = 4;
   }
-  KrylovOutcome r;
-  r.m = host->m;
-  r.hit_limit = host->hit_limit != 0;
-  if (r.hit_limit && !keep_on_limit) return r;
   qca::lanczos_finish(n, x, lw, s);
   QCA_HIP(hipStreamSynchronize(s));
-  return r;
+  return host->m;
 }
 
 }  // namespace
@@ -599,7 +588,7 @@ int qca_krylov_expm(int precision, int kind, void* x, const void* L, const void*
                                   wp ? &wp->d64 : nullptr, Din, Dout, chil, chir, ws,
                                   qca::lanczos_done_flag(lw), s);
           qca::lanczos_iteration_tail<double>(y, n, j, tau, tl, lw, s);
-        }, s).m;
+        }, s);
       } else {
         auto ws = contract_ws<float>(tsize, n);
         qca::c64* x32 = sbuf<qca::c64>("kr_x32", n);
@@ -610,7 +599,7 @@ int qca_krylov_expm(int precision, int kind, void* x, const void* L, const void*
                                  wp ? &wp->d32 : nullptr, Din, Dout, chil, chir, ws,
                                  qca::lanczos_done_flag(lw), s);
           qca::lanczos_iteration_tail<float>(y, n, j, tau, tl, lw, s);
-        }, s).m;
+        }, s);
       }
       if (iters) *iters = m;
     }
@@ -724,47 +713,23 @@ int qca_exact_expm(void* psi, int ncells, int distance, int lo, int hi, double d
                    int* iters, void* stream) {
   return guarded([&] {
     QCA_CHECK(psi, "null vector");
-    QCA_CHECK(ncells >= 2 && ncells <= 28, "ncells out of range for the Krylov exponential (2..28)");
+    QCA_CHECK(ncells >= 2 && ncells <= 28, "ncells out of range for the state-vector exponential (2..28)");
     QCA_CHECK(distance >= 1, "distance must be positive");
     QCA_CHECK(std::isfinite(dt), "time step must be finite");
     hipStream_t s = as_stream(stream);
     const long n = 1L << ncells;
-    // Krylov basis capped at 16 GiB (at least 24 vectors)
-    const int max_m = (int)std::max<long>(24, std::min<long>(qca::LZ_MAXK, (16L << 30) / (16L * n)));
-    qca::LanczosCtrl* host = nullptr;
-    qca::LanczosWork lw = lanczos_ws(n, &host, max_m);
-    qca::c128* y = sbuf<qca::c128>("ex_y", n);
-    const double tl = tol > 0 ? tol : 1e-14;
-    // The time step is split into 2^level equal substeps.  A short basis
-    // starts from about one substep per 8 units of |tau| * N (each row of H
-    // has at most N unit entries, so ||H|| <= N); a substep whose exponential
-    // reaches the basis limit leaves psi untouched and is retried at half the
-    // length.  Progress is counted in units of dt / 2^level, so every substep
-    // is an exact binary fraction of dt.
-    const double tau_full = 1.5707963267948966 * dt;
-    int level = 0;
-    if (max_m < 48) {
-      const double est = std::fabs(tau_full) * ncells / 8.0;
-      while (level < 20 && (double)(1L << level) < est) ++level;
-    }
-    long done_units = 0;
-    int total = 0;
-    while (done_units < (1L << level)) {
-      const double tau = tau_full / (double)(1L << level);
-      const KrylovOutcome r = krylov_loop((qca::c128*)psi, n, lw, host, [&](int j, const qca::c128* vj) {
-        qca::launch_exact_apply<double>(vj, y, ncells, distance, lo, hi, s);
-        qca::lanczos_iteration_tail<double>(y, n, j, tau, tl, lw, s);
-      }, s, /*keep_on_limit=*/false);
-      total += r.m;
-      if (r.hit_limit) {
-        QCA_CHECK(level < 30, "Krylov exponential of the state vector did not converge");
-        ++level;
-        done_units *= 2;
-        continue;
-      }
-      ++done_units;
-    }
-    if (iters) *iters = total;
+    qca::c128* bufa = sbuf<qca::c128>("ex_a", n);
+    qca::c128* bufb = sbuf<qca::c128>("ex_b", n);
+    qca::c128* acc = sbuf<qca::c128>("ex_acc", n);
+    int* bad = sbuf<int>("ex_bad", 1);
+    const int m = qca::launch_exact_expm((qca::c128*)psi, ncells, distance, lo, hi, 1.5707963267948966 * dt,
+                                         tol > 0 ? tol : 1e-14, bufa, bufb, acc, bad, s);
+    int hbad = 0;
+    QCA_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+    QCA_HIP(hipStreamSynchronize(s));
+    if (hbad)
+      throw qca::Error(qca::QCA_ERR_NOT_CONVERGED_CODE, "exponential of a state vector with non-finite amplitudes");
+    if (iters) *iters = m;
   });
 }
 

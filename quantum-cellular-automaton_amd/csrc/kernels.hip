@@ -6,7 +6,6 @@
 //                 the tridiagonal exponential runs on one wave (Taylor with
 //                 scaling) so no host round trip is needed per iteration
 //  * measure   -- <n_i> and the single-site density matrix from the transfer
-//  * exact     -- closed-form 2^N rule-Hamiltonian application
 #include "grouped.hpp"
 #include "wave.hpp"
 
@@ -266,7 +265,6 @@ __global__ void qr_gather_right(const c128* __restrict__ Q, const c128* __restri
 
 // ------------------------------------------------------------------ lanczos
 constexpr int LZ_BLOCK = 256;
-constexpr int LZ_DIRECT_BLOCKS = 4096;   // in-kernel partial reductions up to this many blocks
 constexpr int LZ_EPT = 1;                     // vector elements per thread
 constexpr int LZ_ELEMS = LZ_BLOCK * LZ_EPT;   // elements per block in the partial reductions
 
@@ -388,15 +386,11 @@ __device__ __forceinline__ void lz_subtract_body(const LanczosCtrl* ctrl, const 
                                                  c128* __restrict__ wout, const c128* __restrict__ V,
                                                  long n, int j, const c128* __restrict__ part_in,
                                                  int nblk, c128* __restrict__ coef_out,
-                                                 c128* __restrict__ part_out, int pass, unsigned blk,
-                                                 const c128* __restrict__ coef_in = nullptr) {
+                                                 c128* __restrict__ part_out, int pass, unsigned blk) {
   const int done = ctrl->done;  // tested after the coefficient loads
   __shared__ double sh[16];
   __shared__ c128 cs[LZ_MAXK];
-  if (coef_in) {
-    // coefficients reduced beforehand by lz_reduce (long vectors)
-    if (threadIdx.x <= j) cs[threadIdx.x] = coef_in[threadIdx.x];
-  } else {
+  {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     for (int i = wv; i <= j; i += LZ_BLOCK / 64) {
       double ar = 0, ai = 0;
@@ -457,34 +451,8 @@ __global__ __launch_bounds__(LZ_BLOCK) void lz_subtract(const LanczosCtrl* ctrl,
                                                         const c128* __restrict__ V, long n, int j,
                                                         const c128* __restrict__ part_in, int nblk,
                                                         c128* __restrict__ coef_out,
-                                                        c128* __restrict__ part_out, int pass,
-                                                        const c128* __restrict__ coef_in) {
-  lz_subtract_body<TW>(ctrl, w, wout, V, n, j, part_in, nblk, coef_out, part_out, pass, blockIdx.x,
-                       coef_in);
-}
-
-// Two-level reduction for long vectors: out[i] = sum_b part[b][i] for the
-// coefficients i = blockIdx.x (a fixed order: lanes stride over the blocks,
-// then the waves are combined in order).  With norm != 0, only the squared
-// norm partials part[b][0].re are summed, into ctrl->wnorm2.
-__global__ __launch_bounds__(256) void lz_reduce(LanczosCtrl* ctrl, const c128* __restrict__ part, int nblk,
-                                                 c128* __restrict__ out, int norm) {
-  if (ctrl->done) return;
-  __shared__ double sh[16];
-  const int i = blockIdx.x;
-  double ar = 0, ai = 0;
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    const c128 v = part[(long)b * LZ_MAXK + i];
-    ar += v.re;
-    ai += v.im;
-  }
-  ar = block_sum(ar, sh);
-  if (norm) {
-    if (threadIdx.x == 0) ctrl->wnorm2 = ar;
-    return;
-  }
-  ai = block_sum(ai, sh);
-  if (threadIdx.x == 0) out[i] = c128{ar, ai};
+                                                        c128* __restrict__ part_out, int pass) {
+  lz_subtract_body<TW>(ctrl, w, wout, V, n, j, part_in, nblk, coef_out, part_out, pass, blockIdx.x);
 }
 
 // beta_j = |w| from the per-block partial norms (one wave, fixed order).
@@ -566,12 +534,11 @@ __device__ __forceinline__ void lz_step_scale_body(LanczosCtrl* ctrl, const c128
                                                    const c128* __restrict__ coef2, int j, double tau,
                                                    double tol, int max_m, const c128* __restrict__ w,
                                                    c128* __restrict__ vnext, c64* __restrict__ v32,
-                                                   long n, unsigned blk, unsigned ngrid,
-                                                   int beta_reduced = 0) {
+                                                   long n, unsigned blk, unsigned ngrid) {
   const int done = ctrl->done;  // tested after beta's loads
   __shared__ double sbeta;
   if (threadIdx.x < 64) {
-    const double b = beta_reduced ? sqrt(ctrl->wnorm2) : lz_beta(part_norm, nblk);
+    const double b = lz_beta(part_norm, nblk);
     if (threadIdx.x == 0) sbeta = b;
   }
   __syncthreads();
@@ -592,9 +559,9 @@ __global__ __launch_bounds__(256) void lz_step_scale(LanczosCtrl* ctrl,
                                                      double tau, double tol, int max_m,
                                                      const c128* __restrict__ w,
                                                      c128* __restrict__ vnext,
-                                                     c64* __restrict__ v32, long n, int beta_reduced) {
+                                                     c64* __restrict__ v32, long n) {
   lz_step_scale_body(ctrl, part_norm, nblk, coef1, coef2, j, tau, tol, max_m, w, vnext, v32, n,
-                     blockIdx.x, gridDim.x, beta_reduced);
+                     blockIdx.x, gridDim.x);
 }
 
 // y = beta0 * sum_{i<m} z_i V_i   (a zero input stays zero)
@@ -722,91 +689,6 @@ __global__ void observables_kernel(const c128* __restrict__ rho, int n, double* 
   out[i] = d;
   out[n + i] = rint(d);
   out[2 * n + i] = sse;
-}
-
-// ------------------------------------------------------------------ exact 2^N
-// (H psi)[x] = sum_i [popcount(x & nbr_i) in [lo, hi)] psi[x ^ bit_i]
-// A workgroup owns one tile of 2^EX_TILE_BITS consecutive basis states (the
-// whole vector when it is shorter), staged in LDS: partners across the low
-// bits come from the tile, only flips of the higher bits gather from memory.
-constexpr int EX_TILE_BITS = 10;
-constexpr int EX_THREADS = 256;
-
-template <typename T>
-__global__ __launch_bounds__(EX_THREADS) void exact_apply_kernel(const cplx<T>* __restrict__ psi,
-                                                                 cplx<T>* __restrict__ out,
-                                                                 int ncells, int distance, int lo,
-                                                                 int hi) {
-  __shared__ cplx<T> tile[1 << EX_TILE_BITS];
-  const int tbits = min(ncells, EX_TILE_BITS);
-  const long tsize = 1L << tbits;
-  const long base = (long)blockIdx.x << tbits;
-  for (long t = threadIdx.x; t < tsize; t += EX_THREADS) tile[t] = psi[base + t];
-  __syncthreads();
-  for (long t = threadIdx.x; t < tsize; t += EX_THREADS) {
-    const long x = base + t;
-    T ar = 0, ai = 0;
-    for (int i = 0; i < ncells; ++i) {
-      const int jlo = max(0, i - distance), jhi = min(ncells - 1, i + distance);
-      // neighbours j in [jlo, jhi], j != i; cell j is bit (N-1-j)
-      const int bhi = ncells - 1 - jlo, blo = ncells - 1 - jhi;
-      const unsigned long long span =
-          ((bhi - blo + 1) >= 64) ? ~0ULL : (((1ULL << (bhi - blo + 1)) - 1ULL) << blo);
-      const unsigned long long self = 1ULL << (ncells - 1 - i);
-      const int cnt = __popcll((unsigned long long)x & span & ~self);
-      if (cnt >= lo && cnt < hi) {
-        const cplx<T> v = ((long)self < tsize) ? tile[t ^ (long)self] : psi[x ^ (long)self];
-        ar += v.re;
-        ai += v.im;
-      }
-    }
-    out[x] = cplx<T>{ar, ai};
-  }
-}
-
-// Single-site reduced density matrices of a 2^N state, two-stage reduction.
-// rho_i[p][q] = sum_{x: x_i = p} psi_x conj(psi_{x with x_i = q}); site i is bit N-1-i.
-// Stage 1: block (bx, i) writes partial (rho00, rho11, Re rho01, Im rho01).
-__global__ void exact_rho_partials(const c128* __restrict__ psi, int ncells, double* __restrict__ part) {
-  __shared__ double sh[16];
-  const int i = blockIdx.y;
-  const long dim = 1L << ncells;
-  const long bit = 1L << (ncells - 1 - i);
-  double d0 = 0, d1 = 0, orr = 0, oi = 0;
-  for (long x = blockIdx.x * (long)blockDim.x + threadIdx.x; x < dim; x += (long)gridDim.x * blockDim.x) {
-    const c128 a = psi[x];
-    const double n2 = a.re * a.re + a.im * a.im;
-    if (x & bit) {
-      d1 += n2;
-    } else {
-      d0 += n2;
-      const c128 b = psi[x | bit];  // conj(b) * a summed into rho01 = sum a conj(b)
-      orr += a.re * b.re + a.im * b.im;
-      oi += a.im * b.re - a.re * b.im;
-    }
-  }
-  d0 = block_sum(d0, sh);
-  d1 = block_sum(d1, sh);
-  orr = block_sum(orr, sh);
-  oi = block_sum(oi, sh);
-  if (threadIdx.x == 0) {
-    double* p = part + ((long)i * gridDim.x + blockIdx.x) * 4;
-    p[0] = d0; p[1] = d1; p[2] = orr; p[3] = oi;
-  }
-}
-
-__global__ void exact_rho_finalize(const double* __restrict__ part, int nbx, int ncells, c128* __restrict__ rho) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ncells) return;
-  double d0 = 0, d1 = 0, orr = 0, oi = 0;
-  for (int b = 0; b < nbx; ++b) {
-    const double* p = part + ((long)i * nbx + b) * 4;
-    d0 += p[0]; d1 += p[1]; orr += p[2]; oi += p[3];
-  }
-  rho[4L * i + 0] = c128{d0, 0.0};
-  rho[4L * i + 1] = c128{orr, oi};
-  rho[4L * i + 2] = c128{orr, -oi};
-  rho[4L * i + 3] = c128{d1, 0.0};
 }
 
 int grid_for(long n, int block = 256, int maxb = 8192) {
@@ -1041,28 +923,14 @@ void lanczos_iteration_tail(const cplx<TW>* w, long n, int j, double tau, double
   QCA_CHECK(j + 1 < lw.max_m && lw.max_m <= LZ_MAXK, "Krylov dimension limit");
   const int nb = lanczos_nblk(n);
   const LanczosCtrl* cc = lw.ctrl;
-  // Up to LZ_DIRECT_BLOCKS blocks every block reduces the previous partials
-  // itself (no extra launch); beyond that (state vectors of the exact path)
-  // that would be quadratic in the block count, so one launch per reduction
-  // sums them first.
-  const bool two_level = nb > LZ_DIRECT_BLOCKS;
   hipLaunchKernelGGL(lz_project<TW>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, w, lw.V, n, j, lw.part);
-  if (two_level)
-    hipLaunchKernelGGL(lz_reduce, dim3(j + 1), dim3(256), 0, s, lw.ctrl, (const c128*)lw.part, nb, lw.coef1, 0);
   hipLaunchKernelGGL(lz_subtract<TW>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, w, lw.w64, lw.V, n, j,
-                     (const c128*)lw.part, nb, lw.coef1, lw.part2, 1,
-                     two_level ? (const c128*)lw.coef1 : nullptr);
-  if (two_level)
-    hipLaunchKernelGGL(lz_reduce, dim3(j + 1), dim3(256), 0, s, lw.ctrl, (const c128*)lw.part2, nb, lw.coef2, 0);
+                     (const c128*)lw.part, nb, lw.coef1, lw.part2, 1);
   hipLaunchKernelGGL(lz_subtract<double>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, lw.w64, lw.w64, lw.V,
-                     n, j, (const c128*)lw.part2, nb, lw.coef2, lw.part, 2,
-                     two_level ? (const c128*)lw.coef2 : nullptr);
-  if (two_level)
-    hipLaunchKernelGGL(lz_reduce, dim3(1), dim3(256), 0, s, lw.ctrl, (const c128*)lw.part, nb, lw.coef2, 1);
+                     n, j, (const c128*)lw.part2, nb, lw.coef2, lw.part, 2);
   hipLaunchKernelGGL(lz_step_scale, dim3(grid_for(n)), dim3(256), 0, s, lw.ctrl,
                      (const c128*)lw.part, nb, (const c128*)lw.coef1, (const c128*)lw.coef2, j, tau,
-                     tol, lw.max_m, (const c128*)lw.w64, lw.V + (long)(j + 1) * n, v32, n,
-                     two_level ? 1 : 0);
+                     tol, lw.max_m, (const c128*)lw.w64, lw.V + (long)(j + 1) * n, v32, n);
   QCA_HIP(hipGetLastError());
 }
 template void lanczos_iteration_tail<double>(const c128*, long, int, double, double, LanczosWork&,
@@ -1085,30 +953,5 @@ void launch_rho(const c128* A, const c128* T, long nxb, c128* rho, hipStream_t s
   hipLaunchKernelGGL(rho_kernel, dim3(1), dim3(256), 0, s, A, T, nxb, rho);
   QCA_HIP(hipGetLastError());
 }
-
-template <typename T>
-void launch_exact_apply(const cplx<T>* psi, cplx<T>* out, int ncells, int distance, int lo, int hi,
-                        hipStream_t s) {
-  QCA_CHECK(ncells >= 1 && ncells <= 34, "ncells out of range for the state vector");
-  const long tiles = 1L << std::max(0, ncells - EX_TILE_BITS);
-  QCA_CHECK(tiles <= 0x7fffffffL, "too many tiles for one launch");
-  hipLaunchKernelGGL(exact_apply_kernel<T>, dim3((unsigned)tiles), dim3(EX_THREADS), 0, s, psi, out,
-                     ncells, distance, lo, hi);
-  QCA_HIP(hipGetLastError());
-}
-template void launch_exact_apply<double>(const c128*, c128*, int, int, int, int, hipStream_t);
-
-int exact_rho_blocks(int ncells) {
-  const long dim = 1L << ncells;
-  return (int)std::max<long>(1, std::min<long>((dim + 255) / 256, 512));
-}
-
-void launch_exact_rho(const c128* psi, int ncells, double* part, c128* rho, hipStream_t s) {
-  const int nbx = exact_rho_blocks(ncells);
-  hipLaunchKernelGGL(exact_rho_partials, dim3(nbx, ncells), dim3(256), 0, s, psi, ncells, part);
-  hipLaunchKernelGGL(exact_rho_finalize, dim3((ncells + 63) / 64), dim3(64), 0, s, part, nbx, ncells, rho);
-  QCA_HIP(hipGetLastError());
-}
-template void launch_exact_apply<float>(const c64*, c64*, int, int, int, int, hipStream_t);
 
 }  // namespace qca

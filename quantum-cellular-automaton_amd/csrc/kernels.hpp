@@ -22,7 +22,6 @@ struct LanczosCtrl {
   double alpha[LZ_MAXK];
   double beta[LZ_MAXK];
   c128 z[LZ_MAXK];
-  double wnorm2;      // |w|^2 of the iteration (two-level reduction of long vectors)
 };
 
 // Workspace of one Lanczos exponential (vectors of length <= max_n).
@@ -155,6 +154,13 @@ void launch_exact_rho(const c128* psi, int ncells, double* part, c128* rho, hipS
 template <typename T>
 void launch_exact_apply(const cplx<T>* psi, cplx<T>* out, int ncells, int distance, int lo, int hi,
                         hipStream_t s);
+// psi <- exp(-i tau H) psi by Chebyshev series of at most CHEB_MAX_Z in tau*N
+// each (a longer step is cut into equal parts), the tail of each below tol;
+// returns the number of H applications.  bufa, bufb, acc: 2^ncells elements
+// each; *bad is set, and psi left as it was, when psi is not finite.
+constexpr double CHEB_MAX_Z = 512;
+int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, double tau, double tol, c128* bufa,
+                      c128* bufb, c128* acc, int* bad, hipStream_t s);
 
 // ---------------------------------------------------------------- SVD / QR
 struct SvdResult {

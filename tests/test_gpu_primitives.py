@@ -267,3 +267,51 @@ def test_exact_expm_and_rho(gpu):
     qn.call("qca_exact_rho", qn.ptr(psi), n, rho.ctypes.data, None)
     assert np.abs(rho[:, 1, 1].real - ex.populations()).max() < 1e-13
     assert np.abs(np.trace(rho, axis1=1, axis2=2) - 1).max() < 1e-12
+
+
+@pytest.mark.parametrize("n,d,iv", [(1, 1, range(0, 1)), (2, 1, range(1, 2)), (7, 3, range(2, 5)),
+                                    (8, 2, range(0, 3)), (9, 9, range(3, 40)), (11, 5, range(1, 7)),
+                                    (18, 2, range(2, 5)), (19, 4, range(3, 6)), (20, 1, range(-1, 2))])
+def test_exact_apply_tiles(gpu, n, d, iv):
+    """Tile edges of the state-vector Hamiltonian (256- and 1024-state tiles,
+    shorter vectors, neighbourhoods reaching above the tile or beyond the
+    chain).  At most n terms per amplitude: n roundings."""
+    import torch
+    psi = crand(np.random.default_rng(n), 1 << n)
+    iv_np = range(max(iv.start, 0), iv.stop)
+    ref = AU.apply_h(psi, n, d, iv_np)
+    pd = dev(torch, psi, np.complex128)
+    out = torch.zeros_like(pd)
+    qn.call("qca_exact_apply_h", 0, qn.ptr(pd), qn.ptr(out), n, d, iv.start, iv.stop, None)
+    assert np.abs(out.cpu().numpy() - ref).max() <= n * np.finfo(float).eps * max(np.abs(ref).max(), 1)
+
+
+@pytest.mark.parametrize("n,d,dt,tol", [(2, 1, 0.3, 1e-12), (9, 3, -0.4, 1e-12), (10, 2, 0.0, 1e-14),
+                                        # 628 units of tau * N: two substeps
+                                        (8, 1, 50.0, 1e-10)])
+def test_exact_expm_series(gpu, n, d, dt, tol):
+    """The Chebyshev evolution against the dense propagator: backward steps, no
+    step, and one longer than a single series; rounding of ~1000 terms and the
+    dense phases (eps * tau * N) stay below 1e-10."""
+    import torch
+    from oracle import exact as OE, mps as OM
+    As = OM.product_state([0.1 + 0.08 * i for i in range(n)])
+    ex = OE.ExactOracle(As, n, d, range(1, 3), dt)
+    psi = dev(torch, ex.psi, np.complex128)
+    it = ctypes.c_int(0)
+    qn.call("qca_exact_expm", qn.ptr(psi), n, d, 1, 3, dt, 0.0, ctypes.byref(it), None)
+    ex.do_time_step()
+    assert it.value >= 2
+    assert np.abs(psi.cpu().numpy() - ex.psi).max() < tol
+
+
+def test_exact_expm_refuses_non_finite(gpu):
+    """A state with a NaN is refused and left as it was."""
+    import torch
+    psi = torch.zeros(1 << 10, dtype=torch.complex128, device="cuda")
+    psi[3], psi[700] = 1.0, float("nan")
+    before = psi.cpu().numpy()
+    with pytest.raises(qn.QcaError) as e:
+        qn.call("qca_exact_expm", qn.ptr(psi), 10, 1, 1, 2, 0.2, 0.0, None, None)
+    assert e.value.code == -4
+    assert np.array_equal(psi.cpu().numpy(), before, equal_nan=True)
