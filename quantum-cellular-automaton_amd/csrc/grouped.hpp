@@ -154,31 +154,28 @@ struct GemmGroup {
 };
 
 // ------------------------------------------------------------------ blocked QR steps
-struct QrPanelArgs {
+struct QrStepArgs {   // launch p: reflector p-1 on the columns from 16 p on, then panel p
   c128* M;
-  int rows, j0, pb;
-  c128* tau;
-  c128* V;
-  c128* T;
-  c128* VT;   // V T of the panel, laid out like V
+  int rows, cols, p;
+  c128* T;            // 16 x 16 per panel
 };
-struct QrIdentArgs {
+struct QrFormArgs {   // Q from the first kk reflectors
+  const c128* M;
+  int rows, kk;
+  const c128* T;
   c128* Q;
-  int rows, cols;
+  int qcols;
 };
-constexpr int QR_MAX_PANELS = 32;                       // 512 / 16
-constexpr int QR_SLOT_FACTOR = 0;                       // 4 per panel
-constexpr int QR_SLOT_IDENTITY = 4 * QR_MAX_PANELS;
-constexpr int QR_SLOT_Q = QR_SLOT_IDENTITY + 1;         // 3 per panel, last panel first
+constexpr int QR_SLOT_Q = QR_MAX_ROWS / 16 + 1;   // after every panel's slot
 struct QrStep {
   int slot;
-  int kind;        // 0 panel factorisation, 1 GEMM, 2 identity start of Q
-  QrPanelArgs panel;
-  GemmJob<double> gemm;
-  QrIdentArgs ident;
+  int kind;           // 0 factorisation, 1 Q
+  int blocks;
+  size_t lds;
+  QrStepArgs step;
+  QrFormArgs form;
 };
-std::vector<QrStep> blocked_qr_steps(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols,
-                                     c128* ws, size_t ws_elems);
+std::vector<QrStep> blocked_qr_steps(c128* M, int rows, int cols, c128* Q, int qcols, c128* ws, size_t ws_elems);
 
 // ------------------------------------------------------------------ SVD
 // One launch_jacobi_svd call of one instance.
@@ -228,6 +225,10 @@ GRec<A> grec(const A& a, unsigned gx, unsigned gy = 1, unsigned gz = 1) {
   r.grid.z = gz;
   return r;
 }
+
+// One slot of the blocked QR of many matrices; rows, lds: the largest of the steps.
+void launch_qr_step_grouped(const KGroup<QrStepArgs>& g, int rows, size_t lds, hipStream_t s);
+void launch_form_q_grouped(const KGroup<QrFormArgs>& g, int rows, size_t lds, hipStream_t s);
 
 struct ConvArgs {          // complex128 -> complex64 copy
   const c128* in;

@@ -1,4 +1,4 @@
-// FP64 factorisations of the TDVP split (gfx950).
+// FP64 SVD of the TDVP split (gfx950).
 //
 // jacobi_svd: block one-sided (Hestenes) Jacobi on the columns of a
 // column-major matrix X, with the rotations of each block pair computed on its
@@ -27,11 +27,6 @@
 // columns of a matrix with more columns than rows would go on indefinitely.  jac_finalize sorts the singular values and evaluates
 // the truncation rank (first i with ||s[i:]|| < eps, capped; reference
 // algorithms/tdvp.py:289-292).
-//
-// householder_qr: zgeqr2 + zung2r semantics (reference tensor_networks/mps.py:86
-// calls numpy.linalg.qr -> LAPACK), including LAPACK's zlarfg sign convention
-// beta = -sign(Re alpha)*|x|, so R has a real diagonal and Q matches LAPACK's
-// complete-QR complement columns.
 #include "grouped.hpp"
 #include "wave.hpp"
 
@@ -660,309 +655,6 @@ __global__ __launch_bounds__(JAC_NT) void jac_small(c128* __restrict__ X, int ro
   jac_small_body(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol);
 }
 
-// ------------------------------------------------------------------ QR
-constexpr int QR_THREADS = 1024;
-constexpr int QR_WAVES = QR_THREADS / 64;
-
-__device__ double qr_block_sum(double v, double* sh) {
-  v = wsum(v);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  __syncthreads();
-  if (l == 0) sh[w] = v;
-  __syncthreads();
-  double r = (l < QR_WAVES) ? sh[l] : 0.0;
-  r = wsum(r);
-  __syncthreads();
-  return r;
-}
-
-// M (rows x cols, column-major) -> reflectors below the diagonal, R on and
-// above it (zgeqr2), then Q's first qcols columns (zung2r) into Q.
-__global__ __launch_bounds__(QR_THREADS) void householder_qr_kernel(c128* __restrict__ M, int rows,
-                                                                    int cols, c128* __restrict__ tau,
-                                                                    c128* __restrict__ Q, int qcols) {
-  __shared__ double sh[QR_WAVES];
-  __shared__ c128 s_tau;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int kmax = min(rows, cols);
-  for (int j = 0; j < kmax; ++j) {
-    c128* x = M + (long)j * rows;
-    double part = 0;
-    for (int r = j + 1 + tid; r < rows; r += QR_THREADS) part += x[r].re * x[r].re + x[r].im * x[r].im;
-    const double xnorm2 = qr_block_sum(part, sh);
-    const c128 alpha = x[j];
-    c128 tj{0.0, 0.0};
-    bool identity = (xnorm2 == 0.0 && alpha.im == 0.0);
-    double beta = 0.0;
-    c128 scale{0.0, 0.0};
-    if (!identity) {
-      const double nrm = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + xnorm2);
-      beta = (alpha.re >= 0.0) ? -nrm : nrm;   // -SIGN(dlapy3, alphr)
-      tj = c128{(beta - alpha.re) / beta, -alpha.im / beta};
-      // scale = 1 / (alpha - beta)
-      const double dr = alpha.re - beta, di = alpha.im;
-      const double den = dr * dr + di * di;
-      scale = c128{dr / den, -di / den};
-    }
-    __syncthreads();
-    if (!identity) {
-      for (int r = j + 1 + tid; r < rows; r += QR_THREADS) {
-        const c128 v = x[r];
-        x[r] = c128{v.re * scale.re - v.im * scale.im, v.re * scale.im + v.im * scale.re};
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      if (!identity) x[j] = c128{beta, 0.0};
-      tau[j] = tj;
-      s_tau = tj;
-    }
-    __syncthreads();
-    if (!identity) {
-      // C <- (I - conj(tau) v v^H) C on columns j+1..cols-1, v_j = 1
-      const c128 ct{s_tau.re, -s_tau.im};
-      for (int c = j + 1 + wave; c < cols; c += QR_WAVES) {
-        c128* y = M + (long)c * rows;
-        double wr = 0, wi = 0;  // w = v^H y
-        for (int r = j + lane; r < rows; r += 64) {
-          const c128 v = (r == j) ? c128{1.0, 0.0} : x[r];
-          wr += v.re * y[r].re + v.im * y[r].im;
-          wi += v.re * y[r].im - v.im * y[r].re;
-        }
-        wr = wsum(wr);
-        wi = wsum(wi);
-        // f = conj(tau) * w
-        const double fr = ct.re * wr - ct.im * wi, fi = ct.re * wi + ct.im * wr;
-        for (int r = j + lane; r < rows; r += 64) {
-          const c128 v = (r == j) ? c128{1.0, 0.0} : x[r];
-          y[r].re -= v.re * fr - v.im * fi;
-          y[r].im -= v.re * fi + v.im * fr;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  if (Q == nullptr || qcols == 0) return;
-  // Q = H_0 ... H_{kk-1} [e_0 .. e_{qcols-1}]; reflectors with index >= qcols
-  // leave those columns unchanged.
-  const int kk = min(kmax, qcols);
-  for (long e = tid; e < (long)rows * qcols; e += QR_THREADS) {
-    const int c = (int)(e / rows), r = (int)(e - (long)c * rows);
-    Q[e] = c128{(r == c) ? 1.0 : 0.0, 0.0};
-  }
-  __syncthreads();
-  for (int i = kk - 1; i >= 0; --i) {
-    const c128* v = M + (long)i * rows;
-    const c128 ti = tau[i];
-    for (int c = i + wave; c < qcols; c += QR_WAVES) {
-      c128* y = Q + (long)c * rows;
-      double wr = 0, wi = 0;
-      for (int r = i + lane; r < rows; r += 64) {
-        const c128 vv = (r == i) ? c128{1.0, 0.0} : v[r];
-        wr += vv.re * y[r].re + vv.im * y[r].im;
-        wi += vv.re * y[r].im - vv.im * y[r].re;
-      }
-      wr = wsum(wr);
-      wi = wsum(wi);
-      const double fr = ti.re * wr - ti.im * wi, fi = ti.re * wi + ti.im * wr;
-      for (int r = i + lane; r < rows; r += 64) {
-        const c128 vv = (r == i) ? c128{1.0, 0.0} : v[r];
-        y[r].re -= vv.re * fr - vv.im * fi;
-        y[r].im -= vv.re * fi + vv.im * fr;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------------------------- blocked QR
-// One panel of the blocked Householder QR (zgeqrf = zgeqr2 on panels of
-// QRB_PB columns + zlarft + zlarfb): columns [j0, j0+pb) of M (rows x cols,
-// column-major), rows [j0, rows), staged in LDS.  Per column: zlarfg with
-// LAPACK's beta = -sign(Re alpha)*|x|, then H^H = I - conj(tau) v v^H applied to
-// the panel's remaining columns.  Writes R (on/above the diagonal) and v
-// (below) back to M, tau, the unit-diagonal V of the panel into V (same
-// layout as M, zero above the diagonal), and T (pb x pb, column-major with
-// leading dimension QRB_PB, upper triangular) with H_j0 ... H_{j0+pb-1} =
-// I - V T V^H (zlarft, forward, columnwise).
-constexpr int QRB_PB = 16;
-constexpr int QRB_MAXROWS = 512;
-
-__device__ __forceinline__ void qr_panel_body(c128* __restrict__ M, int rows, int j0, int pb,
-                                              c128* __restrict__ tau, c128* __restrict__ V,
-                                              c128* __restrict__ T, c128* __restrict__ VT) {
-  __shared__ c128 P[QRB_PB][QRB_MAXROWS];   // panel, local row r = global row j0 + r
-  __shared__ c128 s_tau[QRB_PB];
-  __shared__ c128 s_vv[QRB_PB][QRB_PB];     // V^H V of the panel
-  __shared__ c128 s_T[QRB_PB][QRB_PB];      // s_T[i][k] = T(k, i)
-  __shared__ double s_xnorm2;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int nr = rows - j0;
-  {
-    // wave w stages column w, lane l rows l, l + 64, ...: all of a thread's
-    // loads are issued before its first LDS store.  Slots past the panel
-    // (columns >= pb, rows >= nr) load a clamped valid element and are never
-    // read, so neither loads nor stores branch.
-    static_assert(QR_WAVES == QRB_PB && QRB_MAXROWS % 64 == 0, "one wave per panel column");
-    constexpr int IT = QRB_MAXROWS / 64;
-    const int c = min(wave, pb - 1);
-    const c128* src = M + (long)(j0 + c) * rows + j0;
-    c128 v[IT];
-#pragma unroll
-    for (int i = 0; i < IT; ++i) v[i] = src[min(lane + 64 * i, nr - 1)];
-#pragma unroll
-    for (int i = 0; i < IT; ++i) P[wave][lane + 64 * i] = v[i];
-  }
-  __syncthreads();
-  for (int c = 0; c < pb; ++c) {
-    c128* x = P[c];
-    // |x[c+1:]|^2 by wave 0 (nr <= 512: at most 8 elements per lane)
-    if (wave == 0) {
-      double part = 0;
-      for (int r = c + 1 + lane; r < nr; r += 64) part += x[r].re * x[r].re + x[r].im * x[r].im;
-      part = wsum(part);
-      if (lane == 0) s_xnorm2 = part;
-    }
-    __syncthreads();
-    // zlarfg, evaluated redundantly by every thread from the shared norm
-    const double xnorm2 = s_xnorm2;
-    const c128 alpha = x[c];
-    const bool identity = (xnorm2 == 0.0 && alpha.im == 0.0);
-    c128 tj{0.0, 0.0};
-    if (!identity) {
-      const double nrm = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + xnorm2);
-      const double beta = (alpha.re >= 0.0) ? -nrm : nrm;
-      tj = c128{(beta - alpha.re) / beta, -alpha.im / beta};
-      const double dr = alpha.re - beta, di = alpha.im;
-      const double den = dr * dr + di * di;
-      const c128 scale{dr / den, -di / den};
-      for (int r = c + 1 + tid; r < nr; r += QR_THREADS) {
-        const c128 v = x[r];
-        x[r] = c128{v.re * scale.re - v.im * scale.im, v.re * scale.im + v.im * scale.re};
-      }
-      __syncthreads();  // uniform: identity is the same in every thread
-      if (tid == 0) x[c] = c128{beta, 0.0};
-    }
-    if (tid == 0) {
-      s_tau[c] = tj;
-      tau[j0 + c] = tj;
-    }
-    if (!identity) {
-      // C <- (I - conj(tau) v v^H) C on the panel's columns c+1.., v_c = 1
-      const c128 ct{tj.re, -tj.im};
-      for (int cc = c + 1 + wave; cc < pb; cc += QR_WAVES) {
-        c128* y = P[cc];
-        double wr = 0, wi = 0;
-        for (int r = c + lane; r < nr; r += 64) {
-          const c128 v = (r == c) ? c128{1.0, 0.0} : x[r];
-          wr += v.re * y[r].re + v.im * y[r].im;
-          wi += v.re * y[r].im - v.im * y[r].re;
-        }
-        wr = wsum(wr);
-        wi = wsum(wi);
-        const double fr = ct.re * wr - ct.im * wi, fi = ct.re * wi + ct.im * wr;
-        for (int r = c + lane; r < nr; r += 64) {
-          const c128 v = (r == c) ? c128{1.0, 0.0} : x[r];
-          y[r].re -= v.re * fr - v.im * fi;
-          y[r].im -= v.re * fi + v.im * fr;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // write back R / v, and the explicit unit-diagonal V of the panel
-  for (int e = tid; e < pb * rows; e += QR_THREADS) {
-    const int c = e / rows, g = e - c * rows;   // g: global row
-    const int r = g - j0;
-    const long idx = (long)(j0 + c) * rows + g;
-    if (r >= 0) M[idx] = P[c][r];
-    c128 v{0.0, 0.0};
-    if (r == c) v = c128{1.0, 0.0};
-    else if (r > c) v = P[c][r];
-    V[idx] = v;
-  }
-  // V^H V of the panel (k < i), one wave per entry
-  for (int e = wave; e < pb * pb; e += QR_WAVES) {
-    const int k = e % pb, i = e / pb;
-    if (k >= i) continue;
-    double wr = 0, wi = 0;
-    for (int r = i + lane; r < nr; r += 64) {   // V_k and V_i overlap on rows >= i
-      const c128 a = (r == k) ? c128{1.0, 0.0} : P[k][r];
-      const c128 b = (r == i) ? c128{1.0, 0.0} : P[i][r];
-      wr += a.re * b.re + a.im * b.im;
-      wi += a.re * b.im - a.im * b.re;
-    }
-    wr = wsum(wr);
-    wi = wsum(wi);
-    if (lane == 0) s_vv[k][i] = c128{wr, wi};
-  }
-  __syncthreads();
-  // T (zlarft forward columnwise): T(i,i) = tau_i,
-  // T(0:i, i) = -tau_i T(0:i, 0:i) (V(:, 0:i)^H v_i); one lane per row k of T,
-  // the columns in order (T(k, l) for l < i written by the same lane earlier)
-  if (tid < pb) {
-    const int k = tid;
-    for (int i = 0; i < pb; ++i) {
-      c128 out{0.0, 0.0};
-      const c128 ti = s_tau[i];
-      if (k < i) {
-        double ar = 0, ai = 0;
-        for (int l = k; l < i; ++l) {
-          const c128 t = s_T[l][k], w = s_vv[l][i];
-          ar += t.re * w.re - t.im * w.im;
-          ai += t.re * w.im + t.im * w.re;
-        }
-        out = c128{-(ti.re * ar - ti.im * ai), -(ti.re * ai + ti.im * ar)};
-      } else if (k == i) {
-        out = ti;
-      }
-      s_T[i][k] = out;
-    }
-  }
-  __syncthreads();
-  if (tid < pb * QRB_PB) {
-    const int i = tid / QRB_PB, k = tid - i * QRB_PB;
-    T[(long)i * QRB_PB + k] = k < pb ? s_T[i][k] : c128{0.0, 0.0};
-  }
-  // VT = V T on the panel's rows (both triangular: V(r, k) = 0 for r < k,
-  // T(k, c) = 0 for k > c), stored like V.  The trailing update uses
-  // A -= V ((V T)^H A) and the accumulation of Q uses Q -= (V T)(V^H Q), so
-  // neither needs a separate product with T.
-  for (int e = tid; e < nr * pb; e += QR_THREADS) {
-    const int c = e / nr, r = e - c * nr;
-    double ar = 0, ai = 0;
-    const int kmax = min(c, r);
-    for (int k = 0; k <= kmax; ++k) {
-      const c128 v = (r == k) ? c128{1.0, 0.0} : P[k][r];
-      const c128 t = s_T[c][k];
-      ar += v.re * t.re - v.im * t.im;
-      ai += v.re * t.im + v.im * t.re;
-    }
-    VT[(long)(j0 + c) * rows + j0 + r] = c128{ar, ai};
-  }
-}
-// One workgroup per CU (the panel fills LDS): a register budget for 4 waves per
-// SIMD lets the panel load keep all its loads in flight.
-__global__ __launch_bounds__(QR_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void qr_panel_kernel(c128* __restrict__ M, int rows, int j0,
-                                                              int pb, c128* __restrict__ tau,
-                                                              c128* __restrict__ V,
-                                                              c128* __restrict__ T,
-                                                              c128* __restrict__ VT) {
-  qr_panel_body(M, rows, j0, pb, tau, V, T, VT);
-}
-
-__device__ __forceinline__ void set_identity_body(c128* __restrict__ Q, int rows, int cols, unsigned blk,
-                                                  unsigned nblk) {
-  for (long e = blk * (long)blockDim.x + threadIdx.x; e < (long)rows * cols;
-       e += (long)nblk * blockDim.x) {
-    const int c = (int)(e / rows), r = (int)(e - (long)c * rows);
-    Q[e] = c128{r == c ? 1.0 : 0.0, 0.0};
-  }
-}
-__global__ void set_identity(c128* __restrict__ Q, int rows, int cols) {
-  set_identity_body(Q, rows, cols, blockIdx.x, gridDim.x);
-}
-
 // ---------------------------------------------------------- QR preconditioning
 // order[c]: columns of X (rows x cols) by descending norm (ties by index).
 __device__ __forceinline__ void col_norm_order_body(const c128* __restrict__ X, int rows, int cols,
@@ -1127,15 +819,6 @@ __global__ void permute_cols_grouped(const GRec<ColOrderArgs>* __restrict__ recs
   const GRec<ColOrderArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
   permute_cols_body(gbl(r.a.X), r.a.rows, r.a.cols, gbl(r.a.order), gbl(r.a.Xp), bx, r.grid.x);
 }
-__global__ __launch_bounds__(QR_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void qr_panel_grouped(const GRec<QrPanelArgs>* __restrict__ recs, int n) {
-  const QrPanelArgs a = recs[blockIdx.x].a;
-  qr_panel_body(gbl(a.M), a.rows, a.j0, a.pb, gbl(a.tau), gbl(a.V), gbl(a.T), gbl(a.VT));
-}
-__global__ void set_identity_grouped(const GRec<QrIdentArgs>* __restrict__ recs, int n) {
-  unsigned bx, by, bz;
-  const GRec<QrIdentArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
-  set_identity_body(gbl(r.a.Q), r.a.rows, r.a.cols, bx, r.grid.x);
-}
 __global__ void rh_from_qr_grouped(const GRec<RhArgs>* __restrict__ recs, int n) {
   unsigned bx, by, bz;
   const GRec<RhArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
@@ -1272,7 +955,6 @@ size_t jacobi_precond_elems(int max_rows, int max_cols) {
   return (size_t)max_rows * max_cols       // column-permuted copy, then R / reflectors
          + (size_t)max_rows * kq           // Q, then Q J
          + (size_t)max_cols * kq           // Y = R^H
-         + (size_t)kq + 64                 // tau
          + qr_workspace_elems(max_rows, max_cols, (int)kq);
 }
 
@@ -1296,14 +978,13 @@ void launch_jacobi_svd(c128* X, int rows, int cols, double* sigma, int* perm, Sv
     c128* Xp = w.pre;
     c128* Q = Xp + (long)rows * cols;
     c128* Y = Q + (long)rows * kq;
-    c128* tau = Y + (long)cols * kq;
-    c128* qws = tau + kq + 64;
+    c128* qws = Y + (long)cols * kq;
     const size_t qws_elems = w.pre_elems - (size_t)(qws - w.pre);
     int* order = perm;  // scratch until the finalize writes the permutation
     hipLaunchKernelGGL(col_norm_order, dim3(1), dim3(JAC_NT), 0, s, (const c128*)X, rows, cols, order);
     hipLaunchKernelGGL(permute_cols, dim3(256), dim3(256), 0, s, (const c128*)X, rows, cols,
                        (const int*)order, Xp);
-    launch_qr(Xp, rows, cols, tau, Q, kq, qws, qws_elems, s);
+    launch_blocked_qr(Xp, rows, cols, Q, kq, qws, qws_elems, s);
     hipLaunchKernelGGL(rh_from_qr, dim3(256), dim3(256), 0, s, (const c128*)Xp, rows, cols, kq, Y);
     JacobiCtrl* ctrl = gram_jacobi(Y, cols, kq, Q, rows, s, w);
     hipLaunchKernelGGL(jac_finalize, dim3(1), dim3(JAC_NT), 0, s, (const c128*)Y, cols, kq, sigma,
@@ -1316,122 +997,6 @@ void launch_jacobi_svd(c128* X, int rows, int cols, double* sigma, int* perm, Sv
   JacobiCtrl* ctrl = gram_jacobi(X, rows, cols, nullptr, 0, s, w);
   hipLaunchKernelGGL(jac_finalize, dim3(1), dim3(JAC_NT), 0, s, (const c128*)X, rows, cols, sigma,
                      perm, res, chi_max, eps, rank_cap, (const JacobiCtrl*)ctrl);
-  QCA_HIP(hipGetLastError());
-}
-
-size_t qr_workspace_elems(int max_rows, int max_cols, int max_qcols) {
-  const long w = std::max(max_cols, max_qcols);
-  const long panels = ceil_div(std::max(1, std::min(max_rows, max_cols)), QRB_PB);
-  return 2L * max_rows * max_cols                    // V, V T
-         + panels * QRB_PB * QRB_PB                  // T per panel
-         + QRB_PB * w                                // W
-         + 32L * QRB_PB * w + 4096;                  // GEMM split-K partials
-}
-
-// The blocked QR as a list of steps (panel factorisations, GEMMs, the
-// identity start of Q), each with a slot number that orders it among the steps
-// of any other matrix: the single-matrix launcher runs the steps in order, the
-// grouped one runs every slot for all matrices that have it.
-std::vector<QrStep> blocked_qr_steps(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols,
-                                     c128* ws, size_t ws_elems) {
-  QCA_CHECK(rows >= 1 && cols >= 1, "empty QR");
-  QCA_CHECK(rows <= QRB_MAXROWS, "blocked QR rows above 512");
-  const int kmax = std::min(rows, cols);
-  const long panels = ceil_div(kmax, QRB_PB);
-  const long wcols = std::max(cols, qcols);
-  c128* V = ws;
-  c128* VT = V + (long)rows * cols;
-  c128* T = VT + (long)rows * cols;
-  c128* W = T + panels * QRB_PB * QRB_PB;
-  c128* gws = W + QRB_PB * wcols;
-  const long used = gws - ws;
-  QCA_CHECK((long)ws_elems > used + 1024, "QR workspace too small");
-  const long gws_elems = (long)ws_elems - used;
-  std::vector<QrStep> out;
-  auto gemm_step = [&](int slot, const GemmDesc& d, const c128* A, const c128* B, c128* C) {
-    QrStep st{};
-    st.slot = slot;
-    st.kind = 1;
-    st.gemm = GemmJob<double>{d, A, B, C, gws, gws_elems};
-    out.push_back(st);
-  };
-  // GEMM descriptors on column-major operands: X(r, c) at X + r + c * ld
-  for (int p = 0; p < panels; ++p) {
-    const int j0 = p * QRB_PB, pb = std::min(QRB_PB, kmax - j0);
-    c128* Tp = T + (long)p * QRB_PB * QRB_PB;
-    QrStep st{};
-    st.slot = QR_SLOT_FACTOR + 4 * p;
-    st.kind = 0;
-    st.panel = QrPanelArgs{M, rows, j0, pb, tau, V, Tp, VT};
-    out.push_back(st);
-    const int nt = cols - (j0 + pb), nr = rows - j0;
-    if (nt <= 0) continue;
-    const c128* Vp = V + (long)j0 * rows + j0;
-    const c128* VTp = VT + (long)j0 * rows + j0;
-    c128* At = M + (long)(j0 + pb) * rows + j0;
-    // W = (V T)^H A_trail = T^H V^H A_trail  (pb x nt)
-    GemmDesc g{};
-    g.M = pb; g.N = nt; g.K = nr; g.K2 = nr; g.NB1 = g.NB2 = 1; g.alpha_re = 1.0;
-    g.a_m = rows; g.a_k2 = 1; g.conj_a = 1;
-    g.b_k2 = 1; g.b_n = rows;
-    g.c_m = 1; g.c_n = pb;
-    gemm_step(QR_SLOT_FACTOR + 4 * p + 1, g, VTp, At, W);
-    // A_trail -= V W
-    GemmDesc u{};
-    u.M = nr; u.N = nt; u.K = pb; u.K2 = pb; u.NB1 = u.NB2 = 1; u.alpha_re = -1.0; u.accumulate = 1;
-    u.a_m = 1; u.a_k2 = rows;
-    u.b_k2 = 1; u.b_n = pb;
-    u.c_m = 1; u.c_n = rows;
-    gemm_step(QR_SLOT_FACTOR + 4 * p + 3, u, Vp, W, At);
-  }
-  if (Q == nullptr || qcols == 0) return out;
-  // Q = H_0 ... H_{kk-1} [e_0 .. e_{qcols-1}], block reflectors applied from
-  // the last panel back: Q(j0:, j0:) <- (I - V T V^H) Q(j0:, j0:)  (zungqr)
-  {
-    QrStep st{};
-    st.slot = QR_SLOT_IDENTITY;
-    st.kind = 2;
-    st.ident = QrIdentArgs{Q, rows, qcols};
-    out.push_back(st);
-  }
-  const int kk = std::min(kmax, qcols);
-  for (int p = (int)ceil_div(kk, QRB_PB) - 1; p >= 0; --p) {
-    const int j0 = p * QRB_PB, pb = std::min(QRB_PB, kk - j0);
-    const int nr = rows - j0, nq = qcols - j0;
-    const c128* Vp = V + (long)j0 * rows + j0;
-    const c128* VTp = VT + (long)j0 * rows + j0;
-    c128* Qs = Q + (long)j0 * rows + j0;
-    const int base = QR_SLOT_Q + 3 * (QR_MAX_PANELS - 1 - p);
-    // W = V^H Q(j0:, j0:), then Q(j0:, j0:) -= (V T) W
-    GemmDesc g{};
-    g.M = pb; g.N = nq; g.K = nr; g.K2 = nr; g.NB1 = g.NB2 = 1; g.alpha_re = 1.0;
-    g.a_m = rows; g.a_k2 = 1; g.conj_a = 1;
-    g.b_k2 = 1; g.b_n = rows;
-    g.c_m = 1; g.c_n = pb;
-    gemm_step(base, g, Vp, Qs, W);
-    GemmDesc u{};
-    u.M = nr; u.N = nq; u.K = pb; u.K2 = pb; u.NB1 = u.NB2 = 1; u.alpha_re = -1.0; u.accumulate = 1;
-    u.a_m = 1; u.a_k2 = rows;
-    u.b_k2 = 1; u.b_n = pb;
-    u.c_m = 1; u.c_n = rows;
-    gemm_step(base + 2, u, VTp, W, Qs);
-  }
-  return out;
-}
-
-void launch_blocked_qr(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols, c128* ws,
-                       size_t ws_elems, hipStream_t s) {
-  for (const QrStep& st : blocked_qr_steps(M, rows, cols, tau, Q, qcols, ws, ws_elems)) {
-    if (st.kind == 0) {
-      const QrPanelArgs& a = st.panel;
-      hipLaunchKernelGGL(qr_panel_kernel, dim3(1), dim3(QR_THREADS), 0, s, a.M, a.rows, a.j0, a.pb, a.tau,
-                         a.V, a.T, a.VT);
-    } else if (st.kind == 1) {
-      gemm_c128(st.gemm.d, st.gemm.A, st.gemm.B, st.gemm.C, s, st.gemm.ws, st.gemm.ws_elems);
-    } else {
-      hipLaunchKernelGGL(set_identity, dim3(256), dim3(256), 0, s, st.ident.Q, st.ident.rows, st.ident.cols);
-    }
-  }
   QCA_HIP(hipGetLastError());
 }
 
@@ -1464,15 +1029,12 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
       c128* Xp = w.pre;
       c128* Q = Xp + (long)j.rows * j.cols;
       c128* Yp = Q + (long)j.rows * kq;
-      c128* tau = Yp + (long)j.cols * kq;
-      c128* qws = tau + kq + 64;
+      c128* qws = Yp + (long)j.cols * kq;
       const size_t qws_elems = w.pre_elems - (size_t)(qws - w.pre);
-      QCA_CHECK(std::min(j.rows, j.cols) > 2 * QRB_PB && qws_elems >= qr_workspace_elems(j.rows, j.cols, kq),
-                "grouped SVD preconditioning needs the blocked QR");
       const ColOrderArgs co{j.X, j.rows, j.cols, j.perm, Xp};
       order1.push_back(grec(co, 1));
       perm.push_back(grec(co, 256));
-      for (QrStep& st : blocked_qr_steps(Xp, j.rows, j.cols, tau, Q, kq, qws, qws_elems)) steps.push_back(st);
+      for (QrStep& st : blocked_qr_steps(Xp, j.rows, j.cols, Q, kq, qws, qws_elems)) steps.push_back(st);
       rh.push_back(grec(RhArgs{Xp, j.rows, j.cols, kq, Yp}, 256));
       Y = Yp;
       Z = Q;
@@ -1523,9 +1085,10 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   std::sort(steps.begin(), steps.end(), [](const QrStep& x, const QrStep& y) { return x.slot < y.slot; });
   struct Slot {
     int kind;
-    KGroup<QrPanelArgs> panel;
-    KGroup<QrIdentArgs> ident;
-    GemmGroup<double> gemm;
+    size_t lds;
+    int rows;
+    KGroup<QrStepArgs> step;
+    KGroup<QrFormArgs> form;
   };
   std::vector<Slot> slots;
   for (size_t i = 0; i < steps.size();) {
@@ -1533,19 +1096,16 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     while (e < steps.size() && steps[e].slot == steps[i].slot) ++e;
     Slot sl{};
     sl.kind = steps[i].kind;
-    if (sl.kind == 0) {
-      std::vector<GRec<QrPanelArgs>> v;
-      for (size_t k = i; k < e; ++k) v.push_back(grec(steps[k].panel, 1));
-      sl.panel.prepare(v, arena);
-    } else if (sl.kind == 1) {
-      std::vector<GemmJob<double>> v;
-      for (size_t k = i; k < e; ++k) v.push_back(steps[k].gemm);
-      sl.gemm.prepare(v, arena);
-    } else {
-      std::vector<GRec<QrIdentArgs>> v;
-      for (size_t k = i; k < e; ++k) v.push_back(grec(steps[k].ident, 256));
-      sl.ident.prepare(v, arena);
+    std::vector<GRec<QrStepArgs>> v;
+    std::vector<GRec<QrFormArgs>> f;
+    for (size_t k = i; k < e; ++k) {
+      sl.lds = std::max(sl.lds, steps[k].lds);
+      sl.rows = std::max(sl.rows, sl.kind == 0 ? steps[k].step.rows : steps[k].form.rows);
+      if (sl.kind == 0) v.push_back(grec(steps[k].step, steps[k].blocks));
+      else f.push_back(grec(steps[k].form, steps[k].blocks));
     }
+    sl.step.prepare(v, arena);
+    sl.form.prepare(f, arena);
     slots.push_back(sl);
     i = e;
   }
@@ -1560,14 +1120,8 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     hipLaunchKernelGGL(permute_cols_grouped, dim3(g_perm.l.blocks), dim3(256), 0, s, g_perm.l.recs, g_perm.l.n);
   }
   for (const Slot& sl : slots) {
-    if (sl.kind == 0)
-      hipLaunchKernelGGL(qr_panel_grouped, dim3(sl.panel.l.blocks), dim3(QR_THREADS), 0, s, sl.panel.l.recs,
-                         sl.panel.l.n);
-    else if (sl.kind == 1)
-      sl.gemm.launch(s);
-    else
-      hipLaunchKernelGGL(set_identity_grouped, dim3(sl.ident.l.blocks), dim3(256), 0, s, sl.ident.l.recs,
-                         sl.ident.l.n);
+    launch_qr_step_grouped(sl.step, sl.rows, sl.lds, s);
+    launch_form_q_grouped(sl.form, sl.rows, sl.lds, s);
   }
   if (!g_rh.empty())
     hipLaunchKernelGGL(rh_from_qr_grouped, dim3(g_rh.l.blocks), dim3(256), 0, s, g_rh.l.recs, g_rh.l.n);
@@ -1602,24 +1156,6 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
       hipLaunchKernelGGL(scale_by_norms_grouped, dim3(g_scale.l.blocks), dim3(JAC_NT), 0, s, g_scale.l.recs,
                          g_scale.l.n);
   }
-  QCA_HIP(hipGetLastError());
-}
-
-void launch_qr(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols, c128* ws,
-               size_t ws_elems, hipStream_t s) {
-  // one workgroup is quicker while the panels would be few
-  if (ws != nullptr && std::min(rows, cols) > 2 * QRB_PB &&
-      ws_elems >= qr_workspace_elems(rows, cols, qcols))
-    launch_blocked_qr(M, rows, cols, tau, Q, qcols, ws, ws_elems, s);
-  else
-    launch_householder_qr(M, rows, cols, tau, Q, qcols, s);
-}
-
-void launch_householder_qr(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols,
-                           hipStream_t s) {
-  QCA_CHECK(rows >= 1 && cols >= 1, "empty QR");
-  hipLaunchKernelGGL(householder_qr_kernel, dim3(1), dim3(QR_THREADS), 0, s, M, rows, cols, tau, Q,
-                     qcols);
   QCA_HIP(hipGetLastError());
 }
 

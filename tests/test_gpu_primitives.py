@@ -315,3 +315,33 @@ def test_exact_expm_refuses_non_finite(gpu):
         qn.call("qca_exact_expm", qn.ptr(psi), 10, 1, 1, 2, 0.2, 0.0, None, None)
     assert e.value.code == -4
     assert np.array_equal(psi.cpu().numpy(), before, equal_nan=True)
+
+
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("chi_row,chi_col,target", [
+    # panel edges: one column more than a panel, ragged last panels, single rows left
+    (9, 9, 9), (8, 16, 16), (17, 17, 17), (33, 31, 31),
+    # fewer rows than columns: a last panel of 10 or 8 reflectors with columns beside and right of it
+    (5, 24, 10), (12, 40, 24), (3, 17, 6),
+    # every register block of the panel (64-row chunks), complement columns up to a square Q
+    (40, 20, 80), (90, 64, 180), (150, 100, 100), (200, 33, 48), (256, 40, 512)])
+def test_qr_panels_match_lapack(gpu, side, chi_row, chi_col, target):
+    """The blocked QR at its panel and register-block edges, against numpy.linalg.qr
+    in LAPACK's conventions (as test_qr_site_matches_lapack)."""
+    import torch
+    from oracle import mps as OM
+    rng = np.random.default_rng(chi_row * 7 + chi_col + side)
+    chil, chir = (chi_row, chi_col) if side == 0 else (chi_col, chi_row)
+    A = crand(rng, 2, chil, chir)
+    if side == 0:
+        Q, R = OM.left_qr(A, reduced=False)
+        refA, refC = OM.truncate_pad(Q, (2, chil, target)), OM.truncate_pad(R, (target, chir))
+    else:
+        Q, R = OM.right_qr(A, reduced=False)
+        refA, refC = OM.truncate_pad(Q, (2, target, chir)), OM.truncate_pad(R, (chil, target))
+    An = torch.zeros(refA.shape, dtype=torch.complex128, device="cuda")
+    C = torch.zeros(refC.shape, dtype=torch.complex128, device="cuda")
+    Ad = dev(torch, A, np.complex128)
+    qn.call("qca_qr_site", side, qn.ptr(Ad), chil, chir, target, qn.ptr(An), qn.ptr(C), None)
+    assert np.abs(An.cpu().numpy() - refA).max() < 1e-12
+    assert np.abs(C.cpu().numpy() - refC).max() < 1e-12
