@@ -40,6 +40,7 @@ constexpr int JAC_MAXCOLS = 512;
 constexpr int JAC_BS = 16;           // block size: pairs of 32 columns
 constexpr int JAC_LMAX = 2 * JAC_BS;
 constexpr int JAC_RC = 64;           // rows per Gram / apply chunk
+constexpr int JAC_INNER_NT = 256;    // jac_inner: one 2x2 block of the Gram per thread
 constexpr int JAC_GRAM_NT = 256;     // jac_gram: one wave per 16x16 block of the 32x32 Gram
 constexpr int JAC_APPLY_NT = 512;    // jac_apply: one wave per 16x16 block of the 32x64 product
 constexpr int JAC_MAX_SWEEPS = 60;
@@ -344,65 +345,244 @@ __device__ int inner_sweep(c128* G, c128* J, JRot (*rot)[JAC_LMAX / 2], int L, i
   return mine;
 }
 
-// Outer rounds 0 and (nb - 1) / 2 of a sweep run the full inner ordering, which
-// also visits the pairs inside each block (every block takes part in every
-// outer round); the other rounds visit only the pairs across their two blocks.
-// A sweep thus meets every column pair at least once, in 2 * 31 + 13 * 16 inner
-// rounds for 16 blocks of 16 instead of 15 * 31.  Inside pairs once per sweep
-// (round 0 only) cost about one sweep more; twice keeps the sweep count of the
-// full ordering within a fraction of a sweep.
+// Rotations of one Jacobi sweep on the Gram G of 2 x 16 columns held in
+// registers by 256 threads (four waves: a barrier of four waves takes 44
+// cycles, of sixteen 815).  Thread (P, Q), P = 4 wave + lane / 16 and Q =
+// (lane + P) % 16, holds the 2x2 block of G of column pairs P and Q and two rows of J:
+//   g = G(iP,iQ), G(iP,jQ), G(jP,iQ), G(jP,jQ);  j = J(P,iQ), J(P,jQ), J(P+16,iQ), J(P+16,jQ).
+// Rotation of columns (i, j), with g = G(i, j) = x_i^H x_j, d = |x_j|^2 - |x_i|^2,
+// h = sqrt(d^2 + 4|g|^2), w = h + |d|:
+//   x_i' = c x_i - conj(s e) x_j,   x_j' = (s e) x_i + c x_j,
+//   c = sqrt(w / (2h)),  s e = sign(d) g sqrt(2 / (h w)),
+// the Rutishauser rotation t = sign(d)/(|zeta| + sqrt(1 + zeta^2)), zeta = d/(2|g|),
+// c = 1/sqrt(1 + t^2), s = t c.  It is evaluated as c = w y, s e = 2 sign(d) g y
+// with y = 1/sqrt(w^2 + 4|g|^2), so that c^2 + |s e|^2 = 1 whatever w is: the
+// accuracy of the angle only sets how far the pair is from zero afterwards, and
+// h comes from the hardware's reciprocal square root as it is (~1e-8).
+// G <- R^H G R and J <- J R.  Every wave computes the rotations of all 16 pairs
+// for itself (of pair Q in each row of lanes; lane 0 of a row has pair P), and
+// carries their squared norms along, so a round costs one barrier and, of LDS,
+// the way of the blocks that change rows and of the next pairs' inner products.
+// What bounds a round is instruction issue: 1740 cycles, of which 114 FP64
+// instructions at 9 cycles each (one wave per SIMD).  16 rounds with loads and
+// stores take 13.7 us; with the Gram in LDS under 1024 threads and two barriers
+// a round they took 16.7.  Squared norms and inner products read from LDS and
+// the row rotation by lane permutes: 14.7.
+struct InnerShared {
+  c128 blk[2][3][256];    // G(iP,jQ), G(jP,iQ), G(jP,jQ) on their way to the next round
+  c128 off[2][16];        // G(i,j) of the pairs of a round
+  double diag[2][16];     // G(i,i), G(j,j) of the first round's pairs
+};
+struct JacRot {
+  double c, sr, si;   // c, s e
+};
+struct InnerThresholds {
+  double tol2, conv2, negl;
+};
+
+// Lane (l + 1) % 16, and lane 0, of each row of 16 lanes.
+__device__ __forceinline__ double row_next(double v) { return dpp_f64<0x12F>(v); }    // row_ror:15
+__device__ __forceinline__ double row_first(double v) { return dpp_f64<0x150>(v); }   // row_newbcast:0
+
+// Rotation of one pair of squared norms a, b (updated) and inner product g;
+// act: it is rotated, sig: above the convergence margin.
+__device__ __forceinline__ JacRot pair_rotation(double& a, double& b, const c128& g, const InnerThresholds& th,
+                                                bool& act, bool& sig) {
+  const double ag2 = g.re * g.re + g.im * g.im;
+  const double d = b - a;
+  const double f = 4.0 * ag2;
+  const double x = fma(d, d, f);
+  const double w = fma(x, __builtin_amdgcn_rsq(x), fabs(d));
+  // y = 1/sqrt(t): a third-order step on the hardware estimate, then one whose
+  // residual 1 - t y^2 includes the exact error of t y, so that y carries no
+  // bias (c and s share y: a biased y drifts the column norms)
+  const double t = fma(w, w, f);
+  double y = __builtin_amdgcn_rsq(t);
+  const double e0 = fma(-t * y, y, 1.0);
+  y = fma(y, e0 * fma(0.375, e0, 0.5), y);
+  const double ty = t * y;
+  const double e = fma(-ty, y, 1.0) - fma(t, y, -ty) * y;
+  y = fma(0.5 * y, e, y);
+  // a pair with a column at the noise floor is done: rotating noise against a
+  // signal column only re-creates noise, and for matrices with more columns
+  // than rows such pairs can rotate indefinitely
+  const double ab = a * b;
+  act = !(ag2 <= th.tol2 * ab || ag2 < 1e-300 || fmin(a, b) < th.negl);
+  sig = act && ag2 > th.conv2 * ab;
+  const double s = d >= 0 ? 2.0 * y : -2.0 * y;
+  // |x_i|^2 and |x_j|^2 change by tan |g| = 2 |g|^2 / w
+  double iw = __builtin_amdgcn_rcp(w);
+  iw = fma(iw, fma(-w, iw, 1.0), iw);
+  const double delta = act ? (d >= 0 ? 0.5 : -0.5) * f * iw : 0.0;
+  a -= delta;
+  b += delta;
+  return act ? JacRot{w * y, s * g.re, s * g.im} : JacRot{1.0, 0.0, 0.0};
+}
+
+// x_i, x_j <- the rotated pair (columns).
+__device__ __forceinline__ void rotate_cols(const JacRot& q, c128& x, c128& y) {
+  const c128 a = x, b = y;
+  x = c128{q.c * a.re - (q.sr * b.re + q.si * b.im), q.c * a.im - (q.sr * b.im - q.si * b.re)};
+  y = c128{(q.sr * a.re - q.si * a.im) + q.c * b.re, (q.sr * a.im + q.si * a.re) + q.c * b.im};
+}
+// The conjugate rotation, for the rows of R^H G.
+__device__ __forceinline__ void rotate_rows(const JacRot& p, c128& x, c128& y) {
+  const c128 a = x, b = y;
+  x = c128{p.c * a.re - (p.sr * b.re - p.si * b.im), p.c * a.im - (p.sr * b.im + p.si * b.re)};
+  y = c128{(p.sr * a.re + p.si * a.im) + p.c * b.re, (p.sr * a.im - p.si * a.re) + p.c * b.im};
+}
+
+// H rounds: pair t of group m (2H columns from 2H m) joins column t of the
+// group's first half and column H + (t + r) mod H of it in round r, so the
+// blocks of the second columns move to the next pair's thread after each
+// round (across lanes of a row by DPP moves or a lane read, across rows
+// through LDS) and are back in place after the last.
+template <int H>
+__device__ __forceinline__ void inner_rounds(c128 (&g)[4], c128 (&j)[4], InnerShared& sh, const InnerThresholds& th,
+                                             int& rotated, int& above) {
+  const int lane = threadIdx.x & 15, P = threadIdx.x >> 4, Q = (lane + P) & 15;
+  const int nP = (P & ~(H - 1)) | ((P + 1) & (H - 1)), nQ = (Q & ~(H - 1)) | ((Q + 1) & (H - 1));
+  const int nl = (nQ - P) & 15;   // the lane of pair nQ
+  const int at = P * 16 + Q, at_i = nP * 16 + Q, at_j = nP * 16 + nQ;
+  int buf = 0;
+  if (lane == 0) {
+    sh.off[0][P] = g[1];
+    sh.diag[0][P] = g[0].re;
+    sh.diag[1][P] = g[3].re;
+  }
+  __syncthreads();
+  double a = sh.diag[0][Q], b = sh.diag[1][Q];
+  c128 off = sh.off[0][Q];
+#pragma unroll 1
+  for (int r = 0; r < H; ++r) {
+    bool act, sig;
+    const JacRot q = pair_rotation(a, b, off, th, act, sig);
+    rotated += __popcll(__ballot(act) & 0xffff);
+    above += __popcll(__ballot(sig) & 0xffff);
+    const JacRot p{row_first(q.c), row_first(q.sr), row_first(q.si)};
+    rotate_cols(q, g[0], g[1]);
+    rotate_cols(q, g[2], g[3]);
+    rotate_rows(p, g[0], g[2]);
+    rotate_rows(p, g[1], g[3]);
+    buf ^= 1;
+    if (Q == nP) sh.off[buf][P] = g[1];
+    sh.blk[buf][1][at] = g[2];
+    sh.blk[buf][2][at] = g[3];
+    if constexpr (H == 16) {
+      g[1] = c128{row_next(g[1].re), row_next(g[1].im)};
+      b = row_next(b);
+    } else {
+      sh.blk[buf][0][at] = g[1];
+      b = __shfl(b, nl, 16);
+    }
+    rotate_cols(q, j[0], j[1]);
+    rotate_cols(q, j[2], j[3]);
+#pragma unroll
+    for (int k = 1; k < 4; k += 2) {
+      if constexpr (H == 16) j[k] = c128{row_next(j[k].re), row_next(j[k].im)};
+      else j[k] = c128{__shfl(j[k].re, nl, 16), __shfl(j[k].im, nl, 16)};
+    }
+    __syncthreads();
+    off = sh.off[buf][Q];
+    g[2] = sh.blk[buf][1][at_i];
+    g[3] = sh.blk[buf][2][at_j];
+    if constexpr (H < 16) g[1] = sh.blk[buf][0][P * 16 + nQ];
+  }
+}
+
+// From the pairs of groups of 2H columns to those of groups of H.
+template <int H>
+__device__ __forceinline__ void inner_regroup(c128 (&g)[4], c128 (&j)[4], InnerShared& sh) {
+  c128* m = &sh.blk[0][0][0];   // 32 x 32
+  const int P = threadIdx.x >> 4, Q = (threadIdx.x + P) & 15;
+  const int iP = (P / H) * 2 * H + P % H, iQ = (Q / H) * 2 * H + Q % H;
+  constexpr int K = H / 2;
+  const int kP = (P / K) * H + P % K, kQ = (Q / K) * H + Q % K;
+  __syncthreads();
+  m[iP * 32 + iQ] = g[0];
+  m[iP * 32 + iQ + H] = g[1];
+  m[(iP + H) * 32 + iQ] = g[2];
+  m[(iP + H) * 32 + iQ + H] = g[3];
+  __syncthreads();
+  g[0] = m[kP * 32 + kQ];
+  g[1] = m[kP * 32 + kQ + K];
+  g[2] = m[(kP + K) * 32 + kQ];
+  g[3] = m[(kP + K) * 32 + kQ + K];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) m[(P + 16 * (k / 2)) * 32 + iQ + (k & 1) * H] = j[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 4; ++k) j[k] = m[(P + 16 * (k / 2)) * 32 + kQ + (k & 1) * K];
+  __syncthreads();
+}
+
+// Outer rounds 0 and (nb - 1) / 2 of a sweep also visit the pairs inside each
+// block (every block takes part in every outer round), by halves: the pairs
+// across two groups of 16 columns, then of 8, 4, 2, 1 (31 rounds); the others
+// visit only the pairs across their two blocks (16 rounds).  A sweep thus meets
+// every column pair at least once, in 2 * 31 + 13 * 16 inner rounds for 16
+// blocks of 16 instead of 15 * 31.  Inside pairs once per sweep (round 0 only)
+// cost about one sweep more; twice keeps the sweep count of a full ordering
+// within a fraction of a sweep.
 __device__ __forceinline__ void jac_inner_body(const JacobiGeom& g, int round, int sweep,
                                                const c128* __restrict__ Gpart,
                                                c128* __restrict__ Jout, int* __restrict__ rotated,
                                                double tol, JacobiCtrl* __restrict__ ctrl, int p) {
   const int done = ctrl->done;  // read alongside the partial Grams
-  constexpr int HM = JAC_LMAX / 2;
-  __shared__ c128 G[JAC_LMAX * JAC_LMAX];
-  __shared__ c128 J[JAC_LMAX * JAC_LMAX];
-  __shared__ JRot rot[2][HM];
-  __shared__ int total, total_sig;
-  const int L = 2 * g.bs, H = g.bs, tid = threadIdx.x;
-  const double negl = JAC_NOISE2 * ctrl->fro;
+  constexpr int L = JAC_LMAX;
+  __shared__ InnerShared sh;
+  const int P = threadIdx.x >> 4, Q = (threadIdx.x + P) & 15;
   const double conv = jac_conv_tol(tol, g.rows);
-  static_assert(JAC_NT >= JAC_LMAX * JAC_LMAX, "one Gram entry per thread");
-  if (tid < L * L) {
-    // all chunk partials are loaded before the first add (one memory latency),
-    // then summed in chunk order
-    c128 v[JAC_MAXKSPL];
+  const InnerThresholds th{tol * tol, conv * conv, JAC_NOISE2 * ctrl->fro};
+  // all chunk partials are loaded before the first add (one memory latency),
+  // then summed in chunk order; G(P, Q) is read as conj(G(Q, P)), contiguous
+  // over the lanes
+  c128 v[JAC_MAXKSPL][4];
 #pragma unroll
-    for (int kc = 0; kc < JAC_MAXKSPL; ++kc)
-      if (kc < g.kspl) v[kc] = Gpart[((long)p * g.kspl + kc) * L * L + tid];
+  for (int kc = 0; kc < JAC_MAXKSPL; ++kc)
+    if (kc < g.kspl)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        v[kc][k] = Gpart[((long)p * g.kspl + kc) * L * L + (P + 16 * (k / 2)) * L + Q + 16 * (k & 1)];
+  c128 G[4], J[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
     double re = 0, im = 0;
 #pragma unroll
     for (int kc = 0; kc < JAC_MAXKSPL; ++kc)
       if (kc < g.kspl) {
-        re += v[kc].re;
-        im += v[kc].im;
+        re += v[kc][k].re;
+        im += v[kc][k].im;
       }
-    G[tid] = c128{re, im};
-    J[tid] = c128{(tid % L) == (tid / L) ? 1.0 : 0.0, 0.0};
+    G[k] = c128{re, -im};
+    J[k] = c128{(k == 0 || k == 3) && P == Q ? 1.0 : 0.0, 0.0};
   }
-  if (tid == 0) {
-    total = 0;
-    total_sig = 0;
-  }
-  __syncthreads();
   if (done) return;
-  const bool cross = round != 0 && round != (g.nb - 1) / 2;
-  const int mine = cross ? inner_sweep<true>(G, J, rot, L, H, tol * tol, conv * conv, negl)
-                         : inner_sweep<false>(G, J, rot, L, H, tol * tol, conv * conv, negl);
-  if (mine & 0xffff) atomicAdd(&total, mine & 0xffff);
-  if (mine >> 16) atomicAdd(&total_sig, mine >> 16);
-  __syncthreads();
+  int total = 0, above = 0, h = 16;
+  inner_rounds<16>(G, J, sh, th, total, above);
+  if (round == 0 || round == (g.nb - 1) / 2) {
+    inner_regroup<16>(G, J, sh);
+    inner_rounds<8>(G, J, sh, th, total, above);
+    inner_regroup<8>(G, J, sh);
+    inner_rounds<4>(G, J, sh, th, total, above);
+    inner_regroup<4>(G, J, sh);
+    inner_rounds<2>(G, J, sh, th, total, above);
+    inner_regroup<2>(G, J, sh);
+    inner_rounds<1>(G, J, sh, th, total, above);
+    h = 1;
+  }
+  // J(k, c) at c * L + k
   c128* jo = Jout + (long)p * L * L;
-  for (int e = tid; e < L * L; e += JAC_NT) jo[e] = J[e];
-  if (tid == 0) {
+  const int iQ = h == 16 ? Q : 2 * Q;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) jo[(iQ + (k & 1) * h) * L + P + 16 * (k / 2)] = J[k];
+  if (threadIdx.x == 0) {
     rotated[p] = total;
-    if (total_sig) atomicAdd(&ctrl->rot[sweep], total_sig);
+    if (above) atomicAdd(&ctrl->rot[sweep], above);
   }
 }
-// Two workgroups per CU (64 VGPRs): grouped launches hold a pair per workgroup.
-__global__ __launch_bounds__(JAC_NT) __attribute__((amdgpu_waves_per_eu(8))) void jac_inner(JacobiGeom g, int round, int sweep,
+__global__ __launch_bounds__(JAC_INNER_NT) void jac_inner(JacobiGeom g, int round, int sweep,
                                                     const c128* __restrict__ Gpart,
                                                     c128* __restrict__ Jout,
                                                     int* __restrict__ rotated, double tol,
@@ -842,7 +1022,7 @@ __global__ __launch_bounds__(JAC_GRAM_NT) void jac_gram_grouped(const GRec<JacAr
   if (round >= g.nb - 1) return;
   jac_gram_body(gbl(r.a.Y), g, round, gbl(r.a.Gpart), gbl(r.a.ctrl), bx, by);
 }
-__global__ __launch_bounds__(JAC_NT) __attribute__((amdgpu_waves_per_eu(8))) void jac_inner_grouped(const GRec<JacArgs>* __restrict__ recs, int n,
+__global__ __launch_bounds__(JAC_INNER_NT) void jac_inner_grouped(const GRec<JacArgs>* __restrict__ recs, int n,
                                                             int round, int sweep) {
   unsigned bx, by, bz;
   const GRec<JacArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
@@ -928,7 +1108,7 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
       for (int r = 0; r < l.nb - 1; ++r) {
         hipLaunchKernelGGL(jac_gram, dim3(np, l.kspl), dim3(JAC_GRAM_NT), 0, s, (const c128*)Y, g, r,
                            Gpart, (const JacobiCtrl*)ctrl);
-        hipLaunchKernelGGL(jac_inner, dim3(np), dim3(JAC_NT), 0, s, g, r, sweep, (const c128*)Gpart,
+        hipLaunchKernelGGL(jac_inner, dim3(np), dim3(JAC_INNER_NT), 0, s, g, r, sweep, (const c128*)Gpart,
                            Jbuf, rotated, tol, ctrl);
         hipLaunchKernelGGL(jac_apply, dim3(np, l.kspl + gz.kspl), dim3(JAC_APPLY_NT), 0, s, Y, g, Z, gz, r,
                            (const c128*)Jbuf, (const int*)rotated, (const JacobiCtrl*)ctrl);
@@ -1135,7 +1315,7 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
         for (int r = 0; r < max_rounds; ++r) {
           hipLaunchKernelGGL(jac_gram_grouped, dim3(g_gram.l.blocks), dim3(JAC_GRAM_NT), 0, s, g_gram.l.recs,
                              g_gram.l.n, r);
-          hipLaunchKernelGGL(jac_inner_grouped, dim3(g_inner.l.blocks), dim3(JAC_NT), 0, s, g_inner.l.recs,
+          hipLaunchKernelGGL(jac_inner_grouped, dim3(g_inner.l.blocks), dim3(JAC_INNER_NT), 0, s, g_inner.l.recs,
                              g_inner.l.n, r, sweep);
           hipLaunchKernelGGL(jac_apply_grouped, dim3(g_apply.l.blocks), dim3(JAC_APPLY_NT), 0, s, g_apply.l.recs,
                              g_apply.l.n, r);
