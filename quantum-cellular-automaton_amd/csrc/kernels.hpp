@@ -174,8 +174,9 @@ struct SvdResult {
 
 // Workspace of the Jacobi SVD: device memory of at least
 // jacobi_workspace_bytes(rows, cols) (control block, partial Grams, block
-// rotations), a pinned host word pair, and the sweep count of the previous call
-// (the number of sweeps launched before the first convergence check).
+// rotations, matrices of the closing phase), 16 bytes of pinned host memory, and
+// the sweep and closing-step counts of the previous call (the number launched
+// before the first look at the device's state).
 struct JacobiWork {
   void* ws = nullptr;
   size_t ws_bytes = 0;
@@ -185,7 +186,8 @@ struct JacobiWork {
   // jacobi_precond_elems(rows, cols) complex128, or null to skip it
   c128* pre = nullptr;
   size_t pre_elems = 0;
-  int pred_sweeps_pre = 6;
+  int pred_sweeps_pre = 4;
+  int pred_newton = 3;      // closing steps of the previous call
   // rotation threshold relative to the column norms; 0: eps * sqrt(rows)
   double tol = 0;
 };

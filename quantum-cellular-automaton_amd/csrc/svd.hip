@@ -14,6 +14,8 @@
 //              the others only those across the two blocks;
 //   jac_apply  X_p <- X_p J_p, each workgroup one chunk of rows, on the
 //              FP64 matrix cores.
+// The last sweeps of a preconditioned matrix are replaced by simultaneous
+// rotations of all pairs as matrix products (closing phase below).
 // Stream order separates the rounds.  The Gram is rebuilt from the columns in
 // every round, so the test for a converged pair, |x_i^H x_j| <=
 // tol*|x_i||x_j|, and the singular values (final column norms) carry the
@@ -45,6 +47,7 @@ constexpr int JAC_GRAM_NT = 256;     // jac_gram: one wave per 16x16 block of th
 constexpr int JAC_APPLY_NT = 512;    // jac_apply: one wave per 16x16 block of the 32x64 product
 constexpr int JAC_MAX_SWEEPS = 60;
 constexpr int JAC_MAXKSPL = 8;       // row chunks of a Gram: rows <= 512
+constexpr size_t JAC_CTRL_BYTES = 512;   // slot of the control block
 // Noise floor of a column, squared and relative to ||X||_F^2: (16 eps)^2.
 // Columns below 16 eps ||X|| (3.6e-15 ||X||) are not orthogonalised further;
 // their singular values are at the accuracy floor of the method, far below any
@@ -99,8 +102,11 @@ __device__ __forceinline__ int rr_player(int t, int r, int n) {
 
 struct JacobiCtrl {
   double fro;                  // ||X||_F^2
-  int done;                    // set by the first sweep without a rotation above jac_conv_tol
+  int done;                    // converged
   int sweeps;                  // sweeps executed
+  int phase;                   // 0: sweeps, 1: closing phase
+  int newton;                  // closing steps executed
+  int schulz;                  // Newton-Schulz steps of the next closing step
   int rot[JAC_MAX_SWEEPS];     // rotations above jac_conv_tol per sweep
 };
 
@@ -160,6 +166,7 @@ __device__ __forceinline__ void jac_init_body(const c128* __restrict__ X, long n
     ctrl->fro = s;
     ctrl->done = 0;
     ctrl->sweeps = 0;
+    ctrl->phase = ctrl->newton = ctrl->schulz = 0;
   }
   if (threadIdx.x < JAC_MAX_SWEEPS) ctrl->rot[threadIdx.x] = 0;
 }
@@ -177,7 +184,7 @@ __device__ __forceinline__ void jac_gram_body(const c128* __restrict__ X, const 
                                               const JacobiCtrl* __restrict__ ctrl, int p, int kc) {
   // the control word is read alongside the tile, not before it: the round
   // kernels are latency bound, and a no-op round only stages a tile
-  const int done = ctrl->done;
+  const int done = ctrl->done | ctrl->phase;
   __shared__ c128 tile[JAC_RC * (JAC_LMAX + 1)];
   const int L = 2 * g.bs;
   const int r0 = kc * JAC_RC, nr = min(JAC_RC, g.rows - r0);
@@ -529,7 +536,7 @@ __device__ __forceinline__ void jac_inner_body(const JacobiGeom& g, int round, i
                                                const c128* __restrict__ Gpart,
                                                c128* __restrict__ Jout, int* __restrict__ rotated,
                                                double tol, JacobiCtrl* __restrict__ ctrl, int p) {
-  const int done = ctrl->done;  // read alongside the partial Grams
+  const int done = ctrl->done | ctrl->phase;  // read alongside the partial Grams
   constexpr int L = JAC_LMAX;
   __shared__ InnerShared sh;
   const int P = threadIdx.x >> 4, Q = (threadIdx.x + P) & 15;
@@ -599,7 +606,7 @@ __device__ __forceinline__ void jac_apply_body(c128* __restrict__ Xa, const Jaco
                                                const int* __restrict__ rotated,
                                                const JacobiCtrl* __restrict__ ctrl, int p, int by) {
   // the control words are read alongside the tile and J, not before them
-  const int skip = ctrl->done | (rotated[p] == 0);
+  const int skip = ctrl->done | ctrl->phase | (rotated[p] == 0);
   const bool second = by >= ga.kspl;
   c128* __restrict__ X = second ? Za : Xa;
   const JacobiGeom g = second ? gz : ga;
@@ -664,6 +671,310 @@ __global__ void jac_check(JacobiCtrl* __restrict__ ctrl, int sweep) {
   if (threadIdx.x != 0 || ctrl->done) return;
   ctrl->sweeps = sweep + 1;
   if (ctrl->rot[sweep] == 0) ctrl->done = 1;
+}
+
+// ------------------------------------------------------------------ closing phase
+// Once the columns of Y are nearly orthogonal, all pairs are rotated at once:
+// with the small rotations of the cyclic sweeps collected in an anti-Hermitian
+// K, K_ij = sign(d) 2 g_ij / w for every pair (d, w as in the sweeps), Y <- Y J
+// with a unitary J = I + K + O(K^2) squares the scaled off-diagonals just as a
+// sweep does, but as products on the matrix cores instead of a chain of n
+// rotation rounds: J starts as I + K + K^2 / 2 and is made unitary by
+// Newton-Schulz steps J <- J (3 I - J^H J) / 2.  Each product keeps the relative
+// accuracy of graded columns: K_ij, K^2 and J^H J - I carry the factor
+// |y_j| / |y_i| of a pair with |y_j| << |y_i|.
+// A matrix enters the phase after a sweep (the second or a later one) that
+// leaves |K|_F <= NEWTON_KF, and goes back to sweeps if |K|_F should exceed it
+// again (clusters of singular values keep K large: those are left to the
+// sweeps).  It has converged when no pair is above the margin of jac_conv_tol.
+// All of this is decided on the device from Y alone, so that a matrix takes the
+// same steps alone and in a group.
+// A step is bound by its eleven dependent launches: 50 us for 256 columns, of
+// which the products (16x16 tiles, one workgroup each, k split over four waves)
+// take 3-11 us each, against 380 us for a sweep's 15 rounds.  A 256x256 random
+// two-site tensor takes 4 sweeps and 3 steps instead of 7 sweeps (split 3.36 ->
+// 2.43 ms), a 154x90 one 2 and 3 instead of 6 (1.22 -> 0.81 ms).  NEWTON_KF: as
+// far as three Newton-Schulz steps reach rounding; at 0.1 the 154x90 split takes
+// a sweep more (0.91 ms).
+constexpr int NEWTON_NT = 256;
+constexpr int NEWTON_SCHULZ_MAX = 3;
+constexpr double NEWTON_KF = 0.4;     // |K|_F up to which a matrix is in the closing phase
+constexpr int NEWTON_MAX = 12;        // steps after which a matrix stays with the sweeps
+
+struct NewtonArgs {
+  c128* Y;            // yrows x n
+  c128* Q;            // qrows x n, same rotations
+  int yrows, qrows, n, ytiles, qtiles, ntiles;   // 16-row and 16-column tiles
+  c128 *K, *W, *J0, *J1;   // K and W also take the new Y and Q (yrows x n, qrows x n)
+  double* kf2;        // per tile: sum of |K|^2
+  int* above;         // per tile: pairs above the convergence margin
+  JacobiCtrl* ctrl;
+  double tol;
+};
+
+struct NewtonShared {
+  c128 part[4][16 * 17];
+  double nrm[2][16][16];
+  double red[4];
+  int cnt[4];
+};
+
+// One 16x16 tile of a product over k < kdim, the four waves taking 16 of every
+// 64 k each; the sum over the waves is left to tile_sum.  a(k, lane16) and
+// b(k, lane16) give the operands' elements (k = row of the lane group).
+template <typename FA, typename FB>
+__device__ __forceinline__ void tile_product(int kdim, NewtonShared& sh, FA&& a, FB&& b) {
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  jac_f64x4 re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+  for (int k0 = 16 * wave; k0 < kdim; k0 += 128) {
+    // two of the wave's blocks of 16 k: 16 loads in flight
+    c128 x[8], y[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int k = k0 + (s / 4) * 64 + 4 * (s & 3) + hi;
+      x[s] = a(k, lo);
+      y[s] = b(k, lo);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      re = jac_mfma(x[s].re, y[s].re, re);
+      im = jac_mfma(x[s].re, y[s].im, im);
+      re = jac_mfma(-x[s].im, y[s].im, re);
+      im = jac_mfma(x[s].im, y[s].re, im);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) sh.part[wave][(hi + 4 * r) * 17 + lo] = c128{re[r], im[r]};
+}
+// Element (i, j) of the tile for thread i + 16 j (after a barrier).
+__device__ __forceinline__ c128 tile_sum(const NewtonShared& sh) {
+  const int e = (threadIdx.x & 15) * 17 + (threadIdx.x >> 4);
+  c128 s{0.0, 0.0};
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    s.re += sh.part[w][e].re;
+    s.im += sh.part[w][e].im;
+  }
+  return s;
+}
+// X(k, c) of a column-major matrix, zero outside rows x cols.
+__device__ __forceinline__ c128 col_elem(const c128* __restrict__ X, int rows, int cols, int k, int c) {
+  const c128 v = X[(unsigned)min(c, cols - 1) * rows + min(k, rows - 1)];
+  return k < rows && c < cols ? v : c128{0.0, 0.0};
+}
+__device__ __forceinline__ c128 conj_of(c128 v) { return c128{v.re, -v.im}; }
+
+// Phase words: a matrix is in sweeps (0) or in the closing phase (1).
+__device__ __forceinline__ bool newton_off(const JacobiCtrl* ctrl) { return ctrl->done || ctrl->phase == 0; }
+
+// K of column tiles (bi, bj), bi <= bj, and its mirror; after a sweep (closing
+// = 0) for matrices in sweeps, after a closing step for those in the phase.
+__device__ __forceinline__ void newton_corr_body(const NewtonArgs& a, const c128* __restrict__ Y,
+                                                 c128* __restrict__ K, int closing, int bi, int bj, NewtonShared& sh) {
+  if (bi > bj || a.ctrl->done || a.ctrl->phase != closing) return;
+  const int n = a.n, rows = a.yrows, i0 = 16 * bi, j0 = 16 * bj;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double na = 0, nb = 0;
+  tile_product(
+      rows, sh,
+      [&](int k, int c) {
+        const c128 v = col_elem(Y, rows, n, k, i0 + c);
+        na += v.re * v.re + v.im * v.im;
+        return conj_of(v);
+      },
+      [&](int k, int c) {
+        const c128 v = col_elem(Y, rows, n, k, j0 + c);
+        nb += v.re * v.re + v.im * v.im;
+        return v;
+      });
+  sh.nrm[0][4 * wave + (lane >> 4)][lane & 15] = na;
+  sh.nrm[1][4 * wave + (lane >> 4)][lane & 15] = nb;
+  __syncthreads();
+  const c128 g = tile_sum(sh);
+  const int i = threadIdx.x & 15, j = threadIdx.x >> 4;
+  double pa = 0, pb = 0;
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    pa += sh.nrm[0][s][i];
+    pb += sh.nrm[1][s][j];
+  }
+  const int gi = i0 + i, gj = j0 + j;
+  const double conv = jac_conv_tol(a.tol, rows);
+  const double ag2 = g.re * g.re + g.im * g.im, ab = pa * pb;
+  const bool pair = gi < gj && gj < n;
+  const bool act = pair && !(ag2 <= a.tol * a.tol * ab || ag2 < 1e-300 || fmin(pa, pb) < JAC_NOISE2 * a.ctrl->fro);
+  const bool sig = act && ag2 > conv * conv * ab;
+  double t = 0;
+  if (act) {
+    const double d = pb - pa;
+    t = (d >= 0 ? 2.0 : -2.0) / (sqrt(fma(d, d, 4.0 * ag2)) + fabs(d));
+  }
+  const c128 kij{t * g.re, t * g.im};
+  if (pair) {
+    K[(unsigned)gj * n + gi] = kij;
+    K[(unsigned)gi * n + gj] = c128{-kij.re, kij.im};
+  } else if (gi == gj && gi < n) {
+    K[(unsigned)gj * n + gi] = c128{0.0, 0.0};
+  }
+  const double kf = wave_sum64(2.0 * (kij.re * kij.re + kij.im * kij.im));
+  const int cnt = __popcll(__ballot(sig));
+  if (lane == 0) {
+    sh.red[wave] = kf;
+    sh.cnt[wave] = cnt;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int tile = bi * a.ntiles + bj;
+    a.kf2[tile] = (sh.red[0] + sh.red[1]) + (sh.red[2] + sh.red[3]);
+    a.above[tile] = sh.cnt[0] + sh.cnt[1] + sh.cnt[2] + sh.cnt[3];
+  }
+}
+
+// After sweep `sweep` (>= 0) or a closing step (-1): converged, closing phase
+// or sweeps.
+__device__ __forceinline__ void newton_decide_body(const NewtonArgs& a, JacobiCtrl* __restrict__ ctrl, int sweep) {
+  const int closing = sweep < 0 ? 1 : 0;
+  if (ctrl->done || ctrl->phase != closing) return;
+  __shared__ double red[NEWTON_NT / 64];
+  __shared__ int cnt[NEWTON_NT / 64];
+  double kf = 0;
+  int above = 0;
+  for (int t = threadIdx.x; t < a.ntiles * a.ntiles; t += NEWTON_NT)
+    if (t / a.ntiles <= t % a.ntiles) {
+      kf += a.kf2[t];
+      above += a.above[t];
+    }
+  kf = wave_sum64(kf);
+  for (int o = 32; o > 0; o >>= 1) above += __shfl_xor(above, o, 64);
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = kf;
+    cnt[threadIdx.x >> 6] = above;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  kf = (red[0] + red[1]) + (red[2] + red[3]);
+  above = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+  if (closing) ctrl->newton += 1;
+  else ctrl->sweeps += 1;   // sweeps launched during the closing phase are no-ops
+  if (closing ? above == 0 : ctrl->rot[sweep] == 0) {
+    ctrl->done = 1;
+    return;
+  }
+  const bool in = kf <= NEWTON_KF * NEWTON_KF && ctrl->newton < NEWTON_MAX;
+  ctrl->phase = in ? 1 : 0;
+  // Newton-Schulz steps until |J^H J - I| <= 1e-17: it is |K|^4 / 4 at first and
+  // 3/4 of its square after a step (4e-19 after three from NEWTON_KF)
+  int schulz = 0;
+  for (double e = 0.25 * kf * kf; e > 1e-17 && schulz < NEWTON_SCHULZ_MAX; e = 0.75 * e * e) ++schulz;
+  ctrl->schulz = schulz;
+}
+
+// J0 = I + K + K^2 / 2, K^2 = -K^H K.
+__device__ __forceinline__ void newton_start_body(const NewtonArgs& a, const c128* __restrict__ K,
+                                                  c128* __restrict__ J, int bi, int bj, NewtonShared& sh) {
+  if (newton_off(a.ctrl)) return;
+  const int n = a.n, i0 = 16 * bi, j0 = 16 * bj;
+  tile_product(n, sh, [&](int k, int c) { return conj_of(col_elem(K, n, n, k, i0 + c)); },
+               [&](int k, int c) { return col_elem(K, n, n, k, j0 + c); });
+  __syncthreads();
+  const c128 s = tile_sum(sh);
+  const int gi = i0 + (threadIdx.x & 15), gj = j0 + (threadIdx.x >> 4);
+  if (gi < n && gj < n) {
+    const c128 k = K[(unsigned)gj * n + gi];
+    J[(unsigned)gj * n + gi] = c128{(gi == gj ? 1.0 : 0.0) + k.re - 0.5 * s.re, k.im - 0.5 * s.im};
+  }
+}
+// W = J^H J (`step`-th Newton-Schulz step, if there is one).
+__device__ __forceinline__ void newton_gram_body(const NewtonArgs& a, const c128* __restrict__ J,
+                                                 c128* __restrict__ W, int step, int bi, int bj, NewtonShared& sh) {
+  if (newton_off(a.ctrl) || a.ctrl->schulz < step) return;
+  const int n = a.n, i0 = 16 * bi, j0 = 16 * bj;
+  tile_product(n, sh, [&](int k, int c) { return conj_of(col_elem(J, n, n, k, i0 + c)); },
+               [&](int k, int c) { return col_elem(J, n, n, k, j0 + c); });
+  __syncthreads();
+  const c128 s = tile_sum(sh);
+  const int gi = i0 + (threadIdx.x & 15), gj = j0 + (threadIdx.x >> 4);
+  if (gi < n && gj < n) W[(unsigned)gj * n + gi] = s;
+}
+// Jn = 1.5 J - 0.5 J W, W Hermitian (W(l, j) read as conj(W(j, l))).
+__device__ __forceinline__ void newton_schulz_body(const NewtonArgs& a, const c128* __restrict__ J,
+                                                   const c128* __restrict__ W, c128* __restrict__ Jn, int step,
+                                                   int bi, int bj, NewtonShared& sh) {
+  if (newton_off(a.ctrl) || a.ctrl->schulz < step) return;
+  const int n = a.n, i0 = 16 * bi, j0 = 16 * bj;
+  tile_product(n, sh, [&](int k, int c) { return col_elem(J, n, n, i0 + c, k); },
+               [&](int k, int c) { return conj_of(col_elem(W, n, n, j0 + c, k)); });
+  __syncthreads();
+  const c128 s = tile_sum(sh);
+  const int gi = i0 + (threadIdx.x & 15), gj = j0 + (threadIdx.x >> 4);
+  if (gi < n && gj < n) {
+    const c128 z = J[(unsigned)gj * n + gi];
+    Jn[(unsigned)gj * n + gi] = c128{1.5 * z.re - 0.5 * s.re, 1.5 * z.im - 0.5 * s.im};
+  }
+}
+// Row tile br of (Y; Q), column tile bj: the new Y to K's buffer, the new Q to
+// W's.
+__device__ __forceinline__ void newton_apply_body(const NewtonArgs& a, const c128* __restrict__ Y,
+                                                  const c128* __restrict__ Q, const c128* __restrict__ J0,
+                                                  const c128* __restrict__ J1, c128* __restrict__ Yn,
+                                                  c128* __restrict__ Qn, int br, int bj, NewtonShared& sh) {
+  if (newton_off(a.ctrl)) return;
+  const c128* __restrict__ J = a.ctrl->schulz & 1 ? J1 : J0;
+  const bool second = br >= a.ytiles;
+  const c128* __restrict__ X = second ? Q : Y;
+  c128* __restrict__ out = second ? Qn : Yn;
+  const int rows = second ? a.qrows : a.yrows, n = a.n;
+  const int i0 = 16 * (second ? br - a.ytiles : br), j0 = 16 * bj;
+  tile_product(n, sh, [&](int k, int c) { return col_elem(X, rows, n, i0 + c, k); },
+               [&](int k, int c) { return col_elem(J, n, n, k, j0 + c); });
+  __syncthreads();
+  const c128 s = tile_sum(sh);
+  const int gi = i0 + (threadIdx.x & 15), gj = j0 + (threadIdx.x >> 4);
+  if (gi < rows && gj < n) out[(unsigned)gj * rows + gi] = s;
+}
+__device__ __forceinline__ void newton_copy_body(const NewtonArgs& a, c128* __restrict__ Y, c128* __restrict__ Q,
+                                                 const c128* __restrict__ Yn, const c128* __restrict__ Qn,
+                                                 unsigned blk, unsigned nblk) {
+  if (newton_off(a.ctrl)) return;
+  const int ny = a.yrows * a.n, nq = a.qrows * a.n;
+  for (int e = blk * NEWTON_NT + threadIdx.x; e < ny + nq; e += nblk * NEWTON_NT) {
+    if (e < ny) Y[e] = Yn[e];
+    else Q[e - ny] = Qn[e - ny];
+  }
+}
+
+// The kernels of the phase, one for a single matrix and one for a group.
+enum NewtonOp { NEWTON_CORR, NEWTON_START, NEWTON_GRAM, NEWTON_SCHULZ, NEWTON_APPLY, NEWTON_COPY };
+template <int OP>
+__device__ __forceinline__ void newton_body(const NewtonArgs& a, int arg, unsigned bx, unsigned by, unsigned nx) {
+  __shared__ NewtonShared sh;
+  c128 *Y = gbl(a.Y), *Q = gbl(a.Q), *K = gbl(a.K), *W = gbl(a.W), *J0 = gbl(a.J0), *J1 = gbl(a.J1);
+  // arg: closing (corr); Newton-Schulz step 1 or 3 (J0 -> J1) or 2 (J1 -> J0)
+  if constexpr (OP == NEWTON_CORR) newton_corr_body(a, Y, K, arg, bx, by, sh);
+  if constexpr (OP == NEWTON_START) newton_start_body(a, K, J0, bx, by, sh);
+  if constexpr (OP == NEWTON_GRAM) newton_gram_body(a, arg & 1 ? J0 : J1, W, arg, bx, by, sh);
+  if constexpr (OP == NEWTON_SCHULZ) newton_schulz_body(a, arg & 1 ? J0 : J1, W, arg & 1 ? J1 : J0, arg, bx, by, sh);
+  if constexpr (OP == NEWTON_APPLY) newton_apply_body(a, Y, Q, J0, J1, K, W, bx, by, sh);
+  if constexpr (OP == NEWTON_COPY) newton_copy_body(a, Y, Q, K, W, bx, nx);
+}
+template <int OP>
+__global__ __launch_bounds__(NEWTON_NT) void newton_kernel(NewtonArgs a, int arg) {
+  newton_body<OP>(a, arg, blockIdx.x, blockIdx.y, gridDim.x);
+}
+template <int OP>
+__global__ __launch_bounds__(NEWTON_NT) void newton_grouped(const GRec<NewtonArgs>* __restrict__ recs, int n, int arg) {
+  unsigned bx, by, bz;
+  const GRec<NewtonArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
+  const NewtonArgs a = r.a;
+  newton_body<OP>(a, arg, bx, by, r.grid.x);
+}
+__global__ __launch_bounds__(NEWTON_NT) void newton_decide(NewtonArgs a, int sweep) {
+  newton_decide_body(a, a.ctrl, sweep);
+}
+__global__ __launch_bounds__(NEWTON_NT) void newton_decide_grouped(const GRec<NewtonArgs>* __restrict__ recs, int sweep) {
+  const NewtonArgs a = recs[blockIdx.x].a;
+  newton_decide_body(a, gbl(a.ctrl), sweep);
 }
 
 // Column norms, descending sort and truncation rank (one workgroup of JAC_NT).
@@ -1044,10 +1355,10 @@ __global__ void jac_check_grouped(const GRec<JacArgs>* __restrict__ recs, int n,
   ctrl->sweeps = sweep + 1;
   if (ctrl->rot[sweep] == 0) ctrl->done = 1;
 }
-// out[i] = done flag of matrix i (one thread per record)
-__global__ void jac_done_gather(const GRec<JacArgs>* __restrict__ recs, int n, int* __restrict__ out) {
+// out[i] = 0: matrix i sweeps, 1: closing phase, 2: converged (one thread per record)
+__global__ void jac_state_gather(const GRec<JacArgs>* __restrict__ recs, int n, int* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = recs[i].a.ctrl->done;
+  if (i < n) out[i] = recs[i].a.ctrl->done ? 2 : recs[i].a.ctrl->phase;
 }
 __global__ __launch_bounds__(JAC_NT) void jac_finalize_grouped(const GRec<FinArgs>* __restrict__ recs, int n) {
   const FinArgs a = recs[blockIdx.x].a;
@@ -1068,15 +1379,64 @@ JacobiLayout jacobi_layout(int rows, int cols) {
   const long L = 2L * l.bs, np = l.nb / 2;
   l.gpart_elems = np * l.kspl * L * L;
   l.j_elems = np * L * L;
-  l.bytes = 256 + sizeof(int) * np + sizeof(c128) * (l.gpart_elems + l.j_elems);
+  l.bytes = JAC_CTRL_BYTES + (sizeof(int) * np + 15) / 16 * 16 + sizeof(c128) * (l.gpart_elems + l.j_elems);
   return l;
 }
 
+// Closing phase of an n-column matrix (preconditioned: n > 32): K, W, J0 and J1,
+// K and W large enough for the new Y and Q, and the per-tile sums.
+size_t newton_bytes(int rows, int n) {
+  const size_t t = ceil_div(n, 16);
+  return 4 * sizeof(c128) * (size_t)rows * n + 16 * t * t;
+}
+
+// Blocks and closing phase of a matrix as it comes or, preconditioned, of the
+// min(rows, cols) columns of R^H.
 size_t jacobi_workspace_bytes(int max_rows, int max_cols) {
-  return jacobi_layout(max_rows, max_cols).bytes + 1024;
+  const int n = std::min(max_rows, max_cols), m = std::max(max_rows, max_cols);
+  return std::max(jacobi_layout(max_rows, max_cols).bytes, jacobi_layout(m, n).bytes) + newton_bytes(m, n) + 1024;
 }
 
 namespace {
+
+NewtonArgs newton_args(c128* Y, int yrows, c128* Q, int qrows, int n, unsigned char* at, const unsigned char* base,
+                       size_t ws_bytes, JacobiCtrl* ctrl, double tol) {
+  NewtonArgs a{};
+  a.Y = Y;
+  a.Q = Q;
+  a.yrows = yrows;
+  a.qrows = qrows;
+  a.n = n;
+  a.ytiles = ceil_div(yrows, 16);
+  a.qtiles = ceil_div(qrows, 16);
+  a.ntiles = ceil_div(n, 16);
+  const long m = (long)std::max(yrows, qrows) * n;
+  a.K = reinterpret_cast<c128*>(at);
+  a.W = a.K + m;
+  a.J0 = a.W + m;
+  a.J1 = a.J0 + m;
+  a.kf2 = reinterpret_cast<double*>(a.J1 + m);
+  a.above = reinterpret_cast<int*>(a.kf2 + (long)a.ntiles * a.ntiles);
+  QCA_CHECK(reinterpret_cast<unsigned char*>(a.above + (long)a.ntiles * a.ntiles) - base <= (long)ws_bytes,
+            "Jacobi workspace too small");
+  a.ctrl = ctrl;
+  a.tol = tol;
+  return a;
+}
+
+// One closing step of one matrix, and the state it leaves.
+void newton_step(const NewtonArgs& a, hipStream_t s) {
+  const dim3 nn(a.ntiles, a.ntiles), t(NEWTON_NT);
+  hipLaunchKernelGGL(newton_kernel<NEWTON_START>, nn, t, 0, s, a, 0);
+  for (int step = 1; step <= NEWTON_SCHULZ_MAX; ++step) {
+    hipLaunchKernelGGL(newton_kernel<NEWTON_GRAM>, nn, t, 0, s, a, step);
+    hipLaunchKernelGGL(newton_kernel<NEWTON_SCHULZ>, nn, t, 0, s, a, step);
+  }
+  hipLaunchKernelGGL(newton_kernel<NEWTON_APPLY>, dim3(a.ytiles + a.qtiles, a.ntiles), t, 0, s, a, 0);
+  hipLaunchKernelGGL(newton_kernel<NEWTON_COPY>, dim3(256), t, 0, s, a, 0);
+  hipLaunchKernelGGL(newton_kernel<NEWTON_CORR>, nn, t, 0, s, a, 1);
+  hipLaunchKernelGGL(newton_decide, dim3(1), t, 0, s, a, -1);
+}
 
 // Gram-based block Jacobi on the columns of Y (rows x cols), the same block
 // rotations applied to the columns of Z (zrows x cols) when Z != null; leaves
@@ -1085,25 +1445,27 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
                         JacobiWork& w) {
   const JacobiLayout l = jacobi_layout(rows, cols);
   QCA_CHECK(l.bytes <= w.ws_bytes, "Jacobi workspace too small");
-  static_assert(sizeof(JacobiCtrl) <= 256, "control block exceeds its slot");
+  static_assert(sizeof(JacobiCtrl) <= JAC_CTRL_BYTES, "control block exceeds its slot");
   unsigned char* base = reinterpret_cast<unsigned char*>(w.ws);
   JacobiCtrl* ctrl = reinterpret_cast<JacobiCtrl*>(base);
-  int* rotated = reinterpret_cast<int*>(base + 256);
-  c128* Gpart = reinterpret_cast<c128*>(base + 256 + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
+  int* rotated = reinterpret_cast<int*>(base + JAC_CTRL_BYTES);
+  c128* Gpart = reinterpret_cast<c128*>(base + JAC_CTRL_BYTES + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
   c128* Jbuf = Gpart + l.gpart_elems;
-  QCA_CHECK((reinterpret_cast<unsigned char*>(Jbuf + l.j_elems) - base) <= (long)w.ws_bytes,
-            "Jacobi workspace too small");
   const JacobiGeom g{rows, cols, l.bs, l.nb, l.kspl};
   const JacobiGeom gz{zrows, cols, l.bs, l.nb, Z ? ceil_div(zrows, JAC_RC) : 0};
   const int np = l.nb / 2;
   const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)rows);
   hipLaunchKernelGGL(jac_init, dim3(1), dim3(JAC_NT), 0, s, Y, (long)rows * cols, ctrl);
-  // launch the sweeps predicted from the previous call, then read the device
-  // flag once per chunk (rounds after convergence are no-ops)
-  int sweep = 0;
+  // Launch the sweeps and closing steps of the previous call, then read the
+  // device's state once per chunk (what is launched beyond it does nothing).
+  const bool closing = Z != nullptr;
+  NewtonArgs na{};
+  if (closing) na = newton_args(Y, rows, Z, zrows, cols, reinterpret_cast<unsigned char*>(Jbuf + l.j_elems), base,
+                                w.ws_bytes, ctrl, tol);
+  int sweep = 0, steps = closing ? std::max(1, w.pred_newton) : 0;
   int& pred = Z ? w.pred_sweeps_pre : w.pred_sweeps;
   int chunk = std::max(2, pred);
-  while (sweep < JAC_MAX_SWEEPS) {
+  while (sweep < JAC_MAX_SWEEPS || steps > 0) {
     for (int c = 0; c < chunk && sweep < JAC_MAX_SWEEPS; ++c, ++sweep) {
       for (int r = 0; r < l.nb - 1; ++r) {
         hipLaunchKernelGGL(jac_gram, dim3(np, l.kspl), dim3(JAC_GRAM_NT), 0, s, (const c128*)Y, g, r,
@@ -1113,17 +1475,27 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
         hipLaunchKernelGGL(jac_apply, dim3(np, l.kspl + gz.kspl), dim3(JAC_APPLY_NT), 0, s, Y, g, Z, gz, r,
                            (const c128*)Jbuf, (const int*)rotated, (const JacobiCtrl*)ctrl);
       }
-      hipLaunchKernelGGL(jac_check, dim3(1), dim3(64), 0, s, ctrl, sweep);
+      if (closing && sweep > 0) {
+        const dim3 nn(na.ntiles, na.ntiles);
+        hipLaunchKernelGGL(newton_kernel<NEWTON_CORR>, nn, dim3(NEWTON_NT), 0, s, na, 0);
+        hipLaunchKernelGGL(newton_decide, dim3(1), dim3(NEWTON_NT), 0, s, na, sweep);
+      } else {
+        hipLaunchKernelGGL(jac_check, dim3(1), dim3(64), 0, s, ctrl, sweep);
+      }
     }
+    for (int q = 0; q < steps; ++q) newton_step(na, s);
     QCA_HIP(hipGetLastError());
-    QCA_HIP(hipMemcpyAsync(w.host, &ctrl->done, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    QCA_HIP(hipMemcpyAsync(w.host, &ctrl->done, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
     QCA_HIP(hipStreamSynchronize(s));
-    const int* hc = reinterpret_cast<const int*>(w.host);
+    const int* hc = reinterpret_cast<const int*>(w.host);   // done, sweeps, phase, newton
     if (hc[0]) {
       pred = hc[1];
+      if (closing) w.pred_newton = hc[3];
       break;
     }
-    chunk = 2;
+    // in the closing phase: more steps; else more sweeps and the steps after them
+    chunk = hc[2] ? 0 : (closing ? 1 : 2);
+    steps = hc[2] ? 1 : (closing && hc[3] < NEWTON_MAX && sweep < JAC_MAX_SWEEPS ? 2 : 0);
   }
   return ctrl;
 }
@@ -1189,7 +1561,9 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   std::vector<GRec<JacArgs>> jac_one, jac_gram_r, jac_inner_r, jac_apply_r;
   std::vector<GRec<FinArgs>> fin;
   std::vector<QrStep> steps;
-  int max_rounds = 0, pred = 2;
+  std::vector<GRec<JacArgs>> jac_plain;                    // without closing phase
+  std::vector<GRec<NewtonArgs>> newton_one, newton_nn, newton_app, newton_cp;
+  int max_rounds = 0, pred = 2, steps_pred = 1;
   for (const SvdJob& j : jobs) {
     QCA_CHECK(j.rows >= 1 && j.rows <= 512, "SVD rows out of range (1..512)");
     QCA_CHECK(j.cols >= 1 && j.cols <= JAC_MAXCOLS, "SVD cols out of range (1..512)");
@@ -1228,8 +1602,8 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     unsigned char* base = reinterpret_cast<unsigned char*>(w.ws);
     JacArgs a{};
     a.ctrl = reinterpret_cast<JacobiCtrl*>(base);
-    a.rotated = reinterpret_cast<int*>(base + 256);
-    a.Gpart = reinterpret_cast<c128*>(base + 256 + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
+    a.rotated = reinterpret_cast<int*>(base + JAC_CTRL_BYTES);
+    a.Gpart = reinterpret_cast<c128*>(base + JAC_CTRL_BYTES + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
     a.Jbuf = a.Gpart + l.gpart_elems;
     a.Y = Y;
     a.g = JacobiGeom{yrows, ycols, l.bs, l.nb, l.kspl};
@@ -1238,6 +1612,17 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     a.tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)yrows);
     const int np = l.nb / 2;
     jac_one.push_back(grec(a, 1));
+    if (pre) {
+      const NewtonArgs na = newton_args(Y, yrows, Z, zrows, ycols, reinterpret_cast<unsigned char*>(a.Jbuf + l.j_elems),
+                                        base, w.ws_bytes, a.ctrl, a.tol);
+      newton_one.push_back(grec(na, 1));
+      newton_nn.push_back(grec(na, na.ntiles, na.ntiles));
+      newton_app.push_back(grec(na, na.ytiles + na.qtiles, na.ntiles));
+      newton_cp.push_back(grec(na, 256));
+      steps_pred = std::max(steps_pred, w.pred_newton);
+    } else {
+      jac_plain.push_back(grec(a, 1));
+    }
     jac_gram_r.push_back(grec(a, np, l.kspl));
     jac_inner_r.push_back(grec(a, np));
     jac_apply_r.push_back(grec(a, np, l.kspl + a.gz.kspl));
@@ -1249,7 +1634,8 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   KGroup<ColOrderArgs> g_order, g_perm;
   KGroup<RhArgs> g_rh;
   KGroup<ScaleArgs> g_scale;
-  KGroup<JacArgs> g_one, g_gram, g_inner, g_apply;
+  KGroup<JacArgs> g_one, g_gram, g_inner, g_apply, g_plain;
+  KGroup<NewtonArgs> n_one, n_nn, n_app, n_cp;
   KGroup<FinArgs> g_fin;
   g_small.prepare(small, arena);
   g_order.prepare(order1, arena);
@@ -1257,6 +1643,11 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   g_rh.prepare(rh, arena);
   g_scale.prepare(scale, arena);
   g_one.prepare(jac_one, arena);
+  g_plain.prepare(jac_plain, arena);
+  n_one.prepare(newton_one, arena);
+  n_nn.prepare(newton_nn, arena);
+  n_app.prepare(newton_app, arena);
+  n_cp.prepare(newton_cp, arena);
   g_gram.prepare(jac_gram_r, arena);
   g_inner.prepare(jac_inner_r, arena);
   g_apply.prepare(jac_apply_r, arena);
@@ -1309,8 +1700,30 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   if (!g_one.empty()) {
     hipLaunchKernelGGL(jac_init_grouped, dim3(g_one.l.blocks), dim3(JAC_NT), 0, s, g_one.l.recs, g_one.l.n);
     const int nj = g_one.l.n;
-    int sweep = 0, chunk = std::max(2, pred);
-    while (sweep < JAC_MAX_SWEEPS) {
+    const dim3 nt(NEWTON_NT);
+    auto check = [&](int sweep) {
+      // sweep 0 never enters the closing phase
+      const KGroup<JacArgs>& c = sweep > 0 ? g_plain : g_one;
+      if (!c.empty())
+        hipLaunchKernelGGL(jac_check_grouped, dim3(c.l.n), dim3(64), 0, s, c.l.recs, c.l.n, sweep);
+      if (sweep > 0 && !n_one.empty()) {
+        hipLaunchKernelGGL(newton_grouped<NEWTON_CORR>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 0);
+        hipLaunchKernelGGL(newton_decide_grouped, dim3(n_one.l.n), nt, 0, s, n_one.l.recs, sweep);
+      }
+    };
+    auto step = [&] {
+      hipLaunchKernelGGL(newton_grouped<NEWTON_START>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 0);
+      for (int q = 1; q <= NEWTON_SCHULZ_MAX; ++q) {
+        hipLaunchKernelGGL(newton_grouped<NEWTON_GRAM>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, q);
+        hipLaunchKernelGGL(newton_grouped<NEWTON_SCHULZ>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, q);
+      }
+      hipLaunchKernelGGL(newton_grouped<NEWTON_APPLY>, dim3(n_app.l.blocks), nt, 0, s, n_app.l.recs, n_app.l.n, 0);
+      hipLaunchKernelGGL(newton_grouped<NEWTON_COPY>, dim3(n_cp.l.blocks), nt, 0, s, n_cp.l.recs, n_cp.l.n, 0);
+      hipLaunchKernelGGL(newton_grouped<NEWTON_CORR>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 1);
+      hipLaunchKernelGGL(newton_decide_grouped, dim3(n_one.l.n), nt, 0, s, n_one.l.recs, -1);
+    };
+    int sweep = 0, chunk = std::max(2, pred), steps = n_one.empty() ? 0 : steps_pred, steps_done = 0;
+    while (sweep < JAC_MAX_SWEEPS || steps > 0) {
       for (int c = 0; c < chunk && sweep < JAC_MAX_SWEEPS; ++c, ++sweep) {
         for (int r = 0; r < max_rounds; ++r) {
           hipLaunchKernelGGL(jac_gram_grouped, dim3(g_gram.l.blocks), dim3(JAC_GRAM_NT), 0, s, g_gram.l.recs,
@@ -1320,16 +1733,22 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
           hipLaunchKernelGGL(jac_apply_grouped, dim3(g_apply.l.blocks), dim3(JAC_APPLY_NT), 0, s, g_apply.l.recs,
                              g_apply.l.n, r);
         }
-        hipLaunchKernelGGL(jac_check_grouped, dim3(nj), dim3(64), 0, s, g_one.l.recs, nj, sweep);
+        check(sweep);
       }
-      hipLaunchKernelGGL(jac_done_gather, dim3(ceil_div(nj, 256)), dim3(256), 0, s, g_one.l.recs, nj, flags.dev);
+      for (int q = 0; q < steps; ++q, ++steps_done) step();
+      hipLaunchKernelGGL(jac_state_gather, dim3(ceil_div(nj, 256)), dim3(256), 0, s, g_one.l.recs, nj, flags.dev);
       QCA_HIP(hipGetLastError());
       QCA_HIP(hipMemcpyAsync(flags.host, flags.dev, sizeof(int) * nj, hipMemcpyDeviceToHost, s));
       QCA_HIP(hipStreamSynchronize(s));
-      bool all = true;
-      for (int i = 0; i < nj; ++i) all = all && flags.host[i] != 0;
-      if (all) break;
-      chunk = 2;
+      bool sweeping = false, closing = false;
+      for (int i = 0; i < nj; ++i) {
+        sweeping = sweeping || flags.host[i] == 0;
+        closing = closing || flags.host[i] == 1;
+      }
+      if (!sweeping && !closing) break;
+      // a matrix takes at most NEWTON_MAX closing steps, wherever its sweeps end
+      chunk = sweeping ? 1 : 0;
+      steps = n_one.empty() ? 0 : (closing ? 1 : (steps_done < 2 * NEWTON_MAX ? 2 : 0));
     }
     hipLaunchKernelGGL(jac_finalize_grouped, dim3(g_fin.l.blocks), dim3(JAC_NT), 0, s, g_fin.l.recs, g_fin.l.n);
     if (!g_scale.empty())

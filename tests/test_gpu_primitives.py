@@ -203,6 +203,43 @@ def test_svd_split(gpu, right, chil, chir, chi_max, eps):
     assert np.abs(I - np.eye(kk)).max() < max(1e-13, 2 * n * np.finfo(float).eps)
 
 
+@pytest.mark.parametrize("spectrum", ["flat", "pairs", "steps"])
+@pytest.mark.parametrize("chil,chir,right", [(17, 17, 1), (24, 24, 0), (24, 25, 1), (40, 25, 0), (45, 77, 0),
+                                             (64, 65, 1), (128, 128, 0), (200, 20, 1)])
+def test_svd_split_closing_steps(gpu, spectrum, chil, chir, right):
+    """Splits whose last sweeps are products on the matrix cores, at column counts
+    around the 16-column tiles (34..256): a flat spectrum (all pairs close),
+    pairs 1e-6 apart and degenerate plateaus 1e-2 apart, against LAPACK within
+    the bounds of test_svd_split."""
+    import torch
+    rng = np.random.default_rng(chil * 3 + chir + right)
+    m, n = 2 * chil, 2 * chir
+    U, _ = np.linalg.qr(crand(rng, m, min(m, n)))
+    V, _ = np.linalg.qr(crand(rng, n, min(m, n)))
+    i = np.arange(min(m, n))
+    s = {"flat": 1 + 0.01 * i / len(i), "pairs": 0.93 ** (i // 2) * (1 + 1e-6 * (i % 2)),
+         "steps": 10.0 ** (-2 * (i // (len(i) // 4 + 1)))}[spectrum]
+    M = (U * s) @ V.conj().T
+    M /= np.linalg.norm(M)
+    ref = np.linalg.svd(M, compute_uv=False)
+    th = dev(torch, M.reshape(2, chil, 2, chir).transpose(0, 2, 1, 3).reshape(4, chil, chir), np.complex128)
+    kmax = min(m, n)
+    Al = torch.zeros(2 * chil * kmax, dtype=torch.complex128, device="cuda")
+    Ar = torch.zeros(2 * kmax * chir, dtype=torch.complex128, device="cuda")
+    k = ctypes.c_int(0)
+    sig = np.zeros(kmax)
+    qn.call("qca_svd_split", qn.ptr(th), qn.ptr(Al), qn.ptr(Ar), chil, chir, kmax, 1e-10, right,
+            ctypes.byref(k), sig.ctypes.data, None)
+    kk = k.value
+    assert kk == LOC.truncation_rank(ref, kmax, 1e-10)
+    assert np.abs(sig - ref).max() < 1e-13
+    A = Al[: m * kk].cpu().numpy().reshape(m, kk)
+    B = Ar[: n * kk].cpu().numpy().reshape(2, kk, chir).transpose(1, 0, 2).reshape(kk, n)
+    Q = A if right else B.conj().T
+    assert np.abs(Q.conj().T @ Q - np.eye(kk)).max() < max(1e-13, 2 * len(Q) * np.finfo(float).eps)
+    assert np.abs(A @ B - M).max() < 1e-12
+
+
 @pytest.mark.parametrize("side", [0, 1])
 @pytest.mark.parametrize("chil,chir,target", [(1, 1, 2), (2, 2, 4), (4, 8, 8), (8, 8, 8), (32, 32, 32),
                                               (8, 4, 4), (16, 64, 32), (128, 256, 256)])
