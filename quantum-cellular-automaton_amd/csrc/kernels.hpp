@@ -172,7 +172,8 @@ struct SvdResult {
   double tail;        // ||s[k:]||
 };
 
-// Workspace of the Jacobi SVD: device memory of at least
+// Workspace of the Jacobi SVD (a matrix for which small_svd holds needs none of
+// it but a non-null ws): device memory of at least
 // jacobi_workspace_bytes(rows, cols) (control block, partial Grams, block
 // rotations, matrices of the closing phase), 16 bytes of pinned host memory, and
 // the sweep and closing-step counts of the previous call (the number launched
@@ -181,13 +182,11 @@ struct JacobiWork {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   void* host = nullptr;
-  int pred_sweeps = 8;
-  // QR preconditioning (matrices wider than 32 columns): at least
-  // jacobi_precond_elems(rows, cols) complex128, or null to skip it
+  int pred_sweeps = 4;
+  int pred_newton = 3;
+  // QR preconditioning: at least jacobi_precond_elems(rows, cols) complex128
   c128* pre = nullptr;
   size_t pre_elems = 0;
-  int pred_sweeps_pre = 4;
-  int pred_newton = 3;      // closing steps of the previous call
   // rotation threshold relative to the column norms; 0: eps * sqrt(rows)
   double tol = 0;
 };
@@ -200,6 +199,8 @@ struct JacobiLayout {
 JacobiLayout jacobi_layout(int rows, int cols);
 size_t jacobi_workspace_bytes(int max_rows, int max_cols);
 size_t jacobi_precond_elems(int max_rows, int max_cols);
+// One workgroup takes the whole SVD.
+bool small_svd(int rows, int cols);
 
 // One-sided (block) Jacobi SVD of the column-major matrix X (rows x cols,
 // FP64), in place.  On exit the columns are orthogonal; sigma (sorted

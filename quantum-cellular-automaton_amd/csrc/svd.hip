@@ -30,6 +30,7 @@
 // the truncation rank (first i with ||s[i:]|| < eps, capped; reference
 // algorithms/tdvp.py:289-292).
 #include "grouped.hpp"
+#include "larfg.hpp"
 #include "wave.hpp"
 
 #include <algorithm>
@@ -216,140 +217,6 @@ __global__ __launch_bounds__(JAC_GRAM_NT) void jac_gram(const c128* __restrict__
                                                    int round, c128* __restrict__ Gpart,
                                                    const JacobiCtrl* __restrict__ ctrl) {
   jac_gram_body(X, g, round, Gpart, ctrl, blockIdx.x, blockIdx.y);
-}
-
-// One cyclic sweep of two-sided Jacobi on the Gram of pair blockIdx.x.
-// Rotation of columns (i, j), with g = G(i, j) = x_i^H x_j, d = |x_j|^2 - |x_i|^2,
-// h = sqrt(d^2 + 4|g|^2), w = h + |d|:
-//   x_i' = c x_i - conj(s e) x_j,   x_j' = (s e) x_i + c x_j,
-//   c = sqrt(w / (2h)),  s e = sign(d) g sqrt(2 / (h w)),
-// the Rutishauser rotation t = sign(d)/(|zeta| + sqrt(1 + zeta^2)), zeta = d/(2|g|),
-// c = 1/sqrt(1 + t^2), s = t c, rewritten so that c^2 + |s e|^2 = 1 exactly in
-// real arithmetic on non-negative operands; c and |s| are evaluated as w y and
-// 2 y with y = 1/sqrt(2hw), so the critical path is sqrt -> rsqrt.
-// G <- R^H G R and J <- J R.
-// Per round: wave 0 computes the rotations of round r while the other waves
-// apply round r-1 to J; after a barrier all threads apply round r to G.
-// The pair indices are recomputed in registers, the rotation of a pair is one
-// 32-byte LDS record.
-struct alignas(16) JRot {
-  double c, sr, si;   // c, s e
-  int act, pad;
-};
-static_assert(JAC_NT >= 64 + JAC_LMAX * (JAC_LMAX / 2), "jac_inner needs one thread per J item");
-static_assert(JAC_NT >= (JAC_LMAX / 2) * (JAC_LMAX / 2), "jac_inner needs one thread per G block");
-
-// Round-robin position rr_player(t, r, n) without integer division (t < n, r < n - 1).
-__device__ __forceinline__ int rr_fast(int t, int r, int n) {
-  if (t == 0) return 0;
-  int x = t - 1 + r;
-  x -= (x >= n - 1) ? (n - 1) : 0;
-  return x + 1;
-}
-// Pair t of inner round r.  Full ordering: the round-robin tournament over all
-// L = 2H columns (L - 1 rounds, every pair once).  Cross ordering: column t of
-// the first block meets column H + (t + r) mod H of the second (H rounds, only
-// the pairs across the two blocks).
-template <bool CROSS>
-__device__ __forceinline__ int pair_first(int t, int r, int L) {
-  return CROSS ? t : rr_fast(t, r, L);
-}
-template <bool CROSS>
-__device__ __forceinline__ int pair_second(int t, int r, int L) {
-  if (!CROSS) return rr_fast(L - 1 - t, r, L);
-  const int H = L >> 1;
-  int x = t + r;
-  x -= (x >= H) ? H : 0;
-  return H + x;
-}
-// One cyclic sweep of the rotations on G (L x L, column-major, in LDS),
-// accumulating J <- J R; rot is a 2 x (L/2) LDS scratch.  CROSS restricts the
-// sweep to the pairs across the two halves (see pair_first).  Needs blockDim.x
-// == JAC_NT and G, J visible to the whole workgroup on entry (it ends with a
-// barrier).  Returns the rotations this thread computed.
-template <bool CROSS>
-__device__ int inner_sweep(c128* G, c128* J, JRot (*rot)[JAC_LMAX / 2], int L, int H, double tol2,
-                           double conv2, double negl) {
-  const int tid = threadIdx.x;
-  const int NR = CROSS ? H : L - 1;
-  int mine = 0;
-  // fixed roles: lanes < H of wave 0 compute the rotations; threads 64.. own
-  // one J item (row r, pair Q) each; threads < H*H own one 2x2 block of G
-  const int jit = tid - 64;
-  const bool has_j = jit >= 0 && jit < L * H;
-  const int jr = has_j ? jit % L : 0, jq = has_j ? jit / L : 0;
-  const bool has_g = tid < H * H;
-  const int gP = tid % H, gQ = tid / H;
-  for (int round = 0; round <= NR; ++round) {
-    const int cur = round & 1, prev = cur ^ 1;
-    if (tid < 64) {
-      if (round < NR && tid < H) {
-        const int i = pair_first<CROSS>(tid, round, L), j = pair_second<CROSS>(tid, round, L);
-        const double a = G[i * L + i].re, b = G[j * L + j].re;
-        const c128 gij = G[j * L + i];
-        const double ag2 = gij.re * gij.re + gij.im * gij.im;
-        // a pair with a column at the noise floor is done: rotating noise
-        // against a signal column only re-creates noise, and for matrices with
-        // more columns than rows such pairs can rotate indefinitely
-        const int act = !(ag2 <= tol2 * a * b || ag2 < 1e-300 || fmin(a, b) < negl);
-        JRot q{1.0, 0.0, 0.0, act, 0};
-        if (act) {
-          const double d = b - a;
-          const double h = sqrt(d * d + 4.0 * ag2);
-          const double w = h + fabs(d);
-          // c = sqrt(w / 2h) = w y and |s| = sqrt(2 / hw) = 2 y with y =
-          // 1/sqrt(2hw): one reciprocal square root in place of two divides
-          // and two square roots on the serial path of the round.  Hardware
-          // estimate, two Newton steps, and a last one whose residual
-          // 1 - t y^2 includes the exact error of t y, so that y carries no
-          // bias (c and s share y: a biased y drifts the column norms)
-          const double t = 2.0 * h * w;
-          double y = __builtin_amdgcn_rsq(t);
-          y = y * fma(-0.5 * t * y, y, 1.5);
-          y = y * fma(-0.5 * t * y, y, 1.5);
-          const double ty = t * y;
-          const double e = fma(-ty, y, 1.0) - fma(t, y, -ty) * y;
-          y = fma(0.5 * y, e, y);
-          q.c = w * y;
-          const double s = (d >= 0 ? 2.0 : -2.0) * y;
-          q.sr = s * gij.re;
-          q.si = s * gij.im;
-          // low half: rotations applied; high half: rotations above the
-          // convergence threshold, which keep the sweeps going
-          mine += ag2 > conv2 * a * b ? 0x10001 : 1;
-        }
-        rot[cur][tid] = q;
-      }
-    } else if (round > 0 && has_j) {
-      const int qi = pair_first<CROSS>(jq, round - 1, L), qj = pair_second<CROSS>(jq, round - 1, L);
-      const c128 x = J[qi * L + jr], y = J[qj * L + jr];
-      const JRot Q = rot[prev][jq];
-      if (Q.act) {
-        J[qi * L + jr] = c128{Q.c * x.re - (Q.sr * y.re + Q.si * y.im), Q.c * x.im - (Q.sr * y.im - Q.si * y.re)};
-        J[qj * L + jr] = c128{(Q.sr * x.re - Q.si * x.im) + Q.c * y.re, (Q.sr * x.im + Q.si * x.re) + Q.c * y.im};
-      }
-    }
-    __syncthreads();
-    if (round == NR) break;
-    if (has_g) {
-      const int pi = pair_first<CROSS>(gP, round, L), pj = pair_second<CROSS>(gP, round, L);
-      const int qi = pair_first<CROSS>(gQ, round, L), qj = pair_second<CROSS>(gQ, round, L);
-      const c128 t00 = G[qi * L + pi], t10 = G[qi * L + pj], t01 = G[qj * L + pi], t11 = G[qj * L + pj];
-      const JRot P = rot[cur][gP], Q = rot[cur][gQ];
-      if (P.act || Q.act) {
-        const c128 u00{Q.c * t00.re - (Q.sr * t01.re + Q.si * t01.im), Q.c * t00.im - (Q.sr * t01.im - Q.si * t01.re)};
-        const c128 u10{Q.c * t10.re - (Q.sr * t11.re + Q.si * t11.im), Q.c * t10.im - (Q.sr * t11.im - Q.si * t11.re)};
-        const c128 u01{(Q.sr * t00.re - Q.si * t00.im) + Q.c * t01.re, (Q.sr * t00.im + Q.si * t00.re) + Q.c * t01.im};
-        const c128 u11{(Q.sr * t10.re - Q.si * t10.im) + Q.c * t11.re, (Q.sr * t10.im + Q.si * t10.re) + Q.c * t11.im};
-        G[qi * L + pi] = c128{P.c * u00.re - (P.sr * u10.re - P.si * u10.im), P.c * u00.im - (P.sr * u10.im + P.si * u10.re)};
-        G[qi * L + pj] = c128{(P.sr * u00.re + P.si * u00.im) + P.c * u10.re, (P.sr * u00.im - P.si * u00.re) + P.c * u10.im};
-        G[qj * L + pi] = c128{P.c * u01.re - (P.sr * u11.re - P.si * u11.im), P.c * u01.im - (P.sr * u11.im + P.si * u11.re)};
-        G[qj * L + pj] = c128{(P.sr * u01.re + P.si * u01.im) + P.c * u11.re, (P.sr * u01.im - P.si * u01.re) + P.c * u11.im};
-      }
-    }
-    __syncthreads();
-  }
-  return mine;
 }
 
 // Rotations of one Jacobi sweep on the Gram G of 2 x 16 columns held in
@@ -667,11 +534,13 @@ __global__ __launch_bounds__(JAC_APPLY_NT) void jac_apply(c128* __restrict__ Xa,
 }
 
 // Closes a sweep: converged when it made no rotation.
-__global__ void jac_check(JacobiCtrl* __restrict__ ctrl, int sweep) {
+__device__ __forceinline__ void jac_check_body(JacobiCtrl* __restrict__ ctrl) {
   if (threadIdx.x != 0 || ctrl->done) return;
-  ctrl->sweeps = sweep + 1;
-  if (ctrl->rot[sweep] == 0) ctrl->done = 1;
+  ctrl->sweeps = 1;
+  if (ctrl->rot[0] == 0) ctrl->done = 1;
 }
+// After sweep 0.
+__global__ void jac_check(JacobiCtrl* __restrict__ ctrl) { jac_check_body(ctrl); }
 
 // ------------------------------------------------------------------ closing phase
 // Once the columns of Y are nearly orthogonal, all pairs are rotated at once:
@@ -1050,100 +919,455 @@ __global__ __launch_bounds__(JAC_NT) void jac_finalize(const c128* __restrict__ 
   finalize_body(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, ctrl->sweeps, ctrl->done);
 }
 
-// The whole SVD of a matrix with at most JAC_LMAX columns in one workgroup:
-// sweeps of (Gram from the columns -> one rotation sweep on it -> X <- X J)
-// until a sweep makes no rotation, then finalize_body.  Same rotations, test
-// and accuracy as the kernel triple, without launches between rounds.
-__device__ __forceinline__ void jac_small_body(c128* __restrict__ X, int rows, int cols,
-                                               double* __restrict__ sigma, int* __restrict__ perm,
-                                               SvdResult* __restrict__ res, int chi_max, double eps,
-                                               int rank_cap, double tol) {
-  constexpr int HM = JAC_LMAX / 2;
-  __shared__ c128 tile[JAC_RC * (JAC_LMAX + 1)];
-  __shared__ c128 G[JAC_LMAX * JAC_LMAX];
-  __shared__ c128 J[JAC_LMAX * JAC_LMAX];
-  __shared__ JRot rot[2][HM];
-  __shared__ double red[JAC_NT / 64];
-  __shared__ int total, total_sig;
-  const int tid = threadIdx.x;
-  const int H = (cols + 1) / 2, L = 2 * H;
-  const double conv = jac_conv_tol(tol, rows);
-  double part = 0;
-  part = strided_norm2(X, (long)rows * cols, tid, JAC_NT);
-  part = wsum(part);
-  if ((tid & 63) == 0) red[tid >> 6] = part;
+// ------------------------------------------------------------------ small matrices
+// The whole SVD of a matrix with min(rows, cols) <= 32 and max(rows, cols) <= 128
+// in one workgroup of four waves.  One-sided Jacobi on the columns of X takes 6
+// to 19 sweeps on the graded spectra of a TDVP split; on the triangle of a
+// pivoted QR it takes one to four, so:
+//   rows >= cols:  X P1 = Q1 R1,  R1^H P2 = Q2 R2,  Y = R2^H,  X <- Q1 P2 (Y J)
+//   rows <  cols:  X^H P1 = Q1 R1,  Y = R1^H,  X <- P1 (Y J)
+// (P: columns by descending norm; Y is at most 32x32).  Y J has orthogonal
+// columns U S, so neither J nor Q2 is needed.  A sweep is that of jac_inner on
+// the Gram of Y; from |K|_F <= NEWTON_KF on, closing steps as above follow.
+// A QR keeps the matrix in registers, column c in the 8 lanes of its group and
+// its rows c' = lane, lane + 8, ...: a reduction is three DPP moves and a
+// column one barrier (0.6 us at 32 rows).  What bounds the kernel is the chain
+// of rounds and reflectors.  32x32, graded over eight decades: load and order 1
+// us, QR 19 + 20, two sweeps 42 + 10 (rounds, products), four closing steps 34, Q1
+// 5, norms and rank 3; a split of that size in all 721 -> 256 us, 24x32 647 ->
+// 246, 60x30 531 -> 265.  Without the second QR 54 us more sweeps, for 25 of QR
+// and Q1.  Rows beyond 128 (register columns) take the launches below.
+constexpr int SMALL_NT = 256;
+constexpr int SMALL_ROWS = 128;
+constexpr int SMALL_LDV = SMALL_ROWS + 1;
+constexpr int SMALL_LD = JAC_LMAX + 1;
+constexpr int SMALL_M = JAC_LMAX * SMALL_LD;   // element (r, c) at c * SMALL_LD + r
+
+struct SmallShared {
+  c128 V[JAC_LMAX * SMALL_LDV];   // columns on their way into order, then the reflectors of Q1
+  c128 Y[SMALL_M], G[SMALL_M], J0[SMALL_M];
+  union {
+    c128 m[2][SMALL_M];           // J1 and W of a closing step; reflectors of Q2
+    InnerShared inner;
+  };
+  c128 tau[JAC_LMAX], tau2[JAC_LMAX];
+  double key[JAC_LMAX], sorted[JAC_LMAX];
+  int rank[JAC_LMAX];
+  double red[SMALL_NT / 64];
+  int cnt[SMALL_NT / 64];
+};
+
+// Sum over the 8 lanes of a group, the same value in each.
+__device__ __forceinline__ double sum8(double v) {
+  v += dpp_f64<0xB1>(v);    // quad_perm(1,0,3,2)
+  v += dpp_f64<0x4E>(v);    // quad_perm(2,3,0,1)
+  v += dpp_f64<0x141>(v);   // row_half_mirror
+  return v;
+}
+
+// Position of key[c] (c = thread / 8) among the 32 keys, largest first.  Keys are
+// compared as bit patterns (they are not negative), which orders NaN too: the
+// positions are a permutation whatever the keys are.
+__device__ __forceinline__ int small_rank(const double* key) {
+  const int c = threadIdx.x >> 3, rl = threadIdx.x & 7;
+  const unsigned long long mine = __builtin_bit_cast(unsigned long long, key[c]);
+  int rank = 0;
+#pragma unroll
+  for (int i = 0; i < JAC_LMAX / 8; ++i) {
+    const int o = rl + 8 * i;
+    const unsigned long long other = __builtin_bit_cast(unsigned long long, key[o]);
+    const unsigned long long b = __ballot(other > mine || (other == mine && o < c));
+    rank += __popc((unsigned)(b >> (threadIdx.x & 56)) & 0xffu);
+  }
+  return rank;
+}
+
+template <int IT>
+__device__ __forceinline__ double small_norm2(const c128 (&x)[IT]) {
+  double s = 0;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) s += x[i].re * x[i].re + x[i].im * x[i].im;
+  return sum8(s);
+}
+
+// Sorts the columns (by `stage`, stride ld) by descending norm; rank[c] is where
+// column c went.
+template <int IT>
+__device__ __forceinline__ void small_sort(c128 (&x)[IT], SmallShared& sh, c128* stage, int ld) {
+  const int c = threadIdx.x >> 3, rl = threadIdx.x & 7;
+  const double n2 = small_norm2(x);
+  if (rl == 0) sh.key[c] = n2;
   __syncthreads();
-  double fro = 0;
-  for (int w = 0; w < JAC_NT / 64; ++w) fro += red[w];
-  const double negl = JAC_NOISE2 * fro;
-  const JacobiGeom g{rows, cols, H, 2, 1};  // one block pair: columns 0..H-1 and H..L-1
-  int sweep = 0, converged = 0;
-  for (; sweep < JAC_MAX_SWEEPS; ++sweep) {
-    // Gram from the current columns, 64-row chunks through the tile
-    double gre = 0, gim = 0;
-    const int gi = tid % L, gj = tid / L;
-    for (int r0 = 0; r0 < rows; r0 += JAC_RC) {
-      const int nr = min(JAC_RC, rows - r0);
-      __syncthreads();
-      stage_tile<JAC_NT>(X, g, 0, 0, r0, nr, tile);
-      __syncthreads();
-      if (tid < L * L)
-        for (int r = 0; r < nr; ++r) {
-          const c128 u = tile[r * (JAC_LMAX + 1) + gi], v = tile[r * (JAC_LMAX + 1) + gj];
-          gre += u.re * v.re + u.im * v.im;
-          gim += u.re * v.im - u.im * v.re;
-        }
-    }
-    if (tid < L * L) {
-      G[tid] = c128{gre, gim};
-      J[tid] = c128{gi == gj ? 1.0 : 0.0, 0.0};
-    }
-    if (tid == 0) {
-      total = 0;
-      total_sig = 0;
-    }
-    __syncthreads();
-    const int mine = inner_sweep<false>(G, J, rot, L, H, tol * tol, conv * conv, negl);
-    if (mine & 0xffff) atomicAdd(&total, mine & 0xffff);
-    if (mine >> 16) atomicAdd(&total_sig, mine >> 16);
-    __syncthreads();
-    if (total == 0) {
-      converged = 1;
-      break;
-    }
-    // X <- X J, chunk by chunk (each chunk is read into the tile before it is written)
-    for (int r0 = 0; r0 < rows; r0 += JAC_RC) {
-      const int nr = min(JAC_RC, rows - r0);
-      stage_tile<JAC_NT>(X, g, 0, 0, r0, nr, tile);
-      __syncthreads();
-      const int r = tid & 63;
-      if (r < nr)
-        for (int c = tid >> 6; c < cols; c += JAC_NT / 64) {
-          double re = 0, im = 0;
-          for (int k = 0; k < L; ++k) {
-            const c128 x = tile[r * (JAC_LMAX + 1) + k], jj = J[c * L + k];
-            re += x.re * jj.re - x.im * jj.im;
-            im += x.re * jj.im + x.im * jj.re;
+  const int rank = small_rank(sh.key);
+  if (rl == 0) sh.rank[c] = rank;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) stage[rank * ld + rl + 8 * i] = x[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < IT; ++i) x[i] = stage[c * ld + rl + 8 * i];
+}
+
+// Householder QR of the columns in x: kq reflectors, to V (column k at k * ld,
+// valid from row 8 (k / 8) on) and tau; x becomes (R, v).  The slot of a
+// reflector is written by the lanes that read that column of the stage, so V may
+// be the stage of small_sort.
+template <int IT>
+__device__ __forceinline__ void small_qr(c128 (&x)[IT], int kq, c128* V, int ld, c128* tau) {
+  const int c = threadIdx.x >> 3, rl = threadIdx.x & 7;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int i0 = 0; i0 < JAC_LMAX / 8; ++i0) {
+#pragma unroll 1
+    for (int k8 = 0; k8 < 8; ++k8) {
+      const int k = 8 * i0 + k8;
+      if (k >= kq) return;
+      if (wave == i0) {   // columns 8 i0 .. 8 i0 + 7
+        double n2 = rl > k8 ? x[i0].re * x[i0].re + x[i0].im * x[i0].im : 0.0;
+#pragma unroll
+        for (int i = i0 + 1; i < IT; ++i) n2 += x[i].re * x[i].re + x[i].im * x[i].im;
+        n2 = sum8(n2);
+        const double ar = sum8(rl == k8 ? x[i0].re : 0.0), ai = sum8(rl == k8 ? x[i0].im : 0.0);
+        const Larfg h = larfg(c128{ar, ai}, n2);
+        if (c == k) {
+#pragma unroll
+          for (int i = i0; i < IT; ++i) {
+            const c128 s{x[i].re * h.scale.re - x[i].im * h.scale.im, x[i].re * h.scale.im + x[i].im * h.scale.re};
+            if (i > i0) {
+              x[i] = s;
+              V[k * ld + rl + 8 * i] = s;
+            } else {
+              V[k * ld + rl + 8 * i] = rl > k8 ? s : c128{rl == k8 ? 1.0 : 0.0, 0.0};
+              if (rl > k8) x[i] = s;
+              if (rl == k8) x[i] = c128{h.beta, 0.0};
+            }
           }
-          X[(long)c * rows + r0 + r] = c128{re, im};
+          if (rl == 0) tau[k] = h.tau;
         }
+      }
       __syncthreads();
+      if (c > k) {
+        c128 v[IT];
+        double dr = 0, di = 0;
+        const c128 t = tau[k];
+#pragma unroll
+        for (int i = i0; i < IT; ++i) v[i] = V[k * ld + rl + 8 * i];
+#pragma unroll
+        for (int i = i0; i < IT; ++i) {
+          dr += v[i].re * x[i].re + v[i].im * x[i].im;
+          di += v[i].re * x[i].im - v[i].im * x[i].re;
+        }
+        dr = sum8(dr);
+        di = sum8(di);
+        const double fr = t.re * dr + t.im * di, fi = t.re * di - t.im * dr;
+#pragma unroll
+        for (int i = i0; i < IT; ++i) {
+          x[i].re -= v[i].re * fr - v[i].im * fi;
+          x[i].im -= v[i].re * fi + v[i].im * fr;
+        }
+      }
     }
-    if (total_sig == 0) {
-      converged = 1;
-      break;
+  }
+}
+
+// z <- H_0 ... H_{kq-1} z for the columns in z.
+template <int IT>
+__device__ __forceinline__ void small_apply_q(c128 (&z)[IT], int kq, const c128* V, int ld, const c128* tau) {
+  const int rl = threadIdx.x & 7;
+#pragma unroll
+  for (int i0 = JAC_LMAX / 8 - 1; i0 >= 0; --i0) {
+#pragma unroll 1
+    for (int k = min(8 * i0 + 7, kq - 1); k >= 8 * i0; --k) {
+      c128 v[IT];
+      double dr = 0, di = 0;
+      const c128 t = tau[k];
+#pragma unroll
+      for (int i = i0; i < IT; ++i) v[i] = V[k * ld + rl + 8 * i];
+#pragma unroll
+      for (int i = i0; i < IT; ++i) {
+        dr += v[i].re * z[i].re + v[i].im * z[i].im;
+        di += v[i].re * z[i].im - v[i].im * z[i].re;
+      }
+      dr = sum8(dr);
+      di = sum8(di);
+      const double fr = t.re * dr - t.im * di, fi = t.re * di + t.im * dr;
+#pragma unroll
+      for (int i = i0; i < IT; ++i) {
+        z[i].re -= v[i].re * fr - v[i].im * fi;
+        z[i].im -= v[i].re * fi + v[i].im * fr;
+      }
+    }
+  }
+}
+
+// This wave's 16x16 tile (wave & 1, wave / 2) of op(A) B of matrices in LDS,
+// inner dimension kd (16 or 32), handed to out(row, col, value).
+template <bool ADJOINT, typename Out>
+__device__ __forceinline__ void small_mm(const c128* A, const c128* B, int kd, Out&& out) {
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i0 = 16 * (wave & 1), j0 = 16 * (wave >> 1);
+  if (i0 >= kd || j0 >= kd) return;
+  jac_f64x4 re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+  for (int k0 = 0; k0 < kd; k0 += 16) {
+    c128 a[4], b[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = k0 + 4 * s + hi;
+      a[s] = ADJOINT ? conj_of(A[(i0 + lo) * SMALL_LD + k]) : A[k * SMALL_LD + i0 + lo];
+      b[s] = B[(j0 + lo) * SMALL_LD + k];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      re = jac_mfma(a[s].re, b[s].re, re);
+      im = jac_mfma(a[s].re, b[s].im, im);
+      re = jac_mfma(-a[s].im, b[s].im, re);
+      im = jac_mfma(a[s].im, b[s].re, im);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) out(i0 + hi + 4 * r, j0 + lo, c128{re[r], im[r]});
+}
+
+// Y <- Y J, G <- Y^H Y.
+__device__ __forceinline__ void small_update(SmallShared& sh, const c128* J, int kd) {
+  c128 y[4];
+  int n = 0, at[4] = {-1, -1, -1, -1};
+  small_mm<false>(sh.Y, J, kd, [&](int r, int c, const c128& v) {
+    y[n] = v;
+    at[n++] = c * SMALL_LD + r;
+  });
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (at[q] >= 0) sh.Y[at[q]] = y[q];
+  __syncthreads();
+}
+__device__ __forceinline__ void small_gram(SmallShared& sh, int kd) {
+  small_mm<true>(sh.Y, sh.Y, kd, [&](int r, int c, const c128& v) { sh.G[c * SMALL_LD + r] = v; });
+  __syncthreads();
+}
+
+// K of the Gram (to m[0]); |K|_F^2 and the pairs above the convergence margin.
+__device__ __forceinline__ void small_corr(SmallShared& sh, int kq, const InnerThresholds& th, double& kf, int& above) {
+  c128* K = sh.m[0];
+  double part = 0;
+  int sig = 0;
+#pragma unroll
+  for (int q = 0; q < JAC_LMAX * JAC_LMAX / SMALL_NT; ++q) {
+    const int i = threadIdx.x & 31, j = (threadIdx.x >> 5) + 8 * q;
+    const int a = min(i, j), b = max(i, j);
+    const c128 g = sh.G[b * SMALL_LD + a];
+    const double pa = sh.G[a * SMALL_LD + a].re, pb = sh.G[b * SMALL_LD + b].re;
+    const double ag2 = g.re * g.re + g.im * g.im, ab = pa * pb, d = pb - pa;
+    const bool act = a < b && b < kq && !(ag2 <= th.tol2 * ab || ag2 < 1e-300 || fmin(pa, pb) < th.negl);
+    const double t = act ? (d >= 0 ? 2.0 : -2.0) / (sqrt(fma(d, d, 4.0 * ag2)) + fabs(d)) : 0.0;
+    const c128 k = act ? c128{i < j ? t * g.re : -t * g.re, t * g.im} : c128{0.0, 0.0};
+    K[j * SMALL_LD + i] = k;
+    part += k.re * k.re + k.im * k.im;
+    sig += __popcll(__ballot(act && i < j && ag2 > th.conv2 * ab));
+  }
+  part = wave_sum64(part);
+  if ((threadIdx.x & 63) == 0) {
+    sh.red[threadIdx.x >> 6] = part;
+    sh.cnt[threadIdx.x >> 6] = sig;
+  }
+  __syncthreads();
+  kf = (sh.red[0] + sh.red[1]) + (sh.red[2] + sh.red[3]);
+  above = (sh.cnt[0] + sh.cnt[1]) + (sh.cnt[2] + sh.cnt[3]);
+}
+
+// One-sided Jacobi on the columns of Y (kq of them, zero elsewhere); returns
+// whether they are orthogonal, and the sweeps it took.
+__device__ __forceinline__ bool small_jacobi(SmallShared& sh, int kq, const InnerThresholds& th, int& sweeps) {
+  const int P = threadIdx.x >> 4, Q = (threadIdx.x + P) & 15;
+  const int kd = kq > 16 ? 32 : 16;
+  int h0 = 16;   // pairs of the first rounds: half the columns
+  while (h0 > 1 && kq <= h0) h0 >>= 1;
+  const int iP = (P / h0) * 2 * h0 + P % h0, iQ = (Q / h0) * 2 * h0 + Q % h0;
+  int steps = 0;
+  small_gram(sh, kd);
+  for (sweeps = 0; sweeps < JAC_MAX_SWEEPS;) {
+    c128 g[4], j[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = iP + h0 * (q / 2), c = iQ + h0 * (q & 1);
+      g[q] = r < kd && c < kd ? sh.G[c * SMALL_LD + r] : c128{0.0, 0.0};
+      j[q] = c128{P + 16 * (q / 2) == c ? 1.0 : 0.0, 0.0};
+    }
+    int total = 0, above = 0;
+    if (h0 == 16) {
+      inner_rounds<16>(g, j, sh.inner, th, total, above);
+      inner_regroup<16>(g, j, sh.inner);
+    }
+    if (h0 >= 8) {
+      inner_rounds<8>(g, j, sh.inner, th, total, above);
+      inner_regroup<8>(g, j, sh.inner);
+    }
+    if (h0 >= 4) {
+      inner_rounds<4>(g, j, sh.inner, th, total, above);
+      inner_regroup<4>(g, j, sh.inner);
+    }
+    if (h0 >= 2) {
+      inner_rounds<2>(g, j, sh.inner, th, total, above);
+      inner_regroup<2>(g, j, sh.inner);
+    }
+    inner_rounds<1>(g, j, sh.inner, th, total, above);
+    ++sweeps;
+    // the counts of one wave decide for all
+    if (threadIdx.x == 0) {
+      sh.cnt[0] = total;
+      sh.cnt[1] = above;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sh.J0[(2 * Q + (q & 1)) * SMALL_LD + P + 16 * (q / 2)] = j[q];
+    __syncthreads();
+    total = sh.cnt[0];
+    above = sh.cnt[1];
+    if (total == 0) return true;
+    small_update(sh, sh.J0, kd);
+    if (above == 0) return true;
+    small_gram(sh, kd);
+    double kf;
+    small_corr(sh, kq, th, kf, above);
+    for (; kf <= NEWTON_KF * NEWTON_KF && steps < NEWTON_MAX; ++steps) {
+      c128 *K = sh.m[0], *W = sh.m[1];
+      small_mm<true>(K, K, kd, [&](int r, int c, const c128& v) {
+        const c128 k = K[c * SMALL_LD + r];
+        sh.J0[c * SMALL_LD + r] = c128{(r == c ? 1.0 : 0.0) + k.re - 0.5 * v.re, k.im - 0.5 * v.im};
+      });
+      __syncthreads();
+      c128 *A = sh.J0, *B = K;
+      int schulz = 0;
+      for (double e = 0.25 * kf * kf; e > 1e-17 && schulz < NEWTON_SCHULZ_MAX; e = 0.75 * e * e, ++schulz) {
+        small_mm<true>(A, A, kd, [&](int r, int c, const c128& v) { W[c * SMALL_LD + r] = v; });
+        __syncthreads();
+        small_mm<false>(A, W, kd, [&](int r, int c, const c128& v) {
+          const c128 z = A[c * SMALL_LD + r];
+          B[c * SMALL_LD + r] = c128{1.5 * z.re - 0.5 * v.re, 1.5 * z.im - 0.5 * v.im};
+        });
+        __syncthreads();
+        c128* t = A;
+        A = B;
+        B = t;
+      }
+      small_update(sh, A, kd);
+      small_gram(sh, kd);
+      small_corr(sh, kq, th, kf, above);
+      if (above == 0) return true;
+    }
+  }
+  return false;
+}
+
+template <int IT>
+__device__ __forceinline__ void jac_small_body(c128* __restrict__ X, int rows, int cols, double* __restrict__ sigma,
+                                               int* __restrict__ perm, SvdResult* __restrict__ res, int chi_max,
+                                               double eps, int rank_cap, double tol, SmallShared& sh) {
+  const int tid = threadIdx.x, c = tid >> 3, rl = tid & 7;
+  const bool wide = rows < cols;
+  const int kq = min(rows, cols), nr = max(rows, cols);
+  c128 x[IT];
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int r = rl + 8 * i, cc = min(c, kq - 1), rr = min(r, nr - 1);
+    x[i] = wide ? conj_of(X[rr * rows + cc]) : X[cc * rows + rr];
+    if (c >= kq || r >= nr) x[i] = c128{0.0, 0.0};
+  }
+  small_sort(x, sh, sh.V, SMALL_LDV);
+  double fro = 0;
+  for (int q = 0; q < JAC_LMAX; ++q) fro += sh.key[q];
+  const double conv = jac_conv_tol(tol, kq);
+  const InnerThresholds th{tol * tol, conv * conv, JAC_NOISE2 * fro};
+  small_qr(x, kq, sh.V, SMALL_LDV, sh.tau);
+  // R^H: column r is the conjugate of row r of R
+  auto adjoint = [&](c128* out, const c128* r4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = rl + 8 * i;
+      out[r * SMALL_LD + c] = r <= c ? conj_of(r4[i]) : c128{0.0, 0.0};
+    }
+    __syncthreads();
+  };
+  if (wide) {
+    adjoint(sh.Y, x);
+  } else {
+    adjoint(sh.G, x);
+    c128 b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = sh.G[c * SMALL_LD + rl + 8 * i];
+    small_sort(b, sh, sh.m[0], SMALL_LD);
+    small_qr(b, kq, sh.m[0], SMALL_LD, sh.tau2);
+    adjoint(sh.Y, b);
+  }
+  int sweeps;
+  const bool converged = small_jacobi(sh, kq, th, sweeps);
+  // left singular vectors times singular values, and their norms
+  c128 z[IT];
+  const int me = c < kq ? c : 0;
+  double n2 = 0;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int r = rl + 8 * i;
+    z[i] = i < 4 && r < kq ? sh.Y[me * SMALL_LD + sh.rank[r & 31]] : c128{0.0, 0.0};
+    n2 += z[i].re * z[i].re + z[i].im * z[i].im;
+  }
+  n2 = sum8(n2);
+  if (rl == 0) sh.key[c] = c < kq ? sqrt(n2) : 0.0;
+  if (!wide) small_apply_q(z, kq, sh.V, SMALL_LDV, sh.tau);
+  if (c < kq)
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+      if (rl + 8 * i < rows) X[c * rows + rl + 8 * i] = z[i];
+  __syncthreads();
+  const int rank = small_rank(sh.key);
+  if (rl == 0) {
+    sh.sorted[rank] = sh.key[c];
+    if (c < kq) {   // padding sorts behind
+      sigma[rank] = sh.key[c];
+      perm[rank] = c;
     }
   }
   __syncthreads();
-  finalize_body(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap,
-                converged ? sweep + 1 : sweep, converged);
+  if (tid >= 64) return;
+  // first i (< cap) with ||s[i:]|| < eps over the values a reduced SVD returns:
+  // lane e sums s[e:] from the smallest value up
+  const int ns = min(rank_cap, kq), cap = min(chi_max, ns);
+  const double s = tid < ns ? sh.sorted[tid] : 0.0, s2 = s * s;
+  double suffix = 0;
+  for (int e = ns - 1; e >= 0; --e) {
+    const double v = readlane_f64(s2, e);
+    if (e >= tid) suffix += v;
+  }
+  const unsigned long long below = __ballot(tid < cap && sqrt(suffix) < eps);
+  const int k = below ? __ffsll((unsigned long long)below) - 1 : cap;
+  double kept = 0, tail = 0;
+  for (int e = 0; e < ns; ++e) {
+    const double v = readlane_f64(s2, e);
+    if (e < k) kept += v;
+    else tail += v;
+  }
+  if (tid == 0) {
+    res->k = k;
+    res->nsweeps = sweeps;
+    res->converged = converged;
+    res->norm_kept = sqrt(kept);
+    res->tail = sqrt(tail);
+  }
 }
-__global__ __launch_bounds__(JAC_NT) void jac_small(c128* __restrict__ X, int rows, int cols,
-                                                    double* __restrict__ sigma,
-                                                    int* __restrict__ perm,
-                                                    SvdResult* __restrict__ res, int chi_max,
-                                                    double eps, int rank_cap, double tol) {
-  jac_small_body(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol);
+// Rows of the tall orientation in registers: 32, 64 or 128.
+__device__ __forceinline__ void jac_small_rows(c128* X, int rows, int cols, double* sigma, int* perm, SvdResult* res,
+                                               int chi_max, double eps, int rank_cap, double tol) {
+  __shared__ SmallShared sh;
+  const int nr = max(rows, cols);
+  if (nr <= 32) jac_small_body<4>(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
+  else if (nr <= 64) jac_small_body<8>(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
+  else jac_small_body<16>(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
+}
+__global__ __launch_bounds__(SMALL_NT) void jac_small(c128* __restrict__ X, int rows, int cols,
+                                                      double* __restrict__ sigma, int* __restrict__ perm,
+                                                      SvdResult* __restrict__ res, int chi_max, double eps,
+                                                      int rank_cap, double tol) {
+  jac_small_rows(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol);
 }
 
 // ---------------------------------------------------------- QR preconditioning
@@ -1295,9 +1519,9 @@ struct FinArgs {
   const JacobiCtrl* ctrl;
 };
 
-__global__ __launch_bounds__(JAC_NT) void jac_small_grouped(const GRec<JacSmallArgs>* __restrict__ recs, int n) {
+__global__ __launch_bounds__(SMALL_NT) void jac_small_grouped(const GRec<JacSmallArgs>* __restrict__ recs, int n) {
   const JacSmallArgs a = recs[blockIdx.x].a;
-  jac_small_body(gbl(a.X), a.rows, a.cols, gbl(a.sigma), gbl(a.perm), gbl(a.res), a.chi_max, a.eps, a.rank_cap,
+  jac_small_rows(gbl(a.X), a.rows, a.cols, gbl(a.sigma), gbl(a.perm), gbl(a.res), a.chi_max, a.eps, a.rank_cap,
                  a.tol);
 }
 __global__ __launch_bounds__(JAC_NT) void col_norm_order_grouped(const GRec<ColOrderArgs>* __restrict__ recs,
@@ -1349,11 +1573,8 @@ __global__ __launch_bounds__(JAC_APPLY_NT) void jac_apply_grouped(const GRec<Jac
   if (round >= g.nb - 1) return;
   jac_apply_body(gbl(r.a.Y), g, gbl(r.a.Z), gz, round, gbl(r.a.Jbuf), gbl(r.a.rotated), gbl(r.a.ctrl), bx, by);
 }
-__global__ void jac_check_grouped(const GRec<JacArgs>* __restrict__ recs, int n, int sweep) {
-  JacobiCtrl* ctrl = recs[blockIdx.x].a.ctrl;
-  if (threadIdx.x != 0 || ctrl->done) return;
-  ctrl->sweeps = sweep + 1;
-  if (ctrl->rot[sweep] == 0) ctrl->done = 1;
+__global__ void jac_check_grouped(const GRec<JacArgs>* __restrict__ recs) {
+  jac_check_body(gbl(recs[blockIdx.x].a.ctrl));
 }
 // out[i] = 0: matrix i sweeps, 1: closing phase, 2: converged (one thread per record)
 __global__ void jac_state_gather(const GRec<JacArgs>* __restrict__ recs, int n, int* __restrict__ out) {
@@ -1371,7 +1592,7 @@ __global__ __launch_bounds__(JAC_NT) void jac_finalize_grouped(const GRec<FinArg
 
 JacobiLayout jacobi_layout(int rows, int cols) {
   JacobiLayout l;
-  l.bs = cols <= JAC_LMAX ? std::max(1, (cols + 1) / 2) : JAC_BS;
+  l.bs = JAC_BS;
   l.nb = std::max(2, ceil_div(cols, l.bs));
   if (l.nb & 1) ++l.nb;
   l.kspl = ceil_div(rows, JAC_RC);
@@ -1383,18 +1604,22 @@ JacobiLayout jacobi_layout(int rows, int cols) {
   return l;
 }
 
-// Closing phase of an n-column matrix (preconditioned: n > 32): K, W, J0 and J1,
-// K and W large enough for the new Y and Q, and the per-tile sums.
+// Closing phase of an n-column matrix: K, W, J0 and J1, K and W large enough for
+// the new Y and Q, and the per-tile sums.
 size_t newton_bytes(int rows, int n) {
   const size_t t = ceil_div(n, 16);
   return 4 * sizeof(c128) * (size_t)rows * n + 16 * t * t;
 }
 
-// Blocks and closing phase of a matrix as it comes or, preconditioned, of the
-// min(rows, cols) columns of R^H.
+// Blocks and closing phase of the min(rows, cols) columns of R^H, in either
+// orientation.
 size_t jacobi_workspace_bytes(int max_rows, int max_cols) {
   const int n = std::min(max_rows, max_cols), m = std::max(max_rows, max_cols);
-  return std::max(jacobi_layout(max_rows, max_cols).bytes, jacobi_layout(m, n).bytes) + newton_bytes(m, n) + 1024;
+  return jacobi_layout(m, n).bytes + newton_bytes(m, n) + 1024;
+}
+
+bool small_svd(int rows, int cols) {
+  return std::min(rows, cols) <= JAC_LMAX && std::max(rows, cols) <= SMALL_ROWS;
 }
 
 namespace {
@@ -1438,8 +1663,8 @@ void newton_step(const NewtonArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(newton_decide, dim3(1), t, 0, s, a, -1);
 }
 
-// Gram-based block Jacobi on the columns of Y (rows x cols), the same block
-// rotations applied to the columns of Z (zrows x cols) when Z != null; leaves
+// Gram-based block Jacobi on the columns of Y (rows x cols) and its closing
+// phase, the same rotations applied to the columns of Z (zrows x cols); leaves
 // the control block in the workspace for the finalize.
 JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStream_t s,
                         JacobiWork& w) {
@@ -1452,19 +1677,16 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
   c128* Gpart = reinterpret_cast<c128*>(base + JAC_CTRL_BYTES + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
   c128* Jbuf = Gpart + l.gpart_elems;
   const JacobiGeom g{rows, cols, l.bs, l.nb, l.kspl};
-  const JacobiGeom gz{zrows, cols, l.bs, l.nb, Z ? ceil_div(zrows, JAC_RC) : 0};
+  const JacobiGeom gz{zrows, cols, l.bs, l.nb, ceil_div(zrows, JAC_RC)};
   const int np = l.nb / 2;
   const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)rows);
+  const NewtonArgs na = newton_args(Y, rows, Z, zrows, cols, reinterpret_cast<unsigned char*>(Jbuf + l.j_elems),
+                                    base, w.ws_bytes, ctrl, tol);
+  const dim3 nn(na.ntiles, na.ntiles);
   hipLaunchKernelGGL(jac_init, dim3(1), dim3(JAC_NT), 0, s, Y, (long)rows * cols, ctrl);
   // Launch the sweeps and closing steps of the previous call, then read the
   // device's state once per chunk (what is launched beyond it does nothing).
-  const bool closing = Z != nullptr;
-  NewtonArgs na{};
-  if (closing) na = newton_args(Y, rows, Z, zrows, cols, reinterpret_cast<unsigned char*>(Jbuf + l.j_elems), base,
-                                w.ws_bytes, ctrl, tol);
-  int sweep = 0, steps = closing ? std::max(1, w.pred_newton) : 0;
-  int& pred = Z ? w.pred_sweeps_pre : w.pred_sweeps;
-  int chunk = std::max(2, pred);
+  int sweep = 0, chunk = std::max(2, w.pred_sweeps), steps = std::max(1, w.pred_newton);
   while (sweep < JAC_MAX_SWEEPS || steps > 0) {
     for (int c = 0; c < chunk && sweep < JAC_MAX_SWEEPS; ++c, ++sweep) {
       for (int r = 0; r < l.nb - 1; ++r) {
@@ -1475,12 +1697,11 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
         hipLaunchKernelGGL(jac_apply, dim3(np, l.kspl + gz.kspl), dim3(JAC_APPLY_NT), 0, s, Y, g, Z, gz, r,
                            (const c128*)Jbuf, (const int*)rotated, (const JacobiCtrl*)ctrl);
       }
-      if (closing && sweep > 0) {
-        const dim3 nn(na.ntiles, na.ntiles);
+      if (sweep == 0) {   // never enters the closing phase
+        hipLaunchKernelGGL(jac_check, dim3(1), dim3(64), 0, s, ctrl);
+      } else {
         hipLaunchKernelGGL(newton_kernel<NEWTON_CORR>, nn, dim3(NEWTON_NT), 0, s, na, 0);
         hipLaunchKernelGGL(newton_decide, dim3(1), dim3(NEWTON_NT), 0, s, na, sweep);
-      } else {
-        hipLaunchKernelGGL(jac_check, dim3(1), dim3(64), 0, s, ctrl, sweep);
       }
     }
     for (int q = 0; q < steps; ++q) newton_step(na, s);
@@ -1489,13 +1710,13 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
     QCA_HIP(hipStreamSynchronize(s));
     const int* hc = reinterpret_cast<const int*>(w.host);   // done, sweeps, phase, newton
     if (hc[0]) {
-      pred = hc[1];
-      if (closing) w.pred_newton = hc[3];
+      w.pred_sweeps = hc[1];
+      w.pred_newton = hc[3];
       break;
     }
-    // in the closing phase: more steps; else more sweeps and the steps after them
-    chunk = hc[2] ? 0 : (closing ? 1 : 2);
-    steps = hc[2] ? 1 : (closing && hc[3] < NEWTON_MAX && sweep < JAC_MAX_SWEEPS ? 2 : 0);
+    // in the closing phase: more steps; else a sweep and the steps after it
+    chunk = hc[2] ? 0 : 1;
+    steps = hc[2] ? 1 : (hc[3] < NEWTON_MAX && sweep < JAC_MAX_SWEEPS ? 2 : 0);
   }
   return ctrl;
 }
@@ -1515,40 +1736,34 @@ void launch_jacobi_svd(c128* X, int rows, int cols, double* sigma, int* perm, Sv
   QCA_CHECK(rows >= 1 && rows <= 512, "SVD rows out of range (1..512)");
   QCA_CHECK(cols >= 1 && cols <= JAC_MAXCOLS, "SVD cols out of range (1..512)");
   QCA_CHECK(w.ws != nullptr && w.host != nullptr, "Jacobi workspace not set");
-  if (cols <= JAC_LMAX) {
-    const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)rows);
-    hipLaunchKernelGGL(jac_small, dim3(1), dim3(JAC_NT), 0, s, X, rows, cols, sigma, perm, res, chi_max,
+  const int kq = std::min(rows, cols);
+  if (small_svd(rows, cols)) {
+    const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)kq);
+    hipLaunchKernelGGL(jac_small, dim3(1), dim3(SMALL_NT), 0, s, X, rows, cols, sigma, perm, res, chi_max,
                        eps, rank_cap, tol);
     QCA_HIP(hipGetLastError());
     return;
   }
-  const int kq = std::min(rows, cols);
-  if (w.pre != nullptr && kq > JAC_LMAX && w.pre_elems >= jacobi_precond_elems(rows, cols)) {
-    // Preconditioned: X P = Q R with the columns by descending norm, one-sided
-    // Jacobi on Y = R^H with the same rotations applied to Q.  Y J = U' S and
-    // Q J = U, the left singular vectors of X, orthonormal by construction.
-    c128* Xp = w.pre;
-    c128* Q = Xp + (long)rows * cols;
-    c128* Y = Q + (long)rows * kq;
-    c128* qws = Y + (long)cols * kq;
-    const size_t qws_elems = w.pre_elems - (size_t)(qws - w.pre);
-    int* order = perm;  // scratch until the finalize writes the permutation
-    hipLaunchKernelGGL(col_norm_order, dim3(1), dim3(JAC_NT), 0, s, (const c128*)X, rows, cols, order);
-    hipLaunchKernelGGL(permute_cols, dim3(256), dim3(256), 0, s, (const c128*)X, rows, cols,
-                       (const int*)order, Xp);
-    launch_blocked_qr(Xp, rows, cols, Q, kq, qws, qws_elems, s);
-    hipLaunchKernelGGL(rh_from_qr, dim3(256), dim3(256), 0, s, (const c128*)Xp, rows, cols, kq, Y);
-    JacobiCtrl* ctrl = gram_jacobi(Y, cols, kq, Q, rows, s, w);
-    hipLaunchKernelGGL(jac_finalize, dim3(1), dim3(JAC_NT), 0, s, (const c128*)Y, cols, kq, sigma,
-                       perm, res, chi_max, eps, rank_cap, (const JacobiCtrl*)ctrl);
-    hipLaunchKernelGGL(scale_by_norms, dim3(ceil_div(kq, JAC_NT / 64)), dim3(JAC_NT), 0, s,
-                       (const c128*)Y, cols, (const c128*)Q, rows, kq, X);
-    QCA_HIP(hipGetLastError());
-    return;
-  }
-  JacobiCtrl* ctrl = gram_jacobi(X, rows, cols, nullptr, 0, s, w);
-  hipLaunchKernelGGL(jac_finalize, dim3(1), dim3(JAC_NT), 0, s, (const c128*)X, rows, cols, sigma,
+  QCA_CHECK(w.pre != nullptr && w.pre_elems >= jacobi_precond_elems(rows, cols), "Jacobi workspace too small");
+  // Preconditioned: X P = Q R with the columns by descending norm, one-sided
+  // Jacobi on Y = R^H with the same rotations applied to Q.  Y J = U' S and
+  // Q J = U, the left singular vectors of X, orthonormal by construction.
+  c128* Xp = w.pre;
+  c128* Q = Xp + (long)rows * cols;
+  c128* Y = Q + (long)rows * kq;
+  c128* qws = Y + (long)cols * kq;
+  const size_t qws_elems = w.pre_elems - (size_t)(qws - w.pre);
+  int* order = perm;  // scratch until the finalize writes the permutation
+  hipLaunchKernelGGL(col_norm_order, dim3(1), dim3(JAC_NT), 0, s, (const c128*)X, rows, cols, order);
+  hipLaunchKernelGGL(permute_cols, dim3(256), dim3(256), 0, s, (const c128*)X, rows, cols,
+                     (const int*)order, Xp);
+  launch_blocked_qr(Xp, rows, cols, Q, kq, qws, qws_elems, s);
+  hipLaunchKernelGGL(rh_from_qr, dim3(256), dim3(256), 0, s, (const c128*)Xp, rows, cols, kq, Y);
+  JacobiCtrl* ctrl = gram_jacobi(Y, cols, kq, Q, rows, s, w);
+  hipLaunchKernelGGL(jac_finalize, dim3(1), dim3(JAC_NT), 0, s, (const c128*)Y, cols, kq, sigma,
                      perm, res, chi_max, eps, rank_cap, (const JacobiCtrl*)ctrl);
+  hipLaunchKernelGGL(scale_by_norms, dim3(ceil_div(kq, JAC_NT / 64)), dim3(JAC_NT), 0, s,
+                     (const c128*)Y, cols, (const c128*)Q, rows, kq, X);
   QCA_HIP(hipGetLastError());
 }
 
@@ -1561,7 +1776,6 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   std::vector<GRec<JacArgs>> jac_one, jac_gram_r, jac_inner_r, jac_apply_r;
   std::vector<GRec<FinArgs>> fin;
   std::vector<QrStep> steps;
-  std::vector<GRec<JacArgs>> jac_plain;                    // without closing phase
   std::vector<GRec<NewtonArgs>> newton_one, newton_nn, newton_app, newton_cp;
   int max_rounds = 0, pred = 2, steps_pred = 1;
   for (const SvdJob& j : jobs) {
@@ -1569,35 +1783,26 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     QCA_CHECK(j.cols >= 1 && j.cols <= JAC_MAXCOLS, "SVD cols out of range (1..512)");
     JacobiWork& w = *j.w;
     QCA_CHECK(w.ws != nullptr, "Jacobi workspace not set");
-    if (j.cols <= JAC_LMAX) {
-      const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)j.rows);
+    const int kq = std::min(j.rows, j.cols);
+    if (small_svd(j.rows, j.cols)) {
+      const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)kq);
       small.push_back(grec(JacSmallArgs{j.X, j.rows, j.cols, j.sigma, j.perm, j.res, j.chi_max, j.eps,
                                         j.rank_cap, tol}, 1));
       continue;
     }
-    const int kq = std::min(j.rows, j.cols);
-    c128 *Y = j.X, *Z = nullptr;
-    int yrows = j.rows, ycols = j.cols, zrows = 0;
-    const bool pre = w.pre != nullptr && kq > JAC_LMAX && w.pre_elems >= jacobi_precond_elems(j.rows, j.cols);
-    if (pre) {
-      c128* Xp = w.pre;
-      c128* Q = Xp + (long)j.rows * j.cols;
-      c128* Yp = Q + (long)j.rows * kq;
-      c128* qws = Yp + (long)j.cols * kq;
-      const size_t qws_elems = w.pre_elems - (size_t)(qws - w.pre);
-      const ColOrderArgs co{j.X, j.rows, j.cols, j.perm, Xp};
-      order1.push_back(grec(co, 1));
-      perm.push_back(grec(co, 256));
-      for (QrStep& st : blocked_qr_steps(Xp, j.rows, j.cols, Q, kq, qws, qws_elems)) steps.push_back(st);
-      rh.push_back(grec(RhArgs{Xp, j.rows, j.cols, kq, Yp}, 256));
-      Y = Yp;
-      Z = Q;
-      yrows = j.cols;
-      ycols = kq;
-      zrows = j.rows;
-      scale.push_back(grec(ScaleArgs{Yp, j.cols, Q, j.rows, kq, j.X}, ceil_div(kq, JAC_NT / 64)));
-    }
-    const JacobiLayout l = jacobi_layout(yrows, ycols);
+    QCA_CHECK(w.pre != nullptr && w.pre_elems >= jacobi_precond_elems(j.rows, j.cols), "Jacobi workspace too small");
+    c128* Xp = w.pre;
+    c128* Z = Xp + (long)j.rows * j.cols;
+    c128* Y = Z + (long)j.rows * kq;
+    c128* qws = Y + (long)j.cols * kq;
+    const size_t qws_elems = w.pre_elems - (size_t)(qws - w.pre);
+    const ColOrderArgs co{j.X, j.rows, j.cols, j.perm, Xp};
+    order1.push_back(grec(co, 1));
+    perm.push_back(grec(co, 256));
+    for (QrStep& st : blocked_qr_steps(Xp, j.rows, j.cols, Z, kq, qws, qws_elems)) steps.push_back(st);
+    rh.push_back(grec(RhArgs{Xp, j.rows, j.cols, kq, Y}, 256));
+    scale.push_back(grec(ScaleArgs{Y, j.cols, Z, j.rows, kq, j.X}, ceil_div(kq, JAC_NT / 64)));
+    const JacobiLayout l = jacobi_layout(j.cols, kq);
     QCA_CHECK(l.bytes <= w.ws_bytes, "Jacobi workspace too small");
     unsigned char* base = reinterpret_cast<unsigned char*>(w.ws);
     JacArgs a{};
@@ -1606,35 +1811,31 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     a.Gpart = reinterpret_cast<c128*>(base + JAC_CTRL_BYTES + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
     a.Jbuf = a.Gpart + l.gpart_elems;
     a.Y = Y;
-    a.g = JacobiGeom{yrows, ycols, l.bs, l.nb, l.kspl};
+    a.g = JacobiGeom{j.cols, kq, l.bs, l.nb, l.kspl};
     a.Z = Z;
-    a.gz = JacobiGeom{zrows, ycols, l.bs, l.nb, Z ? ceil_div(zrows, JAC_RC) : 0};
-    a.tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)yrows);
+    a.gz = JacobiGeom{j.rows, kq, l.bs, l.nb, ceil_div(j.rows, JAC_RC)};
+    a.tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)j.cols);
     const int np = l.nb / 2;
     jac_one.push_back(grec(a, 1));
-    if (pre) {
-      const NewtonArgs na = newton_args(Y, yrows, Z, zrows, ycols, reinterpret_cast<unsigned char*>(a.Jbuf + l.j_elems),
-                                        base, w.ws_bytes, a.ctrl, a.tol);
-      newton_one.push_back(grec(na, 1));
-      newton_nn.push_back(grec(na, na.ntiles, na.ntiles));
-      newton_app.push_back(grec(na, na.ytiles + na.qtiles, na.ntiles));
-      newton_cp.push_back(grec(na, 256));
-      steps_pred = std::max(steps_pred, w.pred_newton);
-    } else {
-      jac_plain.push_back(grec(a, 1));
-    }
+    const NewtonArgs na = newton_args(Y, j.cols, Z, j.rows, kq, reinterpret_cast<unsigned char*>(a.Jbuf + l.j_elems),
+                                      base, w.ws_bytes, a.ctrl, a.tol);
+    newton_one.push_back(grec(na, 1));
+    newton_nn.push_back(grec(na, na.ntiles, na.ntiles));
+    newton_app.push_back(grec(na, na.ytiles + na.qtiles, na.ntiles));
+    newton_cp.push_back(grec(na, 256));
     jac_gram_r.push_back(grec(a, np, l.kspl));
     jac_inner_r.push_back(grec(a, np));
     jac_apply_r.push_back(grec(a, np, l.kspl + a.gz.kspl));
-    fin.push_back(grec(FinArgs{Y, yrows, ycols, j.sigma, j.perm, j.res, j.chi_max, j.eps, j.rank_cap, a.ctrl}, 1));
+    fin.push_back(grec(FinArgs{Y, j.cols, kq, j.sigma, j.perm, j.res, j.chi_max, j.eps, j.rank_cap, a.ctrl}, 1));
     max_rounds = std::max(max_rounds, l.nb - 1);
-    pred = std::max(pred, pre ? w.pred_sweeps_pre : w.pred_sweeps);
+    pred = std::max(pred, w.pred_sweeps);
+    steps_pred = std::max(steps_pred, w.pred_newton);
   }
   KGroup<JacSmallArgs> g_small;
   KGroup<ColOrderArgs> g_order, g_perm;
   KGroup<RhArgs> g_rh;
   KGroup<ScaleArgs> g_scale;
-  KGroup<JacArgs> g_one, g_gram, g_inner, g_apply, g_plain;
+  KGroup<JacArgs> g_one, g_gram, g_inner, g_apply;
   KGroup<NewtonArgs> n_one, n_nn, n_app, n_cp;
   KGroup<FinArgs> g_fin;
   g_small.prepare(small, arena);
@@ -1643,7 +1844,6 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   g_rh.prepare(rh, arena);
   g_scale.prepare(scale, arena);
   g_one.prepare(jac_one, arena);
-  g_plain.prepare(jac_plain, arena);
   n_one.prepare(newton_one, arena);
   n_nn.prepare(newton_nn, arena);
   n_app.prepare(newton_app, arena);
@@ -1684,7 +1884,7 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   arena.upload(s);
 
   if (!g_small.empty())
-    hipLaunchKernelGGL(jac_small_grouped, dim3(g_small.l.blocks), dim3(JAC_NT), 0, s, g_small.l.recs, g_small.l.n);
+    hipLaunchKernelGGL(jac_small_grouped, dim3(g_small.l.blocks), dim3(SMALL_NT), 0, s, g_small.l.recs, g_small.l.n);
   if (!g_order.empty()) {
     hipLaunchKernelGGL(col_norm_order_grouped, dim3(g_order.l.blocks), dim3(JAC_NT), 0, s, g_order.l.recs,
                        g_order.l.n);
@@ -1702,14 +1902,12 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     const int nj = g_one.l.n;
     const dim3 nt(NEWTON_NT);
     auto check = [&](int sweep) {
-      // sweep 0 never enters the closing phase
-      const KGroup<JacArgs>& c = sweep > 0 ? g_plain : g_one;
-      if (!c.empty())
-        hipLaunchKernelGGL(jac_check_grouped, dim3(c.l.n), dim3(64), 0, s, c.l.recs, c.l.n, sweep);
-      if (sweep > 0 && !n_one.empty()) {
-        hipLaunchKernelGGL(newton_grouped<NEWTON_CORR>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 0);
-        hipLaunchKernelGGL(newton_decide_grouped, dim3(n_one.l.n), nt, 0, s, n_one.l.recs, sweep);
+      if (sweep == 0) {
+        hipLaunchKernelGGL(jac_check_grouped, dim3(g_one.l.n), dim3(64), 0, s, g_one.l.recs);
+        return;
       }
+      hipLaunchKernelGGL(newton_grouped<NEWTON_CORR>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 0);
+      hipLaunchKernelGGL(newton_decide_grouped, dim3(n_one.l.n), nt, 0, s, n_one.l.recs, sweep);
     };
     auto step = [&] {
       hipLaunchKernelGGL(newton_grouped<NEWTON_START>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 0);
@@ -1722,7 +1920,7 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
       hipLaunchKernelGGL(newton_grouped<NEWTON_CORR>, dim3(n_nn.l.blocks), nt, 0, s, n_nn.l.recs, n_nn.l.n, 1);
       hipLaunchKernelGGL(newton_decide_grouped, dim3(n_one.l.n), nt, 0, s, n_one.l.recs, -1);
     };
-    int sweep = 0, chunk = std::max(2, pred), steps = n_one.empty() ? 0 : steps_pred, steps_done = 0;
+    int sweep = 0, chunk = std::max(2, pred), steps = steps_pred, steps_done = 0;
     while (sweep < JAC_MAX_SWEEPS || steps > 0) {
       for (int c = 0; c < chunk && sweep < JAC_MAX_SWEEPS; ++c, ++sweep) {
         for (int r = 0; r < max_rounds; ++r) {
@@ -1748,7 +1946,7 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
       if (!sweeping && !closing) break;
       // a matrix takes at most NEWTON_MAX closing steps, wherever its sweeps end
       chunk = sweeping ? 1 : 0;
-      steps = n_one.empty() ? 0 : (closing ? 1 : (steps_done < 2 * NEWTON_MAX ? 2 : 0));
+      steps = closing ? 1 : (steps_done < 2 * NEWTON_MAX ? 2 : 0);
     }
     hipLaunchKernelGGL(jac_finalize_grouped, dim3(g_fin.l.blocks), dim3(JAC_NT), 0, s, g_fin.l.recs, g_fin.l.n);
     if (!g_scale.empty())

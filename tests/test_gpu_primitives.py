@@ -218,7 +218,8 @@ def test_svd_split_closing_steps(gpu, spectrum, chil, chir, right):
     V, _ = np.linalg.qr(crand(rng, n, min(m, n)))
     i = np.arange(min(m, n))
     s = {"flat": 1 + 0.01 * i / len(i), "pairs": 0.93 ** (i // 2) * (1 + 1e-6 * (i % 2)),
-         "steps": 10.0 ** (-2 * (i // (len(i) // 4 + 1)))}[spectrum]
+         "steps": 10.0 ** (-2 * (i // (len(i) // 4 + 1))),
+         "graded": 10.0 ** (-14 * i / len(i)), "rank1": 1.0 * (i == 0)}[spectrum]
     M = (U * s) @ V.conj().T
     M /= np.linalg.norm(M)
     ref = np.linalg.svd(M, compute_uv=False)
@@ -237,7 +238,23 @@ def test_svd_split_closing_steps(gpu, spectrum, chil, chir, right):
     B = Ar[: n * kk].cpu().numpy().reshape(2, kk, chir).transpose(1, 0, 2).reshape(kk, n)
     Q = A if right else B.conj().T
     assert np.abs(Q.conj().T @ Q - np.eye(kk)).max() < max(1e-13, 2 * len(Q) * np.finfo(float).eps)
-    assert np.abs(A @ B - M).max() < 1e-12
+    # the truncated state, normalised (reference tdvp.py:286-296)
+    u, _, vh = np.linalg.svd(M, full_matrices=False)
+    kept = (u[:, :kk] * ref[:kk] / np.linalg.norm(ref[:kk])) @ vh[:kk]
+    assert np.abs(A @ B - kept).max() < 1e-12
+
+
+@pytest.mark.parametrize("right", [1, 0])
+@pytest.mark.parametrize("spectrum", ["flat", "graded", "rank1"])
+@pytest.mark.parametrize("chil,chir", [(1, 1), (1, 2), (2, 2), (2, 1), (4, 4), (5, 4), (8, 8), (8, 9), (16, 16),
+                                       (12, 16), (16, 17), (16, 33), (16, 64), (1, 64),
+                                       # just past one workgroup's range: 130 and 200 long
+                                       (16, 65), (3, 100)])
+def test_svd_split_one_workgroup(gpu, spectrum, chil, chir, right):
+    """Splits up to 32 x 128 take one workgroup: every half of the round-robin
+    (2..32 columns), tall and wide, at the register sizes of the QR (32, 64, 128
+    long), against LAPACK within the bounds of test_svd_split."""
+    test_svd_split_closing_steps(gpu, spectrum, chil, chir, right)
 
 
 @pytest.mark.parametrize("side", [0, 1])
