@@ -392,7 +392,6 @@ void Engine::fused_run(int kind, int site, c128* x, long n, int chil, int chir, 
   a.x = x;
   a.V = lw_.V;
   a.T1 = reinterpret_cast<cplx<T>*>(T_);
-  a.U = reinterpret_cast<cplx<T>*>(U_);
   a.tally = tally_;
   a.tau = kHalfPi * delta;
   a.tol = p_.krylov_tol;

@@ -359,6 +359,7 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
   constexpr bool mixed = !std::is_same<T, double>::value;
   std::vector<GRec<FusedKrylovArgs<T>>> fused;
   size_t fused_lds = 0;
+  long fused_n = 0;
   std::vector<LzArgs> lz;
   std::vector<int> lz_item;
   std::vector<GemmJob<T>> g1, g3;
@@ -393,7 +394,6 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
       a.x = x[i];
       a.V = e->lw_.V;
       a.T1 = reinterpret_cast<cplx<T>*>(e->T_);
-      a.U = reinterpret_cast<cplx<T>*>(e->U_);
       a.tally = e->tally_;
       a.tau = tau;
       a.tol = e->p_.krylov_tol;
@@ -401,6 +401,7 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
       a.flops_per_matvec = heff_flops(k, chil[i], chir[i], std::max(a.Din, a.Dout));
       FusedKrylovArgs<T> placed;
       fused_lds = std::max(fused_lds, fused_krylov_place(a, placed));
+      fused_n = std::max(fused_n, a.n);
       fused.push_back(grec(placed, 1));
       continue;
     }
@@ -456,7 +457,7 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
     G3.prepare(g3, arena_);
   }
   arena_.upload(s_);
-  launch_fused_krylov_grouped<T>(gf, fused_lds, s_);
+  launch_fused_krylov_grouped<T>(gf, fused_n, fused_lds, s_);
   if (lz.empty()) return;
   QCA_HIP(hipEventRecord(ev2_, s_));
   glz.begin(s_);

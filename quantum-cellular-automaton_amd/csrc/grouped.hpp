@@ -318,6 +318,6 @@ void launch_gather_words(const void* const* src, int words, int n, unsigned long
 template <typename TE>
 size_t fused_krylov_place(const FusedKrylovArgs<TE>& a, FusedKrylovArgs<TE>& placed);
 template <typename TE>
-void launch_fused_krylov_grouped(const KGroup<FusedKrylovArgs<TE>>& g, size_t lds, hipStream_t s);
+void launch_fused_krylov_grouped(const KGroup<FusedKrylovArgs<TE>>& g, long max_n, size_t lds, hipStream_t s);
 
 }  // namespace qca

@@ -92,8 +92,8 @@ void lanczos_iteration_tail(const cplx<TW>* w, long n, int j, double tau, double
 void lanczos_finish(long n, c128* y, LanczosWork& lw, hipStream_t s);
 
 // ---------------------------------------------------------------- one-launch Krylov
-// Longest vector of the one-workgroup exponential (4 residual elements per
-// thread of 1024).
+// Longest vector of the one-workgroup exponential (8 residual elements per
+// thread of 512).
 constexpr long FUSED_KRYLOV_MAX_N = 4096;
 
 // Device-side running totals of the one-launch exponentials of one engine.
@@ -125,19 +125,17 @@ struct FusedKrylovArgs {
   c128* x = nullptr;           // in/out, n elements
   c128* V = nullptr;           // basis, (max_m - 1) * n elements
   cplx<TE>* T1 = nullptr;      // dq * Din * chil * chir elements
-  cplx<TE>* U = nullptr;       // dq * Dout * chil * chir elements
   LanczosCtrl* ctrl = nullptr; // optional: m, error, limit flag of this call
   KrylovTally* tally = nullptr;// optional running totals
   double tau = 0, tol = 0;
   double flops_per_matvec = 0;
   int max_m = LZ_MAXK;
-  // Placement in the workgroup's LDS, filled by launch_fused_krylov: byte
-  // offsets into the dynamic LDS (-1: the operand stays in global memory) and
-  // the number of leading basis vectors held there.
-  long offL = -1, offR = -1, offRow = -1, offCol = -1, offVal = -1, offU = -1, offT1 = -1;
-  long offV = -1;
-  long offW = 0;               // residual staging (n elements), always in LDS
-  int vcap = 0;
+  // Filled by fused_krylov_place: byte offsets into the workgroup's LDS, whether T1
+  // and the MPO, and the environments, lie there, the number of leading basis
+  // vectors held there, the waves that share a tile of H_eff x (a power of two),
+  // and whether the result goes over T1.
+  long offW = 0, offRow = 0, offCol = 0, offVal = 0, offL = 0, offR = 0, offV = 0;
+  int t1_lds = 0, env_lds = 0, vcap = 0, parts = 1, overlay = 0;
 };
 
 template <typename TE>

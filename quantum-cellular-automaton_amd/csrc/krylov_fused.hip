@@ -4,317 +4,325 @@
 // Hamiltonians of reference algorithms/tdvp.py:298-326 (applied matrix-free)
 // with the Lanczos scheme of lautils.py:44-81, entirely inside one workgroup:
 //
-//   * H_eff: L-contraction -> sparse MPO mixing -> R-contraction, the three
-//     stages separated by workgroup barriers, in the environments' type
-//     (complex128, or complex64 on FP32 for the mixed path, as on the
-//     multi-launch path); the result lands, in FP64, in the registers of the
-//     threads that own its elements;
-//   * recurrence: FP64, classical Gram-Schmidt applied twice against the whole
-//     basis (the multi-launch path's scheme), the residual in registers
-//     (element e belongs to thread e % 1024);
+//   * H_eff: T1 = L-contraction -> sparse MPO mixing -> R-contraction on the
+//     matrix cores, in the environments' type (complex128, or complex64 on FP32
+//     for the mixed path, as on the multi-launch path).  T1 lies in LDS with the
+//     left index fastest, the layout of the second product's A operand, so the
+//     mixing is a sparse sum of operands on their way into registers;
+//   * recurrence: FP64, the three-term step and then one classical Gram-Schmidt
+//     pass against the whole basis (a second pass: what the first leaves is
+//     the non-Hermitian rounding of H_eff), the residual and the last two
+//     basis vectors in registers (element e belongs to thread e % 512);
 //   * tridiagonal exponential and the stopping test on wave 0, as in the
-//     multi-launch path (Taylor with scaling, lane = row of T).
+//     multi-launch path (Taylor with scaling, lane = row of T), from the
+//     iteration on in which it can pass at all (fk_unconverged).
 //
 // The multi-launch path needs ~11 launches and a host round trip per Krylov
 // iteration; at small bond dimension those dominate. This kernel needs one
 // launch and no host round trip per exponential; it works on one CU, so it is
-// used only below a size limit chosen by the engine.  Its iterations are bound
-// by memory latency, so the launcher places the operands in LDS as far as
-// they fit (environments, sparse MPO, both intermediates, then leading basis
-// vectors) and the kernel reaches each one through a generic pointer.
+// used only below a size limit chosen by the engine.
+// What bounds it: the two products (FP64 matrix rate of one CU: 2.6 us each for
+// 4 x 16 x 16 with MPO bond 6) and the passes over the basis.  Eight waves: two
+// per SIMD hide the operand loads, and a barrier takes 268 cycles where sixteen
+// waves take 815.  Per iteration at bond 16 (averages over a 15-cell run, MPO bond 6): left
+// product 3.1 us, mixing and right product 4.4, three-term step 1.1, projection
+// 1.4, subtraction and norm 1.5, basis vector 0.5: 12 us, before 22 (sixteen
+// waves, vector products from LDS and global memory, two full Gram-Schmidt
+// passes, a tridiagonal exponential of 3.6 us every time).  The run: 155 -> 104
+// ms.  Above FUSED_KRYLOV_DEFAULT_N elements the whole chip is faster: bond 30,
+// 82 ms with this limit and 86 with all blocks here.
 #include "grouped.hpp"
 #include "wave.hpp"
 
 namespace qca {
 namespace {
 
-constexpr int FK_THREADS = 1024;
+constexpr int FK_THREADS = 512;
 constexpr int FK_WAVES = FK_THREADS / 64;
-constexpr int FK_EPT = FUSED_KRYLOV_MAX_N / FK_THREADS;  // residual elements per thread
+// Residual elements per thread: blocks up to FK_SMALL_N and up to the limit.
+constexpr long FK_SMALL_N = 2 * FK_THREADS;
+constexpr int FK_EPT_MAX = FUSED_KRYLOV_MAX_N / FK_THREADS;
 // Dynamic LDS of one launch (the static part, FkShared, adds ~3 KB; 160 KB per CU).
 constexpr long FK_LDS_BYTES = 152 * 1024;
-
-__device__ __forceinline__ double fk_wave_sum(double v) { return wave_sum64(v); }
-
-// Element i of p in the compute type TC.
-template <typename TC, typename TS>
-__device__ __forceinline__ cplx<TC> ldc(const cplx<TS>* __restrict__ p, unsigned i) {
-  const cplx<TS> v = p[i];
-  return cplx<TC>{TC(v.re), TC(v.im)};
-}
 
 struct FkShared {
   c128 coef[LZ_MAXK];
   double alpha[LZ_MAXK];
   double beta[LZ_MAXK];
   c128 z[LZ_MAXK];
-  double red[FK_WAVES];
-  int flag;
+  c128 red[2][FK_WAVES];
+  double err;
+  int flag, limit;
+  unsigned long long used;     // channels (q, w) that the MPO reads, as bits
+  unsigned char channel[64];   // and as a list
 };
 
-// Operands of one launch, each in LDS or global memory.
-template <typename TE>
-struct FkCtx {
-  const cplx<TE>* L;
-  const cplx<TE>* R;
-  const int* rowptr;
-  const int* col;
-  const cplx<TE>* val;
-  cplx<TE>* T1;
-  cplx<TE>* U;
-  c128* Vl;  // leading vcap basis vectors (LDS)
-  c128* Vg;  // the others (global)
-  c128* wbuf;  // residual staging for the projections (LDS, n elements)
-  int vcap;
-  long n;
-  __device__ __forceinline__ c128* basis(int i) const {
-    return i < vcap ? Vl + (long)i * n : Vg + (long)i * n;
+// Matrix-core tile of the element type: A[i][k] from lane i + 16 k, B[k][j] from
+// lane j + 16 k, k < 4; register r of lane l holds D[row(r, l / 16)][l % 16].
+template <typename T> struct FkMfma;
+template <> struct FkMfma<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ int row(int r, int hi) { return hi + 4 * r; }
 };
-
+template <> struct FkMfma<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ acc mul(float a, float b, acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int r, int hi) { return 4 * hi + r; }
+};
 template <typename T>
-__device__ T* place(unsigned char* arena, long off, T* global) {
-  return off >= 0 ? reinterpret_cast<T*>(arena + off) : global;
-}
-
-// Copies `bytes` (a multiple of 8: complex elements) from global memory into LDS.
-__device__ void stage(void* dst, const void* src, long bytes) {
-  const uint2* s = reinterpret_cast<const uint2*>(src);
-  uint2* d = reinterpret_cast<uint2*>(dst);
-  for (long i = threadIdx.x; i < bytes / 8; i += FK_THREADS) d[i] = s[i];
-}
-
-// Sum of v over the workgroup, returned to every thread.
-__device__ double fk_block_sum(double v, FkShared& sh) {
-  v = fk_wave_sum(v);
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (l == 0) sh.red[w] = v;
-  __syncthreads();
-  double r = 0;
-#pragma unroll
-  for (int i = 0; i < FK_WAVES; ++i) r += sh.red[i];
-  __syncthreads();
-  return r;
-}
-
-// sh.coef[i] = <V_i, w> for i = 0..j; w is this thread's residual elements.
-// The residual goes to LDS once; wave v then reduces the coefficients
-// i = v, v + 16, ... over the whole vector, so the j+1 cross-lane reductions
-// run side by side instead of one after another (fixed order: deterministic).
-template <typename TE>
-__device__ void fk_project(const FkCtx<TE>& f, int j, const double* wr, const double* wi,
-                           FkShared& sh) {
-  const long n = f.n;
-#pragma unroll
-  for (int r = 0; r < FK_EPT; ++r) {
-    const long e = threadIdx.x + (long)r * FK_THREADS;
-    if (e < n) f.wbuf[e] = c128{wr[r], wi[r]};
+struct FkTile {
+  typename FkMfma<T>::acc re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+  __device__ __forceinline__ void add(const cplx<T>& a, const cplx<T>& b) {
+    re = FkMfma<T>::mul(a.re, b.re, re);
+    im = FkMfma<T>::mul(a.re, b.im, im);
+    re = FkMfma<T>::mul(-a.im, b.im, re);
+    im = FkMfma<T>::mul(a.im, b.re, im);
   }
+};
+
+__device__ __forceinline__ double lane_value(double v, int lane) { return readlane_f64(v, lane); }
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+// Sum of (re, im) over the workgroup, returned to every thread; calls alternate
+// between the halves of sh.red, so one barrier per sum is enough.
+__device__ __forceinline__ c128 fk_block_sum(double re, double im, int half, FkShared& sh) {
+  re = wave_sum64(re);
+  im = wave_sum64(im);
+  if ((threadIdx.x & 63) == 0) sh.red[half][threadIdx.x >> 6] = c128{re, im};
   __syncthreads();
-  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int i = wv; i <= j; i += FK_WAVES) {
-    const c128* vi = f.basis(i);
-    double ar = 0, ai = 0;
-    for (long e = l; e < n; e += 64) {
-      const c128 a = vi[e], x = f.wbuf[e];
-      ar += a.re * x.re + a.im * x.im;
-      ai += a.re * x.im - a.im * x.re;
+  c128 t{0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < FK_WAVES; ++i) {
+    t.re += sh.red[half][i].re;
+    t.im += sh.red[half][i].im;
+  }
+  return t;
+}
+
+// T1[q][w][c][x] = sum_a v[q][a][c] L[a][w][x] for the nch channels q * Din + w in
+// `channel` (null: all): 16x16 tiles (c, x), one wave each, the operands of the
+// next 16 a on their way while the products of these run.
+template <typename TE>
+__device__ __forceinline__ void fk_left(const FusedKrylovArgs<TE>& a, const c128* v, const cplx<TE>* L, cplx<TE>* T1,
+                                        const unsigned char* channel, int nch) {
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chil = a.chil, chir = a.chir, Din = a.Din;
+  const int xt = (chil + 15) >> 4, ct = (chir + 15) >> 4, tiles = nch * xt * ct;
+  auto fetch = [&](int t, int k0, c128(&av)[4], cplx<TE>(&bv)[4]) {
+    const int n = t % nch, r1 = t / nch, ci = r1 % ct, xi = r1 / ct;
+    const int qw = channel ? __builtin_amdgcn_readfirstlane((int)channel[n]) : n;
+    const int q = qw / Din, w = qw - q * Din;
+    const c128* vp = v + (unsigned)(q * chil * chir + min(16 * ci + lo, chir - 1));
+    const cplx<TE>* lp = L + (unsigned)(w * chil + min(16 * xi + lo, chil - 1));
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const unsigned k = min(k0 + 4 * s + hi, chil - 1);
+      av[s] = vp[k * chir];
+      bv[s] = lp[k * (unsigned)(Din * chil)];
     }
-    ar = fk_wave_sum(ar);
-    ai = fk_wave_sum(ai);
-    if (l == 0) sh.coef[i] = c128{ar, ai};
-  }
-  __syncthreads();
-}
-
-// w -= sum_{i<=j} coef_i V_i
-template <typename TE>
-__device__ void fk_subtract(const FkCtx<TE>& f, int j, double* wr, double* wi, const FkShared& sh) {
-  const long n = f.n;
-  for (int i = 0; i <= j; ++i) {
-    const c128 c = sh.coef[i];
-    const c128* vi = f.basis(i);
+  };
+  c128 av[4], an[4];
+  cplx<TE> bv[4], bn[4];
+  FkTile<TE> acc;
+  if (wave < tiles) fetch(wave, 0, av, bv);
+  for (int t = wave, k0 = 0; t < tiles;) {
+    const int kn = k0 + 16 < chil ? k0 + 16 : 0, tn = kn ? t : t + FK_WAVES;
+    if (tn < tiles) fetch(tn, kn, an, bn);
 #pragma unroll
-    for (int r = 0; r < FK_EPT; ++r) {
-      const long e = threadIdx.x + (long)r * FK_THREADS;
-      if (e < n) {
-        const c128 a = vi[e];
-        wr[r] -= c.re * a.re - c.im * a.im;
-        wi[r] -= c.re * a.im + c.im * a.re;
+    for (int s = 0; s < 4; ++s) {
+      const bool in = k0 + 4 * s + hi < chil;
+      if (k0 + 4 * s < chil)
+        acc.add(cplx<TE>{in ? TE(av[s].re) : TE(0), in ? TE(av[s].im) : TE(0)}, bv[s]);
+    }
+    if (kn == 0) {
+      const int n = t % nch, r1 = t / nch, ci = r1 % ct, xi = r1 / ct;
+      const int qw = channel ? __builtin_amdgcn_readfirstlane((int)channel[n]) : n;
+      const int x = 16 * xi + lo;
+      cplx<TE>* out = T1 + (unsigned)(qw * chir * chil);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int cc = 16 * ci + FkMfma<TE>::row(r, hi);
+        if (cc < chir && x < chil) out[(unsigned)(cc * chil + x)] = cplx<TE>{acc.re[r], acc.im[r]};
       }
+      acc = FkTile<TE>();
     }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      av[s] = an[s];
+      bv[s] = bn[s];
+    }
+    t = tn;
+    k0 = kn;
   }
 }
 
-// Sum over the S lanes of a group (S a power of two); every lane gets it.
-template <typename T>
-__device__ __forceinline__ void fk_segment_sum(T& re, T& im, unsigned S) {
-  for (int d = (int)S >> 1; d > 0; d >>= 1) {
-    re += __shfl_xor(re, d, 64);
-    im += __shfl_xor(im, d, 64);
-  }
-}
-
-// The H_eff result was written to wbuf by output; each thread takes its own
-// elements into registers.
+// Lane i holds entry z0 + i of the sparse MPO's rows (q', 0..Dout-1): its row v,
+// column and value, so that a wave-uniform lookup is a lane read instead of a
+// chain of three memory reads (kind 2: one entry per v).
 template <typename TE>
-__device__ void fk_collect(const FkCtx<TE>& f, double* yr, double* yi) {
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < FK_EPT; ++r) {
-    const long e = threadIdx.x + (long)r * FK_THREADS;
-    const c128 y = e < f.n ? f.wbuf[e] : c128{0.0, 0.0};
-    yr[r] = y.re;
-    yi[r] = y.im;
-  }
+struct FkEntries {
+  int first, last;   // entries of q'
+  int v, c;
+  cplx<TE> x;
+};
+template <typename TE>
+__device__ __forceinline__ void fk_entries(const FusedKrylovArgs<TE>& a, int q, int z0, const int* rowptr,
+                                           const int* col, const cplx<TE>* val, FkEntries<TE>& e) {
+  const int z = min(z0 + (int)(threadIdx.x & 63), e.last - 1);
+  e.v = e.c = z;
+  e.x = cplx<TE>{TE(1), TE(0)};
+  if (a.kind == 2 || z < z0) return;
+  e.v = 0;
+  for (int r = 1; r < a.Dout; ++r) e.v += rowptr[q * a.Dout + r] <= z ? 1 : 0;
+  e.c = col[z];
+  e.x = val[z];
+}
+template <typename TE>
+__device__ __forceinline__ FkEntries<TE> fk_rows(const FusedKrylovArgs<TE>& a, int q, const int* rowptr,
+                                                 const int* col, const cplx<TE>* val) {
+  FkEntries<TE> e;
+  e.first = a.kind == 2 ? 0 : __builtin_amdgcn_readfirstlane(rowptr[q * a.Dout]);
+  e.last = a.kind == 2 ? a.Dout : __builtin_amdgcn_readfirstlane(rowptr[(q + 1) * a.Dout]);
+  fk_entries(a, q, e.first, rowptr, col, val, e);
+  return e;
+}
+// q' of this wave's first tile of y.
+template <typename TE>
+__device__ __forceinline__ int fk_first_q(const FusedKrylovArgs<TE>& a, int dq) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  return min((wave / a.parts) / (((a.chil + 15) >> 4) * ((a.chir + 15) >> 4)), dq - 1);
 }
 
-// y = H_eff v (v in LDS or global memory); y is left in this thread's registers.
-// C(m, n) = sum_{k1 < K1, k2 < K2} A(m, k) B(k, n) over the workgroup, with
-// A(m, k) = A[m*am + k1*ak1 + k2*ak2], B(k, n) = B[k1*bk1 + k2*bk2 + n*bn],
-// C(m, n) = C[b*cb + m*cm + n] for batch b < NB (A, B shifted by ab, bb).
-// Each group of S lanes owns a TM x TN output tile (register blocking: TM + TN
-// loads per TM*TN complex multiply-adds) and splits its K range S ways.
-struct FkGemm {
-  unsigned M, N, K1, K2, NB;
-  unsigned am, ak1, ak2, ab;
-  unsigned bk1, bk2, bn, bb;
-  unsigned cm, cb;
-};
-
-template <int TM, int TN, typename TC, typename TA, typename TB, typename TO>
-__device__ void fk_gemm_tiled(const FkGemm& g, const cplx<TA>* A, const cplx<TB>* B, cplx<TO>* C,
-                              unsigned S) {
-  const unsigned tm = (g.M + TM - 1) / TM, tn = (g.N + TN - 1) / TN;
-  const unsigned per_b = tm * tn, tiles = per_b * g.NB;
-  const unsigned s = threadIdx.x & (S - 1);
-  const unsigned K = g.K1 * g.K2;
-  for (unsigned t = threadIdx.x / S; t < tiles; t += FK_THREADS / S) {
-    const unsigned b = t / per_b, r = t - b * per_b;
-    const unsigned im = r / tn, in = r - im * tn;
-    const unsigned m0 = im * TM, n0 = in * TN;
-    unsigned aoff[TM], boff[TN];
+// y[q'][x][yy] = sum_{v,c} U[q'][x][c][v] R[c][v][yy], U[q'][x][c][v] the sum of
+// val * T1[col][c][x] over row (q', v) of the sparse MPO (kind 2: U = T1[v]).
+// Tiles (x, yy) of q', the rows v of each dealt to `parts` waves; partial sums go
+// to part[p][e].  `mine` holds the entries of the wave's first tile (they are the
+// same in every iteration).  With one tile per wave `part` lies over T1, hence
+// the barrier.
+template <typename TE>
+__device__ __forceinline__ void fk_right(const FusedKrylovArgs<TE>& a, const cplx<TE>* T1, const cplx<TE>* R,
+                                         const int* rowptr, const int* col, const cplx<TE>* val,
+                                         const FkEntries<TE>& mine, c128* part) {
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chil = a.chil, chir = a.chir, Dout = a.Dout, parts = a.parts;
+  const int dq = a.kind == 0 ? 4 : (a.kind == 1 ? 2 : 1);
+  const int xt = (chil + 15) >> 4, yt = (chir + 15) >> 4, lr = chil * chir;
+  const int p = wave & (parts - 1), ntiles = dq * xt * yt;
+  auto compute = [&](int t, FkEntries<TE> e, FkTile<TE>& acc) {
+    const int yi = t % yt, r1 = t / yt, xi = r1 % xt, q = r1 / xt;
+    const cplx<TE>* tp = T1 + min(16 * xi + lo, chil - 1);
+    const cplx<TE>* rp = R + min(16 * yi + lo, chir - 1);
+    for (int z0 = e.first; z0 < e.last; z0 += 64) {
+      if (z0 > e.first) fk_entries(a, q, z0, rowptr, col, val, e);
+      const int nz = min(64, e.last - z0);
+      for (int k0 = 0; k0 < chir; k0 += 16) {
+        unsigned at[4], ar[4];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) aoff[i] = b * g.ab + min(m0 + i, g.M - 1) * g.am;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) boff[j] = b * g.bb + min(n0 + j, g.N - 1) * g.bn;
-    TC cr[TM][TN], ci[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) cr[i][j] = ci[i][j] = TC(0);
-    unsigned k1 = 0, k2 = s;
-    while (k2 >= g.K2 && k1 < g.K1) {
-      k2 -= g.K2;
-      ++k1;
-    }
-    for (unsigned k = s; k < K; k += S) {
-      const unsigned ka = k1 * g.ak1 + k2 * g.ak2, kb = k1 * g.bk1 + k2 * g.bk2;
-      cplx<TC> av[TM], bv[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) av[i] = ldc<TC>(A, aoff[i] + ka);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bv[j] = ldc<TC>(B, boff[j] + kb);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          cr[i][j] += av[i].re * bv[j].re - av[i].im * bv[j].im;
-          ci[i][j] += av[i].re * bv[j].im + av[i].im * bv[j].re;
+        for (int s = 0; s < 4; ++s) {
+          const unsigned c = min(k0 + 4 * s + hi, chir - 1);
+          at[s] = c * chil;
+          ar[s] = c * (unsigned)(Dout * chir);
         }
-      k2 += S;
-      while (k2 >= g.K2) {
-        k2 -= g.K2;
-        ++k1;
+        // the wave's entries are i with row v = p, p + parts, ...
+        auto next = [&](int i) {
+          while (i < nz && (__builtin_amdgcn_readlane(e.v, i) & (parts - 1)) != p) ++i;
+          return i;
+        };
+        auto fetch = [&](int i, cplx<TE>(&u)[4], cplx<TE>(&av)[4]) {
+          const cplx<TE>* tz = tp + (unsigned)(__builtin_amdgcn_readlane(e.c, i) * lr);
+          const cplx<TE>* rz = rp + (unsigned)(__builtin_amdgcn_readlane(e.v, i) * chir);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            u[s] = tz[at[s]];
+            av[s] = rz[ar[s]];
+          }
+        };
+        cplx<TE> u[4], av[4], un[4], an[4], bv[4];
+        int i = next(0);
+        if (i < nz) fetch(i, u, av);
+        bool fresh = true;
+        while (i < nz) {
+          const int in = next(i + 1);
+          const bool more = in < nz && __builtin_amdgcn_readlane(e.v, in) == __builtin_amdgcn_readlane(e.v, i);
+          if (in < nz) fetch(in, un, an);
+          const cplx<TE> wv{lane_value(e.x.re, i), lane_value(e.x.im, i)};
+          if (wv.re != TE(1) || wv.im != TE(0))   // the rules' MPOs have ones only
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+              u[s] = cplx<TE>{wv.re * u[s].re - wv.im * u[s].im, wv.re * u[s].im + wv.im * u[s].re};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) bv[s] = fresh ? u[s] : cplx<TE>{bv[s].re + u[s].re, bv[s].im + u[s].im};
+          fresh = !more;
+          if (!more) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+              const bool inside = k0 + 4 * s + hi < chir;
+              if (k0 + 4 * s < chir)
+                acc.add(bv[s], cplx<TE>{inside ? av[s].re : TE(0), inside ? av[s].im : TE(0)});
+            }
+          }
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            u[s] = un[s];
+            av[s] = an[s];
+          }
+          i = in;
+        }
       }
     }
+  };
+  auto store = [&](int t, const FkTile<TE>& acc) {
+    const int yi = t % yt, r1 = t / yt, xi = r1 % xt, q = r1 / xt;
+    const int yy = 16 * yi + lo;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) fk_segment_sum(cr[i][j], ci[i][j], S);
-    if (s == 0) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          if (m0 + i < g.M && n0 + j < g.N)
-            C[b * g.cb + (m0 + i) * g.cm + n0 + j] = cplx<TO>{TO(cr[i][j]), TO(ci[i][j])};
+    for (int r = 0; r < 4; ++r) {
+      const int x = 16 * xi + FkMfma<TE>::row(r, hi);
+      if (yy < chir && x < chil)
+        part[(unsigned)(p * dq * lr + (q * chil + x) * chir + yy)] = c128{double(acc.re[r]), double(acc.im[r])};
+    }
+  };
+  int t = wave / parts;
+  if (a.overlay) {
+    FkTile<TE> acc;
+    if (t < ntiles) compute(t, mine, acc);
+    __syncthreads();
+    if (t < ntiles) store(t, acc);
+  } else {
+    for (; t < ntiles; t += FK_WAVES / parts) {
+      FkTile<TE> acc;
+      compute(t, fk_rows(a, t / (xt * yt), rowptr, col, val), acc);
+      store(t, acc);
     }
   }
 }
 
-// Picks the tile (4x2, 2x2 or 1x1: the largest that still gives most of the
-// workgroup a tile; 4x4 would not fit the 128 registers of a 1024-thread
-// workgroup) and the K split, then runs the GEMM.
-template <typename TC, typename TA, typename TB, typename TO>
-__device__ void fk_gemm(const FkGemm& g, const cplx<TA>* A, const cplx<TB>* B, cplx<TO>* C) {
-  auto tiles = [&](unsigned tm, unsigned tn) {
-    return ((g.M + tm - 1) / tm) * ((g.N + tn - 1) / tn) * g.NB;
-  };
-  auto split = [&](unsigned n) {
-    unsigned S = 1;
-    while (S < 16 && n * S * 2 <= FK_THREADS) S *= 2;
-    return S;
-  };
-  if (tiles(4, 2) >= FK_THREADS / 2) fk_gemm_tiled<4, 2, TC>(g, A, B, C, 1);
-  else if (tiles(2, 2) >= FK_THREADS / 4) fk_gemm_tiled<2, 2, TC>(g, A, B, C, split(tiles(2, 2)));
-  else fk_gemm_tiled<1, 1, TC>(g, A, B, C, split(tiles(1, 1)));
+// Lane l + 1 and lane l - 1 of the wave, 0 beyond its ends.
+template <int CTRL>
+__device__ __forceinline__ double wave_shift(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
+__device__ __forceinline__ double lane_above(double v) { return wave_shift<0x130>(v); }   // wave_shl:1
+__device__ __forceinline__ double lane_below(double v) { return wave_shift<0x138>(v); }   // wave_shr:1
 
-template <typename TE>
-__device__ void fk_heff(const FusedKrylovArgs<TE>& a, const FkCtx<TE>& f, const c128* v, double* yr,
-                        double* yi) {
-  // all index arithmetic in 32 bits: every extent here is below 2^20
-  const unsigned chil = a.chil, chir = a.chir, Din = a.Din, Dout = a.Dout;
-  const unsigned lr = chil * chir;
-  const unsigned dq = a.kind == 0 ? 4 : (a.kind == 1 ? 2 : 1);
-  // T1[q][(w,x)][c] = sum_a L[a][(w,x)] v[q][a][c]
-  {
-    FkGemm g;
-    g.M = Din * chil; g.N = chir; g.K1 = 1; g.K2 = chil; g.NB = dq;
-    g.am = 1; g.ak1 = 0; g.ak2 = Din * chil; g.ab = 0;
-    g.bk1 = 0; g.bk2 = chir; g.bn = 1; g.bb = lr;
-    g.cm = chir; g.cb = Din * lr;
-    fk_gemm<TE>(g, f.L, v, f.T1);
-  }
-  __syncthreads();
-  if (a.kind == 2) {
-    // y[x][yy] = sum_{w,c} T1[w][x][c] R[c][w][yy]
-    FkGemm g;
-    g.M = chil; g.N = chir; g.K1 = Din; g.K2 = chir; g.NB = 1;
-    g.am = chir; g.ak1 = lr; g.ak2 = 1; g.ab = 0;
-    g.bk1 = chir; g.bk2 = Din * chir; g.bn = 1; g.bb = 0;
-    g.cm = chir; g.cb = 0;
-    fk_gemm<TE>(g, f.T1, f.R, f.wbuf);
-    fk_collect(f, yr, yi);
-    return;
-  }
-  // U[q'][xc][v] = sum over the sparse row (q',v) of W * T1[(q,w)][xc]
-  const unsigned e2 = dq * Dout * lr;
-  for (unsigned e = threadIdx.x; e < e2; e += FK_THREADS) {
-    const unsigned o = e / lr, xc = e - o * lr;
-    TE re = 0, im = 0;
-    const int z1 = f.rowptr[o + 1];
-    for (int zz = f.rowptr[o]; zz < z1; ++zz) {
-      const cplx<TE> wv = f.val[zz];
-      const cplx<TE> t = f.T1[(unsigned)f.col[zz] * lr + xc];
-      re += wv.re * t.re - wv.im * t.im;
-      im += wv.re * t.im + wv.im * t.re;
-    }
-    const unsigned qp = o / Dout, vv = o - qp * Dout;
-    f.U[(qp * lr + xc) * Dout + vv] = cplx<TE>{re, im};
-  }
-  __syncthreads();
-  // y[(q',x)][yy] = sum_{(c,v)} U[(q',x)][(c,v)] R[(c,v)][yy]
-  {
-    FkGemm g;
-    g.M = dq * chil; g.N = chir; g.K1 = 1; g.K2 = chir * Dout; g.NB = 1;
-    g.am = chir * Dout; g.ak1 = 0; g.ak2 = 1; g.ab = 0;
-    g.bk1 = 0; g.bk2 = chir; g.bn = 1; g.bb = 0;
-    g.cm = chir; g.cb = 0;
-    fk_gemm<TE>(g, f.U, f.R, f.wbuf);
-  }
-  fk_collect(f, yr, yi);
+// Largest v of the wave, in every lane.
+__device__ __forceinline__ double wave_max64(double v) {
+  v = fmax(v, dpp_f64<0xB1>(v));    // quad_perm(1,0,3,2)
+  v = fmax(v, dpp_f64<0x4E>(v));    // quad_perm(2,3,0,1)
+  v = fmax(v, dpp_f64<0x141>(v));   // row_half_mirror
+  v = fmax(v, dpp_f64<0x140>(v));   // row_mirror
+  return fmax(fmax(readlane_f64(v, 0), readlane_f64(v, 16)), fmax(readlane_f64(v, 32), readlane_f64(v, 48)));
 }
 
 // Wave 0: z = exp(-i tau T_m) e_0 for the m = j+1 leading rows of the
@@ -327,8 +335,7 @@ __device__ double fk_tridiag_exp(const FkShared& sh, int j, double beta, double 
   const double al = (l < m) ? sh.alpha[l] : 0.0;
   const double bup = (l + 1 < m) ? sh.beta[l] : 0.0;
   const double bdn = (l >= 1 && l < m) ? sh.beta[l - 1] : 0.0;
-  double rown = fabs(al) + fabs(bup) + fabs(bdn);
-  for (int o = 32; o > 0; o >>= 1) rown = fmax(rown, __shfl_xor(rown, o, 64));
+  const double rown = wave_max64(fabs(al) + fabs(bup) + fabs(bdn));
   const double h = fabs(tau) * rown;
   const int nsub = (h < 2048.0) ? max(1, (int)ceil(h / 0.5)) : 1;
   const double dt = tau / nsub;
@@ -337,8 +344,8 @@ __device__ double fk_tridiag_exp(const FkShared& sh, int j, double beta, double 
   for (int sstep = 0; sstep < nsub; ++sstep) {
     double ar = zr, ai = zi, tr = zr, ti = zi;
     for (int k = 1; k < 60; ++k) {
-      const double upr = __shfl_down(tr, 1, 64), upi = __shfl_down(ti, 1, 64);
-      const double dnr = __shfl_up(tr, 1, 64), dni = __shfl_up(ti, 1, 64);
+      const double upr = lane_above(tr), upi = lane_above(ti);
+      const double dnr = lane_below(tr), dni = lane_below(ti);
       double yr = al * tr + bup * upr + bdn * dnr;
       double yi = al * ti + bup * upi + bdn * dni;
       if (l >= m) {
@@ -357,126 +364,243 @@ __device__ double fk_tridiag_exp(const FkShared& sh, int j, double beta, double 
     zr = ar;
     zi = ai;
   }
-  const double zlr = __shfl(zr, j, 64), zli = __shfl(zi, j, 64);
+  const double zlr = readlane_f64(zr, j), zli = readlane_f64(zi, j);
   return beta * sqrt(zlr * zlr + zli * zli);
 }
 
-template <typename TE>
+// Whether the error estimate beta_j |z_j| of iteration j is certainly above 2 tol,
+// from a lower bound: z_j is the product of the betas times a divided difference
+// of exp(-i tau .) over the eigenvalues of T, (-i tau)^j times the mean of
+// exp(-i tau s) / j! over a simplex of points s between them (Hermite-Genocchi),
+// so |z_j| >= prod |tau|^j / j! cos(tau width / 2) with Gershgorin's width.  The
+// tridiagonal exponential (1.6 us) is evaluated when this does not decide: one or
+// two times per call instead of m.
+struct FkBound {
+  double prod = 1.0, low = 0.0, high = 0.0, last = 0.0;
+  __device__ __forceinline__ bool unconverged(int j, double alpha, double beta, double tau, double tol) {
+    tau = fabs(tau);
+    if (j > 0) prod *= last * tau / j;
+    const double r = last + beta;
+    low = j > 0 ? fmin(low, alpha - r) : alpha - r;
+    high = j > 0 ? fmax(high, alpha + r) : alpha + r;
+    last = beta;
+    const double h = 0.5 * tau * (high - low);
+    return h < 1.4 && beta * prod * (1.0 - 0.5 * h * h) >= 2.0 * tol;   // cos h >= 1 - h^2 / 2
+  }
+};
+
+template <typename TE, int EPT>
 __device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, unsigned char* arena) {
   __shared__ FkShared sh;
-  const long n = a.n;
+  const int n = (int)a.n, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned long long t0 = wall_clock64();
-  FkCtx<TE> f;
-  f.L = place(arena, a.offL, a.L);
-  f.R = place(arena, a.offR, a.R);
-  f.rowptr = place(arena, a.offRow, a.rowptr);
-  f.col = place(arena, a.offCol, a.col);
-  f.val = place(arena, a.offVal, a.val);
-  f.T1 = place(arena, a.offT1, a.T1);
-  f.U = place(arena, a.offU, a.U);
-  f.Vl = place(arena, a.offV, a.V);
-  f.Vg = a.V;
-  f.wbuf = reinterpret_cast<c128*>(arena + a.offW);
-  f.vcap = a.vcap;
-  f.n = n;
+  // LDS: T1, the partial sums of y and then the residual (over T1 where that is
+  // used up), the MPO; T1 and the MPO stay in global memory when they don't fit
+  cplx<TE>* T1l = reinterpret_cast<cplx<TE>*>(arena);
+  c128* wbuf = reinterpret_cast<c128*>(arena + a.offW);
+  int* rowptr = reinterpret_cast<int*>(arena + a.offRow);
+  int* col = reinterpret_cast<int*>(arena + a.offCol);
+  cplx<TE>* val = reinterpret_cast<cplx<TE>*>(arena + a.offVal);
+  cplx<TE>* Ll = reinterpret_cast<cplx<TE>*>(arena + a.offL);
+  cplx<TE>* Rl = reinterpret_cast<cplx<TE>*>(arena + a.offR);
+  c128* Vl = reinterpret_cast<c128*>(arena + a.offV);   // leading vcap basis vectors
+  c128* __restrict__ Vg = a.V;                          // the others
   const int dq = a.kind == 0 ? 4 : (a.kind == 1 ? 2 : 1);
-  if (a.offL >= 0) stage(arena + a.offL, a.L, (long)a.chil * a.Din * a.chil * sizeof(cplx<TE>));
-  if (a.offR >= 0) stage(arena + a.offR, a.R, (long)a.chir * a.Dout * a.chir * sizeof(cplx<TE>));
-  if (a.offVal >= 0) stage(arena + a.offVal, a.val, (long)a.nnz * sizeof(cplx<TE>));
-  if (a.offRow >= 0) {
-    int* rp = reinterpret_cast<int*>(arena + a.offRow);
-    for (int i = threadIdx.x; i <= dq * a.Dout; i += FK_THREADS) rp[i] = a.rowptr[i];
+  if (a.t1_lds && a.kind != 2) {
+    for (int i = tid; i <= dq * a.Dout; i += FK_THREADS) rowptr[i] = a.rowptr[i];
+    for (int i = tid; i < a.nnz; i += FK_THREADS) {
+      col[i] = a.col[i];
+      val[i] = a.val[i];
+    }
   }
-  if (a.offCol >= 0) {
-    int* cp = reinterpret_cast<int*>(arena + a.offCol);
-    for (int i = threadIdx.x; i < a.nnz; i += FK_THREADS) cp[i] = a.col[i];
+  if (a.env_lds) {
+    const int nL = a.chil * a.Din * a.chil, nR = a.chir * a.Dout * a.chir;
+#pragma unroll 4
+    for (int i = tid; i < nL; i += FK_THREADS) Ll[i] = a.L[i];
+#pragma unroll 4
+    for (int i = tid; i < nR; i += FK_THREADS) Rl[i] = a.R[i];
   }
-  double wr[FK_EPT], wi[FK_EPT];
-#pragma unroll
-  for (int r = 0; r < FK_EPT; ++r) {
-    const long e = threadIdx.x + (long)r * FK_THREADS;
-    wr[r] = e < n ? a.x[e].re : 0.0;
-    wi[r] = e < n ? a.x[e].im : 0.0;
-  }
+  // channels of T1 that some row of the MPO reads
+  const int ncol = dq * a.Din;
+  const bool listed = a.kind != 2 && ncol <= 64;
+  if (tid == 0) sh.used = 0;
+  __syncthreads();
+  if (listed)
+    for (int i = tid; i < a.nnz; i += FK_THREADS) atomicOr(&sh.used, 1ull << a.col[i]);
+  __syncthreads();
+  const unsigned long long used = sh.used;
+  if (listed && tid < 64 && (used >> tid & 1)) sh.channel[__popcll(used & ((1ull << tid) - 1))] = (unsigned char)tid;
+  const unsigned char* channel = listed ? sh.channel : nullptr;
+  const int nch = listed ? __popcll(used) : ncol;
+  const int q0 = fk_first_q(a, dq);
+  const FkEntries<TE> mine = a.t1_lds ? fk_rows(a, q0, rowptr, col, val) : fk_rows(a, q0, a.rowptr, a.col, a.val);
+  // f(V_i) with the basis vector in its own address space
+  auto with_basis = [&](int i, auto&& f) {
+    if (i < a.vcap) f(Vl + (unsigned)(i * n));
+    else f(Vg + (unsigned)(i * n));
+  };
+  c128 w[EPT], v0[EPT], v1[EPT];   // residual, V_j, V_{j-1}: elements tid, tid + 512, ...
   double nrm = 0;
 #pragma unroll
-  for (int r = 0; r < FK_EPT; ++r) nrm += wr[r] * wr[r] + wi[r] * wi[r];
-  const double beta0 = sqrt(fk_block_sum(nrm, sh));
+  for (int r = 0; r < EPT; ++r) {
+    const int e = tid + r * FK_THREADS;
+    w[r] = e < n ? a.x[e] : c128{0.0, 0.0};
+    v0[r] = c128{0.0, 0.0};
+    nrm += w[r].re * w[r].re + w[r].im * w[r].im;
+  }
+  const double beta0 = sqrt(fk_block_sum(nrm, 0.0, 0, sh).re);
   int m = 0, hit_limit = 0;
   double err = 0;
   if (beta0 > 0.0) {
-    const double inv0 = 1.0 / beta0;
-#pragma unroll
-    for (int r = 0; r < FK_EPT; ++r) {
-      const long e = threadIdx.x + (long)r * FK_THREADS;
-      if (e < n) f.basis(0)[e] = c128{wr[r] * inv0, wi[r] * inv0};
-    }
-    __syncthreads();
+    FkBound bound;
+    double beta = beta0;
     for (int j = 0;; ++j) {
-      fk_heff<TE>(a, f, f.basis(j), wr, wi);
-      fk_project(f, j, wr, wi, sh);
-      const double c1 = sh.coef[j].re;
-      fk_subtract(f, j, wr, wi, sh);
-      fk_project(f, j, wr, wi, sh);
-      const double c2 = sh.coef[j].re;
-      fk_subtract(f, j, wr, wi, sh);
+      // V_j
+      const double inv = 1.0 / beta;
+#pragma unroll
+      for (int r = 0; r < EPT; ++r) {
+        v1[r] = v0[r];
+        v0[r] = c128{w[r].re * inv, w[r].im * inv};
+      }
+      with_basis(j, [&](c128* vj) {
+#pragma unroll
+        for (int r = 0; r < EPT; ++r)
+          if (tid + r * FK_THREADS < n) vj[tid + r * FK_THREADS] = v0[r];
+      });
+      __syncthreads();
+      // w = H_eff V_j
+      const c128* vj = j < a.vcap ? Vl + (unsigned)(j * n) : Vg + (unsigned)(j * n);
+      if (a.env_lds) {
+        fk_left<TE>(a, vj, Ll, T1l, channel, nch);
+        __syncthreads();
+        fk_right<TE>(a, T1l, Rl, rowptr, col, val, mine, wbuf);
+      } else if (a.t1_lds) {
+        fk_left<TE>(a, vj, a.L, T1l, channel, nch);
+        __syncthreads();
+        fk_right<TE>(a, T1l, a.R, rowptr, col, val, mine, wbuf);
+      } else {
+        fk_left<TE>(a, vj, a.L, a.T1, channel, nch);
+        __syncthreads();
+        fk_right<TE>(a, a.T1, a.R, a.rowptr, a.col, a.val, mine, wbuf);
+      }
+      __syncthreads();
+      double ar = 0, ai = 0;
+#pragma unroll
+      for (int r = 0; r < EPT; ++r) {
+        const int e = tid + r * FK_THREADS;
+        w[r] = c128{0.0, 0.0};
+        if (e < n)
+          for (int p = 0; p < a.parts; ++p) {
+            const c128 y = wbuf[p * n + e];
+            w[r].re += y.re;
+            w[r].im += y.im;
+          }
+        ar += v0[r].re * w[r].re + v0[r].im * w[r].im;
+        ai += v0[r].re * w[r].im - v0[r].im * w[r].re;
+      }
+      // three-term step
+      const c128 c1 = fk_block_sum(ar, ai, 1, sh);
+      const double bp = j > 0 ? beta : 0.0;
+#pragma unroll
+      for (int r = 0; r < EPT; ++r) {
+        w[r].re -= c1.re * v0[r].re - c1.im * v0[r].im + bp * v1[r].re;
+        w[r].im -= c1.re * v0[r].im + c1.im * v0[r].re + bp * v1[r].im;
+        if (tid + r * FK_THREADS < n) wbuf[tid + r * FK_THREADS] = w[r];
+      }
+      __syncthreads();
+      // coef_i = <V_i, w>: the residual is in LDS, wave k takes i = k, k + 8, ...
+      for (int i = wave; i <= j; i += FK_WAVES) {
+        double pr = 0, pi = 0;
+        with_basis(i, [&](const c128* vi) {
+#pragma unroll 8
+          for (int e = lane; e < n; e += 64) {
+            const c128 b = vi[e], x = wbuf[e];
+            pr += b.re * x.re + b.im * x.im;
+            pi += b.re * x.im - b.im * x.re;
+          }
+        });
+        pr = wave_sum64(pr);
+        pi = wave_sum64(pi);
+        if (lane == 0) sh.coef[i] = c128{pr, pi};
+      }
+      __syncthreads();
+      // w -= sum_i coef_i V_i
+      auto subtract = [&](const c128* vi, const c128& c) {
+#pragma unroll
+        for (int r = 0; r < EPT; ++r) {
+          const c128 b = vi[min(tid + r * FK_THREADS, n - 1)];
+          w[r].re -= c.re * b.re - c.im * b.im;
+          w[r].im -= c.re * b.im + c.im * b.re;
+        }
+      };
+      const int nl = min(j, a.vcap);
+#pragma unroll 2
+      for (int i = 0; i < nl; ++i) subtract(Vl + (unsigned)(i * n), sh.coef[i]);
+#pragma unroll 4
+      for (int i = nl; i < j; ++i) subtract(Vg + (unsigned)(i * n), sh.coef[i]);
+      const c128 c2 = sh.coef[j];
       double s = 0;
 #pragma unroll
-      for (int r = 0; r < FK_EPT; ++r) s += wr[r] * wr[r] + wi[r] * wi[r];
-      const double beta = sqrt(fk_block_sum(s, sh));
-      const double alpha_j = c1 + c2;
-      if (threadIdx.x < 64) {
-        if (threadIdx.x == 0) {
-          sh.alpha[j] = alpha_j;
-          sh.beta[j] = beta;
-        }
+      for (int r = 0; r < EPT; ++r) {
+        w[r].re -= c2.re * v0[r].re - c2.im * v0[r].im;
+        w[r].im -= c2.re * v0[r].im + c2.im * v0[r].re;
+        if (tid + r * FK_THREADS >= n) w[r] = c128{0.0, 0.0};
+        s += w[r].re * w[r].re + w[r].im * w[r].im;
+      }
+      beta = sqrt(fk_block_sum(s, 0.0, 0, sh).re);
+      const double alpha_j = c1.re + c2.re;
+      if (tid == 0) {
+        sh.alpha[j] = alpha_j;
+        sh.beta[j] = beta;
+      }
+      const bool breakdown = beta <= 1e-13 * fmax(1.0, fabs(alpha_j));
+      const bool unconverged = bound.unconverged(j, alpha_j, beta, a.tau, a.tol);
+      if (unconverged && !breakdown && j + 1 < a.max_m - 1) continue;
+      if (wave == 0) {
         // wave 0 reads its own writes: wave-local LDS order holds
         __builtin_amdgcn_wave_barrier();
         double zr, zi;
         const double e = fk_tridiag_exp(sh, j, beta, a.tau, zr, zi);
-        const bool breakdown = beta <= 1e-13 * fmax(1.0, fabs(alpha_j));
         const bool conv = breakdown || e < a.tol || j + 1 >= a.max_m - 1;
-        if ((int)threadIdx.x <= j) sh.z[threadIdx.x] = c128{zr, zi};
-        if (threadIdx.x == 0) {
+        if (lane <= j) sh.z[lane] = c128{zr, zi};
+        if (lane == 0) {
           sh.flag = conv ? 1 : 0;
-          sh.red[0] = e;
-          sh.red[1] = (!breakdown && e >= a.tol) ? 1.0 : 0.0;
+          sh.err = e;
+          sh.limit = !breakdown && e >= a.tol;
         }
       }
       __syncthreads();
-      const bool done = sh.flag != 0;
-      err = sh.red[0];
-      hit_limit = sh.red[1] != 0.0;
-      __syncthreads();
-      if (done) {
+      err = sh.err;
+      hit_limit = sh.limit;
+      if (sh.flag) {
         m = j + 1;
         break;
       }
-      const double inv = 1.0 / beta;
-      c128* vn = f.basis(j + 1);
-#pragma unroll
-      for (int r = 0; r < FK_EPT; ++r) {
-        const long e = threadIdx.x + (long)r * FK_THREADS;
-        if (e < n) vn[e] = c128{wr[r] * inv, wi[r] * inv};
-      }
-      __syncthreads();
     }
   }
   // x = beta0 * sum_{i<m} z_i V_i  (a zero input stays zero)
 #pragma unroll
-  for (int r = 0; r < FK_EPT; ++r) {
-    const long e = threadIdx.x + (long)r * FK_THREADS;
-    if (e >= n) continue;
-    double re = 0, im = 0;
-    for (int i = 0; i < m; ++i) {
-      const c128 zc = sh.z[i];
-      const c128 v = f.basis(i)[e];
-      re += zc.re * v.re - zc.im * v.im;
-      im += zc.re * v.im + zc.im * v.re;
+  for (int r = 0; r < EPT; ++r) w[r] = c128{0.0, 0.0};
+  auto add = [&](const c128* vi, const c128& z) {
+#pragma unroll
+    for (int r = 0; r < EPT; ++r) {
+      const c128 b = vi[min(tid + r * FK_THREADS, n - 1)];
+      w[r].re += z.re * b.re - z.im * b.im;
+      w[r].im += z.re * b.im + z.im * b.re;
     }
-    a.x[e] = c128{beta0 * re, beta0 * im};
+  };
+  const int nl = min(m, a.vcap);
+#pragma unroll 2
+  for (int i = 0; i < nl; ++i) add(Vl + (unsigned)(i * n), sh.z[i]);
+#pragma unroll 4
+  for (int i = nl; i < m; ++i) add(Vg + (unsigned)(i * n), sh.z[i]);
+#pragma unroll
+  for (int r = 0; r < EPT; ++r) {
+    const int e = tid + r * FK_THREADS;
+    if (e < n) a.x[e] = c128{beta0 * w[r].re, beta0 * w[r].im};
   }
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     if (a.ctrl) {
       a.ctrl->beta0 = beta0;
       a.ctrl->err = err;
@@ -496,15 +620,15 @@ __device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, 
   }
 }
 
-template <typename TE>
+template <typename TE, int EPT>
 __global__ __launch_bounds__(FK_THREADS) void fused_krylov_kernel(FusedKrylovArgs<TE> a) {
   extern __shared__ __align__(16) unsigned char arena[];
-  fused_krylov_body<TE>(a, arena);
+  fused_krylov_body<TE, EPT>(a, arena);
 }
 
 // One exponential per workgroup, each with its own arguments and LDS placement
 // (the dynamic LDS of the launch is the largest placement).
-template <typename TE>
+template <typename TE, int EPT>
 __global__ __launch_bounds__(FK_THREADS) void fused_krylov_grouped(const GRec<FusedKrylovArgs<TE>>* __restrict__ recs,
                                                                    int n) {
   extern __shared__ __align__(16) unsigned char arena[];
@@ -517,10 +641,9 @@ __global__ __launch_bounds__(FK_THREADS) void fused_krylov_grouped(const GRec<Fu
   a.x = gbl(a.x);
   a.V = gbl(a.V);
   a.T1 = gbl(a.T1);
-  a.U = gbl(a.U);
   a.ctrl = gbl(a.ctrl);
   a.tally = gbl(a.tally);
-  fused_krylov_body<TE>(a, arena);
+  fused_krylov_body<TE, EPT>(a, arena);
 }
 
 }  // namespace
@@ -536,32 +659,45 @@ size_t fused_krylov_place(const FusedKrylovArgs<TE>& a, FusedKrylovArgs<TE>& b) 
   QCA_CHECK(a.kind != 2 || a.Din == a.Dout, "bond block needs equal MPO bonds");
   QCA_CHECK(a.kind == 2 || a.nnz >= 0, "negative MPO entry count");
   QCA_CHECK(a.kind == 2 || a.Dout <= 16, "MPO bond dimension above 16");
-  // LDS placement, in order of use per Krylov iteration
+  // tiles of y and the waves that share one, splitting its MPO rows
   b = a;
   const long lr = (long)a.chil * a.chir;
-  long off = a.n * (long)sizeof(c128);  // residual staging first: always in LDS
-  b.offW = 0;
-  auto take = [&](long bytes) -> long {
-    bytes = (bytes + 15) / 16 * 16;
-    if (off + bytes > FK_LDS_BYTES) return -1;
+  const long tiles = (long)dq * ceil_div(a.chil, 16) * ceil_div(a.chir, 16);
+  b.parts = 1;
+  while (2 * b.parts * tiles <= FK_WAVES && 2 * b.parts <= a.Dout) b.parts *= 2;
+  // LDS: T1 and the MPO if both fit (else they stay in global memory), the partial
+  // sums of y (over T1 if every wave has its tiles in registers by then), leading
+  // basis vectors
+  b.overlay = tiles * b.parts <= FK_WAVES;
+  long off = 0;
+  auto take = [&](long bytes) {
     const long o = off;
-    off += bytes;
+    off += (bytes + 15) / 16 * 16;
     return o;
   };
-  b.offL = take((long)a.chil * a.Din * a.chil * sizeof(cplx<TE>));
-  b.offR = take((long)a.chir * a.Dout * a.chir * sizeof(cplx<TE>));
-  b.offRow = b.offCol = b.offVal = b.offU = -1;
-  if (a.kind != 2) {
-    b.offRow = take((long)(dq * a.Dout + 1) * sizeof(int));
-    b.offCol = take((long)a.nnz * sizeof(int));
-    b.offVal = take((long)a.nnz * sizeof(cplx<TE>));
-    b.offU = take((long)dq * a.Dout * lr * sizeof(cplx<TE>));
+  const long py = b.parts * a.n * (long)sizeof(c128);
+  const long t1 = (long)dq * a.Din * lr * sizeof(cplx<TE>);
+  const long nnz = a.kind == 2 ? 0 : a.nnz, nrow = a.kind == 2 ? 0 : dq * a.Dout + 1;
+  const long work = b.overlay ? std::max(t1, py) : t1 + 16 + py;
+  b.t1_lds = work + 64 + nrow * (long)sizeof(int) + nnz * (long)(sizeof(int) + sizeof(cplx<TE>)) <= FK_LDS_BYTES;
+  if (b.t1_lds) {
+    take(b.overlay ? std::max(t1, py) : t1);
+    b.offW = b.overlay ? 0 : take(py);
+    b.offVal = take(nnz * sizeof(cplx<TE>));
+    b.offRow = take(nrow * sizeof(int));
+    b.offCol = take(nnz * sizeof(int));
+  } else {
+    b.offW = take(py);
   }
-  b.offT1 = take((long)dq * a.Din * lr * sizeof(cplx<TE>));
+  // environments: both, ahead of the basis (their latency is in the way of every
+  // product; the basis is streamed)
+  const long envL = (long)a.chil * a.Din * a.chil * sizeof(cplx<TE>), envR = (long)a.chir * a.Dout * a.chir * sizeof(cplx<TE>);
+  b.env_lds = b.t1_lds && off + envL + envR + 32 <= FK_LDS_BYTES;
+  b.offL = b.env_lds ? take(envL) : 0;
+  b.offR = b.env_lds ? take(envR) : 0;
   const long vbytes = a.n * (long)sizeof(c128);
   b.vcap = (int)std::min<long>(a.max_m - 1, (FK_LDS_BYTES - off) / vbytes);
-  b.offV = b.vcap > 0 ? off : -1;
-  if (b.vcap > 0) off += b.vcap * vbytes;
+  b.offV = take(b.vcap * vbytes);
   return (size_t)off;
 }
 template size_t fused_krylov_place<double>(const FusedKrylovArgs<double>&, FusedKrylovArgs<double>&);
@@ -571,21 +707,29 @@ template <typename TE>
 void launch_fused_krylov(const FusedKrylovArgs<TE>& a, hipStream_t s) {
   FusedKrylovArgs<TE> b;
   const size_t off = fused_krylov_place(a, b);
-  ensure_dynamic_lds((const void*)fused_krylov_kernel<TE>, off);
-  hipLaunchKernelGGL(fused_krylov_kernel<TE>, dim3(1), dim3(FK_THREADS), off, s, b);
+  auto run = [&](auto kernel) {
+    ensure_dynamic_lds((const void*)kernel, off);
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(FK_THREADS), off, s, b);
+  };
+  if (a.n <= FK_SMALL_N) run(fused_krylov_kernel<TE, 2>);
+  else run(fused_krylov_kernel<TE, FK_EPT_MAX>);
   QCA_HIP(hipGetLastError());
 }
 template void launch_fused_krylov<double>(const FusedKrylovArgs<double>&, hipStream_t);
 template void launch_fused_krylov<float>(const FusedKrylovArgs<float>&, hipStream_t);
 
 template <typename TE>
-void launch_fused_krylov_grouped(const KGroup<FusedKrylovArgs<TE>>& g, size_t lds, hipStream_t s) {
+void launch_fused_krylov_grouped(const KGroup<FusedKrylovArgs<TE>>& g, long max_n, size_t lds, hipStream_t s) {
   if (g.empty()) return;
-  ensure_dynamic_lds((const void*)fused_krylov_grouped<TE>, lds);
-  hipLaunchKernelGGL(fused_krylov_grouped<TE>, dim3(g.l.blocks), dim3(FK_THREADS), lds, s, g.l.recs, g.l.n);
+  auto run = [&](auto kernel) {
+    ensure_dynamic_lds((const void*)kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3(g.l.blocks), dim3(FK_THREADS), lds, s, g.l.recs, g.l.n);
+  };
+  if (max_n <= FK_SMALL_N) run(fused_krylov_grouped<TE, 2>);
+  else run(fused_krylov_grouped<TE, FK_EPT_MAX>);
   QCA_HIP(hipGetLastError());
 }
-template void launch_fused_krylov_grouped<double>(const KGroup<FusedKrylovArgs<double>>&, size_t, hipStream_t);
-template void launch_fused_krylov_grouped<float>(const KGroup<FusedKrylovArgs<float>>&, size_t, hipStream_t);
+template void launch_fused_krylov_grouped<double>(const KGroup<FusedKrylovArgs<double>>&, long, size_t, hipStream_t);
+template void launch_fused_krylov_grouped<float>(const KGroup<FusedKrylovArgs<float>>&, long, size_t, hipStream_t);
 
 }  // namespace qca

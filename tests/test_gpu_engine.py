@@ -137,6 +137,31 @@ def test_one_launch_krylov_equals_multi_launch(gpu, monkeypatch, prec):
     assert s1["flops"] > 0
 
 
+@pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("alg,d,chi", [("2tdvp", 1, 3), ("2tdvp", 1, 9), ("2tdvp", 1, 17), ("2tdvp", 1, 31),
+                                       ("2tdvp", 2, 16), ("2tdvp", 2, 24), ("1tdvp", 1, 32), ("1tdvp", 2, 15),
+                                       ("1tdvp", 2, 33)])
+def test_one_launch_krylov_placements(gpu, alg, d, chi, prec):
+    """The one-launch exponential with its operands in LDS, in part, or in global
+    memory, and blocks on and off the 16 x 16 tiles (bonds 1..33, MPO bonds 6
+    and 13), against the multi-launch one within the bounds of
+    test_one_launch_krylov_equals_multi_launch."""
+    n = 11
+    runs = []
+    for limit in (0, 4096):
+        e = make_engine(initial("padded", n, chi), AU.mpo_tensors(n, d, range(d, 2 * d + 1)), ALG_CODE[alg], chi,
+                        0.1, 1e-10, prec=prec)
+        e.set_fused_krylov_limit(limit)
+        runs.append(gpu_trajectory(e, 3))
+        e.close()
+    (p0, b0), (p1, b1) = runs
+    if prec == 0:
+        assert np.array_equal(b0, b1)
+        assert np.abs(p0 - p1).max() < 1e-12
+    else:
+        assert np.abs(p0 - p1).max() < 1e-6
+
+
 def check_against_oracle(case):
     alg, n, d, iv, kind, dt, steps, chi, eps = case
     As = initial(kind, n, chi)
