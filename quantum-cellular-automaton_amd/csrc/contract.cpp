@@ -66,6 +66,7 @@ ContractPlan<T> heff_plan(int kind, const cplx<T>* x, cplx<T>* y, const cplx<T>*
   g.a_m = 1; g.a_k2 = chir; g.a_b1 = lr;
   g.b_k2 = (long)Din * chil; g.b_n = 1; g.b_b2 = chil;
   g.c_m = chil; g.c_n = 1; g.c_b1 = (long)Din * lr; g.c_b2 = lr;
+  g.batch_used = W->used;
   g.skip = skip;
   p.g1 = GemmJob<T>{g, x, L, ws.T1, ws.splitk, ws.splitk_elems};
   // GEMM3 with the MPO mixing gathered into its K loop:
@@ -281,8 +282,8 @@ void WSparsePair::upload(const HostSparse& h, int nin) {
   d32.outv = d64.outv;
   d64.group_rows = d32.group_rows = h.group_rows;
   d64.group_max = d32.group_max = h.group_max;
-  set_group_starts(d64, h.rowptr, h.group_rows);
-  set_group_starts(d32, h.rowptr, h.group_rows);
+  set_group_starts(d64, h.rowptr, h.col, nin, h.group_rows);
+  set_group_starts(d32, h.rowptr, h.col, nin, h.group_rows);
   d64.nout = d32.nout = nout;
   d64.nin = d32.nin = nin;
   d64.nnz = d32.nnz = nnz;

@@ -4,8 +4,8 @@
 // and the mixed path (complex64 on v_mfma_f32_16x16x4f32).  A complex product
 // is four real MFMAs on planar (re, im) LDS tiles:
 //   Cre += Are*Bre - Aim*Bim,   Cim += Are*Bim + Aim*Bre.
-// Tile 64x64x16, 256 threads = 4 wave64s in a 2x2 grid, each wave owning a
-// 32x32 block = 2x2 MFMA 16x16 tiles.  Operands are read with generic two-level
+// Tiles of 64x64x16 or 32x32x16, 256 threads = 4 wave64s in a 2x2 grid, each wave
+// owning 2x2 or one MFMA tile of 16x16.  Operands are read with generic two-level
 // strides (see GemmDesc) so that every TDVP contraction is a single launch with
 // no permutation copies; the load loop walks the unit-stride index so global
 // reads stay coalesced; the next K-tile is loaded into registers while the
@@ -13,7 +13,12 @@
 // lets the MPO mixing of the effective Hamiltonian be gathered into the
 // operand loads (GemmDesc's gather form) instead of a separate pass.
 // Launches with too few output tiles to fill 256 CUs split K and reduce the
-// partial tiles in a second, deterministic pass.
+// partial tiles in a second, deterministic pass.  Tile side and splits come from a
+// model of the launch time (gemm_time).
+// What bounds it: at large sizes the matrix rate and whole rounds over the CUs (a
+// 64x64x128 FP32 tile takes 6.8 us of MFMAs, 3.4 us of staging that the barrier
+// keeps out of step with them, 4.3 us of first loads, exchange and stores), at
+// small sizes the latency of one workgroup and of the reduce launch.
 #include <cstdlib>
 
 #include "grouped.hpp"
@@ -21,8 +26,7 @@
 namespace qca {
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16;
-constexpr int LOADS = BM * BK / 256;  // operand elements per thread per K-tile
+constexpr int BK = 16;   // k of a K-tile
 
 template <typename T>
 struct Mfma;
@@ -54,10 +58,10 @@ struct Mfma<float> {
 // the coalesced loads and the MFMA operand reads (16 consecutive mn at each of
 // 4 k per wave) free of bank conflicts: LDS serves a wave64 b32 access 32
 // lanes per cycle and a b64 access 16 lanes per cycle over 32 banks.
-template <typename T, bool MNCONT>
+template <typename T, bool MNCONT, int TS>
 struct Plane {
-  static constexpr int LS = MNCONT ? (sizeof(T) == 4 ? BM + 16 : BM) : (sizeof(T) == 4 ? BK + 2 : BK + 1);
-  static constexpr int SIZE = MNCONT ? BK * LS : BM * LS;
+  static constexpr int LS = MNCONT ? (sizeof(T) == 4 ? TS + 16 : TS) : (sizeof(T) == 4 ? BK + 2 : BK + 1);
+  static constexpr int SIZE = MNCONT ? BK * LS : TS * LS;
   static __device__ __forceinline__ int at(int k, int mn) { return MNCONT ? k * LS + mn : mn * LS + k; }
 };
 
@@ -81,18 +85,20 @@ __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
 // registers during iteration i-1 is stored into stage i%2 while stage
 // (i-1)%2 may still be read, so one barrier per K-tile suffices, and the
 // global loads of tile i+1 are in flight during the MFMAs of tile i.
-template <typename T, bool A_MCONT, bool B_NCONT, int KG, bool FUSED>
+template <typename T, bool A_MCONT, bool B_NCONT, int TS, int KG, bool FUSED>
 __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __restrict__ A,
                                           const cplx<T>* __restrict__ B, cplx<T>* __restrict__ C,
                                           cplx<T>* __restrict__ ws, int splits, int tiles_per_split,
                                           unsigned bx, unsigned by, unsigned bz) {
   constexpr bool fused = FUSED;
   using acc_t = typename Mfma<T>::acc_t;
-  using PA = Plane<T, A_MCONT>;
-  using PB = Plane<T, B_NCONT>;
+  constexpr int MI = TS / 32;                // 16x16 tiles per wave and dimension
+  constexpr int LOADS = TS * BK / 256;       // operand elements per thread per K-tile
+  using PA = Plane<T, A_MCONT, TS>;
+  using PB = Plane<T, B_NCONT, TS>;
   constexpr int STAGE = 2 * PA::SIZE + 2 * PB::SIZE;  // [A re, A im, B re, B im]
   __shared__ T smem[KG * 2 * STAGE];
-  static_assert(KG == 1 || KG * 2 * STAGE >= 4 * 32 * 64, "partial-tile exchange fits the operand LDS");
+  static_assert(KG == 1 || KG * 2 * STAGE >= 4 * 8 * MI * MI * 64, "partial-tile exchange fits the operand LDS");
   // the skip word is read here and tested once the first tile's loads are in
   // flight: the two memory latencies overlap (a skipped launch only loads)
   const int skipped = d.skip ? *d.skip : 0;
@@ -103,15 +109,19 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = (wave >> 1) * 32;
-  const int wn = (wave & 1) * 32;
-  const int m0 = by * BM;
-  const int n0 = bx * BN;
+  const int wm = (wave >> 1) * (16 * MI);
+  const int wn = (wave & 1) * (16 * MI);
+  const int m0 = by * TS;
+  const int n0 = bx * TS;
   // fused: this workgroup takes every split of its output tile in turn (bz is
   // the batch) and sums them in split order itself; otherwise bz = batch *
   // splits + split and the partial tile goes to the split-K workspace
   const int zb = fused ? (int)bz : (int)bz / splits;
   const int split = fused ? 0 : (int)bz - zb * splits;
+  // nobody reads this batch (64x64 tiles fill one round of the CUs with or without
+  // such batches, and the test costs 0.3 us)
+  if constexpr (TS == 32)
+    if (d.batch_used && !(d.batch_used >> zb & 1)) return;
   const int b1 = zb / d.NB2;
   const int b2 = zb - b1 * d.NB2;
 
@@ -159,10 +169,10 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
 #pragma unroll
   for (int r = 0; r < LOADS; ++r) {
     const int e = tid + 256 * r;
-    const int ml = A_MCONT ? (e % BM) : (e / BK);
-    const int ka = A_MCONT ? (e / BM) : (e % BK);
-    const int nl = B_NCONT ? (e % BN) : (e / BK);
-    const int kb = B_NCONT ? (e / BN) : (e % BK);
+    const int ml = A_MCONT ? (e % TS) : (e / BK);
+    const int ka = A_MCONT ? (e / TS) : (e % BK);
+    const int nl = B_NCONT ? (e % TS) : (e / BK);
+    const int kb = B_NCONT ? (e / TS) : (e % BK);
     oka[r] = m0 + ml < d.M;
     okb[r] = n0 + nl < d.N;
     kla[r] = ka;
@@ -171,11 +181,11 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
     offb[r] = (unsigned)(nl * d.b_n + kb * d.b_k2);
   }
 
-  acc_t acc_re[2][2], acc_im[2][2];
+  acc_t acc_re[MI][MI], acc_im[MI][MI];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < MI; ++j) {
       acc_re[i][j] = acc_t{0, 0, 0, 0};
       acc_im[i][j] = acc_t{0, 0, 0, 0};
     }
@@ -237,15 +247,15 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
 
   auto stage_ptr = [&](int stage) { return smem + (grp * 2 + stage) * STAGE; };
 
-  acc_t tot_re[2][2], tot_im[2][2];   // fused: sum of the finished splits
+  acc_t tot_re[MI][MI], tot_im[MI][MI];   // fused: sum of the finished splits
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < MI; ++j) {
       tot_re[i][j] = acc_t{0, 0, 0, 0};
       tot_im[i][j] = acc_t{0, 0, 0, 0};
     }
-  T* const xs = smem + (wave * 32) * 64 + lane;  // partial-tile exchange: [wave][value][lane]
+  T* const xs = smem + (wave * 8 * MI * MI) * 64 + lane;  // partial-tile exchange: [wave][value][lane]
 
   load_tile(ch_begin < ch_end ? tile_at(ch_begin, 0) : -1);
   if (skipped) return;
@@ -264,8 +274,8 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
 #pragma unroll
       for (int r = 0; r < LOADS; ++r) {
         const int e = tid + 256 * r;
-        const int ml = A_MCONT ? (e % BM) : (e / BK);
-        const int kl = A_MCONT ? (e / BM) : (e % BK);
+        const int ml = A_MCONT ? (e % TS) : (e / BK);
+        const int kl = A_MCONT ? (e / TS) : (e % BK);
         const cplx<T> v = gather ? cmul(pa[r], w) : pa[r];
         a_re[PA::at(kl, ml)] = v.re;
         a_im[PA::at(kl, ml)] = sa * v.im;
@@ -273,8 +283,8 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
 #pragma unroll
       for (int r = 0; r < LOADS; ++r) {
         const int e = tid + 256 * r;
-        const int nl = B_NCONT ? (e % BN) : (e / BK);
-        const int kl = B_NCONT ? (e / BN) : (e % BK);
+        const int nl = B_NCONT ? (e % TS) : (e / BK);
+        const int kl = B_NCONT ? (e / TS) : (e % BK);
         b_re[PB::at(kl, nl)] = pb[r].re;
         b_im[PB::at(kl, nl)] = sb * pb[r].im;
       }
@@ -298,11 +308,11 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
       if (t >= 0) {
         const int c = lane & 15;
         const int q = lane >> 4;
-        T ar[4][2], ai[4][2], br[4][2], bi[4][2];
+        T ar[4][MI], ai[4][MI], br[4][MI], bi[4][MI];
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
+          for (int i = 0; i < MI; ++i) {
             ar[kk][i] = a_re[PA::at(4 * kk + q, wm + 16 * i + c)];
             ai[kk][i] = a_im[PA::at(4 * kk + q, wm + 16 * i + c)];
             br[kk][i] = b_re[PB::at(4 * kk + q, wn + 16 * i + c)];
@@ -311,16 +321,16 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+          for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < MI; ++j) {
               acc_re[i][j] = Mfma<T>::mac(ar[kk][i], br[kk][j], acc_re[i][j]);
               acc_im[i][j] = Mfma<T>::mac(ar[kk][i], bi[kk][j], acc_im[i][j]);
             }
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+          for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < MI; ++j) {
               acc_re[i][j] = Mfma<T>::mac(-ai[kk][i], bi[kk][j], acc_re[i][j]);
               acc_im[i][j] = Mfma<T>::mac(ai[kk][i], br[kk][j], acc_im[i][j]);
             }
@@ -335,25 +345,25 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
       __syncthreads();
       if (grp == 1) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < MI; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              xs[(((i * 2 + j) * 4 + r) * 2 + 0) * 64] = acc_re[i][j][r];
-              xs[(((i * 2 + j) * 4 + r) * 2 + 1) * 64] = acc_im[i][j][r];
+              xs[(((i * MI + j) * 4 + r) * 2 + 0) * 64] = acc_re[i][j][r];
+              xs[(((i * MI + j) * 4 + r) * 2 + 1) * 64] = acc_im[i][j][r];
             }
       }
       __syncthreads();
       if (grp == 0) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < MI; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              acc_re[i][j][r] += xs[(((i * 2 + j) * 4 + r) * 2 + 0) * 64];
-              acc_im[i][j][r] += xs[(((i * 2 + j) * 4 + r) * 2 + 1) * 64];
+              acc_re[i][j][r] += xs[(((i * MI + j) * 4 + r) * 2 + 0) * 64];
+              acc_im[i][j][r] += xs[(((i * MI + j) * 4 + r) * 2 + 1) * 64];
             }
       }
       __syncthreads();
@@ -361,9 +371,9 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
     if (fused) {
       // the split's partial tile joins the sum in split order, as splitk_reduce adds it
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < MI; ++j) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             tot_re[i][j][r] += acc_re[i][j][r];
@@ -389,9 +399,9 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
   if (grp == 0) {
     const int col = lane & 15;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < MI; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int m = m0 + wm + 16 * i + Mfma<T>::row(lane, r);
@@ -408,13 +418,13 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
   }
 }
 
-template <typename T, bool A_MCONT, bool B_NCONT, int KG>
+template <typename T, bool A_MCONT, bool B_NCONT, int TS, int KG>
 __global__ __launch_bounds__(256 * KG) void gemm_kernel(GemmDesc d, const cplx<T>* __restrict__ A,
                                                         const cplx<T>* __restrict__ B,
                                                         cplx<T>* __restrict__ C,
                                                         cplx<T>* __restrict__ ws, int splits,
                                                         int tiles_per_split) {
-  gemm_body<T, A_MCONT, B_NCONT, KG, false>(d, A, B, C, ws, splits, tiles_per_split, blockIdx.x, blockIdx.y,
+  gemm_body<T, A_MCONT, B_NCONT, TS, KG, false>(d, A, B, C, ws, splits, tiles_per_split, blockIdx.x, blockIdx.y,
                                             blockIdx.z);
 }
 
@@ -473,17 +483,41 @@ __global__ void splitk_reduce(GemmDesc d, const cplx<T>* __restrict__ ws, cplx<T
 // workspace only (so a GEMM computes the same whether launched alone or
 // grouped with others).
 // Output tiles of a grouped GEMM launch from which split GEMMs run fused (one
-// workgroup per output tile over all splits): four per CU.
+// workgroup per output tile over all splits): four per CU (512 and 4096: no
+// difference in a group of eight).
 constexpr long GEMM_GROUP_FUSE_TILES = 1024;
+
+// Time in us of a GEMM of `tiles` tiles with side ts and `ktiles` K-tiles under
+// `splits` splits: what the choice of tile and splits minimises.  A 32x32 tile takes
+// 0.22 us (FP32) or 0.46 (FP64) of a CU per K-tile at the matrix rate and a third to
+// 40% more with its operand traffic, a 64x64 one four times the matrix time; a
+// workgroup alone on its CU is bound by latency (0.8 us), and a split costs a
+// reduce launch.  The small tile wins where 64x64 tiles pad (203 -> 256), come in
+// uneven rounds or are too few to go without splits (one-site block of 64: 31.4
+// -> 19.7 us, two-site FP64 of 64: 36.0 -> 20.9, bond block of 16: 20.8 -> 14.0,
+// environments of 117x96: 53.4 -> 38.3 and 256x200: 188 -> 150, two-site FP32 of
+// 160x150: 88 -> 70, one-site FP64 of 203x256: 146 -> 125); the large one at 128
+// and 256 (two-site FP32 of 128: 38.7 against 40.5 with small tiles only, bond
+// block of 256: 92 against 97).
+constexpr int GEMM_CUS = 256;
+constexpr double GEMM_LAT = 0.8, COST32_F64 = 1.33, COST32_F32 = 1.42, REDUCE_US = 6.5, REDUCE_BW = 3e6;
+double gemm_time(int ts, long tiles, long ktiles, long splits, long out_bytes, bool fp64) {
+  const double unit = (fp64 ? 0.46 : 0.22) * (ts == 32 ? (fp64 ? COST32_F64 : COST32_F32) : 4.0);
+  const long rounds = ceil_div(tiles * splits, GEMM_CUS), kps = ceil_div(ktiles, splits);
+  const int kg = ts == 64 && kps >= 4 ? 2 : 1;
+  const double t = ceil_div(kps, kg) * std::max(rounds * kg * unit, GEMM_LAT);
+  return splits > 1 ? t + REDUCE_US + (double)splits * out_bytes / REDUCE_BW : t;
+}
 
 struct GemmPlan {
   bool empty = false;
   int tm = 0, tn = 0, batch = 1, splits = 1, kps = 0;
+  int ts = 0;   // tile side
   bool am = false, bn = false, kg2 = false;
   int reduce_blocks = 0;
 };
 
-GemmPlan gemm_plan(const GemmDesc& d, long ws_elems) {
+GemmPlan gemm_plan(const GemmDesc& d, long ws_elems, bool fp64) {
   QCA_CHECK(d.M >= 0 && d.N >= 0 && d.K >= 0, "negative GEMM extent");
   QCA_CHECK(d.K2 >= 1 && (d.K == 0 || d.K % d.K2 == 0), "K2 must divide K");
   QCA_CHECK(d.NB1 >= 1 && d.NB2 >= 1, "empty batch");
@@ -497,7 +531,7 @@ GemmPlan gemm_plan(const GemmDesc& d, long ws_elems) {
   // per-thread element offsets within a tile are 32-bit and non-negative
   QCA_CHECK(d.a_m >= 0 && d.a_k2 >= 0 && d.b_n >= 0 && d.b_k2 >= 0 && d.a_k1 >= 0 && d.b_k1 >= 0,
             "GEMM strides must be non-negative");
-  QCA_CHECK((BM - 1) * d.a_m + (BK - 1) * d.a_k2 < (1L << 31) && (BN - 1) * d.b_n + (BK - 1) * d.b_k2 < (1L << 31),
+  QCA_CHECK((64 - 1) * d.a_m + (BK - 1) * d.a_k2 < (1L << 31) && (64 - 1) * d.b_n + (BK - 1) * d.b_k2 < (1L << 31),
             "GEMM tile spans more than 2^31 elements");
   GemmPlan p;
   p.batch = d.NB1 * d.NB2;
@@ -505,19 +539,32 @@ GemmPlan gemm_plan(const GemmDesc& d, long ws_elems) {
     p.empty = true;
     return p;
   }
-  p.tm = ceil_div(d.M, BM);
-  p.tn = ceil_div(d.N, BN);
-  const long tiles = (long)p.tm * p.tn * p.batch;
+  QCA_CHECK(!d.batch_used || p.batch <= 64, "a batch mask covers at most 64 batches");
+  const int used = d.batch_used ? __builtin_popcountll(d.batch_used) : p.batch;
   // K-tiles of the longest batch: segments of K2, each cut into BK tiles
   const long ktiles = (long)(d.K / d.K2) * ceil_div(d.K2, BK);
   QCA_CHECK(ktiles < (1L << 30), "GEMM K too long");
-  // split K when the output tiles alone cannot occupy the chip
+  const long out_elems = (long)p.batch * d.M * d.N, out_bytes = out_elems * (fp64 ? 16 : 8);
+  // tile side and splits of K: the best of every tile under a few fills
   int splits = 1;
-  if (tiles < 192 && ktiles >= 4) {
-    splits = (int)std::min<long>((256 + tiles - 1) / tiles, ktiles / 2);
-    while (splits > 1 && (long)splits * p.batch * d.M * d.N > ws_elems) --splits;
-    if (splits < 1) splits = 1;
+  double best = 0;
+  p.ts = 0;
+  for (int ts : {64, 32}) {
+    const long tiles = (long)ceil_div(d.M, ts) * ceil_div(d.N, ts) * (ts == 32 ? used : p.batch);
+    for (long fill : {0, GEMM_CUS, 2 * GEMM_CUS, 3 * GEMM_CUS}) {   // workgroups that splits bring it to
+      long sp = ktiles >= 4 && tiles < fill ? std::min<long>(ceil_div(fill, tiles), ktiles / 2) : 1;
+      while (sp > 1 && sp * out_elems > ws_elems) --sp;
+      const double t = gemm_time(ts, tiles, ktiles, sp, out_bytes, fp64);
+      if (p.ts == 0 || t < best) {
+        best = t;
+        p.ts = ts;
+        splits = (int)sp;
+      }
+    }
   }
+  p.tm = ceil_div(d.M, p.ts);
+  p.tn = ceil_div(d.N, p.ts);
+  const long tiles = (long)p.tm * p.tn * p.batch;
   int kps = (int)ktiles;  // K-tiles per split
   if (splits > 1) {
     kps = ceil_div(ktiles, splits);
@@ -530,7 +577,7 @@ GemmPlan gemm_plan(const GemmDesc& d, long ws_elems) {
   p.am = (d.a_m == 1);
   p.bn = (d.b_n == 1);
   // two K-groups per workgroup when each has at least two K-tiles to take
-  p.kg2 = kps >= 4;
+  p.kg2 = p.ts == 64 && kps >= 4;
   if (splits > 1) {
     const long total = (long)d.M * d.N * p.batch;
     p.reduce_blocks = (int)std::min<long>(ceil_div(total, 256), 4096);
@@ -541,18 +588,21 @@ GemmPlan gemm_plan(const GemmDesc& d, long ws_elems) {
 template <typename T>
 void gemm_launch(const GemmDesc& d, const cplx<T>* A, const cplx<T>* B, cplx<T>* C,
                  hipStream_t s, cplx<T>* ws, long ws_elems) {
-  const GemmPlan p = gemm_plan(d, ws_elems);
+  const GemmPlan p = gemm_plan(d, ws_elems, sizeof(T) == 8);
   if (p.empty) return;
   const int splits = p.splits, kps = p.kps;
   dim3 grid(p.tn, p.tm, p.batch * splits);
   const bool am = p.am, bn = p.bn, kg2 = p.kg2;
 #define QCA_GEMM_L(AM, BNC)                                                                     \
   do {                                                                                         \
-    if (kg2)                                                                                   \
-      hipLaunchKernelGGL((gemm_kernel<T, AM, BNC, 2>), grid, dim3(512), 0, s, d, A, B, C, ws,  \
+    if (p.ts == 32)                                                                             \
+      hipLaunchKernelGGL((gemm_kernel<T, AM, BNC, 32, 1>), grid, dim3(256), 0, s, d, A, B, C, ws, \
+                         splits, kps);                                                         \
+    else if (kg2)                                                                                   \
+      hipLaunchKernelGGL((gemm_kernel<T, AM, BNC, 64, 2>), grid, dim3(512), 0, s, d, A, B, C, ws,  \
                          splits, kps);                                                         \
     else                                                                                       \
-      hipLaunchKernelGGL((gemm_kernel<T, AM, BNC, 1>), grid, dim3(256), 0, s, d, A, B, C, ws,  \
+      hipLaunchKernelGGL((gemm_kernel<T, AM, BNC, 64, 1>), grid, dim3(256), 0, s, d, A, B, C, ws,  \
                          splits, kps);                                                         \
   } while (0)
   if (am && bn) QCA_GEMM_L(true, true);
@@ -579,13 +629,13 @@ __device__ __forceinline__ GemmDesc global_desc(GemmDesc d) {
   return d;
 }
 
-template <typename T, bool A_MCONT, bool B_NCONT, int KG, bool FUSED>
+template <typename T, bool A_MCONT, bool B_NCONT, int TS, int KG, bool FUSED>
 __global__ __launch_bounds__(256 * KG) void gemm_grouped_kernel(const GRec<GemmArgs<T>>* __restrict__ recs,
                                                                 int n, int j) {
   unsigned bx, by, bz;
   const GRec<GemmArgs<T>>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
   const GemmDesc d = global_desc(r.a.d);
-  gemm_body<T, A_MCONT, B_NCONT, KG, FUSED>(d, gbl(r.a.A + (long)j * r.a.a_jstride),
+  gemm_body<T, A_MCONT, B_NCONT, TS, KG, FUSED>(d, gbl(r.a.A + (long)j * r.a.a_jstride),
                                             gbl(r.a.B + (long)j * r.a.b_jstride), gbl(r.a.C),
                                             gbl(r.a.ws), r.a.splits, r.a.kps, bx, by, bz);
 }
@@ -602,7 +652,7 @@ __global__ void splitk_reduce_grouped(const GRec<GemmArgs<T>>* __restrict__ recs
 
 template <typename T>
 void GemmGroup<T>::prepare(const std::vector<GemmJob<T>>& jobs, RecordArena& arena) {
-  std::vector<GRec<GemmArgs<T>>> var[16], red;
+  std::vector<GRec<GemmArgs<T>>> var[24], red;
   // A GEMM's splits (and K-groups) are fixed by its own plan, so that it sums
   // in the same order whether launched alone or grouped.  When the group's
   // output tiles alone fill the GPU, each split GEMM runs one workgroup per
@@ -611,7 +661,7 @@ void GemmGroup<T>::prepare(const std::vector<GemmJob<T>>& jobs, RecordArena& are
   // without the partial tiles' round trip through memory and the reduce.
   long out_tiles = 0;
   for (const auto& j : jobs) {
-    const GemmPlan p = gemm_plan(j.d, j.ws_elems);
+    const GemmPlan p = gemm_plan(j.d, j.ws_elems, sizeof(T) == 8);
     if (!p.empty) out_tiles += (long)p.tm * p.tn * p.batch;
   }
   // QCA_GEMM_GROUP_FUSE_TILES overrides the threshold (0: always), so that the
@@ -620,7 +670,7 @@ void GemmGroup<T>::prepare(const std::vector<GemmJob<T>>& jobs, RecordArena& are
   if (const char* e = std::getenv("QCA_GEMM_GROUP_FUSE_TILES")) fuse_tiles = std::atol(e);
   const bool fuse = out_tiles >= fuse_tiles;
   for (const auto& j : jobs) {
-    const GemmPlan p = gemm_plan(j.d, j.ws_elems);
+    const GemmPlan p = gemm_plan(j.d, j.ws_elems, sizeof(T) == 8);
     if (p.empty) continue;
     GRec<GemmArgs<T>> r{};
     r.a.d = j.d;
@@ -636,14 +686,14 @@ void GemmGroup<T>::prepare(const std::vector<GemmJob<T>>& jobs, RecordArena& are
     r.grid.x = p.tn;
     r.grid.y = p.tm;
     r.grid.z = r.a.fused ? p.batch : p.batch * p.splits;
-    var[(p.am ? 8 : 0) + (p.bn ? 4 : 0) + (p.kg2 ? 2 : 0) + r.a.fused].push_back(r);
+    var[((p.am ? 2 : 0) + (p.bn ? 1 : 0)) * 6 + (p.ts == 32 ? 4 : p.kg2 ? 2 : 0) + r.a.fused].push_back(r);
     if (p.splits > 1 && !r.a.fused) {
       r.grid = VGrid{};
       r.grid.x = p.reduce_blocks;
       red.push_back(r);
     }
   }
-  for (int v = 0; v < 16; ++v) {
+  for (int v = 0; v < 24; ++v) {
     launches[v].n = (int)var[v].size();
     launches[v].blocks = grec_layout(var[v]);
     launches[v].recs = var[v].empty() ? nullptr : arena.push(var[v]);
@@ -655,26 +705,34 @@ void GemmGroup<T>::prepare(const std::vector<GemmJob<T>>& jobs, RecordArena& are
 
 template <typename T>
 void GemmGroup<T>::launch(hipStream_t s, int j) const {
-#define QCA_GG_L(V, AM, BNC, KG, F)                                                            \
+#define QCA_GG_L(V, AM, BNC, TS, KG, F)                                                        \
   if (launches[V].n)                                                                          \
-    hipLaunchKernelGGL((gemm_grouped_kernel<T, AM, BNC, KG, F>), dim3(launches[V].blocks),     \
+    hipLaunchKernelGGL((gemm_grouped_kernel<T, AM, BNC, TS, KG, F>), dim3(launches[V].blocks), \
                        dim3(256 * KG), 0, s, launches[V].recs, launches[V].n, j);
-  QCA_GG_L(0, false, false, 1, false)
-  QCA_GG_L(1, false, false, 1, true)
-  QCA_GG_L(2, false, false, 2, false)
-  QCA_GG_L(3, false, false, 2, true)
-  QCA_GG_L(4, false, true, 1, false)
-  QCA_GG_L(5, false, true, 1, true)
-  QCA_GG_L(6, false, true, 2, false)
-  QCA_GG_L(7, false, true, 2, true)
-  QCA_GG_L(8, true, false, 1, false)
-  QCA_GG_L(9, true, false, 1, true)
-  QCA_GG_L(10, true, false, 2, false)
-  QCA_GG_L(11, true, false, 2, true)
-  QCA_GG_L(12, true, true, 1, false)
-  QCA_GG_L(13, true, true, 1, true)
-  QCA_GG_L(14, true, true, 2, false)
-  QCA_GG_L(15, true, true, 2, true)
+  QCA_GG_L(0, false, false, 64, 1, false)
+  QCA_GG_L(1, false, false, 64, 1, true)
+  QCA_GG_L(2, false, false, 64, 2, false)
+  QCA_GG_L(3, false, false, 64, 2, true)
+  QCA_GG_L(4, false, false, 32, 1, false)
+  QCA_GG_L(5, false, false, 32, 1, true)
+  QCA_GG_L(6, false, true, 64, 1, false)
+  QCA_GG_L(7, false, true, 64, 1, true)
+  QCA_GG_L(8, false, true, 64, 2, false)
+  QCA_GG_L(9, false, true, 64, 2, true)
+  QCA_GG_L(10, false, true, 32, 1, false)
+  QCA_GG_L(11, false, true, 32, 1, true)
+  QCA_GG_L(12, true, false, 64, 1, false)
+  QCA_GG_L(13, true, false, 64, 1, true)
+  QCA_GG_L(14, true, false, 64, 2, false)
+  QCA_GG_L(15, true, false, 64, 2, true)
+  QCA_GG_L(16, true, false, 32, 1, false)
+  QCA_GG_L(17, true, false, 32, 1, true)
+  QCA_GG_L(18, true, true, 64, 1, false)
+  QCA_GG_L(19, true, true, 64, 1, true)
+  QCA_GG_L(20, true, true, 64, 2, false)
+  QCA_GG_L(21, true, true, 64, 2, true)
+  QCA_GG_L(22, true, true, 32, 1, false)
+  QCA_GG_L(23, true, true, 32, 1, true)
 #undef QCA_GG_L
   QCA_HIP(hipGetLastError());
   if (reduce.n) {

@@ -147,7 +147,7 @@ struct GLaunch {
 // arena has been uploaded.
 template <typename T>
 struct GemmGroup {
-  GLaunch<GemmArgs<T>> launches[16];   // by (A m-contiguous, B n-contiguous, two K-groups, fused)
+  GLaunch<GemmArgs<T>> launches[24];   // by (A m-contiguous, B n-contiguous, tile and K-groups, fused)
   GLaunch<GemmArgs<T>> reduce;
   void prepare(const std::vector<GemmJob<T>>& jobs, RecordArena& arena);
   void launch(hipStream_t s, int j = 0) const;

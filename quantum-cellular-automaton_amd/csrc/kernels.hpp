@@ -52,10 +52,15 @@ struct WSparseDev {
   int group_max = 0;     // most nonzeros in any group of group_rows rows
   int ngroups = 0;       // nout / group_rows when at most SEG_STARTS_MAX, else 0
   int group_start[SEG_STARTS_MAX + 1] = {};  // rowptr[g * group_rows], g <= ngroups
+  unsigned long long used = 0;   // columns with an entry, as bits (0: more than 64 columns)
 };
-// Fills ngroups and group_start of w from the host row pointer.
+// Fills ngroups, group_start and used of w from the host row pointer and columns.
 template <typename T>
-inline void set_group_starts(WSparseDev<T>& w, const std::vector<int>& rowptr, int group_rows) {
+inline void set_group_starts(WSparseDev<T>& w, const std::vector<int>& rowptr, const std::vector<int>& col, int nin,
+                             int group_rows) {
+  w.used = 0;
+  if (nin <= 64)
+    for (int c : col) w.used |= 1ull << c;
   const int nout = (int)rowptr.size() - 1;
   w.ngroups = 0;
   if (group_rows <= 0 || nout % group_rows != 0 || nout / group_rows > SEG_STARTS_MAX) return;

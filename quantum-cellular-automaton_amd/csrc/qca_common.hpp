@@ -99,6 +99,9 @@ struct GemmDesc {
   // from its arguments instead of from memory
   int seg_starts;
   int seg_start[SEG_STARTS_MAX + 1];
+  // bit b set: batch b (= b1 * NB2 + b2) is read by the caller, the others need not
+  // be computed; 0: every batch is
+  unsigned long long batch_used;
 };
 
 void gemm_c128(const GemmDesc& d, const c128* A, const c128* B, c128* C, hipStream_t s,

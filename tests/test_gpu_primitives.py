@@ -70,6 +70,15 @@ def test_heff_apply(gpu, prec, kind, chil, chir, rule):
 
 
 @pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("chil,chir,rule", [(31, 33, 1), (33, 64, 3), (65, 31, 1), (96, 97, 1), (160, 129, 3)])
+def test_heff_apply_tiles(gpu, prec, kind, chil, chir, rule):
+    """Blocks around the 32- and 64-wide tiles, on both sides of the choice between
+    them and with and without K splits, with MPO channels that no row reads."""
+    test_heff_apply(gpu, prec, kind, chil, chir, rule)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("side", [0, 1])
 @pytest.mark.parametrize("chil,chir", [(1, 2), (5, 7), (32, 64), (128, 128)])
 def test_env_update(gpu, prec, side, chil, chir):
