@@ -119,11 +119,10 @@ qca::LanczosWork lanczos_ws(long n, qca::LanczosCtrl** ctrl_host) {
   lw.ctrl = sbuf<qca::LanczosCtrl>("lz_ctrl", 1);
   lw.V = sbuf<qca::c128>("lz_V", (long)lw.max_m * n);
   lw.w64 = sbuf<qca::c128>("lz_w", n);
-  lw.part = sbuf<qca::c128>("lz_part", (long)lw.max_blocks * qca::LZ_MAXK);
+  lw.part = sbuf<qca::c128>("lz_part", lw.max_blocks);
   lw.part2 = sbuf<qca::c128>("lz_part2", (long)lw.max_blocks * qca::LZ_MAXK);
   lw.part_norm = sbuf<double>("lz_pnorm", lw.max_blocks);
-  lw.coef1 = sbuf<qca::c128>("lz_c1", qca::LZ_MAXK);
-  lw.coef2 = sbuf<qca::c128>("lz_c2", qca::LZ_MAXK);
+  lw.coef = sbuf<qca::c128>("lz_coef", qca::LZ_MAXK);
   // ordinary host memory: the control block is read once per exponential
   // after a stream synchronisation, and no HIP resource outlives the calls
   static thread_local qca::LanczosCtrl host;
@@ -133,11 +132,12 @@ qca::LanczosWork lanczos_ws(long n, qca::LanczosCtrl** ctrl_host) {
 
 // Runs the Krylov loop: mv(j, V_j) must enqueue w = H V_j and the iteration
 // tail.  Iterations j = 0 .. max_m-2 may run; the device closes the
-// exponential at the latest at dimension max_m-1.  x is overwritten with the
-// result.  Returns the Krylov dimension used.
+// exponential at the latest at dimension max_m-1.  v32: complex64 copy of V_0, or
+// null.  x is overwritten with the result.  Returns the Krylov dimension used.
 template <typename MV>
-int krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::LanczosCtrl* host, MV&& mv, hipStream_t s) {
-  qca::lanczos_begin(x, n, lw, s);
+int krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::LanczosCtrl* host, qca::c64* v32, MV&& mv,
+                hipStream_t s) {
+  qca::lanczos_begin(x, n, lw, s, v32);
   int j = 0, chunk = 8;
   while (true) {
     for (int c = 0; c < chunk && j < lw.max_m - 1; ++c, ++j) mv(j, lw.V + (long)j * n);
@@ -583,7 +583,7 @@ int qca_krylov_expm(int precision, int kind, void* x, const void* L, const void*
       if (precision == 0) {
         auto ws = contract_ws<double>(tsize, n);
         qca::c128* y = sbuf<qca::c128>("kr_y", n);
-        m = krylov_loop((qca::c128*)x, n, lw, host, [&](int j, const qca::c128* vj) {
+        m = krylov_loop((qca::c128*)x, n, lw, host, nullptr, [&](int j, const qca::c128* vj) {
           qca::heff_apply<double>(kind, vj, y, (const qca::c128*)L, (const qca::c128*)R,
                                   wp ? &wp->d64 : nullptr, Din, Dout, chil, chir, ws,
                                   qca::lanczos_done_flag(lw), s);
@@ -593,12 +593,12 @@ int qca_krylov_expm(int precision, int kind, void* x, const void* L, const void*
         auto ws = contract_ws<float>(tsize, n);
         qca::c64* x32 = sbuf<qca::c64>("kr_x32", n);
         qca::c64* y = sbuf<qca::c64>("kr_y32", n);
-        m = krylov_loop((qca::c128*)x, n, lw, host, [&](int j, const qca::c128* vj) {
-          qca::launch_convert_c128_c64(vj, x32, n, s, qca::lanczos_done_flag(lw));
+        // the Lanczos kernels write x32, the complex64 copy of each new basis vector
+        m = krylov_loop((qca::c128*)x, n, lw, host, x32, [&](int j, const qca::c128*) {
           qca::heff_apply<float>(kind, x32, y, (const qca::c64*)L, (const qca::c64*)R,
                                  wp ? &wp->d32 : nullptr, Din, Dout, chil, chir, ws,
                                  qca::lanczos_done_flag(lw), s);
-          qca::lanczos_iteration_tail<float>(y, n, j, tau, tl, lw, s);
+          qca::lanczos_iteration_tail<float>(y, n, j, tau, tl, lw, s, x32);
         }, s);
       }
       if (iters) *iters = m;

@@ -230,11 +230,10 @@ void Engine::init(const std::vector<const c128*>& W_host, const std::vector<int>
   lw_.ctrl = dmalloc<LanczosCtrl>(1);
   lw_.V = dmalloc<c128>((long)LZ_MAXK * nmax);
   lw_.w64 = dmalloc<c128>(nmax);
-  lw_.part = dmalloc<c128>((long)lw_.max_blocks * LZ_MAXK);
+  lw_.part = dmalloc<c128>(lw_.max_blocks);
   lw_.part2 = dmalloc<c128>((long)lw_.max_blocks * LZ_MAXK);
   lw_.part_norm = dmalloc<double>(lw_.max_blocks);
-  lw_.coef1 = dmalloc<c128>(LZ_MAXK);
-  lw_.coef2 = dmalloc<c128>(LZ_MAXK);
+  lw_.coef = dmalloc<c128>(LZ_MAXK);
   tally_ = dmalloc<KrylovTally>(1);
   if (!count_only_) QCA_HIP(hipMemset(tally_, 0, sizeof(KrylovTally)));
   fused_max_n_ = FUSED_KRYLOV_DEFAULT_N;

@@ -414,8 +414,7 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
     z.part = e->lw_.part;
     z.part2 = e->lw_.part2;
     z.part_norm = e->lw_.part_norm;
-    z.coef1 = e->lw_.coef1;
-    z.coef2 = e->lw_.coef2;
+    z.coef = e->lw_.coef;
     z.n = n[i];
     z.nblk = lanczos_nblk(n[i]);
     QCA_CHECK(z.nblk <= e->lw_.max_blocks, "Lanczos vector longer than the workspace");

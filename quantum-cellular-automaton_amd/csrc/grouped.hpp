@@ -287,8 +287,7 @@ struct LzArgs {
   c128* part;
   c128* part2;
   double* part_norm;
-  c128* coef1;
-  c128* coef2;
+  c128* coef;
   const void* w;          // matvec output, cplx<TW>
   c64* v32;               // complex64 copy of each new basis vector (mixed path) or null
   long n;
@@ -300,13 +299,13 @@ struct LzArgs {
 // The Krylov exponentials of many instances in lockstep: the same kernels
 // and reductions as lanczos_begin / lanczos_iteration_tail / lanczos_finish.
 struct LzGroup {
-  KGroup<LzArgs> nb, gf, one;   // grids lanczos_nblk(n), grid_for(n), 1
+  KGroup<LzArgs> nb, gf;   // grids lanczos_nblk(n), grid_for(n)
   void prepare(const std::vector<LzArgs>& jobs, RecordArena& arena);
   void begin(hipStream_t s) const;
   template <typename TW>
   void tail(int j, hipStream_t s) const;
   void finish(hipStream_t s) const;
-  bool empty() const { return one.empty(); }
+  bool empty() const { return nb.empty(); }
 };
 
 // out[i * words + w] = ((const unsigned long long*)src[i])[w], w < words:

@@ -264,17 +264,26 @@ __global__ void qr_gather_right(const c128* __restrict__ Q, const c128* __restri
 }
 
 // ------------------------------------------------------------------ lanczos
-constexpr int LZ_BLOCK = 256;
-constexpr int LZ_EPT = 1;                     // vector elements per thread
-constexpr int LZ_ELEMS = LZ_BLOCK * LZ_EPT;   // elements per block in the partial reductions
+// Per iteration three launches after the matvec: lz_dot, <V_j, w>; lz_three_term,
+// w <- w - c V_j - beta_{j-1} V_{j-1} with the partial projections of the result
+// on the whole basis and its partial norm; lz_next, the Gram-Schmidt pass with
+// those, normalisation and the stopping test.  What the three-term step leaves
+// along the older vectors is rounding (of the matvec's precision), so one pass
+// restores orthogonality, and beta^2 = |w|^2 - sum |c_i|^2 loses nothing.  Two
+// full Gram-Schmidt passes with the norm between launches took four launches and
+// twice the basis traffic: 22.8 us an iteration at 65536 elements (12 vectors), 3.4 +
+// 5.4 + 6.1 us here; what bounds these is launch and memory latency, not traffic.
+// Sums over the blocks are taken by every block that needs them, in one fixed
+// order: no reduction launch.
+constexpr int LZ_BLOCK = 256;   // one vector element per thread
+constexpr int LZ_NORM = LZ_MAXK - 1;   // row of the partial sums that holds |w|^2 (j < LZ_NORM)
 
 __device__ __forceinline__ void lz_norm_partials_body(const c128* __restrict__ x, long n,
                                                       double* __restrict__ part, unsigned blk) {
   __shared__ double sh[16];
   double acc = 0;
-  const long base = (long)blk * LZ_ELEMS;
-  for (long i = base + threadIdx.x; i < min(n, base + LZ_ELEMS); i += blockDim.x)
-    acc += x[i].re * x[i].re + x[i].im * x[i].im;
+  const long i = (long)blk * LZ_BLOCK + threadIdx.x;
+  if (i < n) acc = x[i].re * x[i].re + x[i].im * x[i].im;
   acc = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blk] = acc;
 }
@@ -282,194 +291,144 @@ __global__ void lz_norm_partials(const c128* __restrict__ x, long n, double* __r
   lz_norm_partials_body(x, n, part, blockIdx.x);
 }
 
-__global__ void lz_init_finalize(LanczosCtrl* ctrl, const double* __restrict__ part, int nblk) {
-  if (threadIdx.x != 0) return;
-  double s = 0;
-  for (int b = 0; b < nblk; ++b) s += part[b];
-  ctrl->beta0 = sqrt(s);
-  ctrl->done = (s == 0.0) ? 1 : 0;
-  ctrl->m = 0;
-  ctrl->err = 0;
-  ctrl->zero = (s == 0.0) ? 1 : 0;
-  ctrl->hit_limit = 0;
-}
-
+// V_0 = x / |x|, and its complex64 copy when v32 is given; block 0 opens the
+// control block.
 __device__ __forceinline__ void lz_scale_first_body(const c128* __restrict__ x, c128* __restrict__ v0,
-                                                    long n, const LanczosCtrl* ctrl,
-                                                    c64* __restrict__ v32, unsigned blk, unsigned nblk) {
-  const double b = ctrl->beta0;
-  const double inv = b > 0 ? 1.0 / b : 0.0;
-  for (long i = blk * (long)blockDim.x + threadIdx.x; i < n; i += (long)nblk * blockDim.x) {
+                                                    long n, const double* __restrict__ part, int nblk,
+                                                    LanczosCtrl* ctrl, c64* __restrict__ v32, unsigned blk) {
+  __shared__ double sum;
+  if (threadIdx.x < 64) {
+    double s = 0;
+    for (int b = threadIdx.x; b < nblk; b += 64) s += part[b];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) sum = s;
+  }
+  __syncthreads();
+  const double b = sqrt(sum), inv = b > 0 ? 1.0 / b : 0.0;
+  const long i = (long)blk * LZ_BLOCK + threadIdx.x;
+  if (i < n) {
     const c128 v{x[i].re * inv, x[i].im * inv};
     v0[i] = v;
     if (v32) v32[i] = c64{float(v.re), float(v.im)};
   }
+  if (blk == 0 && threadIdx.x == 0) {
+    ctrl->beta0 = b;
+    ctrl->done = ctrl->zero = (sum == 0.0) ? 1 : 0;
+    ctrl->m = 0;
+    ctrl->err = 0;
+    ctrl->hit_limit = 0;
+  }
 }
-__global__ void lz_scale_first(const c128* __restrict__ x, c128* __restrict__ v0, long n,
-                               const LanczosCtrl* ctrl, c64* __restrict__ v32) {
-  lz_scale_first_body(x, v0, n, ctrl, v32, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(LZ_BLOCK) void lz_scale_first(const c128* __restrict__ x, c128* __restrict__ v0, long n,
+                                                           const double* __restrict__ part, int nblk,
+                                                           LanczosCtrl* ctrl, c64* __restrict__ v32) {
+  lz_scale_first_body(x, v0, n, part, nblk, ctrl, v32, blockIdx.x);
 }
 
-// This block's partial projections part[blk][i] = sum_e conj(V_i[e]) x[e],
-// i = 0..j, with x held in registers (LZ_EPT elements per thread).  Each
-// projection is reduced inside its wave; one barrier then combines the waves.
-__device__ void block_projections(const c128* __restrict__ V, long n, int j, long base,
-                                  const double* xr, const double* xi,
-                                  c128* __restrict__ part_blk) {
+// part[blk] = this block's share of <V_j, w>.
+template <typename TW>
+__device__ __forceinline__ void lz_dot_body(const LanczosCtrl* ctrl, const cplx<TW>* __restrict__ w,
+                                            const c128* __restrict__ vj, long n, c128* __restrict__ part,
+                                            unsigned blk) {
+  const int done = ctrl->done;  // tested once the loads are in flight
+  __shared__ c128 sh[LZ_BLOCK / 64];
+  const long e = (long)blk * LZ_BLOCK + threadIdx.x;
+  double ar = 0, ai = 0;
+  if (e < n) {
+    const c128 a = vj[e];
+    const cplx<TW> x = w[e];
+    ar = a.re * double(x.re) + a.im * double(x.im);
+    ai = a.re * double(x.im) - a.im * double(x.re);
+  }
+  if (done) return;
+  ar = wave_sum(ar);
+  ai = wave_sum(ai);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = c128{ar, ai};
+  __syncthreads();
+  if (threadIdx.x == 0) part[blk] = c128{(sh[0].re + sh[1].re) + (sh[2].re + sh[3].re),
+                                         (sh[0].im + sh[1].im) + (sh[2].im + sh[3].im)};
+}
+template <typename TW>
+__global__ __launch_bounds__(LZ_BLOCK) void lz_dot(const LanczosCtrl* ctrl, const cplx<TW>* __restrict__ w,
+                                                   const c128* __restrict__ vj, long n, c128* __restrict__ part) {
+  lz_dot_body<TW>(ctrl, w, vj, n, part, blockIdx.x);
+}
+
+// One wave: the sum of part[0..nblk), in every lane.
+__device__ __forceinline__ c128 lz_sum(const c128* __restrict__ part, int nblk) {
+  double ar = 0, ai = 0;
+  for (int b = threadIdx.x & 63; b < nblk; b += 64) {
+    const c128 p = part[b];
+    ar += p.re;
+    ai += p.im;
+  }
+  return c128{wave_sum(ar), wave_sum(ai)};
+}
+
+// w64 = w - c V_j - beta_{j-1} V_{j-1} (promoting w to FP64), c = <V_j, w> from
+// lz_dot's shares; this block's shares of <V_i, w64>, i <= j, go to
+// part_out[i * nblk + blk], its share of |w64|^2 to row LZ_NORM.
+template <typename TW>
+__device__ __forceinline__ void lz_three_term_body(const LanczosCtrl* ctrl, const cplx<TW>* __restrict__ w,
+                                                   c128* __restrict__ w64, const c128* __restrict__ V, long n,
+                                                   int j, const c128* __restrict__ part_in, int nblk,
+                                                   c128* __restrict__ coef, c128* __restrict__ part_out,
+                                                   unsigned blk) {
+  const int done = ctrl->done;  // tested after the loads
   constexpr int NW = LZ_BLOCK / 64;
   __shared__ double sh[NW][LZ_MAXK][2];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const c128 c = lz_sum(part_in, nblk);   // every wave for itself
+  const double bp = j > 0 ? ctrl->beta[j - 1] : 0.0;
+  const long e = (long)blk * LZ_BLOCK + threadIdx.x;
+  const bool in = e < n;
+  const long ec = in ? e : n - 1;
+  const c128 vj = V[(long)j * n + ec], vp = V[(long)(j > 0 ? j - 1 : 0) * n + ec];
+  const cplx<TW> y = w[ec];
+  if (done) return;
+  const double xr = in ? double(y.re) - (c.re * vj.re - c.im * vj.im + bp * vp.re) : 0.0;
+  const double xi = in ? double(y.im) - (c.re * vj.im + c.im * vj.re + bp * vp.im) : 0.0;
+  if (in) w64[e] = c128{xr, xi};
+  if (blk == 0 && threadIdx.x == 0) coef[j] = c;
+  const double nrm = wave_sum(xr * xr + xi * xi);
+  if (lane == 0) {
+    sh[wv][LZ_NORM][0] = nrm;
+    sh[wv][LZ_NORM][1] = 0.0;
+  }
+#pragma unroll 4
   for (int i = 0; i <= j; ++i) {
-    const c128* vi = V + (long)i * n;
-    double ar = 0, ai = 0;
-#pragma unroll
-    for (int r = 0; r < LZ_EPT; ++r) {
-      const long e = base + (long)r * LZ_BLOCK;
-      if (e < n) {
-        const c128 a = vi[e];
-        ar += a.re * xr[r] + a.im * xi[r];
-        ai += a.re * xi[r] - a.im * xr[r];
-      }
-    }
-    ar = wave_sum(ar);
-    ai = wave_sum(ai);
+    const c128 a = V[(long)i * n + ec];
+    const double pr = wave_sum(a.re * xr + a.im * xi), pi = wave_sum(a.re * xi - a.im * xr);
     if (lane == 0) {
-      sh[wv][i][0] = ar;
-      sh[wv][i][1] = ai;
+      sh[wv][i][0] = pr;
+      sh[wv][i][1] = pi;
     }
   }
   __syncthreads();
-  if (threadIdx.x <= j) {
+  const int t = threadIdx.x;
+  if (t <= j || t == LZ_NORM) {
     double ar = 0, ai = 0;
-    for (int w = 0; w < NW; ++w) {
-      ar += sh[w][threadIdx.x][0];
-      ai += sh[w][threadIdx.x][1];
+    for (int k = 0; k < NW; ++k) {
+      ar += sh[k][t][0];
+      ai += sh[k][t][1];
     }
-    part_blk[threadIdx.x] = c128{ar, ai};
+    part_out[(long)t * nblk + blk] = c128{ar, ai};
   }
-}
-
-// Partial projections c_i = <V_i, w> over this block's chunk.  Each thread
-// keeps its LZ_EPT elements of w in registers across the i loop.
-template <typename TW>
-__device__ __forceinline__ void lz_project_body(const LanczosCtrl* ctrl, const cplx<TW>* __restrict__ w,
-                                                const c128* __restrict__ V, long n, int j,
-                                                c128* __restrict__ part, unsigned blk) {
-  const int done = ctrl->done;  // tested once w's loads are in flight
-  const long base = (long)blk * LZ_ELEMS + threadIdx.x;
-  double wr[LZ_EPT], wi[LZ_EPT];
-#pragma unroll
-  for (int r = 0; r < LZ_EPT; ++r) {
-    const long e = base + (long)r * LZ_BLOCK;
-    wr[r] = e < n ? double(w[e].re) : 0.0;
-    wi[r] = e < n ? double(w[e].im) : 0.0;
-  }
-  if (done) return;
-  block_projections(V, n, j, base, wr, wi, part + (long)blk * LZ_MAXK);
 }
 template <typename TW>
-__global__ __launch_bounds__(LZ_BLOCK) void lz_project(const LanczosCtrl* ctrl,
-                                                       const cplx<TW>* __restrict__ w,
-                                                       const c128* __restrict__ V, long n, int j,
-                                                       c128* __restrict__ part) {
-  lz_project_body<TW>(ctrl, w, V, n, j, part, blockIdx.x);
-}
-
-// coef_i = sum over blocks of part_in[b][i] (i = 0..j), reduced by every block
-// in one fixed order (one wave per coefficient, lanes striding over the
-// blocks, then a butterfly: deterministic), so no separate reduction launch is
-// needed; block 0 also stores them in coef_out.  Then wout = w - sum_i coef_i V_i (promoting w to
-// FP64), and the partial projections of wout (pass 1) or its partial squared
-// norm (pass 2) go to part_out, a different buffer from part_in.
-template <typename TW>
-__device__ __forceinline__ void lz_subtract_body(const LanczosCtrl* ctrl, const cplx<TW>* __restrict__ w,
-                                                 c128* __restrict__ wout, const c128* __restrict__ V,
-                                                 long n, int j, const c128* __restrict__ part_in,
-                                                 int nblk, c128* __restrict__ coef_out,
-                                                 c128* __restrict__ part_out, int pass, unsigned blk) {
-  const int done = ctrl->done;  // tested after the coefficient loads
-  __shared__ double sh[16];
-  __shared__ c128 cs[LZ_MAXK];
-  {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int i = wv; i <= j; i += LZ_BLOCK / 64) {
-      double ar = 0, ai = 0;
-      for (int b = lane; b < nblk; b += 64) {
-        ar += part_in[(long)b * LZ_MAXK + i].re;
-        ai += part_in[(long)b * LZ_MAXK + i].im;
-      }
-      ar = wave_sum(ar);
-      ai = wave_sum(ai);
-      if (lane == 0) {
-        cs[i] = c128{ar, ai};
-        if (blk == 0 && !done) coef_out[i] = c128{ar, ai};
-      }
-    }
-  }
-  __syncthreads();
-  if (done) return;
-  const long base = (long)blk * LZ_ELEMS + threadIdx.x;
-  double xr[LZ_EPT], xi[LZ_EPT];
-#pragma unroll
-  for (int r = 0; r < LZ_EPT; ++r) {
-    const long e = base + (long)r * LZ_BLOCK;
-    xr[r] = e < n ? double(w[e].re) : 0.0;
-    xi[r] = e < n ? double(w[e].im) : 0.0;
-  }
-  for (int i = 0; i <= j; ++i) {
-    const c128 c = cs[i];
-#pragma unroll
-    for (int r = 0; r < LZ_EPT; ++r) {
-      const long e = base + (long)r * LZ_BLOCK;
-      if (e < n) {
-        const c128 a = V[(long)i * n + e];
-        xr[r] -= c.re * a.re - c.im * a.im;
-        xi[r] -= c.re * a.im + c.im * a.re;
-      }
-    }
-  }
-  double nrm = 0;
-#pragma unroll
-  for (int r = 0; r < LZ_EPT; ++r) {
-    const long e = base + (long)r * LZ_BLOCK;
-    if (e < n) {
-      wout[e] = c128{xr[r], xi[r]};
-      nrm += xr[r] * xr[r] + xi[r] * xi[r];
-    }
-  }
-  if (pass == 2) {
-    nrm = block_sum(nrm, sh);
-    if (threadIdx.x == 0) part_out[(long)blk * LZ_MAXK] = c128{nrm, 0};
-    return;
-  }
-  block_projections(V, n, j, base, xr, xi, part_out + (long)blk * LZ_MAXK);
-}
-template <typename TW>
-__global__ __launch_bounds__(LZ_BLOCK) void lz_subtract(const LanczosCtrl* ctrl,
-                                                        const cplx<TW>* __restrict__ w,
-                                                        c128* __restrict__ wout,
-                                                        const c128* __restrict__ V, long n, int j,
-                                                        const c128* __restrict__ part_in, int nblk,
-                                                        c128* __restrict__ coef_out,
-                                                        c128* __restrict__ part_out, int pass) {
-  lz_subtract_body<TW>(ctrl, w, wout, V, n, j, part_in, nblk, coef_out, part_out, pass, blockIdx.x);
-}
-
-// beta_j = |w| from the per-block partial norms (one wave, fixed order).
-__device__ __forceinline__ double lz_beta(const c128* __restrict__ part_norm, int nblk) {
-  double s = 0;
-  for (int b = threadIdx.x & 63; b < nblk; b += 64) s += part_norm[(long)b * LZ_MAXK].re;
-  return sqrt(wave_sum(s));
+__global__ __launch_bounds__(LZ_BLOCK) void lz_three_term(const LanczosCtrl* ctrl, const cplx<TW>* __restrict__ w,
+                                                          c128* __restrict__ w64, const c128* __restrict__ V, long n,
+                                                          int j, const c128* __restrict__ part_in, int nblk,
+                                                          c128* __restrict__ coef, c128* __restrict__ part_out) {
+  lz_three_term_body<TW>(ctrl, w, w64, V, n, j, part_in, nblk, coef, part_out, blockIdx.x);
 }
 
 // One wave: close iteration j.  alpha_j = Re(c_j + c'_j), beta_j = |w|;
 // z = exp(-i tau T_{j+1}) e_0 by scaled Taylor steps on the tridiagonal
 // (lane = row); converged when beta0*beta_j*|z_j| < tol*beta0.
-__device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, const c128* __restrict__ coef1,
-                                   const c128* __restrict__ coef2, int j, double tau, double tol,
+__device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, double alpha_j, int j, double tau, double tol,
                                    int max_m) {
   const int l = threadIdx.x & 63;
-  const double alpha_j = coef1[j].re + coef2[j].re;
   if (l == 0) {
     ctrl->alpha[j] = alpha_j;
     ctrl->beta[j] = beta;
@@ -479,6 +438,23 @@ __device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, const c128* _
   const double al = (l < j) ? ctrl->alpha[l] : ((l == j) ? alpha_j : 0.0);
   const double bup = (l + 1 < m) ? ctrl->beta[l] : 0.0;     // T[l][l+1]
   const double bdn = (l >= 1 && l < m) ? ctrl->beta[l - 1] : 0.0;  // T[l][l-1]
+  const bool breakdown = beta <= 1e-13 * fmax(1.0, fabs(alpha_j));
+  // The estimate is at least 2 tol by a lower bound of |z_j| (the product of the
+  // betas and |tau|^j / j! times the cosine of half the spectrum's phase width,
+  // from the divided-difference form of z_j as a mean of exp(-i tau s) over s
+  // between Gershgorin's bounds): not converged, without the exponential (2.5 us).
+  if (!breakdown && m < max_m - 1) {
+    const double r = fabs(bdn) + (l == j ? beta : fabs(bup));
+    double prod = l < j ? bup * fabs(tau) / (l + 1) : 1.0;
+    double high = l < m ? al + r : -1e300, low = l < m ? r - al : -1e300;   // low: minus the lower bound
+    for (int o = 32; o > 0; o >>= 1) {
+      prod *= __shfl_xor(prod, o, 64);
+      high = fmax(high, __shfl_xor(high, o, 64));
+      low = fmax(low, __shfl_xor(low, o, 64));
+    }
+    const double half = 0.5 * fabs(tau) * (high + low);
+    if (half < 1.4 && beta * prod * (1.0 - 0.5 * half * half) >= 2.0 * tol) return;   // cos x >= 1 - x^2 / 2
+  }
   double rown = fabs(al) + fabs(bup) + fabs(bdn);
   for (int o = 32; o > 0; o >>= 1) rown = fmax(rown, __shfl_xor(rown, o, 64));
   const double h = fabs(tau) * rown;
@@ -509,7 +485,6 @@ __device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, const c128* _
   }
   const double zlr = __shfl(zr, j, 64), zli = __shfl(zi, j, 64);
   const double err = beta * sqrt(zlr * zlr + zli * zli);
-  const bool breakdown = beta <= 1e-13 * fmax(1.0, fabs(alpha_j));
   const bool conv = breakdown || err < tol || m >= max_m - 1;
   if (l < m) {
     ctrl->z[l] = c128{zr, zi};
@@ -524,44 +499,47 @@ __device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, const c128* _
   }
 }
 
-// Closes iteration j and forms the next basis vector in one launch: every
-// block reduces beta_j itself (same order everywhere), the first wave of block
-// 0 closes the iteration, and all blocks write V_{j+1} = w / beta_j, plus its
-// complex64 copy for the mixed path's next matvec when v32 is given.  Blocks
-// that start after convergence skip the write; V_{j+1} is not read then.
-__device__ __forceinline__ void lz_step_scale_body(LanczosCtrl* ctrl, const c128* __restrict__ part_norm,
-                                                   int nblk, const c128* __restrict__ coef1,
-                                                   const c128* __restrict__ coef2, int j, double tau,
-                                                   double tol, int max_m, const c128* __restrict__ w,
-                                                   c128* __restrict__ vnext, c64* __restrict__ v32,
-                                                   long n, unsigned blk, unsigned ngrid) {
-  const int done = ctrl->done;  // tested after beta's loads
-  __shared__ double sbeta;
-  if (threadIdx.x < 64) {
-    const double b = lz_beta(part_norm, nblk);
-    if (threadIdx.x == 0) sbeta = b;
+// Closes iteration j: every block sums the projections c_i and the norm, the
+// first wave of block 0 takes alpha_j, beta_j and the stopping test, and all
+// blocks write V_{j+1} = (w - sum_i c_i V_i) / beta_j, plus its complex64 copy for
+// the mixed path's next matvec when v32 is given.  Blocks that start after
+// convergence skip the write; V_{j+1} is not read then.
+__device__ __forceinline__ void lz_next_body(LanczosCtrl* ctrl, const c128* __restrict__ part, int nblk,
+                                             const c128* __restrict__ coef, int j, double tau, double tol, int max_m,
+                                             const c128* __restrict__ w, c128* V, c64* __restrict__ v32, long n,
+                                             unsigned blk) {
+  const int done = ctrl->done;  // tested after the loads
+  __shared__ c128 cs[LZ_MAXK];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  for (int i = wv; i <= j + 1; i += LZ_BLOCK / 64) {
+    const int row = i <= j ? i : LZ_NORM;
+    const c128 c = lz_sum(part + (long)row * nblk, nblk);
+    if (lane == 0) cs[row] = c;
   }
+  const long e = (long)blk * LZ_BLOCK + threadIdx.x, ec = e < n ? e : n - 1;
+  c128 x = w[ec];
   __syncthreads();
   if (done) return;
-  const double beta = sbeta;
-  if (blk == 0 && threadIdx.x < 64) lz_close_iteration(ctrl, beta, coef1, coef2, j, tau, tol, max_m);
-  const double inv = 1.0 / beta;
-  for (long i = blk * (long)blockDim.x + threadIdx.x; i < n; i += (long)ngrid * blockDim.x) {
-    const c128 v{w[i].re * inv, w[i].im * inv};
-    vnext[i] = v;
-    if (v32) v32[i] = c64{float(v.re), float(v.im)};
+  double b2 = cs[LZ_NORM].re;
+  for (int i = 0; i <= j; ++i) b2 -= cs[i].re * cs[i].re + cs[i].im * cs[i].im;
+  const double beta = sqrt(fmax(b2, 0.0)), inv = 1.0 / beta;
+  if (blk == 0 && threadIdx.x < 64) lz_close_iteration(ctrl, beta, coef[j].re + cs[j].re, j, tau, tol, max_m);
+#pragma unroll 4
+  for (int i = 0; i <= j; ++i) {
+    const c128 a = V[(long)i * n + ec], c = cs[i];
+    x.re -= c.re * a.re - c.im * a.im;
+    x.im -= c.re * a.im + c.im * a.re;
   }
+  if (e >= n) return;
+  const c128 v{x.re * inv, x.im * inv};
+  V[(long)(j + 1) * n + e] = v;
+  if (v32) v32[e] = c64{float(v.re), float(v.im)};
 }
-__global__ __launch_bounds__(256) void lz_step_scale(LanczosCtrl* ctrl,
-                                                     const c128* __restrict__ part_norm, int nblk,
-                                                     const c128* __restrict__ coef1,
-                                                     const c128* __restrict__ coef2, int j,
-                                                     double tau, double tol, int max_m,
-                                                     const c128* __restrict__ w,
-                                                     c128* __restrict__ vnext,
-                                                     c64* __restrict__ v32, long n) {
-  lz_step_scale_body(ctrl, part_norm, nblk, coef1, coef2, j, tau, tol, max_m, w, vnext, v32, n,
-                     blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(LZ_BLOCK) void lz_next(LanczosCtrl* ctrl, const c128* __restrict__ part, int nblk,
+                                                    const c128* __restrict__ coef, int j, double tau, double tol,
+                                                    int max_m, const c128* __restrict__ w, c128* V,
+                                                    c64* __restrict__ v32, long n) {
+  lz_next_body(ctrl, part, nblk, coef, j, tau, tol, max_m, w, V, v32, n, blockIdx.x);
 }
 
 // y = beta0 * sum_{i<m} z_i V_i   (a zero input stays zero)
@@ -596,52 +574,33 @@ __global__ void lz_norm_partials_grouped(const GRec<LzArgs>* __restrict__ recs, 
   const GRec<LzArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
   lz_norm_partials_body(gbl(r.a.x), r.a.n, gbl(r.a.part_norm), bx);
 }
-__global__ void lz_init_finalize_grouped(const GRec<LzArgs>* __restrict__ recs, int n) {
-  if (threadIdx.x != 0) return;
-  const LzArgs& a = recs[blockIdx.x].a;
-  double sum = 0;
-  for (int b = 0; b < a.nblk; ++b) sum += a.part_norm[b];
-  LanczosCtrl* ctrl = a.ctrl;
-  ctrl->beta0 = sqrt(sum);
-  ctrl->done = (sum == 0.0) ? 1 : 0;
-  ctrl->m = 0;
-  ctrl->err = 0;
-  ctrl->zero = (sum == 0.0) ? 1 : 0;
-  ctrl->hit_limit = 0;
-}
-__global__ void lz_scale_first_grouped(const GRec<LzArgs>* __restrict__ recs, int n) {
+__global__ __launch_bounds__(LZ_BLOCK) void lz_scale_first_grouped(const GRec<LzArgs>* __restrict__ recs, int n) {
   unsigned bx, by, bz;
   const GRec<LzArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
-  lz_scale_first_body(gbl(r.a.x), gbl(r.a.V), r.a.n, gbl(r.a.ctrl), gbl(r.a.v32), bx, r.grid.x);
+  lz_scale_first_body(gbl(r.a.x), gbl(r.a.V), r.a.n, gbl(r.a.part_norm), r.a.nblk, gbl(r.a.ctrl), gbl(r.a.v32), bx);
 }
 template <typename TW>
-__global__ __launch_bounds__(LZ_BLOCK) void lz_project_grouped(const GRec<LzArgs>* __restrict__ recs, int n,
-                                                               int j) {
+__global__ __launch_bounds__(LZ_BLOCK) void lz_dot_grouped(const GRec<LzArgs>* __restrict__ recs, int n, int j) {
   unsigned bx, by, bz;
   const GRec<LzArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
-  lz_project_body<TW>(gbl(r.a.ctrl), gbl(reinterpret_cast<const cplx<TW>*>(r.a.w)), gbl(r.a.V), r.a.n, j,
-                      gbl(r.a.part), bx);
+  lz_dot_body<TW>(gbl(r.a.ctrl), gbl(reinterpret_cast<const cplx<TW>*>(r.a.w)), gbl(r.a.V + (long)j * r.a.n), r.a.n,
+                  gbl(r.a.part), bx);
 }
 template <typename TW>
-__global__ __launch_bounds__(LZ_BLOCK) void lz_subtract_grouped(const GRec<LzArgs>* __restrict__ recs, int n,
-                                                                int j, int pass) {
+__global__ __launch_bounds__(LZ_BLOCK) void lz_three_term_grouped(const GRec<LzArgs>* __restrict__ recs, int n,
+                                                                  int j) {
   unsigned bx, by, bz;
   const GRec<LzArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
   const LzArgs a = r.a;
-  if (pass == 1)
-    lz_subtract_body<TW>(gbl(a.ctrl), gbl(reinterpret_cast<const cplx<TW>*>(a.w)), gbl(a.w64), gbl(a.V), a.n,
-                         j, gbl(a.part), a.nblk, gbl(a.coef1), gbl(a.part2), 1, bx);
-  else
-    lz_subtract_body<double>(gbl(a.ctrl), gbl(a.w64), gbl(a.w64), gbl(a.V), a.n, j, gbl(a.part2), a.nblk,
-                             gbl(a.coef2), gbl(a.part), 2, bx);
+  lz_three_term_body<TW>(gbl(a.ctrl), gbl(reinterpret_cast<const cplx<TW>*>(a.w)), gbl(a.w64), gbl(a.V), a.n, j,
+                         gbl(a.part), a.nblk, gbl(a.coef), gbl(a.part2), bx);
 }
-__global__ __launch_bounds__(256) void lz_step_scale_grouped(const GRec<LzArgs>* __restrict__ recs, int n,
-                                                             int j) {
+__global__ __launch_bounds__(LZ_BLOCK) void lz_next_grouped(const GRec<LzArgs>* __restrict__ recs, int n, int j) {
   unsigned bx, by, bz;
   const GRec<LzArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
   const LzArgs a = r.a;
-  lz_step_scale_body(gbl(a.ctrl), gbl(a.part), a.nblk, gbl(a.coef1), gbl(a.coef2), j, a.tau, a.tol, a.max_m,
-                     gbl(a.w64), gbl(a.V + (long)(j + 1) * a.n), gbl(a.v32), a.n, bx, r.grid.x);
+  lz_next_body(gbl(a.ctrl), gbl(a.part2), a.nblk, gbl(a.coef), j, a.tau, a.tol, a.max_m, gbl(a.w64), gbl(a.V),
+               gbl(a.v32), a.n, bx);
 }
 __global__ void lz_combine_grouped(const GRec<LzArgs>* __restrict__ recs, int n) {
   unsigned bx, by, bz;
@@ -801,32 +760,28 @@ template void launch_wmix_grouped<double>(const KGroup<WmixArgs<double>>&, size_
 template void launch_wmix_grouped<float>(const KGroup<WmixArgs<float>>&, size_t, hipStream_t);
 
 void LzGroup::prepare(const std::vector<LzArgs>& jobs, RecordArena& arena) {
-  std::vector<GRec<LzArgs>> a, b, c;
+  std::vector<GRec<LzArgs>> a, b;
   for (const LzArgs& j : jobs) {
     QCA_CHECK(j.nblk == lanczos_nblk(j.n), "Lanczos block count does not match the vector");
     a.push_back(grec(j, j.nblk));
     b.push_back(grec(j, grid_for(j.n)));
-    c.push_back(grec(j, 1));
   }
   nb.prepare(a, arena);
   gf.prepare(b, arena);
-  one.prepare(c, arena);
 }
 void LzGroup::begin(hipStream_t s) const {
   if (empty()) return;
   hipLaunchKernelGGL(lz_norm_partials_grouped, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n);
-  hipLaunchKernelGGL(lz_init_finalize_grouped, dim3(one.l.blocks), dim3(64), 0, s, one.l.recs, one.l.n);
-  hipLaunchKernelGGL(lz_scale_first_grouped, dim3(gf.l.blocks), dim3(256), 0, s, gf.l.recs, gf.l.n);
+  hipLaunchKernelGGL(lz_scale_first_grouped, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n);
   QCA_HIP(hipGetLastError());
 }
 template <typename TW>
 void LzGroup::tail(int j, hipStream_t s) const {
   if (empty()) return;
   QCA_CHECK(j + 1 < LZ_MAXK, "Krylov dimension limit");
-  hipLaunchKernelGGL(lz_project_grouped<TW>, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n, j);
-  hipLaunchKernelGGL(lz_subtract_grouped<TW>, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n, j, 1);
-  hipLaunchKernelGGL(lz_subtract_grouped<TW>, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n, j, 2);
-  hipLaunchKernelGGL(lz_step_scale_grouped, dim3(gf.l.blocks), dim3(256), 0, s, gf.l.recs, gf.l.n, j);
+  hipLaunchKernelGGL(lz_dot_grouped<TW>, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n, j);
+  hipLaunchKernelGGL(lz_three_term_grouped<TW>, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n, j);
+  hipLaunchKernelGGL(lz_next_grouped, dim3(nb.l.blocks), dim3(LZ_BLOCK), 0, s, nb.l.recs, nb.l.n, j);
   QCA_HIP(hipGetLastError());
 }
 template void LzGroup::tail<double>(int, hipStream_t) const;
@@ -903,7 +858,7 @@ void launch_gather_isometry(const c128* X, const int* perm, const double* sigma,
   QCA_HIP(hipGetLastError());
 }
 
-int lanczos_nblk(long n) { return (int)std::max<long>(1, (n + LZ_ELEMS - 1) / LZ_ELEMS); }
+int lanczos_nblk(long n) { return (int)std::max<long>(1, (n + LZ_BLOCK - 1) / LZ_BLOCK); }
 
 const int* lanczos_done_flag(const LanczosWork& lw) { return &lw.ctrl->done; }
 
@@ -911,9 +866,8 @@ void lanczos_begin(const c128* x, long n, LanczosWork& lw, hipStream_t s, c64* v
   const int nb = lanczos_nblk(n);
   QCA_CHECK(nb <= lw.max_blocks, "Lanczos vector longer than the workspace");
   hipLaunchKernelGGL(lz_norm_partials, dim3(nb), dim3(LZ_BLOCK), 0, s, x, n, lw.part_norm);
-  hipLaunchKernelGGL(lz_init_finalize, dim3(1), dim3(64), 0, s, lw.ctrl, lw.part_norm, nb);
-  hipLaunchKernelGGL(lz_scale_first, dim3(grid_for(n)), dim3(256), 0, s, x, lw.V, n,
-                     (const LanczosCtrl*)lw.ctrl, v32);
+  hipLaunchKernelGGL(lz_scale_first, dim3(nb), dim3(LZ_BLOCK), 0, s, x, lw.V, n, (const double*)lw.part_norm, nb,
+                     lw.ctrl, v32);
   QCA_HIP(hipGetLastError());
 }
 
@@ -923,14 +877,12 @@ void lanczos_iteration_tail(const cplx<TW>* w, long n, int j, double tau, double
   QCA_CHECK(j + 1 < lw.max_m && lw.max_m <= LZ_MAXK, "Krylov dimension limit");
   const int nb = lanczos_nblk(n);
   const LanczosCtrl* cc = lw.ctrl;
-  hipLaunchKernelGGL(lz_project<TW>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, w, lw.V, n, j, lw.part);
-  hipLaunchKernelGGL(lz_subtract<TW>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, w, lw.w64, lw.V, n, j,
-                     (const c128*)lw.part, nb, lw.coef1, lw.part2, 1);
-  hipLaunchKernelGGL(lz_subtract<double>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, lw.w64, lw.w64, lw.V,
-                     n, j, (const c128*)lw.part2, nb, lw.coef2, lw.part, 2);
-  hipLaunchKernelGGL(lz_step_scale, dim3(grid_for(n)), dim3(256), 0, s, lw.ctrl,
-                     (const c128*)lw.part, nb, (const c128*)lw.coef1, (const c128*)lw.coef2, j, tau,
-                     tol, lw.max_m, (const c128*)lw.w64, lw.V + (long)(j + 1) * n, v32, n);
+  hipLaunchKernelGGL(lz_dot<TW>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, w, (const c128*)(lw.V + (long)j * n), n,
+                     lw.part);
+  hipLaunchKernelGGL(lz_three_term<TW>, dim3(nb), dim3(LZ_BLOCK), 0, s, cc, w, lw.w64, (const c128*)lw.V, n, j,
+                     (const c128*)lw.part, nb, lw.coef, lw.part2);
+  hipLaunchKernelGGL(lz_next, dim3(nb), dim3(LZ_BLOCK), 0, s, lw.ctrl, (const c128*)lw.part2, nb,
+                     (const c128*)lw.coef, j, tau, tol, lw.max_m, (const c128*)lw.w64, lw.V, v32, n);
   QCA_HIP(hipGetLastError());
 }
 template void lanczos_iteration_tail<double>(const c128*, long, int, double, double, LanczosWork&,

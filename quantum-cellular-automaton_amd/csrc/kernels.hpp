@@ -29,11 +29,10 @@ struct LanczosWork {
   LanczosCtrl* ctrl = nullptr;
   c128* V = nullptr;      // [LZ_MAXK][max_n] Krylov basis
   c128* w64 = nullptr;    // [max_n] orthogonalised residual
-  c128* part = nullptr;   // [max_blocks][LZ_MAXK] partial projections
-  c128* part2 = nullptr;  // same size: the second pass's partials (read and written apart)
+  c128* part = nullptr;   // [max_blocks] partial sums of <V_j, w>
+  c128* part2 = nullptr;  // [LZ_MAXK][max_blocks] partial projections on the basis, and the norm's
   double* part_norm = nullptr;
-  c128* coef1 = nullptr;  // [LZ_MAXK]
-  c128* coef2 = nullptr;
+  c128* coef = nullptr;   // [LZ_MAXK] <V_j, w> of each iteration
   long max_n = 0;
   int max_blocks = 0;
   int max_m = LZ_MAXK;    // Krylov dimension limit of this workspace (<= LZ_MAXK)

@@ -160,6 +160,34 @@ def test_krylov_expm(gpu, prec, kind, chil, chir, delta):
     assert abs(np.linalg.norm(got) - 1.0) < (1e-12 if prec == 0 else 1e-5)
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("kind,chil,chir,delta", [(2, 1, 1, 0.05), (2, 15, 17, -0.05), (2, 16, 16, 0.1),
+                                                 (2, 1, 257, 0.05), (1, 9, 57, 0.1), (0, 1, 2, 0.05),
+                                                 (2, 16, 16, 0.0)])
+def test_krylov_expm_blocks(gpu, prec, kind, chil, chir, delta):
+    """Vectors just below, at and above one and several 256-element blocks, a zero
+    step, and steps long enough that the convergence bound does not apply (phase
+    widths of 19 and 28, against 2.8)."""
+    if delta == 0.0 or chil * chir == 1:
+        # one iteration at least: the state itself, up to a phase
+        import torch
+        rng = np.random.default_rng(chil)
+        D = AU.bulk_tensor(2, range(2, 5)).shape[2]
+        x = crand(rng, chil, chir)
+        x /= np.linalg.norm(x)
+        L, R = herm_env(rng, chil, D), herm_env(rng, chir, D)
+        dt = np.complex128 if prec == 0 else np.complex64
+        xd = dev(torch, x, np.complex128)
+        Ld, Rd = dev(torch, L, dt), dev(torch, R, dt)
+        it = ctypes.c_int(0)
+        qn.call("qca_krylov_expm", prec, kind, qn.ptr(xd), qn.ptr(Ld), qn.ptr(Rd), None, D, D, chil, chir, delta,
+                0.0, ctypes.byref(it), None)
+        ref = LOC.expm_dense(LOC.dense_keff(L, R), x.reshape(-1), delta).reshape(x.shape)
+        assert np.abs(xd.cpu().numpy() - ref).max() < (1e-12 if prec == 0 else 2e-5)
+    else:
+        test_krylov_expm(gpu, prec, kind, chil, chir, delta)
+
+
 @pytest.mark.parametrize("right", [1, 0])
 @pytest.mark.parametrize("chil,chir,chi_max,eps", [(1, 1, 4, 1e-10), (2, 4, 8, 1e-10), (8, 8, 16, 1e-10),
                                                    (8, 8, 5, 1e-10), (16, 32, 64, 1e-3),
