@@ -1,10 +1,9 @@
 """Exact state-vector evolution on the GPU (drop-in for reference algorithms/exact.py:9-28).
 
 The reference forms the dense 2^N x 2^N propagator; here the 2^N amplitudes
-live in a device buffer and every step applies exp(-i (pi/2) dt H) by a Krylov
-exponential whose matrix-vector product is the closed-form rule Hamiltonian
-(one bit flip per active cell), so N is bounded by memory for vectors, not
-matrices.  ``args.step_size`` is the propagation time per ``do_time_step``;
+live in a device buffer and every step applies exp(-i (pi/2) dt H) as a
+Chebyshev series in the closed-form rule Hamiltonian (one bit flip per active
+cell), so N is bounded by memory for three vectors, not matrices.  ``args.step_size`` is the propagation time per ``do_time_step``;
 the reference driver scales it by the plot interval before construction
 (quantum_game.py:70-73) and that contract is kept.
 """
