@@ -8,7 +8,7 @@
 //              workgroup one chunk of 64 rows on the FP64 matrix cores,
 //              partial Grams to a workspace;
 //   jac_inner  one workgroup per pair sums its partial Grams and runs one
-//              cyclic sweep of two-sided Jacobi rotations on G_p in LDS
+//              cyclic sweep of two-sided Jacobi rotations on G_p in registers
 //              (G <- R^H G R), accumulating J_p = product of the rotations;
 //              two rounds of a sweep sweep all pairs of the 2bs columns,
 //              the others only those across the two blocks;
@@ -26,9 +26,9 @@
 // A pair whose smaller column is below 16 eps of the matrix norm is left alone
 // (JAC_NOISE2): such columns are rounding noise of the rotations, their
 // contribution to any tail is < 4e-15, and rotating them against the signal
-// columns of a matrix with more columns than rows would go on indefinitely.  jac_finalize sorts the singular values and evaluates
-// the truncation rank (first i with ||s[i:]|| < eps, capped; reference
-// algorithms/tdvp.py:289-292).
+// columns of a matrix with more columns than rows would go on indefinitely.
+// jac_finalize sorts the singular values and evaluates the truncation rank (first
+// i with ||s[i:]|| < eps, capped; reference algorithms/tdvp.py:289-292).
 #include "grouped.hpp"
 #include "larfg.hpp"
 #include "wave.hpp"
