@@ -240,9 +240,30 @@ __device__ __forceinline__ void factor_panel(const c128* __restrict__ src, int l
 #pragma unroll
     for (int i = 0; i < IT; ++i)
       if (i > 0 || lane > c) part += y[i].re * y[i].re + y[i].im * y[i].im;
-    const double xnorm2 = wave_sum64(part);
-    const c128 alpha{readlane_f64(y[0].re, c), readlane_f64(y[0].im, c)};
-    const Larfg h = larfg(alpha, xnorm2);
+    double xnorm2 = wave_sum64(part);
+    c128 alpha{readlane_f64(y[0].re, c), readlane_f64(y[0].im, c)};
+    int ex = 0;
+    if (!larfg_in_range(alpha.re * alpha.re + alpha.im * alpha.im + xnorm2)) {
+      // a column whose squares over- or underflow (all zero in most cases): the
+      // reflector of the scaled column is the same
+      double top = 0;
+#pragma unroll
+      for (int i = 0; i < IT; ++i)
+        if (i > 0 || lane >= c) top = fmax(top, fmax(fabs(y[i].re), fabs(y[i].im)));
+      for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 64));
+      ex = larfg_exponent(top);
+      part = 0;
+#pragma unroll
+      for (int i = 0; i < IT; ++i)
+        if (i > 0 || lane >= c) {
+          y[i] = c128{ldexp(y[i].re, -ex), ldexp(y[i].im, -ex)};
+          if (i > 0 || lane > c) part += y[i].re * y[i].re + y[i].im * y[i].im;
+        }
+      xnorm2 = wave_sum64(part);
+      alpha = c128{ldexp(alpha.re, -ex), ldexp(alpha.im, -ex)};
+    }
+    Larfg h = larfg(alpha, xnorm2);
+    if (ex) h.beta = ldexp(h.beta, ex);
     c128* v = vs + c * LDV;
 #pragma unroll
     for (int i = 0; i < IT; ++i) {

@@ -1048,8 +1048,29 @@ __device__ __forceinline__ void small_qr(c128 (&x)[IT], int kq, c128* V, int ld,
 #pragma unroll
         for (int i = i0 + 1; i < IT; ++i) n2 += x[i].re * x[i].re + x[i].im * x[i].im;
         n2 = sum8(n2);
-        const double ar = sum8(rl == k8 ? x[i0].re : 0.0), ai = sum8(rl == k8 ? x[i0].im : 0.0);
-        const Larfg h = larfg(c128{ar, ai}, n2);
+        c128 alpha{sum8(rl == k8 ? x[i0].re : 0.0), sum8(rl == k8 ? x[i0].im : 0.0)};
+        int ex = 0;
+        if (c == k && !larfg_in_range(alpha.re * alpha.re + alpha.im * alpha.im + n2)) {
+          // squares over- or underflow (all zero in most cases): the reflector of the
+          // scaled column is the same
+          double top = 0;
+#pragma unroll
+          for (int i = i0; i < IT; ++i)
+            if (i > i0 || rl >= k8) top = fmax(top, fmax(fabs(x[i].re), fabs(x[i].im)));
+          for (int o = 4; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o, 8));
+          ex = larfg_exponent(top);
+          n2 = 0;
+#pragma unroll
+          for (int i = i0; i < IT; ++i)
+            if (i > i0 || rl >= k8) {
+              x[i] = c128{ldexp(x[i].re, -ex), ldexp(x[i].im, -ex)};
+              if (i > i0 || rl > k8) n2 += x[i].re * x[i].re + x[i].im * x[i].im;
+            }
+          n2 = sum8(n2);
+          alpha = c128{ldexp(alpha.re, -ex), ldexp(alpha.im, -ex)};
+        }
+        Larfg h = larfg(alpha, n2);
+        if (ex) h.beta = ldexp(h.beta, ex);
         if (c == k) {
 #pragma unroll
           for (int i = i0; i < IT; ++i) {

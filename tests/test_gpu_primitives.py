@@ -436,3 +436,63 @@ def test_qr_panels_match_lapack(gpu, side, chi_row, chi_col, target):
     qn.call("qca_qr_site", side, qn.ptr(Ad), chil, chir, target, qn.ptr(An), qn.ptr(C), None)
     assert np.abs(An.cpu().numpy() - refA).max() < 1e-12
     assert np.abs(C.cpu().numpy() - refC).max() < 1e-12
+
+
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("chi_row,chi_col,col", [(1, 2, 0), (9, 9, 3), (40, 20, 17), (150, 33, 32)])
+@pytest.mark.parametrize("scale", [1e-156, 1e-160, 1e-170, 1e-300, 0.0, 1e160])
+def test_qr_column_out_of_range(gpu, scale, side, chi_row, chi_col, col):
+    """A column whose squares under- or overflow (a vanishing Schmidt direction):
+    numpy.linalg.qr's factors within the bound of test_qr_panels_match_lapack,
+    each column of R relative to its own size."""
+    import torch
+    from oracle import mps as OM
+    rng = np.random.default_rng(chi_row + chi_col + side)
+    chil, chir = (chi_row, chi_col) if side == 0 else (chi_col, chi_row)
+    A = crand(rng, 2, chil, chir)
+    (A[:, :, col] if side == 0 else A[:, col])[...] *= scale
+    target = 2 * chi_row
+    Q, R = OM.left_qr(A, reduced=False) if side == 0 else OM.right_qr(A, reduced=False)
+    refA = OM.truncate_pad(Q, (2, chil, target) if side == 0 else (2, target, chir))
+    refC = OM.truncate_pad(R, (target, chir) if side == 0 else (chil, target))
+    An = torch.zeros(refA.shape, dtype=torch.complex128, device="cuda")
+    C = torch.zeros(refC.shape, dtype=torch.complex128, device="cuda")
+    Ad = dev(torch, A, np.complex128)
+    qn.call("qca_qr_site", side, qn.ptr(Ad), chil, chir, target, qn.ptr(An), qn.ptr(C), None)
+    assert np.abs(An.cpu().numpy() - refA).max() < 1e-12
+    got, ref = (C.cpu().numpy(), refC) if side == 0 else (C.cpu().numpy().T, refC.T)
+    size = np.abs(ref).max(axis=0)
+    assert (np.abs(got - ref).max(axis=0) <= 1e-12 * size).all()
+
+
+@pytest.mark.parametrize("right", [1, 0])
+@pytest.mark.parametrize("chil,chir", [(4, 5), (12, 16), (16, 40), (40, 33)])
+@pytest.mark.parametrize("scale", [1e-156, 1e-160, 0.0])
+def test_svd_split_column_out_of_range(gpu, scale, chil, chir, right):
+    """Splits with a column and a row whose squares underflow, against LAPACK within
+    the bounds of test_svd_split."""
+    import torch
+    rng = np.random.default_rng(chil + chir)
+    m, n = 2 * chil, 2 * chir
+    M = crand(rng, m, n)
+    M[:, 1] *= scale
+    M[2] *= scale
+    M /= np.linalg.norm(M)
+    th = dev(torch, M.reshape(2, chil, 2, chir).transpose(0, 2, 1, 3).reshape(4, chil, chir), np.complex128)
+    kmax = min(m, n)
+    Al = torch.zeros(m * kmax, dtype=torch.complex128, device="cuda")
+    Ar = torch.zeros(n * kmax, dtype=torch.complex128, device="cuda")
+    k = ctypes.c_int(0)
+    sig = np.zeros(kmax)
+    qn.call("qca_svd_split", qn.ptr(th), qn.ptr(Al), qn.ptr(Ar), chil, chir, kmax, 1e-10, right, ctypes.byref(k),
+            sig.ctypes.data, None)
+    u, ref, vh = np.linalg.svd(M, full_matrices=False)
+    kk = k.value
+    assert kk == LOC.truncation_rank(ref, kmax, 1e-10)
+    assert np.abs(sig - ref).max() < 1e-13
+    A = Al[: m * kk].cpu().numpy().reshape(m, kk)
+    B = Ar[: n * kk].cpu().numpy().reshape(2, kk, chir).transpose(1, 0, 2).reshape(kk, n)
+    Q = A if right else B.conj().T
+    assert np.abs(Q.conj().T @ Q - np.eye(kk)).max() < 1e-13
+    kept = (u[:, :kk] * ref[:kk] / np.linalg.norm(ref[:kk])) @ vh[:kk]
+    assert np.abs(A @ B - kept).max() < 1e-12
