@@ -133,7 +133,8 @@ qca::LanczosWork lanczos_ws(long n, qca::LanczosCtrl** ctrl_host) {
 // Runs the Krylov loop: mv(j, V_j) must enqueue w = H V_j and the iteration
 // tail.  Iterations j = 0 .. max_m-2 may run; the device closes the
 // exponential at the latest at dimension max_m-1.  v32: complex64 copy of V_0, or
-// null.  x is overwritten with the result.  Returns the Krylov dimension used.
+// null.  x is overwritten with the result (and left alone where the start or a
+// matvec is not finite, an error).  Returns the Krylov dimension used.
 template <typename MV>
 int krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::LanczosCtrl* host, qca::c64* v32, MV&& mv,
                 hipStream_t s) {
@@ -144,11 +145,11 @@ int krylov_loop(qca::c128* x, long n, qca::LanczosWork& lw, qca::LanczosCtrl* ho
     QCA_HIP(hipMemcpyAsync(host, lw.ctrl, sizeof(qca::LanczosCtrl), hipMemcpyDeviceToHost, s));
     QCA_HIP(hipStreamSynchronize(s));
     if (host->done) break;
-    if (j >= lw.max_m - 1)
-      throw qca::Error(qca::QCA_ERR_NOT_CONVERGED_CODE,
-                       "Krylov exponential did not converge (non-finite input?)");
+    QCA_CHECK(j < lw.max_m - 1, "Krylov exponential left open at its dimension limit");
     chunk = 4;
   }
+  if (host->hit_limit == qca::LZ_NON_FINITE)
+    throw qca::Error(qca::QCA_ERR_NOT_CONVERGED_CODE, "Krylov exponential fed non-finite numbers");
   qca::lanczos_finish(n, x, lw, s);
   QCA_HIP(hipStreamSynchronize(s));
   return host->m;

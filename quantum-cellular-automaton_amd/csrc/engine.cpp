@@ -429,10 +429,12 @@ void Engine::lanczos_run(int kind, int site, c128* x, long n, int chil, int chir
     sync();
     if (ctrl_host_->done) break;
     // the device closes the exponential at the dimension limit (m = max_m - 1)
-    // at the latest, so this only fires on non-finite input
-    QCA_CHECK(j < lw_.max_m - 1, "Krylov exponential did not converge (non-finite input?)");
+    // at the latest
+    QCA_CHECK(j < lw_.max_m - 1, "Krylov exponential left open at its dimension limit");
     chunk = 2;
   }
+  if (ctrl_host_->hit_limit == LZ_NON_FINITE)
+    throw Error(QCA_ERR_NOT_CONVERGED_CODE, "Krylov exponential fed non-finite numbers");
   stats_.krylov_ms += elapsed_ms();
   const int m = ctrl_host_->m;
   kpred_[kind] = std::max(2, m);

@@ -479,9 +479,13 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
       all = all && head.done != 0;
     }
     if (all) break;
-    if (j >= max_m - 1)
-      throw Error(QCA_ERR_NOT_CONVERGED_CODE, "Krylov exponential did not converge (non-finite input?)");
+    QCA_CHECK(j < max_m - 1, "Krylov exponential left open at its dimension limit");
     chunk = 2;
+  }
+  for (size_t q = 0; q < lz.size(); ++q) {
+    LanczosCtrl head;
+    std::memcpy(&head, gather_host_ + kGatherWords * q, 32);
+    if (head.hit_limit == LZ_NON_FINITE) fail(inst[lz_item[q]], "Krylov exponential fed non-finite numbers");
   }
   glz.finish(s_);
   QCA_HIP(hipEventRecord(ev3_, s_));

@@ -313,10 +313,12 @@ __device__ __forceinline__ void lz_scale_first_body(const c128* __restrict__ x, 
   }
   if (blk == 0 && threadIdx.x == 0) {
     ctrl->beta0 = b;
-    ctrl->done = ctrl->zero = (sum == 0.0) ? 1 : 0;
+    const bool finite = b < __builtin_inf();
+    ctrl->zero = (sum == 0.0) ? 1 : 0;
+    ctrl->done = sum == 0.0 || !finite ? 1 : 0;
     ctrl->m = 0;
     ctrl->err = 0;
-    ctrl->hit_limit = 0;
+    ctrl->hit_limit = finite ? 0 : LZ_NON_FINITE;
   }
 }
 __global__ __launch_bounds__(LZ_BLOCK) void lz_scale_first(const c128* __restrict__ x, c128* __restrict__ v0, long n,
@@ -434,6 +436,14 @@ __device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, double alpha_
     ctrl->beta[j] = beta;
   }
   const int m = j + 1;
+  if (!(beta < __builtin_inf())) {   // a non-finite start or matvec: the host reports it
+    if (l == 0) {
+      ctrl->m = m;
+      ctrl->done = 1;
+      ctrl->hit_limit = LZ_NON_FINITE;
+    }
+    return;
+  }
   // alpha[0..j-1] and beta[0..j-1] were written by earlier launches
   const double al = (l < j) ? ctrl->alpha[l] : ((l == j) ? alpha_j : 0.0);
   const double bup = (l + 1 < m) ? ctrl->beta[l] : 0.0;     // T[l][l+1]
@@ -458,8 +468,6 @@ __device__ void lz_close_iteration(LanczosCtrl* ctrl, double beta, double alpha_
   double rown = fabs(al) + fabs(bup) + fabs(bdn);
   for (int o = 32; o > 0; o >>= 1) rown = fmax(rown, __shfl_xor(rown, o, 64));
   const double h = fabs(tau) * rown;
-  // bounded even for non-finite input (h = NaN/inf gives one substep and a
-  // non-finite error estimate, which the host reports as non-convergence)
   const int nsub = (h < 2048.0) ? max(1, (int)ceil(h / 0.5)) : 1;
   const double dt = tau / nsub;
   // z <- exp(-i dt T) z, nsub times;  multiplying by -i dt: (x+iy)*(-i dt) = dt*y - i dt*x
@@ -522,7 +530,7 @@ __device__ __forceinline__ void lz_next_body(LanczosCtrl* ctrl, const c128* __re
   if (done) return;
   double b2 = cs[LZ_NORM].re;
   for (int i = 0; i <= j; ++i) b2 -= cs[i].re * cs[i].re + cs[i].im * cs[i].im;
-  const double beta = sqrt(fmax(b2, 0.0)), inv = 1.0 / beta;
+  const double beta = sqrt(b2 < 0.0 ? 0.0 : b2), inv = 1.0 / beta;   // a NaN stays one
   if (blk == 0 && threadIdx.x < 64) lz_close_iteration(ctrl, beta, coef[j].re + cs[j].re, j, tau, tol, max_m);
 #pragma unroll 4
   for (int i = 0; i <= j; ++i) {

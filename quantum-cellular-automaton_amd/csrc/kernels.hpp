@@ -9,6 +9,9 @@ namespace qca {
 
 // Maximum Krylov dimension (one wave holds the tridiagonal matrix).
 constexpr int LZ_MAXK = 64;
+// LanczosCtrl::hit_limit: the last vector's error estimate was above the tolerance,
+// or the start or a matvec was not finite.
+constexpr int LZ_NON_FINITE = 2;
 
 // Lanczos control block, device resident.  Written by the reduction kernels,
 // read back by the host only once per exponential.

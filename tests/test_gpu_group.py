@@ -119,3 +119,25 @@ def test_group_rejects_mixed_sets(gpu):
         qn.Group([e2, em])
     with pytest.raises(qn.QcaError, match="twice"):
         qn.Group([e2, e2])
+
+
+@pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "mixed"])
+def test_non_finite_krylov_is_reported(gpu, prec, monkeypatch):
+    """A Hamiltonian with a NaN: the multi-launch exponentials report it, alone and
+    in a group."""
+    monkeypatch.setenv("QCA_FUSED_KRYLOV_MAX_N", "0")
+    n = 6
+    W = [w.copy() for w in AU.mpo_tensors(n, 1, range(1, 2))]
+    W[3][np.nonzero(W[3])] = float("nan")
+    engines = [qn.Engine(W, OM.product_state([0.3] * n), algorithm=2, precision=prec, chi_max=8, dt=0.1, eps=1e-10,
+                         krylov_tol=0.0) for _ in range(3)]
+    with pytest.raises(qn.QcaError) as e:
+        engines[0].step(1)
+    assert e.value.code == -4
+    g = qn.Group(engines[1:])
+    with pytest.raises(qn.QcaError) as e:
+        g.step(1)
+    assert e.value.code == -4
+    g.close()
+    for e in engines:
+        e.close()

@@ -496,3 +496,30 @@ def test_svd_split_column_out_of_range(gpu, scale, chil, chir, right):
     assert np.abs(Q.conj().T @ Q - np.eye(kk)).max() < 1e-13
     kept = (u[:, :kk] * ref[:kk] / np.linalg.norm(ref[:kk])) @ vh[:kk]
     assert np.abs(A @ B - kept).max() < 1e-12
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("kind,chil,chir", [(0, 3, 4), (1, 24, 24), (2, 33, 17)])
+@pytest.mark.parametrize("where", ["L", "R", "x", "huge"])
+def test_krylov_expm_refuses_non_finite(gpu, where, kind, chil, chir, prec):
+    """A NaN in an environment or in the state, or a state whose norm overflows, is
+    QCA_ERR_NOT_CONVERGED, and the state is left as it was."""
+    import torch
+    rng = np.random.default_rng(chil)
+    W = AU.bulk_tensor(2, range(2, 5))
+    D = W.shape[2]
+    Wk = None if kind == 2 else np.ascontiguousarray(LOC.merge_w(W, W) if kind == 0 else W, dtype=np.complex128)
+    x = crand(rng, {0: 4, 1: 2, 2: 1}[kind], chil, chir)
+    L, R = herm_env(rng, chil, D), herm_env(rng, chir, D)
+    if where == "huge":
+        x *= 1e200
+    else:
+        # channel 0 of an environment carries the finished terms: it is always read
+        {"L": L[:, 0], "R": R[:, -1], "x": x[0]}[where][0, 0] = float("nan")
+    dt = np.complex128 if prec == 0 else np.complex64
+    xd, Ld, Rd = dev(torch, x, np.complex128), dev(torch, L, dt), dev(torch, R, dt)
+    with pytest.raises(qn.QcaError) as e:
+        qn.call("qca_krylov_expm", prec, kind, qn.ptr(xd), qn.ptr(Ld), qn.ptr(Rd),
+                Wk.ctypes.data if Wk is not None else None, D, D, chil, chir, 0.05, 0.0, None, None)
+    assert e.value.code == -4
+    assert np.array_equal(xd.cpu().numpy(), x, equal_nan=True)
