@@ -264,8 +264,9 @@ int qca_exact_apply_h(int precision, const void* psi, void* out, int ncells, int
 
 /* psi <- exp(-i (pi/2) dt H) psi on the 2^N basis (complex128, device) by a
  * Chebyshev series with the closed-form H (|H| <= ncells), cut where its tail
- * falls below tol * |psi|.  Replaces reference exact.py:15-28.  A step with
- * (pi/2) |dt| ncells > 512 is cut into equal substeps.  Uses three vectors of
+ * falls well below tol * |psi|.  Replaces reference exact.py:15-28.  A step with
+ * (pi/2) |dt| ncells > 512 is cut into equal substeps, tol holding for all of
+ * them together.  Uses three vectors of
  * workspace.  *iters receives the number of H applications.  Amplitudes that
  * are not finite are an error (-4), and psi is left as it was. */
 int qca_exact_expm(void* psi, int ncells, int distance, int lo, int hi, double dt, double tol,

@@ -230,24 +230,24 @@ void launch_step(const cplx<T>* phi, int ncells, int distance, int lo, int hi, c
 
 // J_0(z) .. J_kmax(z), z >= 0, by Miller's downward recurrence normalised with
 // J_0 + 2 (J_2 + J_4 + ...) = 1; for tiny z by the first two series terms.
-std::vector<double> bessel_j(double z, int kmax) {
+std::vector<double> bessel_j(long double z, int kmax) {
   std::vector<double> f(kmax + 1, 0.0);
-  if (z < 1e-3) {
+  if (z < 1e-3L) {
     double t = 1.0;   // (z/2)^k / k!
     for (int k = 0; k <= kmax; ++k) {
-      const double q = z * z / 4;
+      const double q = (double)(z * z / 4);
       f[k] = t * (1.0 - q / (k + 1) * (1.0 - q / (2.0 * (k + 2))));
-      t *= z / 2 / (k + 1);
+      t *= (double)z / 2 / (k + 1);
     }
     return f;
   }
-  const int start = 2 * ((std::max(kmax, (int)z) + 40 + (int)(12 * std::cbrt(z))) / 2);
+  const int start = 2 * ((std::max(kmax, (int)z) + 40 + (int)(12 * std::cbrt((double)z))) / 2);
   long double up = 0, cur = 1e-300L, sum = 0;
   for (int k = start; k >= 0; --k) {
     // cur = J_k up to the common factor
     if (k <= kmax) f[k] = (double)cur;
     sum += k == 0 ? cur : ((k & 1) ? 0.0L : 2 * cur);
-    const long double down = 2.0L * k / z * cur - up;
+    const long double down = 2 * k / z * cur - up;
     up = cur;
     cur = down;
     if (std::fabs((double)cur) > 1e200) {
@@ -318,9 +318,9 @@ void launch_exact_apply(const cplx<T>* psi, cplx<T>* out, int ncells, int distan
 template void launch_exact_apply<double>(const c128*, c128*, int, int, int, int, hipStream_t);
 template void launch_exact_apply<float>(const c64*, c64*, int, int, int, int, hipStream_t);
 
-std::vector<double> chebyshev_coefficients(double z, double tol) {
+std::vector<double> chebyshev_coefficients(long double z, double tol) {
   // the tail beyond k = z + 20 cbrt(z) + 40 is below 1e-40
-  const int top = (int)z + (int)(20 * std::cbrt(z)) + 40;
+  const int top = (int)z + (int)(20 * std::cbrt((double)z)) + 40;
   std::vector<double> j = bessel_j(z, top);
   // smallest K >= 2 with 2 sum_{k > K} |J_k| < tol
   int K = top;
@@ -333,12 +333,15 @@ std::vector<double> chebyshev_coefficients(double z, double tol) {
 
 int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, double tau, double tol, c128* bufa,
                       c128* bufb, c128* acc, int* bad, hipStream_t s) {
-  const double R = ncells;
-  const double total = std::fabs(tau) * R;
+  // the recurrence multiplies by 2/R as rounded: the series is that of the R this
+  // factor stands for (a relative error of 1e-16 in R shifts every phase by z times
+  // as much)
+  const double scale = 2.0 / ncells;
+  const double total = (double)(2.0L * std::fabs(tau) / scale);
   QCA_CHECK(total < 4e10, "time step too long for the state vector");
   const long substeps = std::max(1L, (long)std::ceil(total / CHEB_MAX_Z));
-  const double z = total / (double)substeps;
-  const std::vector<double> c = chebyshev_coefficients(z, tol);
+  const long double z = 2.0L * std::fabs(tau) / scale / substeps;
+  const std::vector<double> c = chebyshev_coefficients(z, CHEB_TAIL * tol / substeps);
   const int K = (int)c.size() - 1;   // >= 2
   // coefficient of T_k: c_k (-i sign(tau))^k; even k real, odd k imaginary
   const double sg = tau < 0 ? -1.0 : 1.0;
@@ -359,7 +362,7 @@ int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, doubl
       const c128* phi = k == 0 ? psi : (k & 1 ? bufb : bufa);
       c128* next = k & 1 ? bufa : bufb;
       st.prev = k == 0 ? nullptr : (k == 1 ? psi : next);
-      st.scale = k == 0 ? 1.0 / R : 2.0 / R;
+      st.scale = k == 0 ? 0.5 * scale : scale;
       st.last = k == K - 1;
       st.first = k == 0 && sub == 0;
       if (st.first || st.last) st.bad = bad;

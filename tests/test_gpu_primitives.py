@@ -523,3 +523,55 @@ def test_krylov_expm_refuses_non_finite(gpu, where, kind, chil, chir, prec):
                 Wk.ctypes.data if Wk is not None else None, D, D, chil, chir, 0.05, 0.0, None, None)
     assert e.value.code == -4
     assert np.array_equal(xd.cpu().numpy(), x, equal_nan=True)
+
+
+def exact_h(n, d, lo, hi):
+    """The rule Hamiltonian on vectors of any numpy type."""
+    x = np.arange(1 << n)
+    bits = [x >> (n - 1 - i) & 1 for i in range(n)]
+    alive = [sum(bits[j] for j in range(max(0, i - d), min(n, i + d + 1)) if j != i) for i in range(n)]
+    return lambda v: sum(v[x ^ (1 << (n - 1 - i))] * ((alive[i] >= lo) & (alive[i] < hi)) for i in range(n))
+
+
+@pytest.mark.parametrize("n,d,lo,hi,dt", [(12, 2, 2, 5, 0.1), (13, 2, 2, 4, 0.1), (13, 1, 1, 3, 0.2), (14, 2, 1, 5, 0.5)])
+def test_exact_expm_rounding(gpu, n, d, lo, hi, dt):
+    """At the default tolerance nothing but the rounding of the series' K terms is
+    left: sqrt(K) unit roundoffs in the 2-norm (they add up like a random walk),
+    against a Taylor series in extended precision."""
+    import torch
+    rng = np.random.default_rng(n)
+    psi = np.ones(1)
+    for alive in rng.random(n) < 0.3:
+        p = abs(float(alive) - 0.2 * rng.random())
+        psi = np.kron(psi, [np.sqrt(1 - p), np.sqrt(p)])
+    H = exact_h(n, d, lo, hi)
+    ref = psi.astype(np.clongdouble)
+    steps = int(np.ceil(np.pi / 2 * dt * n))
+    h = -1j * np.longdouble(1.5707963267948966 * dt) / steps
+    for _ in range(steps):
+        term = ref
+        for k in range(1, 30):
+            term = H(term) * (h / k)
+            ref = ref + term
+    pd = dev(torch, psi, np.complex128)
+    it = ctypes.c_int(0)
+    qn.call("qca_exact_expm", qn.ptr(pd), n, d, lo, hi, dt, 0.0, ctypes.byref(it), None)
+    err = np.sqrt(float((np.abs(pd.cpu().numpy() - ref) ** 2).sum()))
+    assert err < np.sqrt(it.value) * 1.1102230246251565e-16
+
+
+def test_exact_expm_tolerance_of_a_long_step(gpu):
+    """The tolerance holds for the whole of a step of 12566 units of tau * N (25
+    substeps), not for each of them."""
+    import torch
+    n, d, lo, hi, dt, tol = 8, 1, 1, 3, 1000.0, 1e-4
+    H = exact_h(n, d, lo, hi)
+    Hm = np.stack([H(e) for e in np.eye(1 << n)])
+    lam, U = np.linalg.eigh(Hm)
+    psi = crand(np.random.default_rng(0), 1 << n)
+    psi /= np.linalg.norm(psi)
+    ref = U @ (np.exp(-1j * np.pi / 2 * dt * lam) * (U.T @ psi))
+    pd = dev(torch, psi, np.complex128)
+    qn.call("qca_exact_expm", qn.ptr(pd), n, d, lo, hi, dt, tol, None, None)
+    # eigenvalues to a few eps N, phases 1570 times as much: 1e-11
+    assert np.linalg.norm(pd.cpu().numpy() - ref) < tol
