@@ -575,3 +575,46 @@ def test_exact_expm_tolerance_of_a_long_step(gpu):
     qn.call("qca_exact_expm", qn.ptr(pd), n, d, lo, hi, dt, tol, None, None)
     # eigenvalues to a few eps N, phases 1570 times as much: 1e-11
     assert np.linalg.norm(pd.cpu().numpy() - ref) < tol
+
+
+def extended_qr(M):
+    """Complete-QR factors (Q's first columns, R) by Householder reflectors with
+    LAPACK's signs, in extended precision."""
+    m, n = M.shape
+    A = M.astype(np.clongdouble)
+    refl = []
+    for j in range(min(m, n)):
+        x = A[j:, j]
+        norm = np.sqrt((np.abs(x) ** 2).sum())
+        beta = -norm if x[0].real >= 0 else norm
+        tau, v = (beta - x[0]) / beta, x / (x[0] - beta)
+        v[0] = 1
+        A[j:, j:] -= np.outer(v, np.conj(tau) * (v.conj()[:, None] * A[j:, j:]).sum(axis=0))
+        refl.append((v, tau))
+    Q = np.eye(m, n, dtype=np.clongdouble)
+    for j in reversed(range(len(refl))):
+        v, tau = refl[j]
+        Q[j:] -= np.outer(v, tau * (v.conj()[:, None] * Q[j:]).sum(axis=0))
+    return Q, np.triu(A[:n])
+
+
+@pytest.mark.parametrize("side,chil,chir", [(0, 180, 200), (0, 256, 256), (1, 256, 256)])
+def test_qr_rounding(gpu, side, chil, chir):
+    """Each of up to 16 block reflectors rounds a column of Q once at its own size
+    and brings the rounding of 16 reflectors as a unit of about the same: 8 unit
+    roundoffs in the 2-norm, 4 in R, whose columns take part in fewer of them."""
+    import torch
+    A = crand(np.random.default_rng(chil), 2, chil, chir)
+    A *= np.logspace(0, -2, chir if side == 0 else chil)[(None, None, slice(None)) if side == 0 else (None, slice(None), None)]
+    M = A.reshape(2 * chil, chir) if side == 0 else A.transpose(0, 2, 1).reshape(2 * chir, chil)
+    Q, R = extended_qr(M)
+    t = M.shape[1]
+    An = torch.zeros((2, chil, t) if side == 0 else (2, t, chir), dtype=torch.complex128, device="cuda")
+    C = torch.zeros((t, t), dtype=torch.complex128, device="cuda")
+    Ad = dev(torch, A, np.complex128)
+    qn.call("qca_qr_site", side, qn.ptr(Ad), chil, chir, t, qn.ptr(An), qn.ptr(C), None)
+    gotq = An.cpu().numpy().reshape(len(M), t) if side == 0 else An.cpu().numpy().transpose(0, 2, 1).reshape(len(M), t)
+    gotr = C.cpu().numpy() if side == 0 else C.cpu().numpy().T
+    u = 1.1102230246251565e-16
+    assert np.sqrt(float((np.abs(gotq - Q) ** 2).sum() / t)) < 8 * u
+    assert np.sqrt(float((np.abs(gotr - R) ** 2).sum() / (np.abs(R) ** 2).sum())) < 4 * u
