@@ -257,6 +257,25 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
     }
   T* const xs = smem + (wave * 8 * MI * MI) * 64 + lane;  // partial-tile exchange: [wave][value][lane]
 
+  // 32x32 tiles take K in one chain where 64x64 ones would have had splits and two
+  // K-groups, so two K-tiles at a time are summed in the accumulators and the rest
+  // in 64 bits (FP32 two-site and bond blocks of 16 to 100 with one chain: 15 to 19%
+  // more error than in splits and groups, environments 57%; in this form 5 to 11% and
+  // 5% less, in the same time)
+  constexpr bool BLOCKED = TS == 32;
+  double blk_re[BLOCKED ? 4 : 1] = {}, blk_im[BLOCKED ? 4 : 1] = {};
+  auto flush = [&] {
+    if constexpr (BLOCKED) {
+      static_assert(MI == 1, "one 16x16 tile per wave");
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        blk_re[r] += double(acc_re[0][0][r]);
+        blk_im[r] += double(acc_im[0][0][r]);
+      }
+      acc_re[0][0] = acc_im[0][0] = acc_t{0, 0, 0, 0};
+    }
+  };
+
   load_tile(ch_begin < ch_end ? tile_at(ch_begin, 0) : -1);
   if (skipped) return;
   int it = 0;  // iterations so far: the LDS stage parity
@@ -303,6 +322,7 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
       load_tile(tn);
       __syncthreads();
 
+      if (BLOCKED && li > 0 && (li & 1) == 0) flush();
       // a group without a tile in the last round skips its MFMAs (the barrier
       // stays outside)
       if (t >= 0) {
@@ -367,6 +387,15 @@ __device__ __forceinline__ void gemm_body(const GemmDesc& d, const cplx<T>* __re
             }
       }
       __syncthreads();
+    }
+    if constexpr (BLOCKED) {
+      flush();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        acc_re[0][0][r] = T(blk_re[r]);
+        acc_im[0][0][r] = T(blk_im[r]);
+        blk_re[r] = blk_im[r] = 0;
+      }
     }
     if (fused) {
       // the split's partial tile joins the sum in split order, as splitk_reduce adds it
@@ -552,6 +581,9 @@ GemmPlan gemm_plan(const GemmDesc& d, long ws_elems, bool fp64) {
   for (int ts : {64, 32}) {
     const long tiles = (long)ceil_div(d.M, ts) * ceil_div(d.N, ts) * (ts == 32 ? used : p.batch);
     for (long fill : {0, GEMM_CUS, 2 * GEMM_CUS, 3 * GEMM_CUS}) {   // workgroups that splits bring it to
+      // FP32 sums of large tiles that leave CUs idle stay in splits: without them
+      // the chains double (bond block of 224: 3.2e-7 -> 3.7e-7)
+      if (!fp64 && ts == 64 && fill == 0 && ktiles >= 4 && tiles < 192) continue;
       long sp = ktiles >= 4 && tiles < fill ? std::min<long>(ceil_div(fill, tiles), ktiles / 2) : 1;
       while (sp > 1 && sp * out_elems > ws_elems) --sp;
       const double t = gemm_time(ts, tiles, ktiles, sp, out_bytes, fp64);

@@ -618,3 +618,36 @@ def test_qr_rounding(gpu, side, chil, chir):
     u = 1.1102230246251565e-16
     assert np.sqrt(float((np.abs(gotq - Q) ** 2).sum() / t)) < 8 * u
     assert np.sqrt(float((np.abs(gotr - R) ** 2).sum() / (np.abs(R) ** 2).sum())) < 4 * u
+
+
+@pytest.mark.parametrize("op,chil,chir", [("left", 128, 128), ("right", 128, 128), ("left", 160, 200), ("right", 200, 160),
+                                          (1, 100, 128), (2, 100, 100), (2, 160, 200)])
+def test_fp32_sums_stay_short(gpu, op, chil, chir):
+    """FP32 contractions in 32x32 tiles, random operands: over a chain of 64 additions
+    the partial sum grows like sqrt(i), and so does its rounding error (u / sqrt(3) of
+    it at each one) like a random walk: u sqrt(64 / 2) / sqrt(3) = 2.0e-7 of the sum
+    in each of the two products, 2.8e-7 together in the 2-norm."""
+    import torch
+    rng = np.random.default_rng(chil + chir)
+    W = AU.bulk_tensor(2, range(2, 5))
+    D = W.shape[2]
+    c64 = lambda a: np.ascontiguousarray(a, dtype=np.complex64)
+    L, R = c64(crand(rng, chil, D, chil) / chil), c64(crand(rng, chir, D, chir) / chir)
+    Wh = np.ascontiguousarray(W, dtype=np.complex128)
+    if op in ("left", "right"):
+        side = int(op == "right")
+        A = c64(crand(rng, 2, chil, chir) / np.sqrt(chil + chir))
+        E = R if side else L
+        ref = (LOC.env_right if side else LOC.env_left)(*[a.astype(np.complex128) for a in (E, A)], W)
+        out = torch.zeros(ref.shape, dtype=torch.complex64, device="cuda")
+        Ad, Ed = dev(torch, A, np.complex64), dev(torch, E, np.complex64)
+        qn.call("qca_env_update", 1, side, qn.ptr(Ad), qn.ptr(Ed), qn.ptr(out), Wh.ctypes.data, D, D, chil, chir, None)
+    else:
+        x = c64(crand(rng, chil, chir) if op == 2 else crand(rng, 2, chil, chir))
+        args = [a.astype(np.complex128) for a in (x, L, R)]
+        ref = LOC.bond_apply(*args) if op == 2 else LOC.heff_apply(*args, W)
+        out = torch.zeros(ref.shape, dtype=torch.complex64, device="cuda")
+        xd, Ld, Rd = dev(torch, x, np.complex64), dev(torch, L, np.complex64), dev(torch, R, np.complex64)
+        qn.call("qca_heff_apply", 1, op, qn.ptr(xd), qn.ptr(out), qn.ptr(Ld), qn.ptr(Rd),
+                None if op == 2 else Wh.ctypes.data, D, D, chil, chir, None)
+    assert np.linalg.norm(out.cpu().numpy() - ref) < 2.8e-7 * np.linalg.norm(ref)
