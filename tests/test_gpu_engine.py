@@ -397,3 +397,37 @@ def test_device_observables_match_host_post_processing(gpu):
         if step:
             assert rows[2].max() > 1e-3        # entanglement has built up
         eng.step(1)
+
+
+def test_one_launch_sums_in_fp32(gpu, monkeypatch):
+    """Mixed precision, bond 30, all Krylov exponentials in one launch each: the
+    distance of the populations from those of the FP64 engine (rms over 16 chains)
+    against that of the multi-launch form.  FP32 sums run in chains of 13 x 16 terms
+    here and of 64 there; the rounding of a chain grows like its square root:
+    sqrt(208 / 64) = 1.8 at most."""
+    n, chi = 13, 30
+    W = AU.mpo_tensors(n, 2, range(2, 5))
+    dims = [min(2 ** i, 2 ** (n - i), chi) for i in range(n + 1)]
+    weight = lambda d: np.logspace(0, -2, d)
+
+    def populations(A, prec, limit):
+        monkeypatch.setenv("QCA_FUSED_KRYLOV_MAX_N", str(limit))
+        e = qn.Engine(W, A, algorithm=2, precision=prec, chi_max=chi, dt=0.1, eps=1e-10,
+                      krylov_tol=1e-14 if prec == 0 else 1e-10)
+        out = []
+        for _ in range(3):
+            e.step(1)
+            out.append(e.rho()[:, 1, 1].real.copy())
+        e.close()
+        return np.array(out)
+
+    far = {0: [], 4096: []}
+    for seed in range(16):
+        rng = np.random.default_rng(500 + seed)
+        A = [(rng.standard_normal((2, a, b)) + 1j * rng.standard_normal((2, a, b))) * weight(a)[:, None] * weight(b)
+             for a, b in zip(dims, dims[1:])]
+        ref = populations(A, 0, 4096)
+        for limit in far:
+            far[limit].append(populations(A, 1, limit) - ref)
+    one, many = (np.sqrt(np.mean(np.square(far[limit]))) for limit in (4096, 0))
+    assert one < 1.8 * many
