@@ -651,3 +651,28 @@ def test_fp32_sums_stay_short(gpu, op, chil, chir):
         qn.call("qca_heff_apply", 1, op, qn.ptr(xd), qn.ptr(out), qn.ptr(Ld), qn.ptr(Rd),
                 None if op == 2 else Wh.ctypes.data, D, D, chil, chir, None)
     assert np.linalg.norm(out.cpu().numpy() - ref) < 2.8e-7 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("right", [1, 0])
+@pytest.mark.parametrize("chi", [4, 6, 8, 10, 16])
+def test_svd_split_small_isometry_is_normalised(gpu, chi, right):
+    """The isometry's columns are divided by their own norms: 6 unit roundoffs in the
+    squared norm (the division, and sum and root of the norm, twice each)."""
+    import torch
+    for seed in range(4):
+        rng = np.random.default_rng(100 * chi + seed)
+        w = np.logspace(0, -7, chi)
+        th = crand(rng, 4, chi, chi) * w[:, None] * w
+        th /= np.linalg.norm(th)
+        Al = torch.zeros(4 * chi * chi, dtype=torch.complex128, device="cuda")
+        Ar = torch.zeros(4 * chi * chi, dtype=torch.complex128, device="cuda")
+        k = ctypes.c_int(0)
+        thd = dev(torch, th, np.complex128)
+        qn.call("qca_svd_split", qn.ptr(thd), qn.ptr(Al), qn.ptr(Ar), chi, chi, 2 * chi, 1e-10, right,
+                ctypes.byref(k), None, None)
+        kk = k.value
+        n = 2 * chi * kk
+        Q = Al[:n].cpu().numpy().reshape(2 * chi, kk) if right else \
+            Ar[:n].cpu().numpy().reshape(2, kk, chi).transpose(0, 2, 1).reshape(2 * chi, kk)
+        norm2 = (np.abs(Q.astype(np.clongdouble)) ** 2).sum(axis=0)
+        assert np.abs(norm2 - 1).max() < 6 * 1.1102230246251565e-16
