@@ -8,7 +8,8 @@
 //     that forms Q.  The launch of panel p applies the block reflector of panel
 //     p-1 to all remaining columns, 16 per workgroup, and its first workgroup
 //     goes on to factor the columns it has just updated;
-//   * one workgroup (householder_qr_kernel), for longer rows.
+//   * one workgroup (householder_qr_kernel), for longer rows and for one or two
+//     reflectors.
 //
 // What bounds the blocked form is the chain of 16 dependent columns of a panel,
 // so a panel lives in registers (wave w holds columns w and w + 8, lane l their rows
@@ -522,6 +523,17 @@ __device__ double qr_block_sum(double v, double* sh) {
   return r;
 }
 
+__device__ double qr_block_max(double v, double* sh) {
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double r = 0;
+  for (int w = 0; w < HH_WAVES; ++w) r = fmax(r, sh[w]);
+  __syncthreads();
+  return r;
+}
+
 // M (rows x cols, column-major) -> reflectors below the diagonal, R on and
 // above it (zgeqr2), then Q's first qcols columns (zung2r) into Q.
 __global__ __launch_bounds__(HH_THREADS) void householder_qr_kernel(c128* __restrict__ M, int rows,
@@ -535,21 +547,26 @@ __global__ __launch_bounds__(HH_THREADS) void householder_qr_kernel(c128* __rest
     c128* x = M + (long)j * rows;
     double part = 0;
     for (int r = j + 1 + tid; r < rows; r += HH_THREADS) part += x[r].re * x[r].re + x[r].im * x[r].im;
-    const double xnorm2 = qr_block_sum(part, sh);
-    const c128 alpha = x[j];
-    c128 tj{0.0, 0.0};
-    bool identity = (xnorm2 == 0.0 && alpha.im == 0.0);
-    double beta = 0.0;
-    c128 scale{0.0, 0.0};
-    if (!identity) {
-      const double nrm = sqrt(alpha.re * alpha.re + alpha.im * alpha.im + xnorm2);
-      beta = (alpha.re >= 0.0) ? -nrm : nrm;   // -SIGN(dlapy3, alphr)
-      tj = c128{(beta - alpha.re) / beta, -alpha.im / beta};
-      // scale = 1 / (alpha - beta)
-      const double dr = alpha.re - beta, di = alpha.im;
-      const double den = dr * dr + di * di;
-      scale = c128{dr / den, -di / den};
+    double xnorm2 = qr_block_sum(part, sh);
+    c128 alpha = x[j];
+    int ex = 0;
+    if (!larfg_in_range(alpha.re * alpha.re + alpha.im * alpha.im + xnorm2)) {
+      // squares over- or underflow: the reflector of the scaled column is the same
+      double top = 0;
+      for (int r = j + tid; r < rows; r += HH_THREADS) top = fmax(top, fmax(fabs(x[r].re), fabs(x[r].im)));
+      ex = larfg_exponent(qr_block_max(top, sh));
+      part = 0;
+      for (int r = j + 1 + tid; r < rows; r += HH_THREADS) {
+        x[r] = c128{ldexp(x[r].re, -ex), ldexp(x[r].im, -ex)};
+        part += x[r].re * x[r].re + x[r].im * x[r].im;
+      }
+      xnorm2 = qr_block_sum(part, sh);
+      alpha = c128{ldexp(alpha.re, -ex), ldexp(alpha.im, -ex)};
     }
+    const bool identity = xnorm2 == 0.0 && alpha.im == 0.0;
+    const Larfg h = larfg(alpha, xnorm2);
+    const c128 scale = h.scale, tj = h.tau;
+    const double beta = ex ? ldexp(h.beta, ex) : h.beta;
     __syncthreads();
     if (!identity) {
       for (int r = j + 1 + tid; r < rows; r += HH_THREADS) {
@@ -689,9 +706,13 @@ void launch_blocked_qr(c128* M, int rows, int cols, c128* Q, int qcols, c128* ws
 
 void launch_qr(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols, c128* ws, size_t ws_elems,
                hipStream_t s) {
-  // the blocked form is the faster one at every size that it takes (8 x 4: 29
-  // against 31 us, 64 x 32: 63 against 147)
-  if (ws != nullptr && rows <= QR_MAX_ROWS && ws_elems >= qr_workspace_elems(rows, cols, qcols))
+  // one or two reflectors are quicker without the second launch: 2 x 2 27.8 us against
+  // 30.2, 512 x 1 27.4 against 40.2, 512 x 2 36.7 against 42.2, 2 x 64 33.2 against
+  // 35.2; with three the forms are equal (4 x 3 30.6 us, 512 x 3 44.6 against 44.2),
+  // with more, or beside many columns, the blocked one is ahead (2 x 256 54 against 36,
+  // 8 x 4 33.5 against 31.3, 64 x 32 147 against 63)
+  const bool few = std::min(rows, cols) <= 2 && cols <= 64;
+  if (!few && ws != nullptr && rows <= QR_MAX_ROWS && ws_elems >= qr_workspace_elems(rows, cols, qcols))
     launch_blocked_qr(M, rows, cols, Q, qcols, ws, ws_elems, s);
   else
     launch_householder_qr(M, rows, cols, tau, Q, qcols, s);

@@ -439,7 +439,7 @@ def test_qr_panels_match_lapack(gpu, side, chi_row, chi_col, target):
 
 
 @pytest.mark.parametrize("side", [0, 1])
-@pytest.mark.parametrize("chi_row,chi_col,col", [(1, 2, 0), (9, 9, 3), (40, 20, 17), (150, 33, 32)])
+@pytest.mark.parametrize("chi_row,chi_col,col", [(1, 2, 0), (9, 9, 3), (40, 20, 17), (150, 33, 32), (260, 5, 2)])
 @pytest.mark.parametrize("scale", [1e-156, 1e-160, 1e-170, 1e-300, 0.0, 1e160])
 def test_qr_column_out_of_range(gpu, scale, side, chi_row, chi_col, col):
     """A column whose squares under- or overflow (a vanishing Schmidt direction):
@@ -676,3 +676,12 @@ def test_svd_split_small_isometry_is_normalised(gpu, chi, right):
             Ar[:n].cpu().numpy().reshape(2, kk, chi).transpose(0, 2, 1).reshape(2 * chi, kk)
         norm2 = (np.abs(Q.astype(np.clongdouble)) ** 2).sum(axis=0)
         assert np.abs(norm2 - 1).max() < 6 * 1.1102230246251565e-16
+
+
+@pytest.mark.parametrize("side", [0, 1])
+@pytest.mark.parametrize("chi_row,chi_col,target", [(1, 1, 1), (64, 1, 1), (256, 2, 4), (1, 64, 2), (1, 65, 2), (2, 3, 4),
+                                                    (256, 3, 3)])
+def test_qr_few_reflectors(gpu, side, chi_row, chi_col, target):
+    """On both sides of the choice between the one-workgroup and the blocked QR: one,
+    two and three reflectors, few and many columns beside them."""
+    test_qr_panels_match_lapack(gpu, side, chi_row, chi_col, target)
