@@ -387,6 +387,7 @@ void Engine::fused_run(int kind, int site, c128* x, long n, int chil, int chir, 
     a.col = wp.d64.col;
     if constexpr (std::is_same<T, double>::value) a.val = wp.d64.val; else a.val = wp.d32.val;
     a.nnz = wp.d64.nnz;
+    a.group_max = wp.d64.group_max;
   }
   a.x = x;
   a.V = lw_.V;

@@ -391,6 +391,7 @@ void Group::evolve(std::vector<int> inst, std::vector<int> kind, std::vector<int
       a.col = wp->d64.col;
       a.val = W->val;
       a.nnz = wp->d64.nnz;
+      a.group_max = wp->d64.group_max;
       a.x = x[i];
       a.V = e->lw_.V;
       a.T1 = reinterpret_cast<cplx<T>*>(e->T_);

@@ -129,6 +129,7 @@ struct FusedKrylovArgs {
   const int* col = nullptr;
   const cplx<TE>* val = nullptr;
   int nnz = 0;                 // entries of the sparse MPO
+  int group_max = 0;           // the most entries of any q' (0: not known)
   c128* x = nullptr;           // in/out, n elements
   c128* V = nullptr;           // basis, (max_m - 1) * n elements
   cplx<TE>* T1 = nullptr;      // dq * Din * chil * chir elements
@@ -140,9 +141,10 @@ struct FusedKrylovArgs {
   // Filled by fused_krylov_place: byte offsets into the workgroup's LDS, whether T1
   // and the MPO, and the environments, lie there, the number of leading basis
   // vectors held there, the waves that share a tile of H_eff x (a power of two),
-  // and whether the result goes over T1.
+  // whether the result goes over T1, and for blocks whose H_eff x is taken element
+  // by element the lanes that share one (a power of two; else 0).
   long offW = 0, offRow = 0, offCol = 0, offVal = 0, offL = 0, offR = 0, offV = 0;
-  int t1_lds = 0, env_lds = 0, vcap = 0, parts = 1, overlay = 0;
+  int t1_lds = 0, env_lds = 0, vcap = 0, parts = 1, overlay = 0, lanes = 0;
 };
 
 template <typename TE>

@@ -323,6 +323,104 @@ __device__ __forceinline__ void fk_right(const FusedKrylovArgs<TE>& a, const cpl
   }
 }
 
+// Small blocks, element by element: a 16x16 tile would be padding for the most part,
+// and its wave would walk the entries one after another.  Thread t takes
+// elements t, t + 512, ... of T1, and S lanes share an element of y, each with every
+// S-th entry of its q'.  What a thread reads is the same in every iteration, so the
+// offsets are kept in registers.
+constexpr int FK_SMALL_LEFT = 8;      // elements of T1 per thread
+constexpr int FK_SMALL_RIGHT = 8;     // entries per thread
+template <typename TE>
+struct FkSmall {
+  int v[FK_SMALL_LEFT], l[FK_SMALL_LEFT], out[FK_SMALL_LEFT];   // out < 0: none
+  int t[FK_SMALL_RIGHT], r[FK_SMALL_RIGHT], entries;
+  cplx<TE> val[FK_SMALL_RIGHT];
+};
+template <typename TE>
+__device__ __forceinline__ void fk_small_init(const FusedKrylovArgs<TE>& a, const unsigned char* channel, int nch,
+                                              const int* rowptr, const int* col, const cplx<TE>* val,
+                                              FkSmall<TE>& m) {
+  const int lr = a.chil * a.chir, tid = threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < FK_SMALL_LEFT; ++k) {
+    const int i = tid + FK_THREADS * k, n = i / lr, rem = i - n * lr, c = rem / a.chil, x = rem - c * a.chil;
+    const bool in = n < nch;
+    const int qw = !in ? 0 : channel ? channel[n] : n, q = qw / a.Din, w = qw - q * a.Din;
+    m.v[k] = q * lr + c;
+    m.l[k] = w * a.chil + x;
+    m.out[k] = in ? qw * lr + rem : -1;
+  }
+  const int e = tid / a.lanes, s = tid & (a.lanes - 1), q = e / lr, rem = e - q * lr, x = rem / a.chir,
+            yy = rem - x * a.chir;
+  m.entries = 0;
+#pragma unroll
+  for (int k = 0; k < FK_SMALL_RIGHT; ++k) {
+    m.t[k] = m.r[k] = 0;
+    m.val[k] = cplx<TE>{TE(1), TE(0)};
+  }
+  if (e >= (int)a.n) return;
+  const int first = a.kind == 2 ? 0 : rowptr[q * a.Dout], last = a.kind == 2 ? a.Dout : rowptr[(q + 1) * a.Dout];
+#pragma unroll
+  for (int k = 0; k < FK_SMALL_RIGHT; ++k) {
+    const int z = first + s + a.lanes * k;
+    if (z >= last) break;
+    int v = z, cz = z;
+    if (a.kind != 2) {
+      v = 0;
+      for (int r = 1; r < a.Dout; ++r) v += rowptr[q * a.Dout + r] <= z ? 1 : 0;
+      cz = col[z];
+      m.val[k] = val[z];
+    }
+    m.t[k] = cz * lr + x;
+    m.r[k] = v * a.chir + yy;
+    m.entries = k + 1;
+  }
+}
+template <typename TE>
+__device__ __forceinline__ void fk_small_left(const FusedKrylovArgs<TE>& a, const c128* v, const cplx<TE>* L,
+                                              cplx<TE>* T1, const FkSmall<TE>& m) {
+  cplx<TE> acc[FK_SMALL_LEFT] = {};
+  const int ls = a.Din * a.chil;
+  for (int i = 0; i < a.chil; ++i) {
+#pragma unroll
+    for (int k = 0; k < FK_SMALL_LEFT; ++k) {
+      if (m.out[k] < 0) continue;
+      const c128 x = v[m.v[k] + i * a.chir];
+      const cplx<TE> y = L[m.l[k] + i * ls], z{TE(x.re), TE(x.im)};
+      acc[k].re += z.re * y.re - z.im * y.im;
+      acc[k].im += z.re * y.im + z.im * y.re;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < FK_SMALL_LEFT; ++k)
+    if (m.out[k] >= 0) T1[m.out[k]] = acc[k];
+}
+template <typename TE>
+__device__ __forceinline__ void fk_small_right(const FusedKrylovArgs<TE>& a, const cplx<TE>* T1, const cplx<TE>* R,
+                                               const FkSmall<TE>& m, c128* y) {
+  double re = 0, im = 0;
+  const int rs = a.Dout * a.chir;
+#pragma unroll
+  for (int k = 0; k < FK_SMALL_RIGHT; ++k) {
+    if (k >= m.entries) continue;
+    cplx<TE> acc{TE(0), TE(0)};
+    for (int c = 0; c < a.chir; ++c) {
+      const cplx<TE> t = T1[m.t[k] + c * a.chil], r = R[m.r[k] + c * rs];
+      acc.re += t.re * r.re - t.im * r.im;
+      acc.im += t.re * r.im + t.im * r.re;
+    }
+    re += double(m.val[k].re * acc.re - m.val[k].im * acc.im);
+    im += double(m.val[k].re * acc.im + m.val[k].im * acc.re);
+  }
+  // over the lanes of an element (a row of 16 at most)
+  if (a.lanes > 1) re += dpp_f64<0xB1>(re), im += dpp_f64<0xB1>(im);      // quad_perm(1,0,3,2)
+  if (a.lanes > 2) re += dpp_f64<0x4E>(re), im += dpp_f64<0x4E>(im);      // quad_perm(2,3,0,1)
+  if (a.lanes > 4) re += dpp_f64<0x141>(re), im += dpp_f64<0x141>(im);    // row_half_mirror
+  if (a.lanes > 8) re += dpp_f64<0x140>(re), im += dpp_f64<0x140>(im);    // row_mirror
+  const int e = threadIdx.x / a.lanes;
+  if ((threadIdx.x & (a.lanes - 1)) == 0 && e < (int)a.n) y[e] = c128{re, im};
+}
+
 // Lane l + 1 and lane l - 1 of the wave, 0 beyond its ends.
 template <int CTRL>
 __device__ __forceinline__ double wave_shift(double v) {
@@ -407,9 +505,8 @@ struct FkBound {
   }
 };
 
-template <typename TE, int EPT>
-__device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, unsigned char* arena) {
-  __shared__ FkShared sh;
+template <typename TE, int EPT, bool SMALL>
+__device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, unsigned char* arena, FkShared& sh) {
   const int n = (int)a.n, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned long long t0 = wall_clock64();
@@ -451,8 +548,15 @@ __device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, 
   if (listed && tid < 64 && (used >> tid & 1)) sh.channel[__popcll(used & ((1ull << tid) - 1))] = (unsigned char)tid;
   const unsigned char* channel = listed ? sh.channel : nullptr;
   const int nch = listed ? __popcll(used) : ncol;
-  const int q0 = fk_first_q(a, dq);
-  const FkEntries<TE> mine = a.t1_lds ? fk_rows(a, q0, rowptr, col, val) : fk_rows(a, q0, a.rowptr, a.col, a.val);
+  FkSmall<TE> sm;
+  FkEntries<TE> mine;
+  if constexpr (SMALL) {
+    __syncthreads();
+    fk_small_init(a, channel, nch, rowptr, col, val, sm);
+  } else {
+    const int q0 = fk_first_q(a, dq);
+    mine = a.t1_lds ? fk_rows(a, q0, rowptr, col, val) : fk_rows(a, q0, a.rowptr, a.col, a.val);
+  }
   // f(V_i) with the basis vector in its own address space
   auto with_basis = [&](int i, auto&& f) {
     if (i < a.vcap) f(Vl + (unsigned)(i * n));
@@ -489,7 +593,11 @@ __device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, 
       __syncthreads();
       // w = H_eff V_j
       const c128* vj = j < a.vcap ? Vl + (unsigned)(j * n) : Vg + (unsigned)(j * n);
-      if (a.env_lds) {
+      if constexpr (SMALL) {
+        fk_small_left(a, vj, Ll, T1l, sm);
+        __syncthreads();
+        fk_small_right(a, T1l, Rl, sm, wbuf);
+      } else if (a.env_lds) {
         fk_left<TE>(a, vj, Ll, T1l, channel, nch);
         __syncthreads();
         fk_right<TE>(a, T1l, Rl, rowptr, col, val, mine, wbuf);
@@ -638,10 +746,11 @@ __device__ __forceinline__ void fused_krylov_body(const FusedKrylovArgs<TE>& a, 
   }
 }
 
-template <typename TE, int EPT>
+template <typename TE, int EPT, bool SMALL>
 __global__ __launch_bounds__(FK_THREADS) void fused_krylov_kernel(FusedKrylovArgs<TE> a) {
   extern __shared__ __align__(16) unsigned char arena[];
-  fused_krylov_body<TE, EPT>(a, arena);
+  __shared__ FkShared sh;
+  fused_krylov_body<TE, EPT, SMALL>(a, arena, sh);
 }
 
 // One exponential per workgroup, each with its own arguments and LDS placement
@@ -661,7 +770,9 @@ __global__ __launch_bounds__(FK_THREADS) void fused_krylov_grouped(const GRec<Fu
   a.T1 = gbl(a.T1);
   a.ctrl = gbl(a.ctrl);
   a.tally = gbl(a.tally);
-  fused_krylov_body<TE, EPT>(a, arena);
+  __shared__ FkShared sh;
+  if (a.lanes > 0) fused_krylov_body<TE, 1, true>(a, arena, sh);
+  else fused_krylov_body<TE, EPT, false>(a, arena, sh);
 }
 
 }  // namespace
@@ -677,16 +788,36 @@ size_t fused_krylov_place(const FusedKrylovArgs<TE>& a, FusedKrylovArgs<TE>& b) 
   QCA_CHECK(a.kind != 2 || a.Din == a.Dout, "bond block needs equal MPO bonds");
   QCA_CHECK(a.kind == 2 || a.nnz >= 0, "negative MPO entry count");
   QCA_CHECK(a.kind == 2 || a.Dout <= 16, "MPO bond dimension above 16");
-  // tiles of y and the waves that share one, splitting its MPO rows
   b = a;
   const long lr = (long)a.chil * a.chir;
+  const long t1 = (long)dq * a.Din * lr * sizeof(cplx<TE>);
+  const long nnz = a.kind == 2 ? 0 : a.nnz, nrow = a.kind == 2 ? 0 : dq * a.Dout + 1;
+  const long mpo = 48 + nrow * (long)sizeof(int) + nnz * (long)(sizeof(int) + sizeof(cplx<TE>));
+  const long envL = (long)a.chil * a.Din * a.chil * sizeof(cplx<TE>), envR = (long)a.chir * a.Dout * a.chir * sizeof(cplx<TE>);
+  // Up to 64 elements of chil x chir, element by element, by as many lanes per
+  // element of y as there are (16 at most), if a thread's share fits its registers and
+  // the operands LDS (MPO bond 13, FP64, tiles -> elements: two-site 1 x 1 64.7 -> 22.7
+  // us, 4 x 4 146 -> 63, 4 x 8 210 -> 118, 8 x 8 221 -> 150, 16 x 4 203 -> 146; one-site 8 x 8
+  // 148 -> 120; from 8 x 16 on tiles: 172 against 186 there).  A bond block has one
+  // entry per row, so only its walk along c is left to shorten: up to 12 (4 x 12 101 ->
+  // 82; 4 x 16 106 against 135).
+  b.lanes = 16;
+  while (b.lanes > 0 && b.lanes * a.n > FK_THREADS) b.lanes /= 2;
+  const int group = a.kind == 2 ? a.Dout : (a.group_max > 0 ? a.group_max : a.nnz);
+  if (b.lanes > 0 && (lr > 64 || (a.kind == 2 && a.chir > 12) ||
+                      (long)dq * a.Din * lr > (long)FK_SMALL_LEFT * FK_THREADS ||
+                      ceil_div(group, b.lanes) > FK_SMALL_RIGHT ||
+                      t1 + 16 + a.n * (long)sizeof(c128) + mpo + envL + envR + 32 > FK_LDS_BYTES))
+    b.lanes = 0;
+  // tiles of y and the waves that share one, splitting its MPO rows
   const long tiles = (long)dq * ceil_div(a.chil, 16) * ceil_div(a.chir, 16);
   b.parts = 1;
-  while (2 * b.parts * tiles <= FK_WAVES && 2 * b.parts <= a.Dout) b.parts *= 2;
+  if (b.lanes == 0)
+    while (2 * b.parts * tiles <= FK_WAVES && 2 * b.parts <= a.Dout) b.parts *= 2;
   // LDS: T1 and the MPO if both fit (else they stay in global memory), the partial
   // sums of y (over T1 if every wave has its tiles in registers by then), leading
   // basis vectors
-  b.overlay = tiles * b.parts <= FK_WAVES;
+  b.overlay = b.lanes == 0 && tiles * b.parts <= FK_WAVES;
   long off = 0;
   auto take = [&](long bytes) {
     const long o = off;
@@ -694,10 +825,8 @@ size_t fused_krylov_place(const FusedKrylovArgs<TE>& a, FusedKrylovArgs<TE>& b) 
     return o;
   };
   const long py = b.parts * a.n * (long)sizeof(c128);
-  const long t1 = (long)dq * a.Din * lr * sizeof(cplx<TE>);
-  const long nnz = a.kind == 2 ? 0 : a.nnz, nrow = a.kind == 2 ? 0 : dq * a.Dout + 1;
   const long work = b.overlay ? std::max(t1, py) : t1 + 16 + py;
-  b.t1_lds = work + 64 + nrow * (long)sizeof(int) + nnz * (long)(sizeof(int) + sizeof(cplx<TE>)) <= FK_LDS_BYTES;
+  b.t1_lds = work + 16 + mpo <= FK_LDS_BYTES;
   if (b.t1_lds) {
     take(b.overlay ? std::max(t1, py) : t1);
     b.offW = b.overlay ? 0 : take(py);
@@ -709,7 +838,6 @@ size_t fused_krylov_place(const FusedKrylovArgs<TE>& a, FusedKrylovArgs<TE>& b) 
   }
   // environments: both, ahead of the basis (their latency is in the way of every
   // product; the basis is streamed)
-  const long envL = (long)a.chil * a.Din * a.chil * sizeof(cplx<TE>), envR = (long)a.chir * a.Dout * a.chir * sizeof(cplx<TE>);
   b.env_lds = b.t1_lds && off + envL + envR + 32 <= FK_LDS_BYTES;
   b.offL = b.env_lds ? take(envL) : 0;
   b.offR = b.env_lds ? take(envR) : 0;
@@ -729,8 +857,9 @@ void launch_fused_krylov(const FusedKrylovArgs<TE>& a, hipStream_t s) {
     ensure_dynamic_lds((const void*)kernel, off);
     hipLaunchKernelGGL(kernel, dim3(1), dim3(FK_THREADS), off, s, b);
   };
-  if (a.n <= FK_SMALL_N) run(fused_krylov_kernel<TE, 2>);
-  else run(fused_krylov_kernel<TE, FK_EPT_MAX>);
+  if (b.lanes > 0) run(fused_krylov_kernel<TE, 1, true>);
+  else if (a.n <= FK_SMALL_N) run(fused_krylov_kernel<TE, 2, false>);
+  else run(fused_krylov_kernel<TE, FK_EPT_MAX, false>);
   QCA_HIP(hipGetLastError());
 }
 template void launch_fused_krylov<double>(const FusedKrylovArgs<double>&, hipStream_t);

@@ -431,3 +431,29 @@ def test_one_launch_sums_in_fp32(gpu, monkeypatch):
             far[limit].append(populations(A, 1, limit) - ref)
     one, many = (np.sqrt(np.mean(np.square(far[limit]))) for limit in (4096, 0))
     assert one < 1.8 * many
+
+
+@pytest.mark.parametrize("algo", [1, 2])
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("d,iv", [(1, range(1, 3)), (2, range(2, 5))])
+@pytest.mark.parametrize("dims", [[1, 2, 4, 4, 2, 1], [1, 2, 4, 8, 8, 8, 4, 2, 1], [1, 2, 4, 8, 9, 7, 9, 5, 4, 2, 1],
+                                  [1, 2, 4, 5, 10, 13, 6, 3, 2, 1], [1, 2, 4, 8, 12, 5, 12, 6, 3, 2, 1]])
+def test_one_launch_small_blocks(gpu, dims, d, iv, prec, algo, monkeypatch):
+    """Krylov exponentials of small blocks in one launch, element by element and in
+    tiles, on both sides of the choice (up to 64 elements per physical index, bond
+    blocks up to 12 columns), against the multi-launch form: 60 exponentials a step to
+    1e-14 (mixed 1e-7, the FP32 contractions) each, the bonds' weights down to 1e-2;
+    relative to the state's norm, which 1TDVP keeps as it is."""
+    n = len(dims) - 1
+    rng = np.random.default_rng(sum(dims))
+    weight = lambda k: np.logspace(0, -2, k)
+    A = [crand(rng, 2, a, b) * weight(a)[:, None] * weight(b) for a, b in zip(dims, dims[1:])]
+    out = []
+    for limit in (0, 4096):
+        monkeypatch.setenv("QCA_FUSED_KRYLOV_MAX_N", str(limit))
+        e = make_engine(A, AU.mpo_tensors(n, d, iv), algo, 16, 0.1, 1e-10, prec)
+        e.step(2)
+        out.append(e.rho())
+        e.close()
+    norm2 = np.abs(np.trace(out[0], axis1=1, axis2=2)).max()
+    assert np.abs(out[0] - out[1]).max() < (1e-11 if prec == 0 else 1e-5) * norm2
