@@ -159,12 +159,13 @@ struct QrStepArgs {   // launch p: reflector p-1 on the columns from 16 p on, th
   int rows, cols, p;
   c128* T;            // 16 x 16 per panel
 };
-struct QrFormArgs {   // Q from the first kk reflectors
+struct QrFormArgs {   // Q from the first kk reflectors, or Q times kk x qcols Z
   const c128* M;
   int rows, kk;
   const c128* T;
   c128* Q;
   int qcols;
+  const c128* Z;
 };
 constexpr int QR_SLOT_Q = QR_MAX_ROWS / 16 + 1;   // after every panel's slot
 struct QrStep {
@@ -176,6 +177,10 @@ struct QrStep {
   QrFormArgs form;
 };
 std::vector<QrStep> blocked_qr_steps(c128* M, int rows, int cols, c128* Q, int qcols, c128* ws, size_t ws_elems);
+// The launch that forms qcols columns of Q (or of Q times Z) from kk reflectors in M
+// and their T (the workspace of blocked_qr_steps).
+QrStep form_q_step(const c128* M, int rows, int kk, const c128* T, c128* Q, int qcols, const c128* Z);
+void launch_form_q(const QrStep& st, hipStream_t s);
 
 // ------------------------------------------------------------------ SVD
 // One launch_jacobi_svd call of one instance.

@@ -209,8 +209,9 @@ struct JacobiLayout {
 JacobiLayout jacobi_layout(int rows, int cols);
 size_t jacobi_workspace_bytes(int max_rows, int max_cols);
 size_t jacobi_precond_elems(int max_rows, int max_cols);
-// One workgroup takes the whole SVD.
+// One workgroup takes the whole SVD, or that of the triangle of a QR.
 bool small_svd(int rows, int cols);
+bool tall_svd(int rows, int cols);
 
 // One-sided (block) Jacobi SVD of the column-major matrix X (rows x cols,
 // FP64), in place.  On exit the columns are orthogonal; sigma (sorted

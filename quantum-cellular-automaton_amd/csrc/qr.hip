@@ -442,13 +442,14 @@ __device__ __forceinline__ void qr_step_body(const QrStepArgs& a, c128* __restri
   }
 }
 
-// Columns 16 blk.. of Q = H_0 ... H_{kk-1} [e_0 .. e_{qcols-1}]: the block
-// reflectors from the last panel back, on columns that stay in registers.  A
-// panel right of the block's columns leaves them as they are.
+// Columns 16 blk.. of Q = H_0 ... H_{kk-1} [e_0 .. e_{qcols-1}], or of H_0 ...
+// H_{kk-1} (Z; 0): the block reflectors from the last panel back, on columns that
+// stay in registers.  A panel right of the block's columns of [e_0 ..] leaves them as
+// they are.
 template <int QR_TILES>
 __device__ __forceinline__ void form_q_body(const QrFormArgs& a, const c128* __restrict__ M,
-                                            const c128* __restrict__ T, c128* __restrict__ Q, int blk, c128* big,
-                                            QrShared& sh) {
+                                            const c128* __restrict__ T, c128* __restrict__ Q,
+                                            const c128* __restrict__ Z, int blk, c128* big, QrShared& sh) {
   const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rows = a.rows, kk = a.kk, c0 = QR_PB * blk;
@@ -457,10 +458,14 @@ __device__ __forceinline__ void form_q_body(const QrFormArgs& a, const c128* __r
   for (int t = 0; t < QR_TILES; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      qre[t][r] = 16 * (wave + QR_WAVES * t) + 4 * r + hi == c0 + lo ? 1.0 : 0.0;
-      qim[t][r] = 0.0;
+      const int row = 16 * (wave + QR_WAVES * t) + 4 * r + hi, col = c0 + lo;
+      c128 z{row == col ? 1.0 : 0.0, 0.0};
+      if (Z) z = row < kk && col < a.qcols ? Z[(long)col * kk + row] : c128{0.0, 0.0};
+      qre[t][r] = z.re;
+      qim[t][r] = z.im;
     }
-  for (int p = min((kk + QR_PB - 1) / QR_PB - 1, blk); p >= 0; --p) {
+  const int last = (kk + QR_PB - 1) / QR_PB - 1;
+  for (int p = Z ? last : min(last, blk); p >= 0; --p) {
     const int j0 = p * QR_PB, pb = min(QR_PB, kk - j0);
     QrOperands<QR_TILES> o;
     load_operands(M, rows, j0, pb, T + (long)p * QR_PB * QR_PB, false, o);
@@ -497,7 +502,7 @@ template <int TILES>
 __global__ QCA_QR_BOUNDS void form_q_kernel(QrFormArgs a) {
   extern __shared__ __align__(16) unsigned char qr_lds[];
   __shared__ QrShared sh;
-  form_q_body<TILES>(a, a.M, a.T, a.Q, blockIdx.x, reinterpret_cast<c128*>(qr_lds), sh);
+  form_q_body<TILES>(a, a.M, a.T, a.Q, a.Z, blockIdx.x, reinterpret_cast<c128*>(qr_lds), sh);
 }
 template <int TILES>
 __global__ QCA_QR_BOUNDS void form_q_grouped(const GRec<QrFormArgs>* __restrict__ recs, int n) {
@@ -505,7 +510,7 @@ __global__ QCA_QR_BOUNDS void form_q_grouped(const GRec<QrFormArgs>* __restrict_
   __shared__ QrShared sh;
   unsigned bx, by, bz;
   const QrFormArgs a = grec_find(recs, n, blockIdx.x, bx, by, bz).a;
-  form_q_body<TILES>(a, gbl(a.M), gbl(a.T), gbl(a.Q), bx, reinterpret_cast<c128*>(qr_lds), sh);
+  form_q_body<TILES>(a, gbl(a.M), gbl(a.T), gbl(a.Q), a.Z ? gbl(a.Z) : nullptr, bx, reinterpret_cast<c128*>(qr_lds), sh);
 }
 
 constexpr int HH_THREADS = 1024;
@@ -644,6 +649,16 @@ size_t qr_workspace_elems(int max_rows, int max_cols, int) {
   return (size_t)ceil_div(std::max(1, std::min(max_rows, max_cols)), QR_PB) * QR_PB * QR_PB;   // T per panel
 }
 
+QrStep form_q_step(const c128* M, int rows, int kk, const c128* T, c128* Q, int qcols, const c128* Z) {
+  QrStep st{};
+  st.slot = QR_SLOT_Q;
+  st.kind = 1;
+  st.blocks = ceil_div(qcols, QR_PB);
+  st.lds = sizeof(c128) * (size_t)QR_WAVES * QR_PB * QR_PB;
+  st.form = QrFormArgs{M, rows, kk, T, Q, qcols, Z};
+  return st;
+}
+
 // The blocked QR as a list of launches, each with a slot number that orders
 // it among those of any other matrix: the single-matrix launcher runs them in
 // order, the grouped one runs every slot for all matrices that have it.
@@ -665,14 +680,7 @@ std::vector<QrStep> blocked_qr_steps(c128* M, int rows, int cols, c128* Q, int q
     st.step = QrStepArgs{M, rows, cols, p, ws};
     out.push_back(st);
   }
-  if (Q == nullptr || qcols == 0) return out;
-  QrStep st{};
-  st.slot = QR_SLOT_Q;
-  st.kind = 1;
-  st.blocks = ceil_div(qcols, QR_PB);
-  st.lds = sizeof(c128) * (size_t)QR_WAVES * QR_PB * QR_PB;
-  st.form = QrFormArgs{M, rows, std::min(kmax, qcols), ws, Q, qcols};
-  out.push_back(st);
+  if (Q != nullptr && qcols > 0) out.push_back(form_q_step(M, rows, std::min(kmax, qcols), ws, Q, qcols, nullptr));
   return out;
 }
 
@@ -696,10 +704,15 @@ void launch_form_q_grouped(const KGroup<QrFormArgs>& g, int rows, size_t lds, hi
   QCA_HIP(hipGetLastError());
 }
 
+void launch_form_q(const QrStep& st, hipStream_t s) {
+  launch_rows(form_q_kernel<2>, form_q_kernel<4>, st.form.rows, st.blocks, st.lds, s, st.form);
+  QCA_HIP(hipGetLastError());
+}
+
 void launch_blocked_qr(c128* M, int rows, int cols, c128* Q, int qcols, c128* ws, size_t ws_elems, hipStream_t s) {
   for (const QrStep& st : blocked_qr_steps(M, rows, cols, Q, qcols, ws, ws_elems)) {
     if (st.kind == 0) launch_rows(qr_step_kernel<2>, qr_step_kernel<4>, rows, st.blocks, st.lds, s, st.step);
-    else launch_rows(form_q_kernel<2>, form_q_kernel<4>, rows, st.blocks, st.lds, s, st.form);
+    else launch_form_q(st, s);
   }
   QCA_HIP(hipGetLastError());
 }

@@ -958,7 +958,8 @@ __global__ __launch_bounds__(JAC_NT) void jac_finalize(const c128* __restrict__ 
 // us, QR 19 + 20, two sweeps 42 + 10 (rounds, products), four closing steps 34, Q1
 // 5, norms and rank 3; a split of that size in all 721 -> 256 us, 24x32 647 ->
 // 246, 60x30 531 -> 265.  Without the second QR 54 us more sweeps, for 25 of QR
-// and Q1.  Rows beyond 128 (register columns) take the launches below.
+// and Q1.  Rows beyond 128 (register columns): the triangle of a QR when there are at
+// most 32 columns (tall_svd), else the launches below.
 constexpr int SMALL_NT = 256;
 constexpr int SMALL_ROWS = 128;
 constexpr int SMALL_LDV = SMALL_ROWS + 1;
@@ -1303,9 +1304,10 @@ __device__ __forceinline__ bool small_jacobi(SmallShared& sh, int kq, const Inne
 }
 
 template <int IT>
-__device__ __forceinline__ void jac_small_body(c128* __restrict__ X, int rows, int cols, double* __restrict__ sigma,
-                                               int* __restrict__ perm, SvdResult* __restrict__ res, int chi_max,
-                                               double eps, int rank_cap, double tol, SmallShared& sh) {
+__device__ __forceinline__ void jac_small_body(const c128* __restrict__ in, int ld, c128* __restrict__ X, int rows,
+                                               int cols, double* __restrict__ sigma, int* __restrict__ perm,
+                                               SvdResult* __restrict__ res, int chi_max, double eps, int rank_cap,
+                                               double tol, SmallShared& sh) {
   const int tid = threadIdx.x, c = tid >> 3, rl = tid & 7;
   const bool wide = rows < cols;
   const int kq = min(rows, cols), nr = max(rows, cols);
@@ -1313,8 +1315,8 @@ __device__ __forceinline__ void jac_small_body(c128* __restrict__ X, int rows, i
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
     const int r = rl + 8 * i, cc = min(c, kq - 1), rr = min(r, nr - 1);
-    x[i] = wide ? conj_of(X[rr * rows + cc]) : X[cc * rows + rr];
-    if (c >= kq || r >= nr) x[i] = c128{0.0, 0.0};
+    x[i] = wide ? conj_of(in[rr * ld + cc]) : in[cc * ld + rr];
+    if (c >= kq || r >= nr || (ld > rows && r > c)) x[i] = c128{0.0, 0.0};
   }
   small_sort(x, sh, sh.V, SMALL_LDV);
   double fro = 0;
@@ -1397,20 +1399,23 @@ __device__ __forceinline__ void jac_small_body(c128* __restrict__ X, int rows, i
     res->tail = sqrt(tail);
   }
 }
-// Rows of the tall orientation in registers: 32, 64 or 128.
-__device__ __forceinline__ void jac_small_rows(c128* X, int rows, int cols, double* sigma, int* perm, SvdResult* res,
-                                               int chi_max, double eps, int rank_cap, double tol) {
+// Rows of the tall orientation in registers: 32, 64 or 128.  `in` is X itself (ld =
+// rows), or the square matrix is the triangle of a QR above the diagonal of a taller
+// matrix (ld > rows).
+__device__ __forceinline__ void jac_small_rows(const c128* in, int ld, c128* X, int rows, int cols, double* sigma,
+                                               int* perm, SvdResult* res, int chi_max, double eps, int rank_cap,
+                                               double tol) {
   __shared__ SmallShared sh;
   const int nr = max(rows, cols);
-  if (nr <= 32) jac_small_body<4>(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
-  else if (nr <= 64) jac_small_body<8>(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
-  else jac_small_body<16>(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
+  if (nr <= 32) jac_small_body<4>(in, ld, X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
+  else if (nr <= 64) jac_small_body<8>(in, ld, X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
+  else jac_small_body<16>(in, ld, X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol, sh);
 }
-__global__ __launch_bounds__(SMALL_NT) void jac_small(c128* __restrict__ X, int rows, int cols,
+__global__ __launch_bounds__(SMALL_NT) void jac_small(const c128* in, int ld, c128* X, int rows, int cols,
                                                       double* __restrict__ sigma, int* __restrict__ perm,
                                                       SvdResult* __restrict__ res, int chi_max, double eps,
                                                       int rank_cap, double tol) {
-  jac_small_rows(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol);
+  jac_small_rows(in, ld, X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, tol);
 }
 
 // ---------------------------------------------------------- QR preconditioning
@@ -1436,14 +1441,14 @@ __global__ __launch_bounds__(JAC_NT) void col_norm_order(const c128* __restrict_
   col_norm_order_body(X, rows, cols, order);
 }
 
-// Xp[:, c] = X[:, order[c]]
+// Xp[:, c] = X[:, order[c]], or a copy (order null)
 __device__ __forceinline__ void permute_cols_body(const c128* __restrict__ X, int rows, int cols,
                                                   const int* __restrict__ order, c128* __restrict__ Xp,
                                                   unsigned blk, unsigned nblk) {
   for (long e = blk * (long)blockDim.x + threadIdx.x; e < (long)rows * cols;
        e += (long)nblk * blockDim.x) {
     const int c = (int)(e / rows), r = (int)(e - (long)c * rows);
-    Xp[e] = X[(long)order[c] * rows + r];
+    Xp[e] = X[(long)(order ? order[c] : c) * rows + r];
   }
 }
 __global__ void permute_cols(const c128* __restrict__ X, int rows, int cols,
@@ -1490,6 +1495,8 @@ __global__ __launch_bounds__(JAC_NT) void scale_by_norms(const c128* __restrict_
 
 // ------------------------------------------------------------------ grouped kernels
 struct JacSmallArgs {
+  const c128* in;
+  int ld;
   c128* X;
   int rows, cols;
   double* sigma;
@@ -1544,7 +1551,7 @@ struct FinArgs {
 
 __global__ __launch_bounds__(SMALL_NT) void jac_small_grouped(const GRec<JacSmallArgs>* __restrict__ recs, int n) {
   const JacSmallArgs a = recs[blockIdx.x].a;
-  jac_small_rows(gbl(a.X), a.rows, a.cols, gbl(a.sigma), gbl(a.perm), gbl(a.res), a.chi_max, a.eps, a.rank_cap,
+  jac_small_rows(gbl(a.in), a.ld, gbl(a.X), a.rows, a.cols, gbl(a.sigma), gbl(a.perm), gbl(a.res), a.chi_max, a.eps, a.rank_cap,
                  a.tol);
 }
 __global__ __launch_bounds__(JAC_NT) void col_norm_order_grouped(const GRec<ColOrderArgs>* __restrict__ recs,
@@ -1555,7 +1562,7 @@ __global__ __launch_bounds__(JAC_NT) void col_norm_order_grouped(const GRec<ColO
 __global__ void permute_cols_grouped(const GRec<ColOrderArgs>* __restrict__ recs, int n) {
   unsigned bx, by, bz;
   const GRec<ColOrderArgs>& r = grec_find(recs, n, blockIdx.x, bx, by, bz);
-  permute_cols_body(gbl(r.a.X), r.a.rows, r.a.cols, gbl(r.a.order), gbl(r.a.Xp), bx, r.grid.x);
+  permute_cols_body(gbl(r.a.X), r.a.rows, r.a.cols, r.a.order ? gbl(r.a.order) : nullptr, gbl(r.a.Xp), bx, r.grid.x);
 }
 __global__ void rh_from_qr_grouped(const GRec<RhArgs>* __restrict__ recs, int n) {
   unsigned bx, by, bz;
@@ -1644,6 +1651,11 @@ size_t jacobi_workspace_bytes(int max_rows, int max_cols) {
 bool small_svd(int rows, int cols) {
   return std::min(rows, cols) <= JAC_LMAX && std::max(rows, cols) <= SMALL_ROWS;
 }
+// Longer than the one workgroup's registers hold, but no wider: the workgroup takes
+// the triangle of a QR.  130 x 2 151 us for the whole split (sweeps in one workgroup
+// 143, the launches 307), 130 x 16 214 (286, 350), 512 x 32 346 (897, 454): at every
+// size ahead of the launches.
+bool tall_svd(int rows, int cols) { return rows > SMALL_ROWS && cols <= JAC_LMAX; }
 
 namespace {
 
@@ -1754,6 +1766,17 @@ size_t jacobi_precond_elems(int max_rows, int max_cols) {
          + qr_workspace_elems(max_rows, max_cols, (int)kq);
 }
 
+namespace {
+// X = Q R, R = U' S V^H in one workgroup, X <- Q (U' S): the copy that becomes V and
+// R, U' S, and T, in the preconditioning workspace.
+struct TallSvd {
+  c128 *Xp, *Z, *T;
+  size_t t_elems;
+  TallSvd(c128* pre, size_t elems, int rows, int cols)
+      : Xp(pre), Z(Xp + (long)rows * cols), T(Z + (long)cols * cols), t_elems(elems - (size_t)(T - pre)) {}
+};
+}  // namespace
+
 void launch_jacobi_svd(c128* X, int rows, int cols, double* sigma, int* perm, SvdResult* res,
                        int chi_max, double eps, int rank_cap, hipStream_t s, JacobiWork& w) {
   QCA_CHECK(rows >= 1 && rows <= 512, "SVD rows out of range (1..512)");
@@ -1762,12 +1785,22 @@ void launch_jacobi_svd(c128* X, int rows, int cols, double* sigma, int* perm, Sv
   const int kq = std::min(rows, cols);
   if (small_svd(rows, cols)) {
     const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)kq);
-    hipLaunchKernelGGL(jac_small, dim3(1), dim3(SMALL_NT), 0, s, X, rows, cols, sigma, perm, res, chi_max,
-                       eps, rank_cap, tol);
+    hipLaunchKernelGGL(jac_small, dim3(1), dim3(SMALL_NT), 0, s, (const c128*)X, rows, X, rows, cols, sigma, perm,
+                       res, chi_max, eps, rank_cap, tol);
     QCA_HIP(hipGetLastError());
     return;
   }
   QCA_CHECK(w.pre != nullptr && w.pre_elems >= jacobi_precond_elems(rows, cols), "Jacobi workspace too small");
+  if (tall_svd(rows, cols)) {
+    const TallSvd t(w.pre, w.pre_elems, rows, cols);
+    hipLaunchKernelGGL(permute_cols, dim3(256), dim3(256), 0, s, (const c128*)X, rows, cols, (const int*)nullptr, t.Xp);
+    launch_blocked_qr(t.Xp, rows, cols, nullptr, 0, t.T, t.t_elems, s);
+    const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)kq);
+    hipLaunchKernelGGL(jac_small, dim3(1), dim3(SMALL_NT), 0, s, (const c128*)t.Xp, rows, t.Z, cols, cols, sigma, perm,
+                       res, chi_max, eps, rank_cap, tol);
+    launch_form_q(form_q_step(t.Xp, rows, cols, t.T, X, cols, t.Z), s);
+    return;
+  }
   // Preconditioned: X P = Q R with the columns by descending norm, one-sided
   // Jacobi on Y = R^H with the same rotations applied to Q.  Y J = U' S and
   // Q J = U, the left singular vectors of X, orthonormal by construction.
@@ -1792,7 +1825,10 @@ void launch_jacobi_svd(c128* X, int rows, int cols, double* sigma, int* perm, Sv
 
 void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, GroupFlags& flags,
                         hipStream_t s) {
-  std::vector<GRec<JacSmallArgs>> small;
+  std::vector<GRec<JacSmallArgs>> small, triangle;
+  std::vector<GRec<QrFormArgs>> back;
+  int back_rows = 0;
+  size_t back_lds = 0;
   std::vector<GRec<ColOrderArgs>> order1, perm;
   std::vector<GRec<RhArgs>> rh;
   std::vector<GRec<ScaleArgs>> scale;
@@ -1809,11 +1845,24 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     const int kq = std::min(j.rows, j.cols);
     if (small_svd(j.rows, j.cols)) {
       const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)kq);
-      small.push_back(grec(JacSmallArgs{j.X, j.rows, j.cols, j.sigma, j.perm, j.res, j.chi_max, j.eps,
+      small.push_back(grec(JacSmallArgs{j.X, j.rows, j.X, j.rows, j.cols, j.sigma, j.perm, j.res, j.chi_max, j.eps,
                                         j.rank_cap, tol}, 1));
       continue;
     }
     QCA_CHECK(w.pre != nullptr && w.pre_elems >= jacobi_precond_elems(j.rows, j.cols), "Jacobi workspace too small");
+    if (tall_svd(j.rows, j.cols)) {
+      const TallSvd t(w.pre, w.pre_elems, j.rows, j.cols);
+      const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)kq);
+      perm.push_back(grec(ColOrderArgs{j.X, j.rows, j.cols, nullptr, t.Xp}, 256));
+      for (QrStep& st : blocked_qr_steps(t.Xp, j.rows, j.cols, nullptr, 0, t.T, t.t_elems)) steps.push_back(st);
+      triangle.push_back(grec(JacSmallArgs{t.Xp, j.rows, t.Z, j.cols, j.cols, j.sigma, j.perm, j.res, j.chi_max, j.eps,
+                                           j.rank_cap, tol}, 1));
+      const QrStep f = form_q_step(t.Xp, j.rows, j.cols, t.T, j.X, j.cols, t.Z);
+      back.push_back(grec(f.form, f.blocks));
+      back_rows = std::max(back_rows, j.rows);
+      back_lds = std::max(back_lds, f.lds);
+      continue;
+    }
     c128* Xp = w.pre;
     c128* Z = Xp + (long)j.rows * j.cols;
     c128* Y = Z + (long)j.rows * kq;
@@ -1854,7 +1903,8 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     pred = std::max(pred, w.pred_sweeps);
     steps_pred = std::max(steps_pred, w.pred_newton);
   }
-  KGroup<JacSmallArgs> g_small;
+  KGroup<JacSmallArgs> g_small, g_triangle;
+  KGroup<QrFormArgs> g_back;
   KGroup<ColOrderArgs> g_order, g_perm;
   KGroup<RhArgs> g_rh;
   KGroup<ScaleArgs> g_scale;
@@ -1862,6 +1912,8 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
   KGroup<NewtonArgs> n_one, n_nn, n_app, n_cp;
   KGroup<FinArgs> g_fin;
   g_small.prepare(small, arena);
+  g_triangle.prepare(triangle, arena);
+  g_back.prepare(back, arena);
   g_order.prepare(order1, arena);
   g_perm.prepare(perm, arena);
   g_rh.prepare(rh, arena);
@@ -1908,14 +1960,19 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
 
   if (!g_small.empty())
     hipLaunchKernelGGL(jac_small_grouped, dim3(g_small.l.blocks), dim3(SMALL_NT), 0, s, g_small.l.recs, g_small.l.n);
-  if (!g_order.empty()) {
+  if (!g_order.empty())
     hipLaunchKernelGGL(col_norm_order_grouped, dim3(g_order.l.blocks), dim3(JAC_NT), 0, s, g_order.l.recs,
                        g_order.l.n);
+  if (!g_perm.empty())
     hipLaunchKernelGGL(permute_cols_grouped, dim3(g_perm.l.blocks), dim3(256), 0, s, g_perm.l.recs, g_perm.l.n);
-  }
   for (const Slot& sl : slots) {
     launch_qr_step_grouped(sl.step, sl.rows, sl.lds, s);
     launch_form_q_grouped(sl.form, sl.rows, sl.lds, s);
+  }
+  if (!g_triangle.empty()) {
+    hipLaunchKernelGGL(jac_small_grouped, dim3(g_triangle.l.blocks), dim3(SMALL_NT), 0, s, g_triangle.l.recs,
+                       g_triangle.l.n);
+    launch_form_q_grouped(g_back, back_rows, back_lds, s);
   }
   if (!g_rh.empty())
     hipLaunchKernelGGL(rh_from_qr_grouped, dim3(g_rh.l.blocks), dim3(256), 0, s, g_rh.l.recs, g_rh.l.n);

@@ -5,6 +5,8 @@ to the reference's algorithm."""
 import numpy as np
 import pytest
 
+from conftest import crand
+
 import qca_native as qn
 from oracle import automaton as AU, mps as OM, tdvp as OT
 
@@ -140,4 +142,47 @@ def test_non_finite_krylov_is_reported(gpu, prec, monkeypatch):
     assert e.value.code == -4
     g.close()
     for e in engines:
+        e.close()
+
+
+UNEVEN = [[1, 2, 4, 8, 16, 32, 64, 128, 70, 12, 4, 2, 1], [1, 2, 4, 8, 16, 32, 64, 160, 160, 100, 24, 4, 1],
+          [1, 2, 4, 8, 16, 8, 4, 2, 1]]
+
+
+def uneven_chains(prec):
+    """Chains whose bonds differ by more than a site can, kept by eps = 0."""
+    out = []
+    for k, dims in enumerate(UNEVEN):
+        n = len(dims) - 1
+        rng = np.random.default_rng(k)
+        weight = lambda d: np.logspace(0, -3, d)
+        A = [crand(rng, 2, a, b) * weight(a)[:, None] * weight(b) for a, b in zip(dims, dims[1:])]
+        out.append(qn.Engine(AU.mpo_tensors(n, 1, range(1, 2)), A, algorithm=2, precision=prec, chi_max=160, dt=0.1,
+                             eps=0.0, krylov_tol=1e-14 if prec == 0 else 1e-10))
+    return out
+
+
+@pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "mixed"])
+def test_group_of_uneven_chains_is_bit_identical(gpu, prec):
+    """Splits of more than 128 rows and at most 32 columns, and QRs below and above 256
+    rows in one launch."""
+    shapes = set()
+    for dims in UNEVEN:
+        chi = list(dims)
+        for s in range(len(chi) - 2):            # the right sweep's splits
+            shapes.add((2 * chi[s], 2 * chi[s + 2]))
+            chi[s + 1] = min(160, 2 * chi[s], 2 * chi[s + 2])
+    assert any(r > 128 and c <= 32 for r, c in shapes) and any(r > 256 and c > 32 for r, c in shapes)
+    grouped, alone = uneven_chains(prec), uneven_chains(prec)
+    g = qn.Group(grouped)
+    g.step(1)
+    for e in alone:
+        e.step(1)
+    for b, a in zip(grouped, alone):
+        assert np.array_equal(b.bond_dims(), a.bond_dims())
+        assert np.array_equal(b.rho(), a.rho())
+        for x, y in zip(b.tensors(), a.tensors()):
+            assert np.array_equal(x, y)
+    g.close()
+    for e in grouped + alone:
         e.close()

@@ -685,3 +685,13 @@ def test_qr_few_reflectors(gpu, side, chi_row, chi_col, target):
     """On both sides of the choice between the one-workgroup and the blocked QR: one,
     two and three reflectors, few and many columns beside them."""
     test_qr_panels_match_lapack(gpu, side, chi_row, chi_col, target)
+
+
+@pytest.mark.parametrize("spectrum", ["flat", "graded", "rank1"])
+@pytest.mark.parametrize("chil,chir", [(65, 1), (65, 8), (72, 9), (128, 16), (129, 4), (256, 16)])
+def test_svd_split_tall(gpu, spectrum, chil, chir):
+    """Splits with more than 128 rows and up to 32 columns (one and two QR panels,
+    up to 256 and up to 512 rows), against LAPACK within the bounds of
+    test_svd_split."""
+    test_svd_split_closing_steps(gpu, spectrum, chil, chir, 1)
+    test_svd_split_closing_steps(gpu, spectrum, chir, chil, 0)
