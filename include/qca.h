@@ -266,9 +266,10 @@ int qca_exact_apply_h(int precision, const void* psi, void* out, int ncells, int
  * Chebyshev series with the closed-form H (|H| <= ncells), cut where its tail
  * falls well below tol * |psi|.  Replaces reference exact.py:15-28.  A step with
  * (pi/2) |dt| ncells > 512 is cut into equal substeps, tol holding for all of
- * them together.  Uses three vectors of
- * workspace.  *iters receives the number of H applications.  Amplitudes that
- * are not finite are an error (-4), and psi is left as it was. */
+ * them together.  Uses three vectors of workspace.  A state on at most 64 basis
+ * states that H maps among themselves is evolved on these alone.  *iters receives
+ * the number of H applications (there, of the H of those states).  Amplitudes
+ * that are not finite are an error (-4), and psi is left as it was. */
 int qca_exact_expm(void* psi, int ncells, int distance, int lo, int hi, double dt, double tol,
                    int* iters, void* stream);
 

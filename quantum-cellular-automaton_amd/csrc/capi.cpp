@@ -79,9 +79,17 @@ struct Scratch {
     for (auto& kv : mpos) kv.second.release();
     mpos.clear();
   }
+  // A word of host memory that kernels write to.
+  int* word = nullptr;
+  int* host_word() {
+    if (!word) QCA_HIP(hipHostMalloc((void**)&word, 64, hipHostMallocCoherent | hipHostMallocMapped));
+    return word;
+  }
   void release() {
     for (auto& kv : bufs) (void)hipFree(kv.second.first);
     bufs.clear();
+    if (word) (void)hipHostFree(word);
+    word = nullptr;
     for (auto& kv : mpos) kv.second.release();
     mpos.clear();
   }
@@ -722,14 +730,9 @@ int qca_exact_expm(void* psi, int ncells, int distance, int lo, int hi, double d
     qca::c128* bufa = sbuf<qca::c128>("ex_a", n);
     qca::c128* bufb = sbuf<qca::c128>("ex_b", n);
     qca::c128* acc = sbuf<qca::c128>("ex_acc", n);
-    int* bad = sbuf<int>("ex_bad", 1);
     const int m = qca::launch_exact_expm((qca::c128*)psi, ncells, distance, lo, hi, 1.5707963267948966 * dt,
-                                         tol > 0 ? tol : 1e-14, bufa, bufb, acc, bad, s);
-    int hbad = 0;
-    QCA_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
-    QCA_HIP(hipStreamSynchronize(s));
-    if (hbad)
-      throw qca::Error(qca::QCA_ERR_NOT_CONVERGED_CODE, "exponential of a state vector with non-finite amplitudes");
+                                         tol > 0 ? tol : 1e-14, bufa, bufb, acc, sbuf<qca::ExactProbe>("ex_probe", 1),
+                                         prim_scratch().host_word(), s);
     if (iters) *iters = m;
   });
 }

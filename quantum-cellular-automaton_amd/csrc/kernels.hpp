@@ -167,10 +167,23 @@ void launch_exact_apply(const cplx<T>* psi, cplx<T>* out, int ncells, int distan
 // (cut at tol itself, the tail was most of the error: 12 to 15 cells, 2.0e-15
 // relative to |psi| on average, against 2.4e-16; one or two terms more);
 // returns the number of H applications.  bufa, bufb, acc: 2^ncells elements
-// each; *bad is set, and psi left as it was, when psi is not finite.
+// each; word: a word of pinned host memory.  psi not finite: an error, psi is left as
+// it was.  Returns with the stream drained.
 constexpr double CHEB_MAX_Z = 512, CHEB_TAIL = 0.03;
+// Basis states up to which the support of psi is told to the host, and up to which a
+// set of them that H maps to itself is evolved there.
+constexpr int EXACT_SUPPORT = 64;
+struct ExactAmplitude {
+  unsigned long long x;
+  double re, im;
+};
+struct ExactProbe {      // device; the first two words are cleared for each call
+  int bad;               // psi is not finite
+  int count;             // nonzero amplitudes (some of them, where there are more than EXACT_SUPPORT)
+  ExactAmplitude e[EXACT_SUPPORT];
+};
 int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, double tau, double tol, c128* bufa,
-                      c128* bufb, c128* acc, int* bad, hipStream_t s);
+                      c128* bufb, c128* acc, ExactProbe* probe, int* word, hipStream_t s);
 
 // ---------------------------------------------------------------- SVD / QR
 struct SvdResult {

@@ -695,3 +695,35 @@ def test_svd_split_tall(gpu, spectrum, chil, chir):
     test_svd_split."""
     test_svd_split_closing_steps(gpu, spectrum, chil, chir, 1)
     test_svd_split_closing_steps(gpu, spectrum, chir, chil, 0)
+
+
+@pytest.mark.parametrize("dt", [0.3, -1.0, 5.0])
+@pytest.mark.parametrize("n,d,lo,hi,states,few", [
+    (10, 1, 2, 3, [0], True),                                   # dead: H psi = 0
+    (10, 1, 2, 3, [0b0001110000], True),                        # a blinker
+    (10, 2, 2, 5, [0, 1, 0b1000000001], True),                  # still lives in superposition
+    (10, 1, 2, 3, [0b0111000111, 0b1110000000], True),          # blinkers side by side
+    (10, 1, 1, 3, [0b0000100000], False),                       # spreads over more than 64 states
+    (6, 2, 1, 4, list(range(64)), True),                        # every state, and just that many
+    (7, 2, 1, 4, list(range(64)), False), (7, 2, 1, 4, list(range(65)), False),
+    (10, 1, 0, 1, list(range(70)), False)])
+def test_exact_expm_few_states(gpu, n, d, lo, hi, states, few, dt):
+    """States on few basis states, closed under the Hamiltonian or not, against the
+    dense propagator (rounding of the phases: eps * tau * N); a closed set takes no
+    more applications than a series for its own few states."""
+    import torch
+    H = exact_h(n, d, lo, hi)
+    lam, U = np.linalg.eigh(np.stack([H(e) for e in np.eye(1 << n)]))
+    psi = np.zeros(1 << n, dtype=complex)
+    psi[states] = crand(np.random.default_rng(len(states)), len(states))
+    psi /= np.linalg.norm(psi)
+    ref = U @ (np.exp(-1j * np.pi / 2 * dt * lam) * (U.T @ psi))
+    pd = dev(torch, psi, np.complex128)
+    it = ctypes.c_int(0)
+    qn.call("qca_exact_expm", qn.ptr(pd), n, d, lo, hi, dt, 0.0, ctypes.byref(it), None)
+    assert np.abs(pd.cpu().numpy() - ref).max() < 1e-12
+    if few:
+        degree = max(int((H(np.eye(1 << n)[x]) != 0).sum()) for x in range(1 << n)) if n < 8 else 4
+        assert it.value <= np.pi / 2 * abs(dt) * degree * 2 + 30
+    if states == [0]:
+        assert it.value == 1
