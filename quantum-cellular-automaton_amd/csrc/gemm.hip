@@ -470,6 +470,8 @@ __device__ __forceinline__ void splitk_reduce_body(const GemmDesc& d, const cplx
   for (long idx = blk * (long)blockDim.x + threadIdx.x; idx < total;
        idx += (long)nblk * blockDim.x) {
     const int zb = (int)(idx / mn);
+    // nobody reads this batch, and 32x32 tiles have left its partials unwritten
+    if (d.batch_used && !(d.batch_used >> zb & 1)) continue;
     const long r = idx - zb * mn;
     const int m = (int)(r / d.N), n = (int)(r - (long)m * d.N);
     T xr = 0, xi = 0;
@@ -573,7 +575,8 @@ GemmPlan gemm_plan(const GemmDesc& d, long ws_elems, bool fp64) {
   // K-tiles of the longest batch: segments of K2, each cut into BK tiles
   const long ktiles = (long)(d.K / d.K2) * ceil_div(d.K2, BK);
   QCA_CHECK(ktiles < (1L << 30), "GEMM K too long");
-  const long out_elems = (long)p.batch * d.M * d.N, out_bytes = out_elems * (fp64 ? 16 : 8);
+  const long out_elems = (long)p.batch * d.M * d.N;
+  const long out_bytes = (long)used * d.M * d.N * (fp64 ? 16 : 8);   // what a reduce reads per split
   // tile side and splits of K: the best of every tile under a few fills
   int splits = 1;
   double best = 0;
