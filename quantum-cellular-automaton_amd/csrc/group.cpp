@@ -218,7 +218,10 @@ void Group::position(std::vector<Bond>& bonds) {
     e->stats_.svd_sweeps += r.nsweeps;
     const int rows = b.right ? 2 * b.chil : 2 * b.chir;
     const int cols = b.right ? 2 * b.chir : 2 * b.chil;
-    if (!small_svd(rows, cols) && !tall_svd(rows, cols)) e->jw_.pred_sweeps = r.nsweeps;
+    if (!small_svd(rows, cols) && !tall_svd(rows, cols)) {
+      e->jw_.pred_sweeps = r.nsweeps;
+      e->jw_.pred_newton = r.nsteps;
+    }
     if (!r.converged) fail(b.inst, "Jacobi SVD of the two-site split did not converge");
     QCA_CHECK(r.k >= 1, "SVD truncation produced an empty bond");
     QCA_CHECK(r.k <= e->cap_[b.s + 1], "truncation rank above bond capacity");

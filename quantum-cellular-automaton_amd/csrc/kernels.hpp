@@ -190,7 +190,7 @@ struct SvdResult {
   int k;              // truncation rank
   int nsweeps;        // Jacobi sweeps used
   int converged;
-  int pad;
+  int nsteps;         // closing steps used
   double norm_kept;   // ||s[:k]||
   double tail;        // ||s[k:]||
 };

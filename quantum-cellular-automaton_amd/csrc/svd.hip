@@ -869,7 +869,7 @@ __device__ __forceinline__ int key_rank(const double* keys, int n, int c) {
 __device__ void finalize_body(const c128* __restrict__ X, int rows, int cols,
                               double* __restrict__ sigma, int* __restrict__ perm,
                               SvdResult* __restrict__ res, int chi_max, double eps, int rank_cap,
-                              int sweeps, int converged) {
+                              const JacobiCtrl* __restrict__ ctrl) {
   __shared__ double skey[JAC_MAXCOLS], sorted[JAC_MAXCOLS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = JAC_NT / 64;
   for (int c = wave; c < cols; c += nw) {
@@ -925,8 +925,9 @@ __device__ void finalize_body(const c128* __restrict__ X, int rows, int cols,
   tail = wsum(tail);
   if (tid == 0) {
     res->k = k;
-    res->nsweeps = sweeps;
-    res->converged = converged;
+    res->nsweeps = ctrl->sweeps;
+    res->converged = ctrl->done;
+    res->nsteps = ctrl->newton;
     res->norm_kept = sqrt(kept);
     res->tail = sqrt(tail);
   }
@@ -938,7 +939,7 @@ __global__ __launch_bounds__(JAC_NT) void jac_finalize(const c128* __restrict__ 
                                                        SvdResult* __restrict__ res, int chi_max,
                                                        double eps, int rank_cap,
                                                        const JacobiCtrl* __restrict__ ctrl) {
-  finalize_body(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, ctrl->sweeps, ctrl->done);
+  finalize_body(X, rows, cols, sigma, perm, res, chi_max, eps, rank_cap, ctrl);
 }
 
 // ------------------------------------------------------------------ small matrices
@@ -1395,6 +1396,7 @@ __device__ __forceinline__ void jac_small_body(const c128* __restrict__ in, int 
     res->k = k;
     res->nsweeps = sweeps;
     res->converged = converged;
+    res->nsteps = 0;
     res->norm_kept = sqrt(kept);
     res->tail = sqrt(tail);
   }
@@ -1613,9 +1615,8 @@ __global__ void jac_state_gather(const GRec<JacArgs>* __restrict__ recs, int n, 
 }
 __global__ __launch_bounds__(JAC_NT) void jac_finalize_grouped(const GRec<FinArgs>* __restrict__ recs, int n) {
   const FinArgs a = recs[blockIdx.x].a;
-  const JacobiCtrl* ctrl = gbl(a.ctrl);
   finalize_body(gbl(a.X), a.rows, a.cols, gbl(a.sigma), gbl(a.perm), gbl(a.res), a.chi_max, a.eps, a.rank_cap,
-                ctrl->sweeps, ctrl->done);
+                gbl(a.ctrl));
 }
 
 }  // namespace
