@@ -178,8 +178,7 @@ void Engine::init(const std::vector<const c128*>& W_host, const std::vector<int>
   qrQ_ = dmalloc<c128>(4 * cmax * cmax);
   qrTau_ = dmalloc<c128>(2 * cmax);
   cbond_ = dmalloc<c128>(cmax * cmax * 2);
-  qr_ws_elems_ = qr_workspace_elems((int)std::min<long>(2 * cmax, 512), (int)cmax,
-                                    (int)std::min<long>(2 * cmax, 512));
+  qr_ws_elems_ = qr_workspace_elems((int)std::min<long>(2 * cmax, 512), (int)cmax);
   qrWs_ = dmalloc<c128>((long)qr_ws_elems_);
   T_ = dmalloc<c128>(tmax);
   U_ = dmalloc<c128>(tmax);

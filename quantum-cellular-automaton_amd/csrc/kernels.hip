@@ -2,7 +2,8 @@
 //
 //  * wmix      -- sparse MPO mixing between the two GEMMs of every contraction
 //  * permute   -- Theta <-> SVD matrix layouts, gathers of singular vectors
-//  * lanczos   -- FP64 Krylov exp(-i tau H) v with CGS2 reorthogonalisation;
+//  * lanczos   -- FP64 Krylov exp(-i tau H) v: the three-term step and one classical
+//                 Gram-Schmidt pass against the whole basis;
 //                 the tridiagonal exponential runs on one wave (Taylor with
 //                 scaling) so no host round trip is needed per iteration
 //  * measure   -- <n_i> and the single-site density matrix from the transfer

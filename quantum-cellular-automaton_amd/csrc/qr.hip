@@ -645,7 +645,7 @@ __global__ __launch_bounds__(HH_THREADS) void householder_qr_kernel(c128* __rest
 
 }  // namespace
 
-size_t qr_workspace_elems(int max_rows, int max_cols, int) {
+size_t qr_workspace_elems(int max_rows, int max_cols) {
   return (size_t)ceil_div(std::max(1, std::min(max_rows, max_cols)), QR_PB) * QR_PB * QR_PB;   // T per panel
 }
 
@@ -665,7 +665,7 @@ QrStep form_q_step(const c128* M, int rows, int kk, const c128* T, c128* Q, int 
 std::vector<QrStep> blocked_qr_steps(c128* M, int rows, int cols, c128* Q, int qcols, c128* ws, size_t ws_elems) {
   QCA_CHECK(rows >= 1 && cols >= 1, "empty QR");
   QCA_CHECK(rows <= QR_MAX_ROWS, "blocked QR rows above 512");
-  QCA_CHECK(ws_elems >= qr_workspace_elems(rows, cols, qcols), "QR workspace too small");
+  QCA_CHECK(ws_elems >= qr_workspace_elems(rows, cols), "QR workspace too small");
   QCA_CHECK(qcols <= rows, "more columns of Q than rows");
   const int kmax = std::min(rows, cols), panels = ceil_div(kmax, QR_PB);
   std::vector<QrStep> out;
@@ -725,7 +725,7 @@ void launch_qr(c128* M, int rows, int cols, c128* tau, c128* Q, int qcols, c128*
   // with more, or beside many columns, the blocked one is ahead (2 x 256 54 against 36,
   // 8 x 4 33.5 against 31.3, 64 x 32 147 against 63)
   const bool few = std::min(rows, cols) <= 2 && cols <= 64;
-  if (!few && ws != nullptr && rows <= QR_MAX_ROWS && ws_elems >= qr_workspace_elems(rows, cols, qcols))
+  if (!few && ws != nullptr && rows <= QR_MAX_ROWS && ws_elems >= qr_workspace_elems(rows, cols))
     launch_blocked_qr(M, rows, cols, Q, qcols, ws, ws_elems, s);
   else
     launch_householder_qr(M, rows, cols, tau, Q, qcols, s);

@@ -2,7 +2,7 @@
 //
 // jacobi_svd: block one-sided (Hestenes) Jacobi on the columns of a
 // column-major matrix X, with the rotations of each block pair computed on its
-// Gram matrix.  The columns are cut into blocks of bs <= 16; the blocks meet in
+// Gram matrix.  The columns are cut into blocks of 16; the blocks meet in
 // the round-robin tournament, one outer round per kernel triple:
 //   jac_gram   G_p = X_p^H X_p for every block pair p (2bs columns), each
 //              workgroup one chunk of 64 rows on the FP64 matrix cores,
@@ -112,12 +112,17 @@ struct JacobiCtrl {
 };
 
 struct JacobiGeom {
-  int rows, cols, bs, nb, kspl;
+  int rows, cols, nb, kspl;
 };
 
-// Stages rows [r0, r0+nr) of the 2bs columns of pair p into a row-major LDS
+// Column of the matrix that is column c of block pair (bi, bj).
+__device__ __forceinline__ int pair_column(int bi, int bj, int c) {
+  return c < JAC_BS ? bi * JAC_BS + c : bj * JAC_BS + (c - JAC_BS);
+}
+
+// Stages rows [r0, r0+nr) of the 32 columns of pair p into a row-major LDS
 // tile with a padded row stride (JAC_LMAX + 1) that spreads the banks; rows
-// beyond nr and columns beyond 2bs (up to JAC_LMAX) are zero.  Lane bits give
+// beyond nr and columns beyond the matrix are zero.  Lane bits give
 // the row, the wave index walks the columns: no divisions, and each wave reads
 // one contiguous 64-row run of a column.  NT is the workgroup size: all of a
 // thread's loads are issued before its first LDS store, so the tile costs one
@@ -128,15 +133,13 @@ __device__ __forceinline__ void stage_tile(const c128* __restrict__ X, const Jac
   static_assert(JAC_RC == 64, "one row per lane");
   static_assert(NT % 64 == 0 && JAC_LMAX % (NT / 64) == 0, "whole columns per wave");
   constexpr int NW = NT / 64, IT = JAC_LMAX / NW;
-  const int L = 2 * g.bs;
   const int bi = rr_player(p, round, g.nb), bj = rr_player(g.nb - 1 - p, round, g.nb);
   const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
   c128 v[IT];
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
-    const int c = w + i * NW;
-    const int gc = c < g.bs ? bi * g.bs + c : bj * g.bs + (c - g.bs);
-    v[i] = (c < L && gc < g.cols && r < nr) ? X[(long)gc * g.rows + r0 + r] : c128{0.0, 0.0};
+    const int gc = pair_column(bi, bj, w + i * NW);
+    v[i] = (gc < g.cols && r < nr) ? X[(long)gc * g.rows + r0 + r] : c128{0.0, 0.0};
   }
 #pragma unroll
   for (int i = 0; i < IT; ++i) tile[r * (JAC_LMAX + 1) + w + i * NW] = v[i];
@@ -186,21 +189,20 @@ __device__ __forceinline__ void jac_gram_body(const c128* __restrict__ X, const 
   // the control word is read alongside the tile, not before it: the round
   // kernels are latency bound, and a no-op round only stages a tile
   const int done = ctrl->done | ctrl->phase;
-  __shared__ c128 tile[JAC_RC * (JAC_LMAX + 1)];
-  const int L = 2 * g.bs;
+  constexpr int L = JAC_LMAX;
+  __shared__ c128 tile[JAC_RC * (L + 1)];
   const int r0 = kc * JAC_RC, nr = min(JAC_RC, g.rows - r0);
   stage_tile<JAC_GRAM_NT>(X, g, p, round, r0, nr, tile);
   __syncthreads();
   if (done) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int tj = (wave >> 1) * 16, ti = (wave & 1) * 16;
-  if (tj >= L || ti >= L) return;
   const int q = lane >> 4, c = lane & 15;
   jac_f64x4 gre = {0, 0, 0, 0}, gim = {0, 0, 0, 0};
   const int kmax = (nr + 3) & ~3;
   for (int k0 = 0; k0 < kmax; k0 += 4) {
-    const c128 a = tile[(k0 + q) * (JAC_LMAX + 1) + tj + c];   // X(r, c_j)
-    const c128 b = tile[(k0 + q) * (JAC_LMAX + 1) + ti + c];   // X(r, c_i), conjugated below
+    const c128 a = tile[(k0 + q) * (L + 1) + tj + c];   // X(r, c_j)
+    const c128 b = tile[(k0 + q) * (L + 1) + ti + c];   // X(r, c_i), conjugated below
     gre = jac_mfma(a.re, b.re, gre);
     gre = jac_mfma(a.im, b.im, gre);
     gim = jac_mfma(a.im, b.re, gim);
@@ -210,7 +212,7 @@ __device__ __forceinline__ void jac_gram_body(const c128* __restrict__ X, const 
 #pragma unroll
   for (int rr = 0; rr < 4; ++rr) {
     const int j = tj + q + 4 * rr, i = ti + c;
-    if (i < L && j < L) out[i + j * L] = c128{gre[rr], gim[rr]};
+    out[i + j * L] = c128{gre[rr], gim[rr]};
   }
 }
 __global__ __launch_bounds__(JAC_GRAM_NT) void jac_gram(const c128* __restrict__ X, JacobiGeom g,
@@ -479,22 +481,19 @@ __device__ __forceinline__ void jac_apply_body(c128* __restrict__ Xa, const Jaco
   const JacobiGeom g = second ? gz : ga;
   const int kc = second ? by - ga.kspl : by;
   __shared__ c128 tile[JAC_RC * (JAC_LMAX + 1)];
-  __shared__ c128 J[JAC_LMAX * (JAC_LMAX + 1)];   // J(k, c) at c * (JAC_LMAX + 1) + k, zero-padded
-  const int L = 2 * g.bs;
+  constexpr int L = JAC_LMAX;
+  __shared__ c128 J[L * (L + 1)];   // J(k, c) at c * (L + 1) + k
   const int r0 = kc * JAC_RC, nr = min(JAC_RC, g.rows - r0);
   stage_tile<JAC_APPLY_NT>(X, g, p, round, r0, nr, tile);
   const c128* jp = Jin + (long)p * L * L;
-  constexpr int JIT = JAC_LMAX * JAC_LMAX / JAC_APPLY_NT;
+  constexpr int JIT = L * L / JAC_APPLY_NT;
   c128 jv[JIT];
 #pragma unroll
-  for (int i = 0; i < JIT; ++i) {
-    const int e = threadIdx.x + i * JAC_APPLY_NT, k = e % JAC_LMAX, c = e / JAC_LMAX;
-    jv[i] = (k < L && c < L) ? jp[c * L + k] : c128{0.0, 0.0};
-  }
+  for (int i = 0; i < JIT; ++i) jv[i] = jp[threadIdx.x + i * JAC_APPLY_NT];
 #pragma unroll
   for (int i = 0; i < JIT; ++i) {
-    const int e = threadIdx.x + i * JAC_APPLY_NT, k = e % JAC_LMAX, c = e / JAC_LMAX;
-    J[c * (JAC_LMAX + 1) + k] = jv[i];
+    const int e = threadIdx.x + i * JAC_APPLY_NT, k = e % L, c = e / L;
+    J[c * (L + 1) + k] = jv[i];
   }
   __syncthreads();
   if (skip) return;
@@ -504,13 +503,12 @@ __device__ __forceinline__ void jac_apply_body(c128* __restrict__ Xa, const Jaco
   const int bi = rr_player(p, round, g.nb), bj = rr_player(g.nb - 1 - p, round, g.nb);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int tc = (wave & 1) * 16, tr = (wave >> 1) * 16;
-  if (tc >= L || tr >= nr) return;
+  if (tr >= nr) return;
   const int q = lane >> 4, cl = lane & 15;
   jac_f64x4 dre = {0, 0, 0, 0}, dim = {0, 0, 0, 0};
-  const int kmax = (L + 3) & ~3;
-  for (int k0 = 0; k0 < kmax; k0 += 4) {
-    const c128 a = J[(tc + cl) * (JAC_LMAX + 1) + k0 + q];      // J(k, c)
-    const c128 b = tile[(tr + cl) * (JAC_LMAX + 1) + k0 + q];   // X(r, k)
+  for (int k0 = 0; k0 < L; k0 += 4) {
+    const c128 a = J[(tc + cl) * (L + 1) + k0 + q];      // J(k, c)
+    const c128 b = tile[(tr + cl) * (L + 1) + k0 + q];   // X(r, k)
     dre = jac_mfma(a.re, b.re, dre);
     dre = jac_mfma(-a.im, b.im, dre);
     dim = jac_mfma(a.re, b.im, dim);
@@ -520,9 +518,8 @@ __device__ __forceinline__ void jac_apply_body(c128* __restrict__ Xa, const Jaco
   if (r < nr)
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
-      const int c = tc + q + 4 * rr;
-      const int gc = c < g.bs ? bi * g.bs + c : bj * g.bs + (c - g.bs);
-      if (c < L && gc < g.cols) X[(long)gc * g.rows + r0 + r] = c128{dre[rr], dim[rr]};
+      const int gc = pair_column(bi, bj, tc + q + 4 * rr);
+      if (gc < g.cols) X[(long)gc * g.rows + r0 + r] = c128{dre[rr], dim[rr]};
     }
 }
 __global__ __launch_bounds__(JAC_APPLY_NT) void jac_apply(c128* __restrict__ Xa, JacobiGeom ga,
@@ -946,7 +943,7 @@ __global__ __launch_bounds__(JAC_NT) void jac_finalize(const c128* __restrict__ 
 // The whole SVD of a matrix with min(rows, cols) <= 32 and max(rows, cols) <= 128
 // in one workgroup of four waves.  One-sided Jacobi on the columns of X takes 6
 // to 19 sweeps on the graded spectra of a TDVP split; on the triangle of a
-// pivoted QR it takes one to four, so:
+// QR with the columns sorted by norm it takes one to four, so:
 //   rows >= cols:  X P1 = Q1 R1,  R1^H P2 = Q2 R2,  Y = R2^H,  X <- Q1 P2 (Y J)
 //   rows <  cols:  X^H P1 = Q1 R1,  Y = R1^H,  X <- P1 (Y J)
 // (P: columns by descending norm; Y is at most 32x32).  Y J has orthogonal
@@ -1623,12 +1620,11 @@ __global__ __launch_bounds__(JAC_NT) void jac_finalize_grouped(const GRec<FinArg
 
 JacobiLayout jacobi_layout(int rows, int cols) {
   JacobiLayout l;
-  l.bs = JAC_BS;
-  l.nb = std::max(2, ceil_div(cols, l.bs));
+  l.nb = std::max(2, ceil_div(cols, JAC_BS));
   if (l.nb & 1) ++l.nb;
   l.kspl = ceil_div(rows, JAC_RC);
   QCA_CHECK(l.kspl <= JAC_MAXKSPL, "Jacobi rows out of range (1..512)");
-  const long L = 2L * l.bs, np = l.nb / 2;
+  const long L = JAC_LMAX, np = l.nb / 2;
   l.gpart_elems = np * l.kspl * L * L;
   l.j_elems = np * L * L;
   l.bytes = JAC_CTRL_BYTES + (sizeof(int) * np + 15) / 16 * 16 + sizeof(c128) * (l.gpart_elems + l.j_elems);
@@ -1712,8 +1708,8 @@ JacobiCtrl* gram_jacobi(c128* Y, int rows, int cols, c128* Z, int zrows, hipStre
   int* rotated = reinterpret_cast<int*>(base + JAC_CTRL_BYTES);
   c128* Gpart = reinterpret_cast<c128*>(base + JAC_CTRL_BYTES + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
   c128* Jbuf = Gpart + l.gpart_elems;
-  const JacobiGeom g{rows, cols, l.bs, l.nb, l.kspl};
-  const JacobiGeom gz{zrows, cols, l.bs, l.nb, ceil_div(zrows, JAC_RC)};
+  const JacobiGeom g{rows, cols, l.nb, l.kspl};
+  const JacobiGeom gz{zrows, cols, l.nb, ceil_div(zrows, JAC_RC)};
   const int np = l.nb / 2;
   const double tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)rows);
   const NewtonArgs na = newton_args(Y, rows, Z, zrows, cols, reinterpret_cast<unsigned char*>(Jbuf + l.j_elems),
@@ -1764,7 +1760,7 @@ size_t jacobi_precond_elems(int max_rows, int max_cols) {
   return (size_t)max_rows * max_cols       // column-permuted copy, then R / reflectors
          + (size_t)max_rows * kq           // Q, then Q J
          + (size_t)max_cols * kq           // Y = R^H
-         + qr_workspace_elems(max_rows, max_cols, (int)kq);
+         + qr_workspace_elems(max_rows, max_cols);
 }
 
 namespace {
@@ -1884,9 +1880,9 @@ void grouped_jacobi_svd(const std::vector<SvdJob>& jobs, RecordArena& arena, Gro
     a.Gpart = reinterpret_cast<c128*>(base + JAC_CTRL_BYTES + ((sizeof(int) * (l.nb / 2) + 15) / 16) * 16);
     a.Jbuf = a.Gpart + l.gpart_elems;
     a.Y = Y;
-    a.g = JacobiGeom{j.cols, kq, l.bs, l.nb, l.kspl};
+    a.g = JacobiGeom{j.cols, kq, l.nb, l.kspl};
     a.Z = Z;
-    a.gz = JacobiGeom{j.rows, kq, l.bs, l.nb, ceil_div(j.rows, JAC_RC)};
+    a.gz = JacobiGeom{j.rows, kq, l.nb, ceil_div(j.rows, JAC_RC)};
     a.tol = w.tol > 0 ? w.tol : 1.1102230246251565e-16 * sqrt((double)j.cols);
     const int np = l.nb / 2;
     jac_one.push_back(grec(a, 1));

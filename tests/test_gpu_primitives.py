@@ -727,3 +727,17 @@ def test_exact_expm_few_states(gpu, n, d, lo, hi, states, few, dt):
         assert it.value <= np.pi / 2 * abs(dt) * degree * 2 + 30
     if states == [0]:
         assert it.value == 1
+
+
+@pytest.mark.parametrize("n,d,iv", [(1, 1, range(0, 1)), (7, 3, range(2, 5)), (8, 2, range(0, 3)), (9, 9, range(3, 40)),
+                                    (18, 2, range(2, 5)), (19, 4, range(3, 6)), (20, 1, range(0, 2))])
+def test_exact_apply_tiles_fp32(gpu, n, d, iv):
+    """The edges of test_exact_apply_tiles in complex64: at most n terms per
+    amplitude, n roundings."""
+    import torch
+    psi = crand(np.random.default_rng(n), 1 << n).astype(np.complex64)
+    ref = AU.apply_h(psi.astype(np.complex128), n, d, iv)
+    pd = dev(torch, psi, np.complex64)
+    out = torch.zeros_like(pd)
+    qn.call("qca_exact_apply_h", 1, qn.ptr(pd), qn.ptr(out), n, d, iv.start, iv.stop, None)
+    assert np.abs(out.cpu().numpy() - ref).max() <= n * np.finfo(np.float32).eps * max(np.abs(ref).max(), 1)
