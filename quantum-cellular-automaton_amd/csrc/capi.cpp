@@ -79,17 +79,18 @@ struct Scratch {
     for (auto& kv : mpos) kv.second.release();
     mpos.clear();
   }
-  // A word of host memory that kernels write to.
-  int* word = nullptr;
-  int* host_word() {
-    if (!word) QCA_HIP(hipHostMalloc((void**)&word, 64, hipHostMallocCoherent | hipHostMallocMapped));
-    return word;
+  // Host memory that kernels write to.
+  qca::ExactReport* report = nullptr;
+  qca::ExactReport* exact_report() {
+    if (!report)
+      QCA_HIP(hipHostMalloc((void**)&report, sizeof(qca::ExactReport), hipHostMallocCoherent | hipHostMallocMapped));
+    return report;
   }
   void release() {
     for (auto& kv : bufs) (void)hipFree(kv.second.first);
     bufs.clear();
-    if (word) (void)hipHostFree(word);
-    word = nullptr;
+    if (report) (void)hipHostFree(report);
+    report = nullptr;
     for (auto& kv : mpos) kv.second.release();
     mpos.clear();
   }
@@ -732,7 +733,7 @@ int qca_exact_expm(void* psi, int ncells, int distance, int lo, int hi, double d
     qca::c128* acc = sbuf<qca::c128>("ex_acc", n);
     const int m = qca::launch_exact_expm((qca::c128*)psi, ncells, distance, lo, hi, 1.5707963267948966 * dt,
                                          tol > 0 ? tol : 1e-14, bufa, bufb, acc, sbuf<qca::ExactProbe>("ex_probe", 1),
-                                         prim_scratch().host_word(), s);
+                                         prim_scratch().exact_report(), s);
     if (iters) *iters = m;
   });
 }

@@ -116,11 +116,19 @@ __device__ __forceinline__ void probe_state(const ExactStep<T>& st, const cplx<T
 }
 
 // The probe to the host: 1 + the nonzero amplitudes (more than EXACT_SUPPORT: just
-// that), or EXACT_BAD.  A launch of its own: by the last workgroup of the first step,
+// that), or EXACT_BAD; and the amplitudes where they are few, so that the host need not
+// copy them, which drains the stream (a set that is not closed, 2^8: 135 -> 81 us).  A launch of its own: by the last workgroup of the first step,
 // with the fence that takes in each of them, it cost 0.7 ms at 2^23.
 constexpr int EXACT_BAD = 1 << 30;
-__global__ void tell_probe(const ExactProbe* p, int* word) {
-  __hip_atomic_store(word, p->bad ? EXACT_BAD : 1 + p->count, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+__global__ __launch_bounds__(EXACT_SUPPORT) void tell_probe(const ExactProbe* p, ExactReport* report) {
+  const int n = p->count, i = threadIdx.x;
+  if (n <= EXACT_SUPPORT && i < n) {
+    report->e[i] = p->e[i];
+    __threadfence_system();
+  }
+  __syncthreads();
+  if (i == 0)
+    __hip_atomic_store(&report->word, p->bad ? EXACT_BAD : 1 + n, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // One workgroup owns a tile of 2^TB consecutive states (the whole vector when
@@ -400,10 +408,11 @@ __global__ void scatter_closed_set(ClosedSet c, c128* __restrict__ psi) {
 // itself, if that has at most EXACT_SUPPORT states; returns the H applications, or 0.
 // (Still lifes, blinkers and the like: the Chebyshev series in the whole space takes
 // as many terms for them as for any state, where H acts on a handful of numbers.)
-int evolve_closed_set(c128* psi, const std::vector<ExactAmplitude>& support, int ncells, int distance, int lo, int hi,
-                      double tau, double tol, hipStream_t s) {
+int evolve_closed_set(c128* psi, const ExactAmplitude* support, int nsupport, int ncells, int distance, int lo,
+                      int hi, double tau, double tol, hipStream_t s) {
   ClosedSet cs;
-  std::vector<std::vector<int>> to;    // neighbours
+  unsigned char to[EXACT_SUPPORT][EXACT_SUPPORT];   // neighbours: at most one for each cell
+  int nto[EXACT_SUPPORT];
   int slot[256];                       // open addressing over the states
   std::fill(slot, slot + 256, -1);
   auto find = [&](unsigned long long x) {
@@ -413,15 +422,15 @@ int evolve_closed_set(c128* psi, const std::vector<ExactAmplitude>& support, int
       if (cs.n == EXACT_SUPPORT) return -1;
       cs.x[cs.n] = x;
       cs.re[cs.n] = cs.im[cs.n] = 0;
+      nto[cs.n] = 0;
       slot[h] = cs.n++;
-      to.emplace_back();
     }
     return slot[h];
   };
-  for (const ExactAmplitude& a : support) {
-    const int i = find(a.x);
-    cs.re[i] = a.re;
-    cs.im[i] = a.im;
+  for (int a = 0; a < nsupport; ++a) {
+    const int i = find(support[a].x);
+    cs.re[i] = support[a].re;
+    cs.im[i] = support[a].im;
   }
   std::vector<unsigned long long> near(ncells);
   for (int b = 0; b < ncells; ++b)
@@ -434,9 +443,9 @@ int evolve_closed_set(c128* psi, const std::vector<ExactAmplitude>& support, int
       if (alive < lo || alive >= hi) continue;
       const int j = find(cs.x[i] ^ (1ull << b));
       if (j < 0) return 0;
-      to[i].push_back(j);
+      to[i][nto[i]++] = (unsigned char)j;
     }
-    R = std::max(R, (int)to[i].size());
+    R = std::max(R, nto[i]);
   }
   if (R == 0) return 1;   // H psi = 0
   const ChebSeries f(tau, R, tol);
@@ -447,9 +456,9 @@ int evolve_closed_set(c128* psi, const std::vector<ExactAmplitude>& support, int
   auto step = [&](const Vec& p, double scale, const Vec* minus, Vec& out) {
     for (int i = 0; i < cs.n; ++i) {
       c128 h{0, 0};
-      for (int j : to[i]) {
-        h.re += p[j].re;
-        h.im += p[j].im;
+      for (int t = 0; t < nto[i]; ++t) {
+        h.re += p[to[i][t]].re;
+        h.im += p[to[i][t]].im;
       }
       out[i] = minus ? c128{scale * h.re - (*minus)[i].re, scale * h.im - (*minus)[i].im}
                      : c128{scale * h.re, scale * h.im};
@@ -483,23 +492,23 @@ int evolve_closed_set(c128* psi, const std::vector<ExactAmplitude>& support, int
 }  // namespace
 
 // The first step looks psi over (finite, and how many amplitudes are not zero) and
-// tells the host through a word of its own memory while the next steps are on their
+// tells the host through memory of its own while the next steps are on their
 // way, so a general state pays no wait for it.  What it learns by the eighth step: a
 // closed set of few states is evolved on the host (dead or blinking cells, dt 5, 12
-// cells: 660 -> 70 us, 23 cells 28 -> 1.0 ms; with the Krylov evolution before the
+// cells: 640 -> 46 us, 23 cells 28 -> 1.0 ms; with the Krylov evolution before the
 // series 0.2 and 3.9 ms).
 int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, double tau, double tol, c128* bufa,
-                      c128* bufb, c128* acc, ExactProbe* probe, int* word, hipStream_t s) {
+                      c128* bufb, c128* acc, ExactProbe* probe, ExactReport* report, hipStream_t s) {
   const ChebSeries f(tau, ncells, tol);
   const int K = f.K;
-  __atomic_store_n(word, 0, __ATOMIC_RELAXED);
+  __atomic_store_n(&report->word, 0, __ATOMIC_RELAXED);
   QCA_HIP(hipMemsetAsync(probe, 0, offsetof(ExactProbe, e), s));
   auto look = [&](bool wait) {
     for (;;) {
-      const int v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+      const int v = __atomic_load_n(&report->word, __ATOMIC_ACQUIRE);
       if (v != 0 || !wait) return v;
       const hipError_t e = hipStreamQuery(s);   // ends with the stream's work, if not before
-      if (e == hipSuccess) return __atomic_load_n(word, __ATOMIC_ACQUIRE);
+      if (e == hipSuccess) return __atomic_load_n(&report->word, __ATOMIC_ACQUIRE);
       if (e != hipErrorNotReady) QCA_HIP(e);
       (void)hipGetLastError();   // "not ready" is no error of the launches below
     }
@@ -511,17 +520,11 @@ int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, doubl
       if (seen == 0 && launched > 0 && launched <= 8) {
         seen = look(launched == 8);
         if (seen == EXACT_BAD) break;
-        if (seen > 0 && seen - 1 <= EXACT_SUPPORT) {   // psi is written by a substep's last step at the earliest
-          std::vector<ExactAmplitude> support(seen - 1);
-          if (!support.empty())
-            QCA_HIP(hipMemcpyAsync(support.data(), probe->e, sizeof(ExactAmplitude) * support.size(),
-                                   hipMemcpyDeviceToHost, s));
-          QCA_HIP(hipStreamSynchronize(s));
-          if (const int m = evolve_closed_set(psi, support, ncells, distance, lo, hi, tau, tol, s)) {
+        if (seen > 0 && seen - 1 <= EXACT_SUPPORT)   // psi is written by a substep's last step at the earliest
+          if (const int m = evolve_closed_set(psi, report->e, seen - 1, ncells, distance, lo, hi, tau, tol, s)) {
             QCA_HIP(hipStreamSynchronize(s));
             return m;
           }
-        }
       }
       ExactStep<double> st;
       const c128* phi = k == 0 ? psi : (k & 1 ? bufb : bufa);
@@ -543,12 +546,13 @@ int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, doubl
         st.e2 = f.coef(k + 1);
       }
       launch_step<double>(phi, ncells, distance, lo, hi, st, s);
-      if (st.first) hipLaunchKernelGGL(tell_probe, dim3(1), dim3(1), 0, s, (const ExactProbe*)probe, word);
+      if (st.first) 
+        hipLaunchKernelGGL(tell_probe, dim3(1), dim3(EXACT_SUPPORT), 0, s, (const ExactProbe*)probe, report);
     }
     if (seen == EXACT_BAD) break;
   }
   QCA_HIP(hipStreamSynchronize(s));
-  if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == EXACT_BAD)
+  if (__atomic_load_n(&report->word, __ATOMIC_ACQUIRE) == EXACT_BAD)
     throw Error(QCA_ERR_NOT_CONVERGED_CODE, "exponential of a state vector with non-finite amplitudes");
   return f.applications();
 }

@@ -167,7 +167,7 @@ void launch_exact_apply(const cplx<T>* psi, cplx<T>* out, int ncells, int distan
 // (cut at tol itself, the tail was most of the error: 12 to 15 cells, 2.0e-15
 // relative to |psi| on average, against 2.4e-16; one or two terms more);
 // returns the number of H applications.  bufa, bufb, acc: 2^ncells elements
-// each; word: a word of pinned host memory.  psi not finite: an error, psi is left as
+// each; report: pinned host memory.  psi not finite: an error, psi is left as
 // it was.  Returns with the stream drained.
 constexpr double CHEB_MAX_Z = 512, CHEB_TAIL = 0.03;
 // Basis states up to which the support of psi is told to the host, and up to which a
@@ -182,8 +182,12 @@ struct ExactProbe {      // device; the first two words are cleared for each cal
   int count;             // nonzero amplitudes (some of them, where there are more than EXACT_SUPPORT)
   ExactAmplitude e[EXACT_SUPPORT];
 };
+struct ExactReport {     // pinned host memory, written by the device
+  int word;
+  ExactAmplitude e[EXACT_SUPPORT];   // the amplitudes, where word says that they fit
+};
 int launch_exact_expm(c128* psi, int ncells, int distance, int lo, int hi, double tau, double tol, c128* bufa,
-                      c128* bufb, c128* acc, ExactProbe* probe, int* word, hipStream_t s);
+                      c128* bufb, c128* acc, ExactProbe* probe, ExactReport* report, hipStream_t s);
 
 // ---------------------------------------------------------------- SVD / QR
 struct SvdResult {
