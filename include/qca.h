@@ -235,7 +235,10 @@ int qca_env_update(int precision, int side, const void* A, const void* Eprev, vo
 
 /* x <- exp(-i (pi/2) delta H_eff) x by Krylov (FP64 recurrence), x complex128
  * on the device.  Replaces reference lautils.py:44-81 (calculate_U/timestep)
- * as used by tdvp.py:147-188, 349-365.  Arguments as qca_heff_apply. */
+ * as used by tdvp.py:147-188, 349-365.  Arguments as qca_heff_apply.  At most 63
+ * basis vectors: a step that needs more (|delta| well above those of a time
+ * evolution) ends there with what they give, *iters is 63 and the tolerance is
+ * not met. */
 int qca_krylov_expm(int precision, int kind, void* x, const void* L, const void* R,
                     const double* W_host, int Din, int Dout, int chil, int chir, double delta,
                     double tol, int* iters, void* stream);

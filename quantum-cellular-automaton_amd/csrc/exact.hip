@@ -10,7 +10,7 @@
 // phi_{k+1} = (2/R) H phi_k - phi_{k-1} needs three vectors and no inner
 // products, where the Krylov basis it replaced read every earlier vector
 // several times per step.  One step of 2^23 amplitudes, tau = 0.785: 41 Krylov
-// vectors 101 ms, 45 Chebyshev terms 7.5 ms; 2^12, tau = 0.31: 1.07 -> 0.15 ms.
+// vectors 101 ms, 47 Chebyshev terms 7.8 ms; 2^12, tau = 0.31: 1.07 -> 0.15 ms.
 #include "kernels.hpp"
 #include "wave.hpp"
 
@@ -117,8 +117,9 @@ __device__ __forceinline__ void probe_state(const ExactStep<T>& st, const cplx<T
 
 // The probe to the host: 1 + the nonzero amplitudes (more than EXACT_SUPPORT: just
 // that), or EXACT_BAD; and the amplitudes where they are few, so that the host need not
-// copy them, which drains the stream (a set that is not closed, 2^8: 135 -> 81 us).  A launch of its own: by the last workgroup of the first step,
-// with the fence that takes in each of them, it cost 0.7 ms at 2^23.
+// copy them, which drains the stream (a set that is not closed, 2^8: 135 -> 81 us).  A
+// launch of its own: by the last workgroup of the first step, with the fence that takes
+// in each of them, it cost 0.7 ms at 2^23.
 constexpr int EXACT_BAD = 1 << 30;
 __global__ __launch_bounds__(EXACT_SUPPORT) void tell_probe(const ExactProbe* p, ExactReport* report) {
   const int n = p->count, i = threadIdx.x;
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(EXACT_SUPPORT) void tell_probe(const ExactProbe* p,
 // 2^23 amplitudes against 109 us for reading phi, prev, half of acc and
 // writing next and half of acc at the rate of a large copy; the rest is the
 // tile reads (half of N - TB of them).  prev and acc are loaded with the tile,
-// before the gathers (2^23: 7.9 -> 7.5 ms per evolution).  Giving each XCD a
+// before the gathers (2^23: 7.9 -> 7.5 ms for 45 steps).  Giving each XCD a
 // contiguous range of tiles cost 9%.
 template <typename T, typename I, int D, int TB>
 __global__ __launch_bounds__((1 << TB) / 4) void exact_kernel(const cplx<T>* __restrict__ phi, int ncells,
@@ -242,8 +243,8 @@ void launch_step_d(const cplx<T>* phi, int ncells, int distance, int lo, int hi,
                    hipStream_t s) {
   // Tiles of 1024 states from two workgroups per CU on, of 256 below, where
   // more and shorter workgroups count.  Tiles of 4096 read fewer partners from
-  // memory and measured the same (2^23: 7.78 ms, 1024: 7.87, 256: 7.94 per
-  // evolution; 2^16: 0.253 against 0.197 and 0.200).
+  // memory and measured the same (2^23: 7.78 ms, 1024: 7.87, 256: 7.94 for 45
+  // steps; 2^16: 0.253 against 0.197 and 0.200).
   auto tiles = [&](int tb) { return 1L << std::max(0, ncells - tb); };
 #define QCA_EXACT_L(TB)                                                                          \
   hipLaunchKernelGGL((exact_kernel<T, I, D, TB>), dim3((unsigned)tiles(TB)), dim3((1 << TB) / 4), 0, s, phi, \

@@ -29,7 +29,7 @@
 // 1.4, subtraction and norm 1.5, basis vector 0.5: 12 us, before 22 (sixteen
 // waves, vector products from LDS and global memory, two full Gram-Schmidt
 // passes, a tridiagonal exponential of 3.6 us every time).  The run: 155 -> 104
-// ms.  Above FUSED_KRYLOV_DEFAULT_N elements the whole chip is faster: bond 30,
+// ms, and 95 with the elements of small blocks on their own.  Above FUSED_KRYLOV_DEFAULT_N elements the whole chip is faster: bond 30,
 // 82 ms with this limit and 86 with all blocks here.
 #include "grouped.hpp"
 #include "wave.hpp"

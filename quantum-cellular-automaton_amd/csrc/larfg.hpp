@@ -22,10 +22,7 @@ __device__ __forceinline__ int larfg_exponent(double largest) {
   return largest > 0.0 && largest < __builtin_inf() ? ilogb(largest) : 0;
 }
 
-// alpha and the squared norm of what is below it, in range (or all zero).  Square
-// root and divisions to the last bit: a refined reciprocal square root and a
-// reciprocal in their place gave Q 4% more error and no time (512 x 256: 777
-// against 784 us, splits equal).
+// alpha and the squared norm of what is below it, in range (or all zero).
 __device__ __forceinline__ Larfg larfg(c128 alpha, double xnorm2) {
   Larfg h;
   h.beta = alpha.re;
@@ -35,9 +32,10 @@ __device__ __forceinline__ Larfg larfg(c128 alpha, double xnorm2) {
   const double s = alpha.re * alpha.re + alpha.im * alpha.im + xnorm2;
   // sqrt and 1 / sqrt from one reciprocal square root and Newton steps:
   // y (1 + e/2 + 3 e^2 / 8), e = 1 - s y^2, then one more step on each.  sqrt() and
-  // divisions by beta are a longer serial chain for no smaller error: QR 32x32 67.3
-  // instead of 65.8 us, split 12x16 218.3 instead of 216.6, triangles 264 instead of 246
-  // (R off by 1.01e-16 instead of 1.04e-16, rms over shapes up to 256x512, both)
+  // divisions to the last bit are a longer serial chain: QR 32x32 67.3 us instead of
+  // 65.8, 512x256 786 instead of 777, split 12x16 264 instead of 246 (left sweep), for
+  // Q of 4.4e-16 instead of 4.6e-16 and R of 1.01e-16 instead of 1.04e-16 (25 shapes up
+  // to 512x256; 4.9e-16 and 1.08e-16 with panel GEMMs in place of register panels)
   double y = __builtin_amdgcn_rsq(s);
   const double e = fma(-s * y, y, 1.0);
   y = fma(y, e * fma(0.375, e, 0.5), y);

@@ -18,8 +18,8 @@
 // The block reflectors run on the FP64 matrix cores with the updated columns in
 // accumulator registers: the accumulator layout (row (l / 16) + 4 r in register
 // r) is the B operand layout of four consecutive rows, so V^H A and A -= V W
-// both use them in place.  512 x 256 with 256 columns of Q: 2.07 -> 0.83 ms
-// (a panel launch 40 us where panel, two GEMMs and a reduce took 102; Q 170 us);
+// both use them in place.  512 x 256 with 256 columns of Q: 2.07 -> 0.78 ms
+// (a panel launch 36 us where panel, two GEMMs and a reduce took 102; Q 165 us);
 // 256 x 256 within a split: 1.6 -> 0.55 ms; 16 x 32: 73 -> 39 us.
 #include "grouped.hpp"
 #include "larfg.hpp"
@@ -197,9 +197,9 @@ __device__ __forceinline__ void block_reflect(const QrOperands<QR_TILES>& o, int
     }
     ure += xr;
     uim += xi;
-    // one rounding at the size of q, not 32: Q of 512 x 256 to 5.7e-16 in the 2-norm
+    // one rounding at the size of q, not 32: Q of 512 x 256 to 6.0e-16 in the 2-norm
     // against 1.33e-15 with the products added to q itself and a reciprocal square
-    // root in larfg, in the same time (829 -> 784 us)
+    // root without its last step in larfg, in less time (829 -> 780 us)
     qre[t] -= ure;
     qim[t] -= uim;
   }
